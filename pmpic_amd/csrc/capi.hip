@@ -161,6 +161,27 @@ void spec_from_device_layout(const Geometry &g, const std::vector<double> &dev, 
         ref[((size_t)ii * g.sy + jj) * g.nzn + k] = dev[((size_t)k * g.sy + jj) * g.sx + ii];
 }
 
+// the same between the reference's layout and the spectral tiles (common.h)
+void spec_to_tiles(const Geometry &g, const double *ref, std::vector<double> &dev) {
+  dev.assign((size_t)spec_tiles(g) * g.nzn * 64, 0.0);
+  for (int ii = 0; ii < g.sx; ii++)
+    for (int jj = 0; jj < g.sy; jj++) {
+      const double *r = ref + ((size_t)ii * g.sy + jj) * g.nzn;
+      double *d = dev.data() + spec_at(g.nzn, g.sx / 2, 0, jj / 2, ii / 2) + 2 * (jj & 1) + (ii & 1);
+      for (int k = 0; k < g.nzn; k++) d[(size_t)k * 64] = r[k];
+    }
+}
+
+void spec_from_tiles(const Geometry &g, const std::vector<double> &dev, double *ref) {
+  for (int ii = 0; ii < g.sx; ii++)
+    for (int jj = 0; jj < g.sy; jj++) {
+      double *r = ref + ((size_t)ii * g.sy + jj) * g.nzn;
+      const double *d =
+          dev.data() + spec_at(g.nzn, g.sx / 2, 0, jj / 2, ii / 2) + 2 * (jj & 1) + (ii & 1);
+      for (int k = 0; k < g.nzn; k++) r[k] = d[(size_t)k * 64];
+    }
+}
+
 void col_to_device_layout(const Geometry &g, const double *ref, std::vector<double> &dev) {
   dev.resize((size_t)g.sy * g.sx);
   for (int jj = 0; jj < g.sy; jj++)
@@ -211,13 +232,14 @@ int free_all(Ctx *c) {
   for (int g = 0; g < NGRIDS; g++) hipFree(c->grid[g]);
   for (int g = 0; g < 8; g++) hipFree(c->gtmp[g]);
   for (int g = 0; g < 6; g++) hipFree(c->kres[g]);
-  double *sp[] = {c->sa, c->sb, c->sc, c->sd, c->se, c->sf, c->su, c->sv, c->sw, c->sbs};
+  double *sp[] = {c->spool, c->sd, c->se, c->sf, c->su, c->sv, c->sw, c->sbs};
   for (double *p : sp) hipFree(p);
-  for (int g = 0; g < 8; g++) hipFree(c->sder[g]);
-  hipFree(c->atop); hipFree(c->abot); hipFree(c->btop); hipFree(c->bbot);
+  for (int g = 1; g < 6; g++) hipFree(c->sder[g]);
+  hipFree(c->atop); hipFree(c->abot);
   hipFree(c->ubar); hipFree(c->vbar);
   hipFree(c->kx); hipFree(c->ky); hipFree(c->k2); hipFree(c->filt); hipFree(c->coords);
-  hipFree(c->dz_den); hipFree(c->dz_cp);
+  hipFree(c->dz_den); hipFree(c->dz_cp); hipFree(c->dz_rcp);
+  hipFree(c->lpool); hipFree(c->lap_bad);
   hipFree(c->fbuf);
   hipFree(c->cbuf); hipFree(c->tw_x); hipFree(c->tw_y); hipFree(c->tw_x32); hipFree(c->tw_y32);
   hipFree(c->scan_tmp); hipFree(c->blk); hipFree(c->maxblk); hipFree(c->dsc);
@@ -257,6 +279,7 @@ int create(const pmpic_config *cf, Ctx *c) {
   if (c->ncell > (int64_t)INT32_MAX) return PMPIC_ERR_ARG;
   c->gsz = (int64_t)g.nzn * g.ny * g.nx;
   c->ssz = (int64_t)g.nzn * g.sy * g.sx;
+  c->bsz = (int64_t)spec_tiles(g) * g.nzn * 64;  // >= ssz
   c->csz = (int64_t)g.nzn * ((int64_t)g.ny * (g.nx / 2 + 1) > (int64_t)(g.ny / 2 + 1) * g.nx
                                   ? (int64_t)g.ny * (g.nx / 2 + 1)
                                   : (int64_t)(g.ny / 2 + 1) * g.nx);
@@ -285,14 +308,16 @@ int create(const pmpic_config *cf, Ctx *c) {
   for (int i = 0; i < NGRIDS; i++) PMPIC_TRY(dalloc(&c->grid[i], c->gsz));
   for (int i = 0; i < 8; i++) PMPIC_TRY(dalloc(&c->gtmp[i], c->gsz));
   for (int i = 0; i < 6; i++) PMPIC_TRY(dalloc(&c->kres[i], c->gsz));
-  double **sp[] = {&c->sa, &c->sb, &c->sc, &c->sd, &c->se, &c->sf, &c->su, &c->sv, &c->sw, &c->sbs};
-  for (double **p : sp) PMPIC_TRY(dalloc(p, c->ssz));
-  for (int i = 0; i < 8; i++) PMPIC_TRY(dalloc(&c->sder[i], c->ssz));
+  double **sp[] = {&c->sd, &c->se, &c->sf, &c->su, &c->sv, &c->sw, &c->sbs};
+  for (double **p : sp) PMPIC_TRY(dalloc(p, c->bsz));
+  for (int i = 1; i < 6; i++) PMPIC_TRY(dalloc(&c->sder[i], c->bsz));
   const int64_t plane = (int64_t)g.sy * g.sx;
+  // the arrays the column kernel reads ahead in, one after another between COLUMN_PAD levels
+  PMPIC_TRY(dalloc(&c->spool, 4 * c->bsz + 2 * COLUMN_PAD * 64));
+  double **rp[] = {&c->sa, &c->sb, &c->sc, &c->sder[0]};
+  for (int i = 0; i < 4; i++) *rp[i] = c->spool + COLUMN_PAD * 64 + i * c->bsz;
   PMPIC_TRY(dalloc(&c->atop, plane));
   PMPIC_TRY(dalloc(&c->abot, plane));
-  PMPIC_TRY(dalloc(&c->btop, plane));
-  PMPIC_TRY(dalloc(&c->bbot, plane));
   PMPIC_TRY(dalloc(&c->ubar, g.nzn));
   PMPIC_TRY(dalloc(&c->vbar, g.nzn));
   PMPIC_TRY(dalloc(&c->kx, plane));
@@ -301,10 +326,20 @@ int create(const pmpic_config *cf, Ctx *c) {
   PMPIC_TRY(dalloc(&c->filt, plane));
   PMPIC_TRY(dalloc(&c->dz_den, 2 * (int64_t)g.nzn));
   PMPIC_TRY(dalloc(&c->dz_cp, 2 * (int64_t)g.nzn));
+  PMPIC_TRY(dalloc(&c->dz_rcp, 2 * (int64_t)g.nzn));
+  const int64_t pivots = 2 * c->bsz / 4, lpad = COLUMN_PAD * 16;
+  PMPIC_TRY(dalloc(&c->lpool, (c->precision == 0 ? 3 : 1) * pivots + 2 * lpad));
+  c->lap_rcp = c->lpool + lpad;
+  if (c->precision == 0) {
+    c->lap_den = c->lap_rcp + pivots;
+    c->lap_cp = c->lap_den + pivots;
+  }
+  PMPIC_TRY(dalloc(&c->lap_bad, 1));
   PMPIC_TRY(dalloc(&c->coords, (int64_t)coords.size()));
   PMPIC_CHECK(hipMemcpy(c->coords, coords.data(), sizeof(double) * coords.size(),
                         hipMemcpyHostToDevice));
-  PMPIC_TRY(dalloc(&c->cbuf, 8 * c->csz));
+  // FP32-bulk form: float2 elements
+  PMPIC_TRY(dalloc(&c->cbuf, (c->precision == 1 ? FFT_FIELDS / 2 : FFT_FIELDS) * c->csz));
   c->nblk_max = cdiv(big, 256) + 1;
   PMPIC_TRY(dalloc(&c->blk, 20 * c->nblk_max + 64));
   PMPIC_TRY(dalloc(&c->maxblk, 4 * 1024));
@@ -318,6 +353,7 @@ int create(const pmpic_config *cf, Ctx *c) {
     }
   PMPIC_TRY(fft_setup(c));
   PMPIC_TRY(spectral_setup(c));
+  PMPIC_TRY(columns_setup(c));
   PMPIC_TRY(set_dev_scalars(c));
   // PMPIC_GRAPH=1: the FP32-bulk form launches stages 1-3 of a step as a HIP graph
   const char *genv = getenv("PMPIC_GRAPH");
@@ -495,20 +531,18 @@ int pmpic_set_time(pmpic_ctx *ctx, double time, double dtm) {
 }
 
 // vort2vel: par2grid of p, q, r (and, fused into the same pass, the total buoyancy that
-// vorticity_tendency grids from the same cached weights), the spectral solve, and at stage 1
-// the grid maxima for the timestep limits
+// vorticity_tendency grids from the same cached weights), the spectral solve and the derivative
+// grids vorticity_tendency multiplies; its stage 1 takes the grid maxima for the timestep limits
 int pmpic_vort2vel(pmpic_ctx *ctx) {
   if (!ctx) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
-  const int stage = stage_of(c->it_v2v);
   PMPIC_TRY(timing_begin(c, T_VORT2VEL));
   if (c->precision == 1) {
     PMPIC_TRY(b32_par2grid(c));
-    PMPIC_TRY(vort2vel_spectral(c, stage));  // also writes the FP32 u, v, w
   } else {
     PMPIC_TRY(par2grid_fused(c, c->n));
-    PMPIC_TRY(vort2vel_spectral(c, stage));
   }
+  PMPIC_TRY(vort2vel_spectral(c));
   PMPIC_TRY(timing_end(c, T_VORT2VEL));
   c->it_v2v++;
   return PMPIC_OK;
@@ -519,7 +553,7 @@ int pmpic_vorticity_tendency(pmpic_ctx *ctx) {
   Ctx *c = &ctx->c;
   const int stage = stage_of(c->it_vt);
   PMPIC_TRY(timing_begin(c, T_VORT_TEND));
-  PMPIC_TRY(vorticity_tendency_spectral(c, stage));  // and the FP32 tendencies
+  PMPIC_TRY(vorticity_tendency_grids(c));
   if (stage == 1) {
     PMPIC_TRY(grid_max_reduce(c));
   }
@@ -830,15 +864,15 @@ int pmpic_get_spectral(pmpic_ctx *ctx, int32_t id, double *spec) {
   std::vector<double> h;
   if (c->precision == 1) {
     // the FP32-bulk form's spectral arrays hold FP32 values; widened exactly
-    std::vector<float> h32((size_t)c->ssz);
-    PMPIC_CHECK(hipMemcpyAsync(h32.data(), src, sizeof(float) * (size_t)c->ssz,
+    std::vector<float> h32((size_t)c->bsz);
+    PMPIC_CHECK(hipMemcpyAsync(h32.data(), src, sizeof(float) * (size_t)c->bsz,
                                hipMemcpyDeviceToHost, c->stream));
     PMPIC_CHECK(hipStreamSynchronize(c->stream));
     h.assign(h32.begin(), h32.end());
   } else {
-    PMPIC_TRY(download(c, h, src, c->ssz));
+    PMPIC_TRY(download(c, h, src, c->bsz));
   }
-  spec_from_device_layout(c->g, h, spec);
+  spec_from_tiles(c->g, h, spec);
   return PMPIC_OK;
 }
 
@@ -847,12 +881,12 @@ int pmpic_fft_forward(pmpic_ctx *ctx, const double *grid, double *spec) {
   Ctx *c = &ctx->c;
   std::vector<double> h;
   grid_to_device_layout(c->g, grid, h);
-  PMPIC_TRY(upload(c, c->gtmp[0], h));
-  const double *src[1] = {c->gtmp[0]};
+  PMPIC_TRY(upload(c, c->kres[0], h));
+  const double *src[1] = {c->kres[0]};
   double *dst[1] = {c->sder[0]};
   PMPIC_TRY(fft_forward(c, 1, src, dst));
-  PMPIC_TRY(download(c, h, c->sder[0], c->ssz));
-  spec_from_device_layout(c->g, h, spec);
+  PMPIC_TRY(download(c, h, c->sder[0], c->bsz));
+  spec_from_tiles(c->g, h, spec);
   return PMPIC_OK;
 }
 
@@ -860,12 +894,12 @@ int pmpic_fft_backward(pmpic_ctx *ctx, const double *spec, double *grid) {
   if (!ctx || !grid || !spec) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
   std::vector<double> h;
-  spec_to_device_layout(c->g, spec, h);
+  spec_to_tiles(c->g, spec, h);
   PMPIC_TRY(upload(c, c->sder[0], h));
   const double *src[1] = {c->sder[0]};
-  double *dst[1] = {c->gtmp[0]};
+  double *dst[1] = {c->kres[0]};
   PMPIC_TRY(fft_backward(c, 1, src, dst));
-  PMPIC_TRY(download(c, h, c->gtmp[0], c->gsz));
+  PMPIC_TRY(download(c, h, c->kres[0], c->gsz));
   grid_from_device_layout(c->g, h, grid);
   return PMPIC_OK;
 }

@@ -6,9 +6,13 @@
 //  * physical grids: interior nodes only, [nzn][ny][nx] (x fastest, z slowest); the reference's
 //    x/y halos (decomposition.F90:449-451) become periodic index arithmetic, so the halo fold of
 //    par2grid (MPIC_Haloswap.F90:188-290) and the fill of grid2par (:95-184) are implicit;
-//  * spectral arrays: [nzn][sy][sx] with sy = (ny/2+1)*2, sx = (nx/2+1)*2 holding the
-//    reference's (Re,Im)-interleaved semi-spectral layout (pencilfft.F90:838-899), z slowest so
-//    that one thread per (kx,ky) column walks z with unit-stride, coalesced across threads;
+//  * spectral arrays: the reference's (Re,Im)-interleaved semi-spectral values
+//    (pencilfft.F90:838-899) in tiles of 16 (m, l) blocks (m, l the y and x wavenumbers, blocks
+//    numbered m (nx/2+1) + l): [tile][nzn][16 blocks][a][b], a and b the Re/Im parts of the y and x
+//    transforms.  A block's four values are one vector for the transforms, and a wavefront's 64
+//    columns of one tile are contiguous through all z levels for the column kernel (columns.hip);
+//    the standalone spectral operators work on planes [nzn][sy][sx] instead, sy = (ny/2+1)*2,
+//    sx = (nx/2+1)*2, as the wavenumber and filter planes [sy][sx] are laid out;
 //  * cells: c = (k*ny + j)*nx + i over ncz*ny*nx cells.
 #pragma once
 #include <hip/hip_ext.h>
@@ -111,6 +115,15 @@ struct DevScalars {
   int32_t novf;      // parcels past their cell's slot capacity in the last FP32 binning
 };
 
+// tiles of the spectral layout, and the place of block (m, l)'s four values at level k
+__host__ __device__ inline int spec_tiles(const Geometry &g) {
+  return ((g.sx / 2) * (g.sy / 2) + 15) / 16;
+}
+__host__ __device__ inline int64_t spec_at(int nzn, int nl, int k, int m, int l) {
+  const int blk = m * nl + l;
+  return ((int64_t)(blk >> 4) * nzn + k) * 64 + 4 * (blk & 15);
+}
+
 enum TimerId { T_ACCUM = 0, T_RK = 1, T_VORT2VEL, T_VORT_TEND, T_RK4, T_SPLIT, T_MIX, NTIMERS };
 
 struct Ctx {
@@ -144,21 +157,28 @@ struct Ctx {
   int32_t *npercell;                  // ncell
   uint8_t *cellflag;                  // ncell
   // grids (interior [nzn][ny][nx])
-  int64_t gsz, ssz, csz;
+  int64_t gsz, ssz, csz;              // grid; spectral (planes); complex transform intermediate
+  int64_t bsz;                        // spectral (tiles)
   double *grid[NGRIDS];
-  double *gtmp[8];                    // vorticity tendency derivative grids
+  double *gtmp[8];                    // vorticity tendency derivative grids (made by vort2vel)
   double *kres[6];                    // mixing residual grids
-  // spectral [nzn][sy][sx]
+  // spectral, in tiles (the standalone operators use the sder arrays as planes)
   double *sa, *sb, *sc, *sd, *se, *sf, *su, *sv, *sw, *sbs;
-  double *sder[8];
-  double *atop, *abot, *btop, *bbot;  // [sy][sx]
+  double *sder[6];
+  double *spool;                      // holds sa, sb, sc and sder[0] (COLUMN_PAD)
+  double *abot, *atop;                // [sy][sx], standalone diffz's boundary planes
   double *ubar, *vbar;                // [nzn]
   double *kx, *ky, *k2, *filt;        // [sy][sx]
   // Thomas elimination: diffz's denominators and c' [bt][k] (the same for every column)
-  double *dz_den, *dz_cp;
+  double *dz_den, *dz_cp, *dz_rcp;
+  // and the inverse Laplacian's by boundary condition, step and (m, l) block of columns:
+  // reciprocal pivots, and for the FP64 form the pivots and c' (lpool holds all three); lap_bad:
+  // one of the pivots is zero
+  double *lap_rcp, *lap_den, *lap_cp, *lpool;
+  int *lap_bad;
   double *coords;                     // x_coords (nx+4), y_coords (ny+4), z_coords (nzn)
   double *fbuf;                       // host-array staging, allocated at first use (ensure_fbuf)
-  double2 *cbuf;                      // complex FFT intermediates, 8 fields
+  double2 *cbuf;                      // complex FFT intermediates, FFT_FIELDS fields
   double2 *tw_x, *tw_y;               // twiddles W_n^e, e in [0,n)
   float2 *tw_x32, *tw_y32;            // the same rounded to FP32
   // scan scratch
@@ -312,6 +332,7 @@ int mixing_grids(Ctx *c, int64_t n);
 int dump_grids_f64(Ctx *c, int64_t n);  // writebinary's b, hg, p, q, r grids
 int hgliq_grid(Ctx *c);                 // hgliq and b += 12.5 hgliq (writebinary.F90:224-233)
 // fft.hip
+constexpr int FFT_FIELDS = 14;  // most fields of one transform call
 int fft_setup(Ctx *c);
 int fft_forward(Ctx *c, int nf, const double *const *src, double *const *dst);
 // dst32 (optional, entries may be NULL): an FP32 copy of each real output.
@@ -328,10 +349,17 @@ int fft_forward_t(Ctx *c, int nf, const S *const *src, S *const *dst);
 template <typename S>
 int fft_backward_t(Ctx *c, int nf, const S *const *src, double *const *dst, float *const *dst32,
                    const int *deriv);
+// levels of a tile readable before and after the arrays and tables that the column kernel reads
+// ahead of its recurrences
+constexpr int COLUMN_PAD = 16;
+// columns.hip: everything of vort2vel between its transforms, in place of sa, sb, sc
+int columns_setup(Ctx *c);
+template <typename S>
+int vort2vel_columns(Ctx *c);
 // spectral.hip
 int spectral_setup(Ctx *c);
-int vort2vel_spectral(Ctx *c, int stage);
-int vorticity_tendency_spectral(Ctx *c, int stage);
+int vort2vel_spectral(Ctx *c);
+int vorticity_tendency_grids(Ctx *c);
 int op_diffx(Ctx *c, const double *in, double *out);
 int op_diffy(Ctx *c, const double *in, double *out);
 int op_filter(Ctx *c, const double *in, double *out);

@@ -53,7 +53,7 @@ __host__ __device__ constexpr Plan make_plan(int n) {
 constexpr int FIXED_N[] = {16, 32, 48, 64, 96, 128, 256, 512};
 
 constexpr int FFT_TPB = 256;
-constexpr int MAXF = 8;
+constexpr int MAXF = FFT_FIELDS;
 
 // The transforms run in the precision S of the spectral arrays: FP64 (double2 complex
 // elements), or FP32 (float2) in the FP32-bulk form, whose LDS buffers then hold twice as many
@@ -328,13 +328,18 @@ __global__ void __launch_bounds__(FFT_TPB) k_rows_r2c(Plan p, const cx_t<S> *__r
   }
 }
 
+// a block's four values (one 16-byte FP32 vector, or two FP64 pairs)
+template <typename S>
+struct alignas(4 * sizeof(S) > 16 ? 16 : 4 * sizeof(S)) Quad {
+  S v[4];  // a = 0: (Re, Im) of the x transform, a = 1: (Re, Im)
+};
+
 // forward pass 2: complex FFT along y of nb adjacent columns l of one z level, then the
 // (Re,Im)-pair split into the semi-spectral layout
 template <typename S, int NT>
 __global__ void __launch_bounds__(FFT_TPB) k_cols_fwd(Plan p, const cx_t<S> *__restrict__ tw,
                                                       FieldPtrs fp, const cx_t<S> *__restrict__ c1,
-                                                      int64_t c1_field, int nl, int nb, int sx,
-                                                      int sy) {
+                                                      int64_t c1_field, int nl, int nb, int nzn) {
   using C = cx_t<S>;
   constexpr int EPT = lds_cols<S>(NT, false) / FFT_TPB;
   __shared__ C A[lds_cols<S>(NT, false)], B[lds_cols<S>(NT, false)], T[512];
@@ -371,7 +376,6 @@ __global__ void __launch_bounds__(FFT_TPB) k_cols_fwd(Plan p, const cx_t<S> *__r
   __syncthreads();
   C *R = lds_fft<false, NT>(A, B, T, p, nbb);
   const int nm = ny / 2 + 1;
-  S *out = dst + (int64_t)k * sy * sx;
   for (int e = threadIdx.x; e < nbd * nm; e += FFT_TPB) {
     const int m = e / nbd, t = e - m * nbd;
     if (t >= nbb) continue;
@@ -380,63 +384,52 @@ __global__ void __launch_bounds__(FFT_TPB) k_cols_fwd(Plan p, const cx_t<S> *__r
     C h = R[t * ny + ((ny - m) % ny)];
     C s = mkc<C, S>(g.x + h.x, g.y + h.y);
     C d = mkc<C, S>(g.x - h.x, g.y - h.y);
-    out[(int64_t)(2 * m) * sx + 2 * l] = s.x / 2;
-    out[(int64_t)(2 * m) * sx + 2 * l + 1] = s.y / 2;
-    out[(int64_t)(2 * m + 1) * sx + 2 * l] = d.y / 2;
-    out[(int64_t)(2 * m + 1) * sx + 2 * l + 1] = -d.x / 2;
+    *reinterpret_cast<Quad<S> *>(dst + spec_at(nzn, nl, k, m, l)) =
+        Quad<S>{s.x / 2, s.y / 2, d.y / 2, -d.x / 2};
   }
 }
 
 // inverse pass 1: per (k, m) build H = A_m + i B_m over l in [0, nx) from the two real
 // x-spectra (imaginary parts of the DC and Nyquist bins dropped as c2r drops them), inverse
-// FFT along x, scale 1/nx -> C2[k][m][x]
+// FFT along x, scale 1/nx -> C2[k][m][x].  A thread loads a block (m, l) once and forms H at l and
+// at nx - l.
 template <typename S, int NT>
 __global__ void __launch_bounds__(FFT_TPB) k_rows_inv(Plan p, const cx_t<S> *__restrict__ tw,
                                                       FieldPtrs fp, cx_t<S> *__restrict__ c2,
                                                       int64_t c2_field, int nrows, int nm,
-                                                      float rnm, int nb, int sx) {
+                                                      float rnm, int nb, int nzn) {
   using C = cx_t<S>;
-  constexpr int EPT = ept_rows<S>();
+  // blocks per thread: nl = nx / 2 + 1 of nb = lds_rows / nx rows
+  constexpr int EPT = NT > 0 ? (lds_rows<S>() / NT * (NT / 2 + 1) + FFT_TPB - 1) / FFT_TPB
+                             : ept_rows<S>();
   __shared__ C A[lds_rows<S>()], B[lds_rows<S>()], T[512];
   const int f = blockIdx.y;
   const S *src = static_cast<const S *>(fp.in[f]);
   const int op = fp.op[f];
   C *dst = c2 + (int64_t)f * c2_field;
-  const int nx = NT ? NT : p.n;
+  const int nx = NT ? NT : p.n, nl = nx / 2 + 1;
   const int r0 = blockIdx.x * nb;
   const int nbb = min(nb, nrows - r0);
-  const int half = nx / 2;
-  const bool even = (nx % 2) == 0;
-  C w[TPT], va[EPT], vb[EPT];
+  C w[TPT];
+  Quad<S> q[EPT];
   load_twiddles(w, tw, nx);
 #pragma unroll
   for (int i = 0; i < EPT; i++) {
     const int e = threadIdx.x + i * FFT_TPB;
-    if (e < nbb * nx) {
-      const int t = e / nx, l = e - t * nx;
-      const int row = r0 + t;  // row = k * nm + m
+    if (e < nbb * nl) {
+      const int t = e / nl, l = e - t * nl;
       int m;
-      const int k = div_small(row, nm, rnm, m);
-      const S *sa = src + ((int64_t)k * (2 * nm) + 2 * m) * sx;
-      const int ll = (l <= half) ? l : nx - l;
-      va[i] = *reinterpret_cast<const C *>(sa + 2 * ll);       // (ar, ai)
-      vb[i] = *reinterpret_cast<const C *>(sa + sx + 2 * ll);  // (br, bi)
+      const int k = div_small(r0 + t, nm, rnm, m);  // row = k * nm + m
+      q[i] = *reinterpret_cast<const Quad<S> *>(src + spec_at(nzn, nl, k, m, l));
       if (op != SPEC_PLAIN) {
-        // the derivative of spectral rows 2m (a) and 2m+1 (b), element for element as the
-        // standalone diffx / diffy compute it (fft_ops.F90:266-269, :366-369); the
-        // wavenumber planes are indexed by (row, x) like the spectral plane
-        const double *kp = (op == SPEC_DX ? fp.kx : fp.ky) + (int64_t)(2 * m) * sx + 2 * ll;
-        const double2 kad = *reinterpret_cast<const double2 *>(kp);
-        const double2 kbd = *reinterpret_cast<const double2 *>(kp + sx);
-        const S kax = (S)kad.x, kay = (S)kad.y, kbx = (S)kbd.x, kby = (S)kbd.y;
-        const C a0 = va[i], b0 = vb[i];
-        if (op == SPEC_DX) {  // pair swap along x within each row
-          va[i] = mkc<C, S>(((S)-1. * a0.y) * kax, a0.x * kay);
-          vb[i] = mkc<C, S>(((S)-1. * b0.y) * kbx, b0.x * kby);
-        } else {  // pair swap along y between the two rows
-          va[i] = mkc<C, S>(((S)-1. * b0.x) * kax, ((S)-1. * b0.y) * kay);
-          vb[i] = mkc<C, S>(a0.x * kbx, a0.y * kby);
-        }
+        // the derivative, element for element as the standalone diffx / diffy compute it
+        // (fft_ops.F90:266-269, :366-369); kx depends on l and ky on m only
+        const S kw = (S)(op == SPEC_DX ? fp.kx[2 * l] : fp.ky[(int64_t)(2 * m) * (2 * nl)]);
+        const Quad<S> u = q[i];
+        if (op == SPEC_DX)  // pair swap along x
+          q[i] = Quad<S>{((S)-1. * u.v[1]) * kw, u.v[0] * kw, ((S)-1. * u.v[3]) * kw, u.v[2] * kw};
+        else  // pair swap along y
+          q[i] = Quad<S>{((S)-1. * u.v[2]) * kw, ((S)-1. * u.v[3]) * kw, u.v[0] * kw, u.v[1] * kw};
       }
     }
   }
@@ -444,16 +437,15 @@ __global__ void __launch_bounds__(FFT_TPB) k_rows_inv(Plan p, const cx_t<S> *__r
 #pragma unroll
   for (int i = 0; i < EPT; i++) {
     const int e = threadIdx.x + i * FFT_TPB;
-    if (e < nbb * nx) {
-      const int t = e / nx, l = e - t * nx;
-      const int ll = (l <= half) ? l : nx - l;
-      const S ar = va[i].x, br = vb[i].x;
-      S ai = va[i].y, bi = vb[i].y;
-      if (ll == 0 || (even && ll == half)) { ai = 0; bi = 0; }
-      C h;
-      if (l <= half) h = mkc<C, S>(ar - bi, ai + br);
-      else h = mkc<C, S>(ar + bi, -ai + br);
-      A[t * nx + l] = h;
+    if (e < nbb * nl) {
+      const int t = e / nl, l = e - t * nl;
+      const S ar = q[i].v[0], ai = q[i].v[1], br = q[i].v[2], bi = q[i].v[3];
+      if (l == 0 || 2 * l == nx) {
+        A[t * nx + l] = mkc<C, S>(ar, br);
+      } else {
+        A[t * nx + l] = mkc<C, S>(ar - bi, ai + br);
+        A[t * nx + nx - l] = mkc<C, S>(ar + bi, -ai + br);
+      }
     }
   }
   __syncthreads();
@@ -615,7 +607,7 @@ int fft_forward_t(Ctx *c, int nf, const S *const *src, S *const *dst) {
   with_length(g.ny, [&](auto N) {
     hipLaunchKernelGGL((k_cols_fwd<S, decltype(N)::value>), dim3(cdiv(nl, nby), g.nzn, nf),
                        dim3(FFT_TPB), 0, c->stream, py, twiddles_y<S>(c), fp, cb, c1f, nl, nby,
-                       g.sx, g.sy);
+                       g.nzn);
     return 0;
   });
   PMPIC_CHECK(hipGetLastError());
@@ -648,7 +640,7 @@ int fft_backward_t(Ctx *c, int nf, const S *const *src, double *const *dst, floa
   with_length(g.nx, [&](auto N) {
     hipLaunchKernelGGL((k_rows_inv<S, decltype(N)::value>), dim3(cdiv(nrows, nbx), nf),
                        dim3(FFT_TPB), 0, c->stream, px, twiddles_x<S>(c), fp, cb, c2f, nrows, nm,
-                       rnm, nbx, g.sx);
+                       rnm, nbx, g.nzn);
     return 0;
   });
   const int nby = col_batch<S>(g.ny, true);  // transforms per workgroup, two x columns each

@@ -5,10 +5,10 @@
 // components/vort2vel/src/vort2vel.F90:98-400 and
 // components/vorticity_tendency/src/vorticity_tendency.F90:107-334.
 //
-// Every operator is memory bound: element-wise kernels over the [nzn][sy][sx] spectral arrays
-// (fused where the reference's sequence allows it without changing any operation) and column
-// kernels with one thread per (kx,ky) column walking z; with z slowest in memory the column
-// walk is coalesced across the threads of a wavefront.  The tridiagonal solves keep the
+// The standalone operators (pmpic_diffx ... pmpic_laplinv), the composition of vort2vel and
+// vorticity_tendency from the transforms (fft.hip) and the fused column kernel (columns.hip), and
+// the grid kernels of vorticity_tendency.  The standalone column solvers walk z with one thread or
+// lane group per (kx,ky) column (z slowest in memory, so the walk is coalesced) and keep the
 // reference's Thomas recurrence operation for operation (FP32-rounded literal coefficients,
 // skipped k^2 = 0 columns).
 #include "common.h"
@@ -23,32 +23,15 @@ namespace {
 
 constexpr int TPB = 256;
 
-struct SpecDims {
-  int sx, sy, nzn;
-  int64_t ssz;
-};
-
-__device__ __forceinline__ SpecDims sdims(const Geometry &g) {
-  SpecDims d;
-  d.sx = g.sx; d.sy = g.sy; d.nzn = g.nzn;
-  d.ssz = (int64_t)g.nzn * g.sy * g.sx;
-  return d;
-}
-
-// The spectral arrays are of type S: FP64, or FP32 in the FP32-bulk form, whose spectral
-// kernels then read and write FP32 values and compute in FP64 between.
-//
 // diffx of element q (fft_ops.F90:266-269, :295): pair swap along x, times kx
-template <typename S>
-__device__ __forceinline__ double dx_at(const S *in, const double *kx, int64_t q, int ii,
+__device__ __forceinline__ double dx_at(const double *in, const double *kx, int64_t q, int ii,
                                         int64_t col) {
-  return ((ii & 1) == 0 ? (-1. * (double)in[q + 1]) : (double)in[q - 1]) * kx[col];
+  return ((ii & 1) == 0 ? (-1. * in[q + 1]) : in[q - 1]) * kx[col];
 }
 // diffy of element q (fft_ops.F90:366-369, :394)
-template <typename S>
-__device__ __forceinline__ double dy_at(const S *in, const double *ky, int64_t q, int jj,
+__device__ __forceinline__ double dy_at(const double *in, const double *ky, int64_t q, int jj,
                                         int sx, int64_t col) {
-  return ((jj & 1) == 0 ? (-1. * (double)in[q + sx]) : (double)in[q - sx]) * ky[col];
+  return ((jj & 1) == 0 ? (-1. * in[q + sx]) : in[q - sx]) * ky[col];
 }
 
 __global__ void k_diffx(Geometry g, const double *__restrict__ in, double *__restrict__ out,
@@ -71,131 +54,19 @@ __global__ void k_diffy(Geometry g, const double *__restrict__ in, double *__res
   out[q] = dy_at(in, ky, q, jj, g.sx, col);
 }
 
-// The element-wise spectral kernels take one thread per element of a z level (blockIdx.y): the
-// column col = (jj, ii) of the level's sy x sx plane and the element q = k plane + col, with no
-// 64-bit division.  SPEC_ELEMENT declares plane, k, col, q, ii, jj and leaves threads past the
-// plane.
-#define SPEC_ELEMENT(g)                                                                      \
-  const int64_t plane = (int64_t)(g).sy * (g).sx;                                            \
-  const int col32 = (int)(blockIdx.x * blockDim.x + threadIdx.x);                            \
-  if (col32 >= plane) return;                                                                \
-  const int k = (int)blockIdx.y;                                                             \
-  const int64_t col = col32;                                                                 \
-  const int64_t q = (int64_t)k * plane + col;                                                \
-  const int ii = col32 % (g).sx, jj = col32 / (g).sx;                                        \
-  (void)k; (void)ii; (void)jj
-inline dim3 spec_grid(const Geometry &g) {
-  return dim3((unsigned)cdiv((int64_t)g.sy * g.sx, TPB), (unsigned)g.nzn);
-}
-
-template <typename S>
-__global__ void k_filter(Geometry g, const S *__restrict__ in, S *__restrict__ out,
+// spectral_filter (fft_ops.F90:176-197)
+__global__ void k_filter(Geometry g, const double *__restrict__ in, double *__restrict__ out,
                          const double *__restrict__ filt) {
-  SPEC_ELEMENT(g);
-  out[q] = (S)((double)in[q] * filt[col]);
-}
-
-// vort2vel.F90:158-174: f = (diffx(a) + diffy(b)) + dc/dz (explicit 2nd order, one-sided at
-// the ends), then the constant column zeroed
-template <typename S>
-__global__ void k_divergence(Geometry g, const S *__restrict__ a, const S *__restrict__ b,
-                             const S *__restrict__ cs, S *__restrict__ f,
-                             const double *__restrict__ kx, const double *__restrict__ ky,
-                             double hdzi) {
-  auto c = [&](int64_t i) { return (double)cs[i]; };
-  SPEC_ELEMENT(g);
-  const int nz = g.nzn;
-  const double d = dx_at(a, kx, q, ii, col);
-  const double e = dy_at(b, ky, q, jj, g.sx, col);
-  double fz;
-  if (k == 0)
-    fz = hdzi * (4. * c(q + plane) - c(q + 2 * plane) - 3. * c(q));
-  else if (k == nz - 1)
-    fz = hdzi * (c(q - 2 * plane) + 3. * c(q) - 4. * c(q - plane));
-  else
-    fz = (c(q + plane) - c(q - plane)) * hdzi;
-  double r = d + e + fz;
-  if (col == 0) r = 0.0;
-  f[q] = (S)r;
-}
-
-// vort2vel.F90:184-194: a -= diffx(f); b -= diffy(f)
-template <typename S>
-__global__ void k_correct_ab(Geometry g, S *__restrict__ a, S *__restrict__ b,
-                             const S *__restrict__ f, const double *__restrict__ kx,
-                             const double *__restrict__ ky) {
-  SPEC_ELEMENT(g);
-  a[q] = (S)((double)a[q] - dx_at(f, kx, q, ii, col));
-  b[q] = (S)((double)b[q] - dy_at(f, ky, q, jj, g.sx, col));
-}
-
-// vort2vel.F90:197-218: c -= dz(f); c(level 1) = 0; d,e,f = filtered a,b,c; cache the top and
-// bottom levels of the unfiltered a, b
-template <typename S>
-__global__ void k_correct_c_filter(Geometry g, const S *__restrict__ a,
-                                   const S *__restrict__ b, S *__restrict__ c,
-                                   const S *__restrict__ dzf, S *__restrict__ d,
-                                   S *__restrict__ e, S *__restrict__ f,
-                                   const double *__restrict__ filt, double *__restrict__ atop,
-                                   double *__restrict__ abot, double *__restrict__ btop,
-                                   double *__restrict__ bbot) {
-  SPEC_ELEMENT(g);
-  double cv = (double)c[q] - (double)dzf[q];
-  if (k == 0) cv = 0.;
-  c[q] = (S)cv;
-  const double fl = filt[col];
-  const double av = a[q], bv = b[q];
-  d[q] = (S)(av * fl);
-  e[q] = (S)(bv * fl);
-  f[q] = (S)((double)(S)cv * fl);
-  if (k == g.nzn - 1) { atop[col] = av; btop[col] = bv; }
-  if (k == 0) { abot[col] = av; bbot[col] = bv; }
-}
-
-// mean flow, vort2vel.F90:230-241 (sequential over z; 1./nz is a default-real quotient)
-template <typename S>
-__global__ void k_mean_flow(Geometry g, const S *__restrict__ d, const S *__restrict__ e,
-                            double *__restrict__ ubar, double *__restrict__ vbar) {
-  // the (1,1) columns are staged in LDS by the whole block; one thread then runs the
-  // reference's sequential recurrences and sums on them, and the block writes the result
-  extern __shared__ double sm[];
-  const int64_t plane = (int64_t)g.sy * g.sx;
-  const int nz = g.nzn;
-  double *se = sm, *sd = sm + nz, *ub = sm + 2 * nz, *vb = sm + 3 * nz, *avg = sm + 4 * nz;
-  for (int k = threadIdx.x; k < nz; k += blockDim.x) {
-    se[k] = e[(int64_t)k * plane];
-    sd[k] = d[(int64_t)k * plane];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const double dz = g.dz;
-    ub[0] = 0;
-    vb[0] = 0;
-    for (int k = 1; k <= nz - 1; k++) {
-      ub[k] = ub[k - 1] + dz / 2. * (se[k - 1] + se[k]);
-      vb[k] = vb[k - 1] - dz / 2. * (sd[k - 1] + sd[k]);
-    }
-    const double rnz = (double)(1.f / (float)nz);
-    double su = 0, sv = 0;
-    for (int k = 1; k <= nz - 1; k++) {
-      su += ub[k - 1] + 0.5 * ub[nz - 1];
-      sv += vb[k - 1] + 0.5 * vb[nz - 1];
-    }
-    avg[0] = rnz * su;
-    avg[1] = rnz * sv;
-  }
-  __syncthreads();
-  for (int k = threadIdx.x; k < nz; k += blockDim.x) {
-    ubar[k] = ub[k] - avg[0];
-    vbar[k] = vb[k] - avg[1];
-  }
+  const int64_t ssz = (int64_t)g.nzn * g.sy * g.sx;
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= ssz) return;
+  out[q] = in[q] * filt[q % ((int64_t)g.sy * g.sx)];
 }
 
 // Column stage-in with many loads in flight: a chunk of LVL levels is read into registers
 // (independent loads, issued back to back) before any is written to the LDS slice.
 constexpr int LVL = 16;
-template <typename S>
-__device__ __forceinline__ void column_to_lds(const S *__restrict__ f, int64_t plane, int nz,
+__device__ __forceinline__ void column_to_lds(const double *__restrict__ f, int64_t plane, int nz,
                                               double *F, int nc) {
   for (int k0 = 0; k0 < nz; k0 += LVL) {
     double t[LVL];
@@ -322,32 +193,27 @@ __device__ __forceinline__ int diffz_column(const Geometry &g, CI F, CO O, CC CP
   return PMPIC_OK;
 }
 
-// up to 4 fields per launch (blockIdx.y); the boundary planes are FP64 in both forms
-template <typename S>
-struct ColFields {
-  const S *in[4];
-  S *out[4];
-  const double *bot[4];
-  const double *top[4];
-  int df0[4];
+struct ColField {
+  const double *in;
+  double *out;
+  const double *bot, *top;
+  int df0;
 };
 
-template <typename S>
-__global__ void k_laplinv(Geometry g, ColFields<S> cf, double *__restrict__ cp,
+__global__ void k_laplinv(Geometry g, ColField cf, double *__restrict__ cp,
                           const double *__restrict__ k2a, DevScalars *sc) {
   const int64_t plane = (int64_t)g.sy * g.sx;
   const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= plane) return;
   const double k2 = k2a[col];
   if (k2 == 0) return;
-  Col<S> F{cf.out[blockIdx.y] + col, plane};
-  Col<double> CP{cp + (int64_t)blockIdx.y * g.nzn * plane + col, plane};
-  const int st = laplinv_column(g, F, CP, k2, cf.df0[blockIdx.y]);
+  Col<double> F{cf.out + col, plane};
+  Col<double> CP{cp + col, plane};
+  const int st = laplinv_column(g, F, CP, k2, cf.df0);
   if (st != PMPIC_OK) raise_status(sc, st);
 }
 
-template <typename S>
-__global__ void __launch_bounds__(64) k_laplinv_lds(Geometry g, ColFields<S> cf,
+__global__ void __launch_bounds__(64) k_laplinv_lds(Geometry g, ColField cf,
                                                     const double *__restrict__ k2a,
                                                     DevScalars *sc) {
   extern __shared__ double sh[];
@@ -357,54 +223,50 @@ __global__ void __launch_bounds__(64) k_laplinv_lds(Geometry g, ColFields<S> cf,
   if (col >= plane) return;  // no barriers below: each thread touches only its own slice
   const double k2 = k2a[col];
   if (k2 == 0) return;
-  S *f = cf.out[blockIdx.y] + col;
+  double *f = cf.out + col;
   Col<double> F{sh + t, nc}, CP{sh + (int64_t)nz * nc + t, nc};
   column_to_lds(f, plane, nz, sh + t, nc);
-  const int st = laplinv_column(g, F, CP, k2, cf.df0[blockIdx.y]);
+  const int st = laplinv_column(g, F, CP, k2, cf.df0);
   if (st != PMPIC_OK) {
     raise_status(sc, st);
     return;
   }
 #pragma unroll 8
-  for (int k = 0; k < nz; k++) f[(int64_t)k * plane] = (S)F[k];
+  for (int k = 0; k < nz; k++) f[(int64_t)k * plane] = F[k];
 }
 
-template <typename S>
-__global__ void k_diffz(Geometry g, ColFields<S> cf, double *__restrict__ cp, DevScalars *sc) {
+__global__ void k_diffz(Geometry g, ColField cf, double *__restrict__ cp, DevScalars *sc) {
   const int64_t plane = (int64_t)g.sy * g.sx;
   const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= plane) return;
-  const int fi = blockIdx.y;
-  const bool bt = cf.bot[fi] != nullptr && cf.top[fi] != nullptr;
-  Col<const S> F{cf.in[fi] + col, plane};
-  Col<S> O{cf.out[fi] + col, plane};
-  Col<double> CP{cp + (int64_t)fi * g.nzn * plane + col, plane};
-  const int st = diffz_column(g, F, O, CP, bt, bt ? cf.bot[fi][col] : 0.0,
-                              bt ? cf.top[fi][col] : 0.0);
+  const bool bt = cf.bot != nullptr && cf.top != nullptr;
+  Col<const double> F{cf.in + col, plane};
+  Col<double> O{cf.out + col, plane};
+  Col<double> CP{cp + col, plane};
+  const int st = diffz_column(g, F, O, CP, bt, bt ? cf.bot[col] : 0.0,
+                              bt ? cf.top[col] : 0.0);
   if (st != PMPIC_OK) raise_status(sc, st);
 }
 
-template <typename S>
-__global__ void __launch_bounds__(64) k_diffz_lds(Geometry g, ColFields<S> cf, DevScalars *sc) {
+__global__ void __launch_bounds__(64) k_diffz_lds(Geometry g, ColField cf, DevScalars *sc) {
   extern __shared__ double sh[];
   const int nc = blockDim.x, t = threadIdx.x, nz = g.nzn;
   const int64_t plane = (int64_t)g.sy * g.sx;
   const int64_t col = (int64_t)blockIdx.x * nc + t;
   if (col >= plane) return;  // no barriers below: each thread touches only its own slice
-  const int fi = blockIdx.y;
-  const bool bt = cf.bot[fi] != nullptr && cf.top[fi] != nullptr;
-  const S *f = cf.in[fi] + col;
-  S *o = cf.out[fi] + col;
+  const bool bt = cf.bot != nullptr && cf.top != nullptr;
+  const double *f = cf.in + col;
+  double *o = cf.out + col;
   Col<double> F{sh + t, nc}, CP{sh + (int64_t)nz * nc + t, nc};
   column_to_lds(f, plane, nz, sh + t, nc);
-  const int st = diffz_column(g, F, F, CP, bt, bt ? cf.bot[fi][col] : 0.0,
-                              bt ? cf.top[fi][col] : 0.0);
+  const int st = diffz_column(g, F, F, CP, bt, bt ? cf.bot[col] : 0.0,
+                              bt ? cf.top[col] : 0.0);
   if (st != PMPIC_OK) {
     raise_status(sc, st);
     return;
   }
 #pragma unroll 8
-  for (int k = 0; k < nz; k++) o[(int64_t)k * plane] = (S)F[k];
+  for (int k = 0; k < nz; k++) o[(int64_t)k * plane] = F[k];
 }
 
 // Register-resident column solvers: the column stays in registers (NZ levels, unrolled) and
@@ -444,8 +306,8 @@ __global__ void k_dz_tables(Geometry g, double *__restrict__ den, double *__rest
 // operation is the one of laplinv_column in the same order: results are bit-identical.  A zero
 // pivot is flagged and raised after the sweeps (the reference stops there; the column's values
 // are then moot).
-template <int Q, int NZ, typename S>
-__global__ void __launch_bounds__(64) k_laplinv_reg(Geometry g, ColFields<S> cf,
+template <int Q, int NZ>
+__global__ void __launch_bounds__(64) k_laplinv_reg(Geometry g, ColField cf,
                                                     const double *__restrict__ k2a,
                                                     DevScalars *sc) {
   static_assert(Q == 1 || Q == 2 || Q == 4, "one, two or four lanes per column");
@@ -458,13 +320,9 @@ __global__ void __launch_bounds__(64) k_laplinv_reg(Geometry g, ColFields<S> cf,
   if (col >= plane) return;
   const double k2 = k2a[col];
   if (k2 == 0) return;
-  const int df0 = cf.df0[blockIdx.y];
-  S *f = cf.out[blockIdx.y] + col;
-  // the FP32-bulk form (S float) forms one reciprocal per pivot and multiplies by it, and
-  // holds the column and the c' values in FP32; the FP64 form divides as the reference does
-  constexpr bool F32 = std::is_same<S, float>::value;
-  using FT = typename std::conditional<F32, float, double>::type;
-  FT F[L], CPl[L];
+  const int df0 = cf.df0;
+  double *f = cf.out + col;
+  double F[L], CPl[L];
 #pragma unroll
   for (int i = 0; i < L; i++) {
     F[i] = 0.0;
@@ -479,15 +337,14 @@ __global__ void __launch_bounds__(64) k_laplinv_reg(Geometry g, ColFields<S> cf,
   const double i2dz2 = 2. / dz / dz, idz2 = 1. / dz / dz;
   const double ai = idz2 - f112 * k2, bi = -i2dz2 - f56 * k2, ci = idz2 - f112 * k2;
   // the original of level q L + L, the next group's first (unused with one lane per column)
-  const double nxt0 = __shfl((double)F[0], (lane + CPW) & 63);
+  const double nxt0 = __shfl(F[0], (lane + CPW) & 63);
   constexpr int PTOP = (NZ - 1) / L;  // group holding level NZ - 1
-  double denominator = 0.0, rden = 0.0, fprev = 0.0, cprev = 0.0, f0 = 0.0, fp = 0.0;
+  double denominator = 0.0, fprev = 0.0, cprev = 0.0, f0 = 0.0, fp = 0.0;
   bool bad = false;
 #pragma unroll
   for (int p = 0; p <= PTOP; p++) {
     if (p > 0) {
       denominator = __shfl(denominator, lane - CPW);
-      if (F32) rden = __shfl(rden, lane - CPW);
       fprev = __shfl(fprev, lane - CPW);
       cprev = __shfl(cprev, lane - CPW);
       f0 = __shfl(f0, lane - CPW);
@@ -506,13 +363,8 @@ __global__ void __launch_bounds__(64) k_laplinv_reg(Geometry g, ColFields<S> cf,
           if (!df0) { b1 = 1.; c1 = 0.; d1 = 0.; }
           else { b1 = -idz2 - f13 * k2; c1 = idz2 - f16 * k2; d1 = f13 * f0 + f16 * fp; }
           denominator = b1;
-          if constexpr (F32) {
-            rden = 1.0 / denominator;
-            fprev = d1 * rden;
-          } else {
-            fprev = d1 / denominator;
-          }
-          F[0] = (FT)fprev;
+          fprev = d1 / denominator;
+          F[0] = fprev;
           cprev = c1;
           continue;
         }
@@ -529,23 +381,18 @@ __global__ void __launch_bounds__(64) k_laplinv_reg(Geometry g, ColFields<S> cf,
           a = idz2 - f16 * k2; b = -idz2 - f13 * k2; c = 0.;
           d = f13 * f0 + f16 * fm;
         }
-        const double cpk = F32 ? cprev * rden : cprev / denominator;
-        CPl[i] = (FT)cpk;
+        const double cpk = cprev / denominator;
+        CPl[i] = cpk;
         denominator = b - a * cpk;
         bad |= (denominator == 0);
-        if constexpr (F32) {
-          rden = 1.0 / denominator;
-          fprev = (d - a * fprev) * rden;
-        } else {
-          fprev = (d - a * fprev) / (denominator);
-        }
-        F[i] = (FT)fprev;
+        fprev = (d - a * fprev) / (denominator);
+        F[i] = fprev;
         cprev = c;
       }
     }
   }
   // backward sweep from the top group down: level j takes c' of level j + 1
-  const double cpn = __shfl((double)CPl[0], (lane + CPW) & 63);
+  const double cpn = __shfl(CPl[0], (lane + CPW) & 63);
   double fnext = fprev;
 #pragma unroll
   for (int p = PTOP; p >= 0; p--) {
@@ -555,9 +402,9 @@ __global__ void __launch_bounds__(64) k_laplinv_reg(Geometry g, ColFields<S> cf,
       for (int i = L - 1; i >= 0; i--) {
         const int j = p * L + i;
         if (j >= NZ - 1) continue;
-        const double cpj1 = (i + 1 < L) ? (double)CPl[i + 1 < L ? i + 1 : 0] : cpn;
-        const double v = (double)F[i] - cpj1 * fnext;
-        F[i] = (FT)v;
+        const double cpj1 = (i + 1 < L) ? CPl[i + 1 < L ? i + 1 : 0] : cpn;
+        const double v = F[i] - cpj1 * fnext;
+        F[i] = v;
         fnext = v;
       }
     }
@@ -565,11 +412,11 @@ __global__ void __launch_bounds__(64) k_laplinv_reg(Geometry g, ColFields<S> cf,
   if (bad) raise_status(sc, PMPIC_ERR_ZERO_PIVOT);
 #pragma unroll
   for (int i = 0; i < L; i++)
-    if (q * L + i < NZ) f[(int64_t)(q * L + i) * plane] = (S)F[i];
+    if (q * L + i < NZ) f[(int64_t)(q * L + i) * plane] = F[i];
 }
 
-template <int NZ, typename S>
-__global__ void __launch_bounds__(64) k_diffz_reg(Geometry g, ColFields<S> cf,
+template <int NZ>
+__global__ void __launch_bounds__(64) k_diffz_reg(Geometry g, ColField cf,
                                                   const double *__restrict__ tden,
                                                   const double *__restrict__ tcp,
                                                   DevScalars *sc) {
@@ -578,64 +425,56 @@ __global__ void __launch_bounds__(64) k_diffz_reg(Geometry g, ColFields<S> cf,
   // stages the pivots' reciprocals and multiplies by them, takes 1/dz and 1/(2 dz) as factors
   // and holds the column in FP32 between the sweeps (the sweeps themselves run in FP64); the
   // FP64 form divides as the reference does
-  constexpr bool F32 = std::is_same<S, float>::value;
-  using FT = typename std::conditional<F32, float, double>::type;
   __shared__ double den[NZ], cpt[NZ];
   const int64_t plane = (int64_t)g.sy * g.sx;
   const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int fi = blockIdx.y;
-  const bool bt = cf.bot[fi] != nullptr && cf.top[fi] != nullptr;
+  const bool bt = cf.bot != nullptr && cf.top != nullptr;
   for (int k = threadIdx.x; k < NZ; k += blockDim.x) {
     const double dn = tden[(bt ? NZ : 0) + k];
-    if (F32 && dn == 0 && blockIdx.x == 0) raise_status(sc, PMPIC_ERR_ZERO_PIVOT);
-    den[k] = F32 ? 1.0 / dn : dn;
+    den[k] = dn;
     cpt[k] = tcp[(bt ? NZ : 0) + k];
   }
   __syncthreads();
   if (col >= plane) return;
-  const S *fin = cf.in[fi] + col;
-  S *o = cf.out[fi] + col;
-  FT F[NZ];
+  const double *fin = cf.in + col;
+  double *o = cf.out + col;
+  double F[NZ];
 #pragma unroll
   for (int k = 0; k < NZ; k++) F[k] = fin[(int64_t)k * plane];
-  const double bot = bt ? cf.bot[fi][col] : 0.0, top = bt ? cf.top[fi][col] : 0.0;
+  const double bot = bt ? cf.bot[col] : 0.0, top = bt ? cf.top[col] : 0.0;
   const double a1 = (double)(1.f / 6.f), al = (double)(1.f / 3.f);
   const double dz = g.dz, idz = 1.0 / dz, ih2dz = 0.5 / dz;
   double fkm2 = F[0], fkm1 = F[1];  // originals f(k-2), f(k-1) of the next row
-  const double d0 = bt ? (F32 ? fkm1 * idz : fkm1 / dz) - a1 * bot * dz : 0.0;
-  double fprev = F32 ? d0 * den[0] : d0 / den[0];
-  F[0] = (FT)fprev;
+  const double d0 = bt ? (fkm1 / dz) - a1 * bot * dz : 0.0;
+  double fprev = d0 / den[0];
+  F[0] = fprev;
 #pragma unroll
   for (int k = 2; k <= NZ; k++) {
     double a, d, fk = 0.0;
     if (k < NZ) {
       a = a1;
       fk = F[k < NZ ? k : 0];
-      d = F32 ? (fk - fkm2) * ih2dz : (fk - fkm2) / 2. / dz;
+      d = (fk - fkm2) / 2. / dz;
     } else {
       a = bt ? al : 0.;
-      d = bt ? (F32 ? -fkm2 * idz : -fkm2 / dz) + a1 * top * dz : 0.0;
+      d = bt ? (-fkm2 / dz) + a1 * top * dz : 0.0;
     }
     const double dn = den[k - 1];
-    if constexpr (F32) {
-      fprev = (d - a * fprev) * dn;
-    } else {
-      if (dn == 0) { raise_status(sc, PMPIC_ERR_ZERO_PIVOT); return; }
-      fprev = (d - a * fprev) / (dn);
-    }
-    F[k - 1] = (FT)fprev;
+    if (dn == 0) { raise_status(sc, PMPIC_ERR_ZERO_PIVOT); return; }
+    fprev = (d - a * fprev) / (dn);
+    F[k - 1] = fprev;
     fkm2 = fkm1;
     fkm1 = fk;
   }
   double fnext = fprev;
 #pragma unroll
   for (int k = NZ - 1; k >= 1; k--) {
-    const double v = (double)F[k - 1] - cpt[k] * fnext;
-    F[k - 1] = (FT)v;
+    const double v = F[k - 1] - cpt[k] * fnext;
+    F[k - 1] = v;
     fnext = v;
   }
 #pragma unroll
-  for (int k = 0; k < NZ; k++) o[(int64_t)k * plane] = (S)F[k];
+  for (int k = 0; k < NZ; k++) o[(int64_t)k * plane] = F[k];
 }
 
 // Long columns (more z nodes than the instances above): Q lanes per column, lane q holding
@@ -643,8 +482,8 @@ __global__ void __launch_bounds__(64) k_diffz_reg(Geometry g, ColFields<S> cf,
 // run time.  The sweeps run lane group after lane group as in k_laplinv_reg, the recurrence
 // state crossing by lane shuffles, every operation the one of laplinv_column / k_diffz_reg in
 // the same order, so results are bit-identical to them.
-template <int Q, int L, typename S>
-__global__ void __launch_bounds__(64) k_laplinv_qn(Geometry g, ColFields<S> cf,
+template <int Q, int L>
+__global__ void __launch_bounds__(64) k_laplinv_qn(Geometry g, ColField cf,
                                                    const double *__restrict__ k2a,
                                                    DevScalars *sc) {
   constexpr int CPW = 64 / Q;  // columns per wavefront
@@ -656,12 +495,9 @@ __global__ void __launch_bounds__(64) k_laplinv_qn(Geometry g, ColFields<S> cf,
   if (col >= plane) return;  // all Q lanes of a column leave together
   const double k2 = k2a[col];
   if (k2 == 0) return;
-  const int df0 = cf.df0[blockIdx.y];
-  S *f = cf.out[blockIdx.y] + col;
-  // the FP32-bulk form as in k_laplinv_reg: one reciprocal per pivot, FP32 column and c'
-  constexpr bool F32 = std::is_same<S, float>::value;
-  using FT = typename std::conditional<F32, float, double>::type;
-  FT F[L], CPl[L];
+  const int df0 = cf.df0;
+  double *f = cf.out + col;
+  double F[L], CPl[L];
 #pragma unroll
   for (int i = 0; i < L; i++) {
     F[i] = 0.0;
@@ -675,14 +511,13 @@ __global__ void __launch_bounds__(64) k_laplinv_qn(Geometry g, ColFields<S> cf,
   const double dz = g.dz;
   const double i2dz2 = 2. / dz / dz, idz2 = 1. / dz / dz;
   const double ai = idz2 - f112 * k2, bi = -i2dz2 - f56 * k2, ci = idz2 - f112 * k2;
-  const double nxt0 = __shfl((double)F[0], lane + CPW);  // the next group's first original
+  const double nxt0 = __shfl(F[0], lane + CPW);  // the next group's first original
   const int PTOP = (NZ - 1) / L;                         // group holding level NZ - 1
-  double denominator = 0.0, rden = 0.0, fprev = 0.0, cprev = 0.0, f0 = 0.0, fp = 0.0;
+  double denominator = 0.0, fprev = 0.0, cprev = 0.0, f0 = 0.0, fp = 0.0;
   bool bad = false;
   for (int p = 0; p <= PTOP; p++) {
     if (p > 0) {
       denominator = __shfl(denominator, lane - CPW);
-      if (F32) rden = __shfl(rden, lane - CPW);
       fprev = __shfl(fprev, lane - CPW);
       cprev = __shfl(cprev, lane - CPW);
       f0 = __shfl(f0, lane - CPW);
@@ -701,13 +536,8 @@ __global__ void __launch_bounds__(64) k_laplinv_qn(Geometry g, ColFields<S> cf,
           if (!df0) { b1 = 1.; c1 = 0.; d1 = 0.; }
           else { b1 = -idz2 - f13 * k2; c1 = idz2 - f16 * k2; d1 = f13 * f0 + f16 * fp; }
           denominator = b1;
-          if constexpr (F32) {
-            rden = 1.0 / denominator;
-            fprev = d1 * rden;
-          } else {
-            fprev = d1 / denominator;
-          }
-          F[0] = (FT)fprev;
+          fprev = d1 / denominator;
+          F[0] = fprev;
           cprev = c1;
           continue;
         }
@@ -724,22 +554,17 @@ __global__ void __launch_bounds__(64) k_laplinv_qn(Geometry g, ColFields<S> cf,
           a = idz2 - f16 * k2; b = -idz2 - f13 * k2; c = 0.;
           d = f13 * f0 + f16 * fm;
         }
-        const double cpk = F32 ? cprev * rden : cprev / denominator;
-        CPl[i] = (FT)cpk;
+        const double cpk = cprev / denominator;
+        CPl[i] = cpk;
         denominator = b - a * cpk;
         bad |= (denominator == 0);
-        if constexpr (F32) {
-          rden = 1.0 / denominator;
-          fprev = (d - a * fprev) * rden;
-        } else {
-          fprev = (d - a * fprev) / (denominator);
-        }
-        F[i] = (FT)fprev;
+        fprev = (d - a * fprev) / (denominator);
+        F[i] = fprev;
         cprev = c;
       }
     }
   }
-  const double cpn = __shfl((double)CPl[0], lane + CPW);
+  const double cpn = __shfl(CPl[0], lane + CPW);
   double fnext = fprev;
   for (int p = PTOP; p >= 0; p--) {
     if (p < PTOP) fnext = __shfl(fnext, lane + CPW);
@@ -748,9 +573,9 @@ __global__ void __launch_bounds__(64) k_laplinv_qn(Geometry g, ColFields<S> cf,
       for (int i = L - 1; i >= 0; i--) {
         const int j = p * L + i;
         if (j >= NZ - 1) continue;
-        const double cpj1 = (i + 1 < L) ? (double)CPl[i + 1 < L ? i + 1 : 0] : cpn;
-        const double v = (double)F[i] - cpj1 * fnext;
-        F[i] = (FT)v;
+        const double cpj1 = (i + 1 < L) ? CPl[i + 1 < L ? i + 1 : 0] : cpn;
+        const double v = F[i] - cpj1 * fnext;
+        F[i] = v;
         fnext = v;
       }
     }
@@ -758,42 +583,38 @@ __global__ void __launch_bounds__(64) k_laplinv_qn(Geometry g, ColFields<S> cf,
   if (bad) raise_status(sc, PMPIC_ERR_ZERO_PIVOT);
 #pragma unroll
   for (int i = 0; i < L; i++)
-    if (q * L + i < NZ) f[(int64_t)(q * L + i) * plane] = (S)F[i];
+    if (q * L + i < NZ) f[(int64_t)(q * L + i) * plane] = F[i];
 }
 
-template <int Q, int L, typename S>
-__global__ void __launch_bounds__(64) k_diffz_qn(Geometry g, ColFields<S> cf,
+template <int Q, int L>
+__global__ void __launch_bounds__(64) k_diffz_qn(Geometry g, ColField cf,
                                                  const double *__restrict__ tden,
                                                  const double *__restrict__ tcp,
                                                  DevScalars *sc) {
   constexpr int CPW = 64 / Q;
-  // the FP32-bulk form as in k_diffz_reg: pivot reciprocals, 1/dz factors, FP32 column
-  constexpr bool F32 = std::is_same<S, float>::value;
-  using FT = typename std::conditional<F32, float, double>::type;
   __shared__ double den[Q * L], cpt[Q * L];
   const int NZ = g.nzn;
   const int lane = threadIdx.x;
   const int q = lane / CPW;
   const int64_t plane = (int64_t)g.sy * g.sx;
   const int64_t col = (int64_t)blockIdx.x * CPW + (lane % CPW);
-  const int fi = blockIdx.y;
-  const bool bt = cf.bot[fi] != nullptr && cf.top[fi] != nullptr;
+  const bool bt = cf.bot != nullptr && cf.top != nullptr;
   for (int k = threadIdx.x; k < NZ; k += blockDim.x) {
     const double dn = tden[(bt ? NZ : 0) + k];
-    den[k] = F32 ? 1.0 / dn : dn;
+    den[k] = dn;
     cpt[k] = tcp[(bt ? NZ : 0) + k];
   }
   __syncthreads();
   if (col >= plane) return;  // all Q lanes of a column leave together
-  const S *fin = cf.in[fi] + col;
-  S *o = cf.out[fi] + col;
-  FT F[L];
+  const double *fin = cf.in + col;
+  double *o = cf.out + col;
+  double F[L];
 #pragma unroll
-  for (int i = 0; i < L; i++) F[i] = (q * L + i < NZ) ? fin[(int64_t)(q * L + i) * plane] : (S)0;
-  const double bot = bt ? cf.bot[fi][col] : 0.0, top = bt ? cf.top[fi][col] : 0.0;
+  for (int i = 0; i < L; i++) F[i] = (q * L + i < NZ) ? fin[(int64_t)(q * L + i) * plane] : 0.0;
+  const double bot = bt ? cf.bot[col] : 0.0, top = bt ? cf.top[col] : 0.0;
   const double a1 = (double)(1.f / 6.f), al = (double)(1.f / 3.f);
   const double dz = g.dz, idz = 1.0 / dz, ih2dz = 0.5 / dz;
-  const double nxt0 = __shfl((double)F[0], lane + CPW);  // the original of the next group's first level
+  const double nxt0 = __shfl(F[0], lane + CPW);  // the original of the next group's first level
   const int PTOP = (NZ - 1) / L;
   double fprev = 0.0, fkm2 = 0.0, fkm1 = 0.0;  // originals f(k-2), f(k-1) of the next row
   bool bad = false;
@@ -812,35 +633,25 @@ __global__ void __launch_bounds__(64) k_diffz_qn(Geometry g, ColFields<S> cf,
         if (j == 0) {
           fkm2 = F[0];
           fkm1 = onext;
-          const double d0 = bt ? (F32 ? fkm1 * idz : fkm1 / dz) - a1 * bot * dz : 0.0;
-          if constexpr (F32) {
-            bad |= !__builtin_isfinite(den[0]);
-            fprev = d0 * den[0];
-          } else {
-            bad |= (den[0] == 0);
-            fprev = d0 / den[0];
-          }
-          F[0] = (FT)fprev;
+          const double d0 = bt ? (fkm1 / dz) - a1 * bot * dz : 0.0;
+          bad |= (den[0] == 0);
+          fprev = d0 / den[0];
+          F[0] = fprev;
           continue;
         }
         double a, d, fk = 0.0;
         if (j + 1 < NZ) {
           a = a1;
           fk = onext;
-          d = F32 ? (fk - fkm2) * ih2dz : (fk - fkm2) / 2. / dz;
+          d = (fk - fkm2) / 2. / dz;
         } else {
           a = bt ? al : 0.;
-          d = bt ? (F32 ? -fkm2 * idz : -fkm2 / dz) + a1 * top * dz : 0.0;
+          d = bt ? (-fkm2 / dz) + a1 * top * dz : 0.0;
         }
         const double dn = den[j];
-        if constexpr (F32) {
-          bad |= !__builtin_isfinite(dn);
-          fprev = (d - a * fprev) * dn;
-        } else {
-          bad |= (dn == 0);
-          fprev = (d - a * fprev) / (dn);
-        }
-        F[i] = (FT)fprev;
+        bad |= (dn == 0);
+        fprev = (d - a * fprev) / (dn);
+        F[i] = fprev;
         fkm2 = fkm1;
         fkm1 = fk;
       }
@@ -854,8 +665,8 @@ __global__ void __launch_bounds__(64) k_diffz_qn(Geometry g, ColFields<S> cf,
       for (int i = L - 1; i >= 0; i--) {
         const int j = p * L + i;
         if (j >= NZ - 1) continue;
-        const double v = (double)F[i] - cpt[j + 1] * fnext;
-        F[i] = (FT)v;
+        const double v = F[i] - cpt[j + 1] * fnext;
+        F[i] = v;
         fnext = v;
       }
     }
@@ -863,30 +674,7 @@ __global__ void __launch_bounds__(64) k_diffz_qn(Geometry g, ColFields<S> cf,
   if (bad) raise_status(sc, PMPIC_ERR_ZERO_PIVOT);
 #pragma unroll
   for (int i = 0; i < L; i++)
-    if (q * L + i < NZ) o[(int64_t)(q * L + i) * plane] = (S)F[i];
-}
-
-// u, v, w spectra (vort2vel.F90:251-320): fu = dzb - diffy(c), column (1,1) = ubar;
-// fv = diffx(c) - dza, column (1,1) = vbar; fw = diffy(a) - diffx(b); u_s.. = filtered
-template <typename S>
-__global__ void k_velocity_spectra(Geometry g, const S *__restrict__ a,
-                                   const S *__restrict__ b, const S *__restrict__ c,
-                                   const S *__restrict__ dzb, const S *__restrict__ dza,
-                                   const double *__restrict__ ubar, const double *__restrict__ vbar,
-                                   S *__restrict__ fu, S *__restrict__ fv,
-                                   S *__restrict__ fw, S *__restrict__ us,
-                                   S *__restrict__ vs, S *__restrict__ ws,
-                                   const double *__restrict__ kx, const double *__restrict__ ky,
-                                   const double *__restrict__ filt) {
-  SPEC_ELEMENT(g);
-  const double fl = filt[col];
-  double u = (double)dzb[q] - dy_at(c, ky, q, jj, g.sx, col);
-  if (col == 0) u = ubar[k];
-  double v = dx_at(c, kx, q, ii, col) - (double)dza[q];
-  if (col == 0) v = vbar[k];
-  const double w = dy_at(a, ky, q, jj, g.sx, col) - dx_at(b, kx, q, ii, col);
-  fu[q] = (S)u; fv[q] = (S)v; fw[q] = (S)w;
-  us[q] = (S)(u * fl); vs[q] = (S)(v * fl); ws[q] = (S)(w * fl);
+    if (q * L + i < NZ) o[(int64_t)(q * L + i) * plane] = F[i];
 }
 
 // vorticity_tendency.F90:169-265, physical interior, accumulation order as written
@@ -1077,185 +865,75 @@ static int lds_cols(const Geometry &g) {
 
 // column lengths (z nodes) with a register-resident solver instance
 #define PMPIC_REG_COLUMNS(X) X(9) X(17) X(33) X(65) X(129)
+// lanes per column of the register-resident laplinv
+constexpr int LAP_Q = 4;
 // longer columns, up to LONG_Q * LONG_L z nodes: LONG_Q lanes per column, LONG_L levels each
 constexpr int LONG_Q = 8, LONG_L = 33;
 // other lengths up to 129 z nodes (48^3 and 96^3 grids, say) in the same lane-group form: four
 // lanes per column with 13 levels each up to 52 nodes, 33 each up to 129
 constexpr int MID_Q = 4, MID_L_SHORT = 13, MID_L = 33;
-// the FP32-bulk form, whose columns sit in registers as FP32, takes long columns up to
-// F32_Q * F32_L z nodes with four lanes per column (sixteen columns a wavefront, twice the FP64
-// form's), and the 257-node columns of 256-cell-deep grids in the register-resident solvers
-constexpr int F32_Q = 4, F32_L = 65, F32_REG_LONG = 257;
-// lanes per column of the register-resident laplinv: four, but two (32 columns a wavefront) for
-// the FP32-bulk form's columns of up to F32_LAP_Q2 nodes, whose column and c' then still fit in
-// registers at three wavefronts per SIMD (18.8 against 24.7 us a call at 65 nodes, 128^2
-// columns).  One lane per column, or two on longer columns, gains nothing (the sweeps are then
-// held at one or two wavefronts per SIMD by their registers)
-constexpr int F32_LAP_Q2 = 65;
-template <typename S>
-constexpr int lap_q(int nz) {
-  return std::is_same<S, float>::value && nz <= F32_LAP_Q2 ? 2 : 4;
-}
 
-template <typename S>
-int op_filter_t(Ctx *c, const S *in, S *out) {
-  hipLaunchKernelGGL(k_filter<S>, spec_grid(c->g), dim3(TPB), 0, c->stream, c->g,
-                     in, out, c->filt);
+int op_filter(Ctx *c, const double *in, double *out) {
+  hipLaunchKernelGGL(k_filter, dim3(cdiv(ssz_of(c->g), TPB)), dim3(TPB), 0, c->stream, c->g, in,
+                     out, c->filt);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
-int op_filter(Ctx *c, const double *in, double *out) { return op_filter_t<double>(c, in, out); }
 
-template <typename S>
-int op_diffz_n(Ctx *c, int nf, const S *const *in, S *const *out, const double *const *bot,
-               const double *const *top) {
-  if (nf < 1 || nf > 4) return PMPIC_ERR_ARG;
+int op_diffz(Ctx *c, const double *in, double *out, const double *bot, const double *top) {
   const int64_t plane = plane_of(c->g);
-  const int nc = lds_cols(c->g);
-  ColFields<S> rf{};
-  for (int f = 0; f < nf; f++) {
-    rf.in[f] = in[f];
-    rf.out[f] = out[f];
-    rf.bot[f] = bot ? bot[f] : nullptr;
-    rf.top[f] = top ? top[f] : nullptr;
-  }
-  switch (c->g.nzn) {
-#define PMPIC_DZ_CASE(NZ)                                                                     \
-  case NZ:                                                                                     \
-    hipLaunchKernelGGL((k_diffz_reg<NZ, S>), dim3(cdiv(plane, 64), nf), dim3(64), 0, c->stream, \
-                       c->g, rf, c->dz_den, c->dz_cp, c->dsc);                                 \
-    PMPIC_CHECK(hipGetLastError());                                                            \
-    return PMPIC_OK;
+  const int nzn = c->g.nzn, nc = lds_cols(c->g);
+  const ColField f{in, out, bot, top, 0};
+  auto run = [&](auto kernel, int columns) {
+    hipLaunchKernelGGL(kernel, dim3(cdiv(plane, columns)), dim3(64), 0, c->stream, c->g, f,
+                       c->dz_den, c->dz_cp, c->dsc);
+  };
+  switch (nzn) {
+#define PMPIC_DZ_CASE(NZ) case NZ: run(k_diffz_reg<NZ>, 64); break;
     PMPIC_REG_COLUMNS(PMPIC_DZ_CASE)
 #undef PMPIC_DZ_CASE
     default:
-      break;
-  }
-  if (c->g.nzn <= MID_Q * MID_L_SHORT) {
-    hipLaunchKernelGGL((k_diffz_qn<MID_Q, MID_L_SHORT, S>), dim3(cdiv(plane, 64 / MID_Q), nf),
-                       dim3(64), 0, c->stream, c->g, rf, c->dz_den, c->dz_cp, c->dsc);
-    PMPIC_CHECK(hipGetLastError());
-    return PMPIC_OK;
-  }
-  if (c->g.nzn <= 129) {
-    hipLaunchKernelGGL((k_diffz_qn<MID_Q, MID_L, S>), dim3(cdiv(plane, 64 / MID_Q), nf),
-                       dim3(64), 0, c->stream, c->g, rf, c->dz_den, c->dz_cp, c->dsc);
-    PMPIC_CHECK(hipGetLastError());
-    return PMPIC_OK;
-  }
-  if constexpr (std::is_same<S, float>::value) {
-    if (c->g.nzn == F32_REG_LONG) {
-      hipLaunchKernelGGL((k_diffz_reg<F32_REG_LONG, S>), dim3(cdiv(plane, 64), nf), dim3(64), 0,
-                         c->stream, c->g, rf, c->dz_den, c->dz_cp, c->dsc);
-      PMPIC_CHECK(hipGetLastError());
-      return PMPIC_OK;
-    }
-    if (c->g.nzn <= F32_Q * F32_L) {
-      hipLaunchKernelGGL((k_diffz_qn<F32_Q, F32_L, S>), dim3(cdiv(plane, 64 / F32_Q), nf),
-                         dim3(64), 0, c->stream, c->g, rf, c->dz_den, c->dz_cp, c->dsc);
-      PMPIC_CHECK(hipGetLastError());
-      return PMPIC_OK;
-    }
-  }
-  if (c->g.nzn <= LONG_Q * LONG_L) {
-    hipLaunchKernelGGL((k_diffz_qn<LONG_Q, LONG_L, S>), dim3(cdiv(plane, 64 / LONG_Q), nf),
-                       dim3(64), 0, c->stream, c->g, rf, c->dz_den, c->dz_cp, c->dsc);
-    PMPIC_CHECK(hipGetLastError());
-    return PMPIC_OK;
-  }
-  if (nc > 0) {
-    hipLaunchKernelGGL(k_diffz_lds<S>, dim3(cdiv(plane, nc), nf), dim3(nc),
-                       (size_t)2 * nc * c->g.nzn * sizeof(double), c->stream, c->g, rf, c->dsc);
-  } else {
-    for (int f = 0; f < nf; f++) {  // one field at a time: sder[7] holds one field's cp
-      ColFields<S> one{};
-      one.in[0] = in[f];
-      one.out[0] = out[f];
-      one.bot[0] = bot ? bot[f] : nullptr;
-      one.top[0] = top ? top[f] : nullptr;
-      hipLaunchKernelGGL(k_diffz<S>, dim3(cdiv(plane, 64), 1), dim3(64), 0, c->stream, c->g, one,
-                         c->sder[7], c->dsc);
-    }
+      if (nzn <= MID_Q * MID_L_SHORT) run(k_diffz_qn<MID_Q, MID_L_SHORT>, 64 / MID_Q);
+      else if (nzn <= 129) run(k_diffz_qn<MID_Q, MID_L>, 64 / MID_Q);
+      else if (nzn <= LONG_Q * LONG_L) run(k_diffz_qn<LONG_Q, LONG_L>, 64 / LONG_Q);
+      else if (nc > 0)
+        hipLaunchKernelGGL(k_diffz_lds, dim3(cdiv(plane, nc)), dim3(nc),
+                           (size_t)2 * nc * nzn * sizeof(double), c->stream, c->g, f, c->dsc);
+      else
+        hipLaunchKernelGGL(k_diffz, dim3(cdiv(plane, 64)), dim3(64), 0, c->stream, c->g, f,
+                           c->sder[5], c->dsc);
   }
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
-int op_diffz(Ctx *c, const double *in, double *out, const double *bot, const double *top) {
-  return op_diffz_n<double>(c, 1, &in, &out, bot ? &bot : nullptr, top ? &top : nullptr);
-}
 
-template <typename S>
-int op_laplinv_n(Ctx *c, int nf, S *const *f, const int *df0) {
-  if (nf < 1 || nf > 4) return PMPIC_ERR_ARG;
+int op_laplinv(Ctx *c, double *data, int df0) {
   const int64_t plane = plane_of(c->g);
-  const int nc = lds_cols(c->g);
-  ColFields<S> rf{};
-  for (int q = 0; q < nf; q++) {
-    rf.out[q] = f[q];
-    rf.df0[q] = df0[q] ? 1 : 0;
-  }
-  switch (c->g.nzn) {
-#define PMPIC_LAP_CASE(NZ)                                                                    \
-  case NZ:                                                                                     \
-    hipLaunchKernelGGL((k_laplinv_reg<lap_q<S>(NZ), NZ, S>), dim3(cdiv(plane, 64 / lap_q<S>(NZ)), \
-                       nf), dim3(64), 0, c->stream, c->g, rf, c->k2, c->dsc);                  \
-    PMPIC_CHECK(hipGetLastError());                                                            \
-    return PMPIC_OK;
+  const int nzn = c->g.nzn, nc = lds_cols(c->g);
+  const ColField f{nullptr, data, nullptr, nullptr, df0 ? 1 : 0};
+  auto run = [&](auto kernel, int columns) {
+    hipLaunchKernelGGL(kernel, dim3(cdiv(plane, columns)), dim3(64), 0, c->stream, c->g, f, c->k2,
+                       c->dsc);
+  };
+  switch (nzn) {
+#define PMPIC_LAP_CASE(NZ) case NZ: run(k_laplinv_reg<LAP_Q, NZ>, 64 / LAP_Q); break;
     PMPIC_REG_COLUMNS(PMPIC_LAP_CASE)
 #undef PMPIC_LAP_CASE
     default:
-      break;
-  }
-  if (c->g.nzn <= MID_Q * MID_L_SHORT) {
-    hipLaunchKernelGGL((k_laplinv_qn<MID_Q, MID_L_SHORT, S>), dim3(cdiv(plane, 64 / MID_Q), nf),
-                       dim3(64), 0, c->stream, c->g, rf, c->k2, c->dsc);
-    PMPIC_CHECK(hipGetLastError());
-    return PMPIC_OK;
-  }
-  if (c->g.nzn <= 129) {
-    hipLaunchKernelGGL((k_laplinv_qn<MID_Q, MID_L, S>), dim3(cdiv(plane, 64 / MID_Q), nf),
-                       dim3(64), 0, c->stream, c->g, rf, c->k2, c->dsc);
-    PMPIC_CHECK(hipGetLastError());
-    return PMPIC_OK;
-  }
-  if constexpr (std::is_same<S, float>::value) {
-    if (c->g.nzn == F32_REG_LONG) {
-      constexpr int Q = lap_q<S>(F32_REG_LONG);
-      hipLaunchKernelGGL((k_laplinv_reg<Q, F32_REG_LONG, S>), dim3(cdiv(plane, 64 / Q), nf),
-                         dim3(64), 0, c->stream, c->g, rf, c->k2, c->dsc);
-      PMPIC_CHECK(hipGetLastError());
-      return PMPIC_OK;
-    }
-    if (c->g.nzn <= F32_Q * F32_L) {
-      hipLaunchKernelGGL((k_laplinv_qn<F32_Q, F32_L, S>), dim3(cdiv(plane, 64 / F32_Q), nf),
-                         dim3(64), 0, c->stream, c->g, rf, c->k2, c->dsc);
-      PMPIC_CHECK(hipGetLastError());
-      return PMPIC_OK;
-    }
-  }
-  if (c->g.nzn <= LONG_Q * LONG_L) {
-    hipLaunchKernelGGL((k_laplinv_qn<LONG_Q, LONG_L, S>), dim3(cdiv(plane, 64 / LONG_Q), nf),
-                       dim3(64), 0, c->stream, c->g, rf, c->k2, c->dsc);
-    PMPIC_CHECK(hipGetLastError());
-    return PMPIC_OK;
-  }
-  if (nc > 0) {
-    hipLaunchKernelGGL(k_laplinv_lds<S>, dim3(cdiv(plane, nc), nf), dim3(nc),
-                       (size_t)2 * nc * c->g.nzn * sizeof(double), c->stream, c->g, rf, c->k2,
-                       c->dsc);
-  } else {
-    for (int q = 0; q < nf; q++) {
-      ColFields<S> one{};
-      one.out[0] = f[q];
-      one.df0[0] = df0[q];
-      hipLaunchKernelGGL(k_laplinv<S>, dim3(cdiv(plane, 64), 1), dim3(64), 0, c->stream, c->g,
-                         one, c->sder[7], c->k2, c->dsc);
-    }
+      if (nzn <= MID_Q * MID_L_SHORT) run(k_laplinv_qn<MID_Q, MID_L_SHORT>, 64 / MID_Q);
+      else if (nzn <= 129) run(k_laplinv_qn<MID_Q, MID_L>, 64 / MID_Q);
+      else if (nzn <= LONG_Q * LONG_L) run(k_laplinv_qn<LONG_Q, LONG_L>, 64 / LONG_Q);
+      else if (nc > 0)
+        hipLaunchKernelGGL(k_laplinv_lds, dim3(cdiv(plane, nc)), dim3(nc),
+                           (size_t)2 * nc * nzn * sizeof(double), c->stream, c->g, f, c->k2,
+                           c->dsc);
+      else
+        hipLaunchKernelGGL(k_laplinv, dim3(cdiv(plane, 64)), dim3(64), 0, c->stream, c->g, f,
+                           c->sder[5], c->k2, c->dsc);
   }
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
-int op_laplinv(Ctx *c, double *f, int df0) { return op_laplinv_n<double>(c, 1, &f, &df0); }
 
 namespace {
 // the spectral scratch arrays as arrays of the form's spectral type (the FP32-bulk form uses
@@ -1263,11 +941,6 @@ namespace {
 template <typename S> S *sp(double *a) { return reinterpret_cast<S *>(a); }
 }  // namespace
 
-// vort2vel timestep_callback (vort2vel.F90:134-320) after par2grid of p, q, r into the grids:
-// corrected and filtered vorticity back into grid[GP..GR], velocities into grid[GU..GW], the
-// filtered velocity spectra into su, sv, sw.  S: the spectral arrays' type (FP32 in the
-// FP32-bulk form: its transforms and spectral arrays are FP32, the mean flow, the boundary
-// planes and the column solvers' arithmetic FP64).
 // the physical p, q, r and total-buoyancy grids (k = 0..3) in the transforms' precision: the
 // FP64 grids GP, GQ, GR, GB, or the FP32-bulk form's FP32 grids
 static_assert(GQ == GP + 1 && GR == GP + 2 && GB == GP + 3, "grid ids p, q, r, b in sequence");
@@ -1275,105 +948,53 @@ template <typename S> S *pqrb(Ctx *c, int k);
 template <> double *pqrb<double>(Ctx *c, int k) { return c->grid[GP + k]; }
 template <> float *pqrb<float>(Ctx *c, int k) { return c->b32.pgrid[k]; }
 
+// vort2vel timestep_callback (vort2vel.F90:134-320) after par2grid of p, q, r (and the total
+// buoyancy) into the grids: corrected and filtered vorticity back into grid[GP..GR], velocities
+// into grid[GU..GW], the filtered velocity spectra into su, sv, sw.  Also what
+// vorticity_tendency.F90:147-232 takes from the same spectra: the transform of the total buoyancy
+// and the eight derivative grids of the tendency (db/dy, du/dx, du/dy, dw/dx, db/dx, dv/dx, dv/dy,
+// dw/dy) into gtmp, each derivative taken while its inverse transform reads the spectrum, so that
+// the two components share one forward and one inverse transform call.  S: the spectral arrays'
+// type (FP32 in the FP32-bulk form, which keeps every grid here in FP32 only).
 template <typename S>
 static int vort2vel_spectral_t(Ctx *c) {
-  const Geometry &g = c->g;
-  const dim3 eb = spec_grid(g), et(TPB);
-  S *sa = sp<S>(c->sa), *sb = sp<S>(c->sb), *sc = sp<S>(c->sc), *sd = sp<S>(c->sd);
-  S *se = sp<S>(c->se), *sf = sp<S>(c->sf);
-  S *sder[5] = {sp<S>(c->sder[0]), sp<S>(c->sder[1]), sp<S>(c->sder[2]), sp<S>(c->sder[3]),
-                sp<S>(c->sder[4])};
+  S *sbs = sp<S>(c->sbs);
   {
-    const S *src[3] = {pqrb<S>(c, 0), pqrb<S>(c, 1), pqrb<S>(c, 2)};
-    S *dst[3] = {sa, sb, sc};
-    PMPIC_TRY(fft_forward_t<S>(c, 3, src, dst));
+    const S *src[4] = {pqrb<S>(c, 0), pqrb<S>(c, 1), pqrb<S>(c, 2), pqrb<S>(c, 3)};
+    S *dst[4] = {sp<S>(c->sa), sp<S>(c->sb), sp<S>(c->sc), sbs};
+    PMPIC_TRY(fft_forward_t<S>(c, 4, src, dst));
   }
-  const double hdzi = 1. / 2. / g.dz;
-  hipLaunchKernelGGL(k_divergence<S>, eb, et, 0, c->stream, g, sa, sb, sc, sf, c->kx, c->ky,
-                     hdzi);
-  {
-    const int df0[1] = {1};
-    PMPIC_TRY(op_laplinv_n<S>(c, 1, &sf, df0));
-  }
-  PMPIC_TRY(op_filter_t<S>(c, sf, sf));
-  hipLaunchKernelGGL(k_correct_ab<S>, eb, et, 0, c->stream, g, sa, sb, sf, c->kx, c->ky);
-  {
-    const S *in[1] = {sf};
-    PMPIC_TRY(op_diffz_n<S>(c, 1, in, &sd, nullptr, nullptr));
-  }
-  hipLaunchKernelGGL(k_correct_c_filter<S>, eb, et, 0, c->stream, g, sa, sb, sc, sd, sd, se, sf,
-                     c->filt, c->atop, c->abot, c->btop, c->bbot);
-  hipLaunchKernelGGL(k_mean_flow<S>, dim3(1), dim3(256), (size_t)(4 * g.nzn + 2) * sizeof(double),
-                     c->stream, g, sd, se, c->ubar, c->vbar);
-  {
-    S *fl[3] = {sa, sb, sc};
-    const int df0[3] = {0, 0, 1};
-    PMPIC_TRY(op_laplinv_n<S>(c, 3, fl, df0));
-  }
-  {
-    // dz(b) with b's cached top/bottom into sder[0], dz(a) into sder[1]
-    const S *in[2] = {sb, sa};
-    S *out[2] = {sder[0], sder[1]};
-    const double *bot[2] = {c->bbot, c->abot}, *top[2] = {c->btop, c->atop};
-    PMPIC_TRY(op_diffz_n<S>(c, 2, in, out, bot, top));
-  }
-  hipLaunchKernelGGL(k_velocity_spectra<S>, eb, et, 0, c->stream, g, sa, sb, sc, sder[0],
-                     sder[1], c->ubar, c->vbar, sder[2], sder[3], sder[4], sp<S>(c->su),
-                     sp<S>(c->sv), sp<S>(c->sw), c->kx, c->ky, c->filt);
-  {
-    const S *src[6] = {sd, se, sf, sder[2], sder[3], sder[4]};
-    // the FP32-bulk form keeps p, q, r in its FP32 grids and u, v, w only as the FP32 grids its
-    // gathers read
-    const bool b32 = c->precision == 1;
-    double *dst[6] = {c->grid[GP], c->grid[GQ], c->grid[GR], c->grid[GU], c->grid[GV],
-                      c->grid[GW]};
-    float *dst32[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    if (b32)
-      for (int a = 0; a < 3; a++) {
-        dst[a] = dst[3 + a] = nullptr;
-        dst32[a] = c->b32.pgrid[a];
-        dst32[3 + a] = c->b32.grid[a];
-      }
-    PMPIC_TRY(fft_backward_t<S>(c, 6, src, dst, dst32, nullptr));
-  }
-  PMPIC_CHECK(hipGetLastError());
-  return PMPIC_OK;
+  PMPIC_TRY(vort2vel_columns<S>(c));
+  S *su = sp<S>(c->su), *sv = sp<S>(c->sv), *sw = sp<S>(c->sw);
+  const S *src[14] = {sp<S>(c->sd), sp<S>(c->se), sp<S>(c->sf), sp<S>(c->sder[2]),
+                      sp<S>(c->sder[3]), sp<S>(c->sder[4]), sbs, su, su, sw, sbs, sv, sv, sw};
+  const int op[14] = {SPEC_PLAIN, SPEC_PLAIN, SPEC_PLAIN, SPEC_PLAIN, SPEC_PLAIN,
+                      SPEC_PLAIN, SPEC_DY,    SPEC_DX,    SPEC_DY,    SPEC_DX,
+                      SPEC_DX,    SPEC_DX,    SPEC_DY,    SPEC_DY};
+  double *dst[14] = {c->grid[GP], c->grid[GQ], c->grid[GR], c->grid[GU], c->grid[GV], c->grid[GW]};
+  float *dst32[14] = {};
+  for (int f = 0; f < 8; f++) dst[6 + f] = c->gtmp[f];
+  if (c->precision == 1)
+    for (int f = 0; f < 14; f++) {
+      // the derivative grids in the first half of each FP64 scratch grid
+      dst32[f] = f < 3 ? c->b32.pgrid[f] : f < 6 ? c->b32.grid[f - 3]
+                                                 : reinterpret_cast<float *>(c->gtmp[f - 6]);
+      dst[f] = nullptr;
+    }
+  return fft_backward_t<S>(c, 14, src, dst, dst32, op);
 }
 
-int vort2vel_spectral(Ctx *c, int stage) {
-  (void)stage;
+int vort2vel_spectral(Ctx *c) {
   return c->precision == 1 ? vort2vel_spectral_t<float>(c) : vort2vel_spectral_t<double>(c);
 }
 
-// vorticity_tendency timestep_callback (vorticity_tendency.F90:147-265) after par2grid of btot
-// into grid[GB]; tendencies into grid[GDP..GDR] (plain FP64 form) or only into the FP32 grids
-// the FP32-bulk gathers read
+// vorticity_tendency timestep_callback (vorticity_tendency.F90:169-265) from the grids of
+// vort2vel; tendencies into grid[GDP..GDR] (plain FP64 form) or only into the FP32 grids the
+// FP32-bulk gathers read
 template <typename S>
-static int vorticity_tendency_spectral_t(Ctx *c) {
+static int vorticity_tendency_t(Ctx *c) {
   const Geometry &g = c->g;
   const bool b32 = c->precision == 1;  // the FP32-bulk form: FP32 grids, FP32 tendencies only
-  S *sbs = sp<S>(c->sbs);
-  {
-    const S *src[1] = {pqrb<S>(c, 3)};
-    S *dst[1] = {sbs};
-    PMPIC_TRY(fft_forward_t<S>(c, 1, src, dst));
-  }
-  {
-    // the eight spectral derivatives of vorticity_tendency.F90:155-232 (db/dy, du/dx, du/dy,
-    // dw/dx, db/dx, dv/dx, dv/dy, dw/dy), each taken while its inverse transform reads it
-    S *su = sp<S>(c->su), *sv = sp<S>(c->sv), *sw = sp<S>(c->sw);
-    const S *src[8] = {sbs, su, su, sw, sbs, sv, sv, sw};
-    const int op[8] = {SPEC_DY, SPEC_DX, SPEC_DY, SPEC_DX, SPEC_DX, SPEC_DX, SPEC_DY, SPEC_DY};
-    // the derivative grids in the transforms' precision (the FP32-bulk form's in the first
-    // half of each FP64 scratch grid)
-    double *dst[8];
-    float *dst32[8];
-    for (int f = 0; f < 8; f++) {
-      dst[f] = b32 ? nullptr : c->gtmp[f];
-      dst32[f] = b32 ? reinterpret_cast<float *>(c->gtmp[f]) : nullptr;
-    }
-    PMPIC_TRY(fft_backward_t<S>(c, 8, src, dst, dst32, op));
-  }
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
   const S *d[8];
   for (int f = 0; f < 8; f++) d[f] = reinterpret_cast<const S *>(c->gtmp[f]);
@@ -1386,10 +1007,8 @@ static int vorticity_tendency_spectral_t(Ctx *c) {
   return PMPIC_OK;
 }
 
-int vorticity_tendency_spectral(Ctx *c, int stage) {
-  (void)stage;
-  return c->precision == 1 ? vorticity_tendency_spectral_t<float>(c)
-                           : vorticity_tendency_spectral_t<double>(c);
+int vorticity_tendency_grids(Ctx *c) {
+  return c->precision == 1 ? vorticity_tendency_t<float>(c) : vorticity_tendency_t<double>(c);
 }
 
 int grid_max_reduce(Ctx *c) {
