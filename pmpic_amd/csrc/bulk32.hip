@@ -147,13 +147,13 @@ __device__ __forceinline__ void corner_nodes(const Geometry &g, int i, int j, in
   o[4] = b10 + i; o[5] = b10 + i1; o[6] = b11 + i; o[7] = b11 + i1;
 }
 
-// trilinear interpolation in the reference's order (parcel_interpolation.F90:309-321)
-__device__ __forceinline__ float interp(const float *__restrict__ G, const int32_t o[8], float ox,
-                                        float oy, float oz) {
-  const float c00 = ld(G, o[0]) * (1 - oz) + ld(G, o[4]) * oz;
-  const float c01 = ld(G, o[1]) * (1 - oz) + ld(G, o[5]) * oz;
-  const float c10 = ld(G, o[2]) * (1 - oz) + ld(G, o[6]) * oz;
-  const float c11 = ld(G, o[3]) * (1 - oz) + ld(G, o[7]) * oz;
+// trilinear interpolation of the eight corner values in the reference's order
+// (parcel_interpolation.F90:309-321)
+__device__ __forceinline__ float interp(const float c[8], float ox, float oy, float oz) {
+  const float c00 = c[0] * (1 - oz) + c[4] * oz;
+  const float c01 = c[1] * (1 - oz) + c[5] * oz;
+  const float c10 = c[2] * (1 - oz) + c[6] * oz;
+  const float c11 = c[3] * (1 - oz) + c[7] * oz;
   const float c0 = c00 * (1 - oy) + c10 * oy;
   const float c1 = c01 * (1 - oy) + c11 * oy;
   return c0 * (1 - ox) + c1 * ox;
@@ -860,10 +860,6 @@ __global__ void k32_grid_to_f64(const float *__restrict__ a, double *__restrict_
 }
 
 // ---- RK4 stage: gather the six tendencies, update, place (wrap x, y; reflect z) ----
-struct Grid32Set {
-  const float *g[6];
-};
-
 struct Scale32 {
   float idx, idy, idz;  // cells per unit length
 };
@@ -913,7 +909,8 @@ __device__ __forceinline__ void bin_lane(const Geometry &g, int32_t cell, uint32
 // the RK stage of parcel p; returns its new cell, or -1 when it left the box (status raised)
 template <int STAGE>
 __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b, int64_t cap,
-                                             const Grid32Set &gs, const Scale32 &sc3,
+                                             const float4 *__restrict__ rec,
+                                             const Scale32 &sc3,
                                              int stretch, uint8_t *__restrict__ split_flag,
                                              DevScalars *sc, uint32_t p) {
   float *F = b.f;
@@ -944,9 +941,16 @@ __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b,
   cell_ijk(g, cell, i, j, k);
   int32_t o[8];
   corner_nodes(g, i, j, k, o);
-  float kv[6];
+  float kv[6], cv[6][8];
 #pragma unroll
-  for (int f = 0; f < 6; f++) kv[f] = interp(gs.g[f], o, ox, oy, oz);
+  for (int q = 0; q < 8; q++) {  // 32-byte records: a 64-bit index, nodes times 32 may pass 2^32
+    const float4 r0 = rec[2 * (int64_t)o[q]];
+    const float2 r1 = *reinterpret_cast<const float2 *>(rec + 2 * (int64_t)o[q] + 1);
+    cv[0][q] = r0.x; cv[1][q] = r0.y; cv[2][q] = r0.z;
+    cv[3][q] = r0.w; cv[4][q] = r1.x; cv[5][q] = r1.y;
+  }
+#pragma unroll
+  for (int f = 0; f < 6; f++) kv[f] = interp(cv[f], ox, oy, oz);
   const double dtd = sc->dtm;
   const float dt = (float)dtd, dt6 = (float)(dtd / 6), dt2 = (float)(dtd / 2),
               dt3 = (float)(dtd / 3);
@@ -1021,7 +1025,8 @@ __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b,
 
 template <int STAGE>
 __global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, int64_t cap, int64_t n,
-                                                    Grid32Set gs, Scale32 sc3, int stretch,
+                                                    const float4 *__restrict__ rec, Scale32 sc3,
+                                                    int stretch,
                                                     uint8_t *__restrict__ split_flag,
                                                     DevScalars *sc, BinOut bo) {
   const int64_t p64 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1031,13 +1036,13 @@ __global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, int64_
   // with bo.on, the parcel's new cell is binned for the next stage's par2grid as k32_bin_slot
   // bins it; every lane of the wavefront then takes part, parcels past the count as empty
   if (bo.on) {
-    const int32_t nc = valid ? rk_update<STAGE>(g, b, cap, gs, sc3, stretch, split_flag, sc, p)
+    const int32_t nc = valid ? rk_update<STAGE>(g, b, cap, rec, sc3, stretch, split_flag, sc, p)
                              : -1;
     bin_lane(g, nc, p, bo, sc);
     return;
   }
   if (!valid) return;
-  rk_update<STAGE>(g, b, cap, gs, sc3, stretch, split_flag, sc, p);
+  rk_update<STAGE>(g, b, cap, rec, sc3, stretch, split_flag, sc, p);
 }
 
 // ---- splitting (parcel_splitting.F90:76-131, then the haloswap's wrap and reflection) ----
@@ -1453,7 +1458,7 @@ int b32_alloc(Ctx *c) {
   // count reads 0 for them, as in the FP64 form's arrays, which are cleared at allocation too
   PMPIC_CHECK(hipMemset(b.f, 0, sizeof(float) * (size_t)NF32 * (size_t)c->cap));
   PMPIC_CHECK(hipMemset(b.tag, 0, sizeof(double) * (size_t)c->cap));
-  for (int i = 0; i < 6; i++) PMPIC_TRY(dalloc32(&b.grid[i], c->gsz));
+  for (int i = 0; i < 3; i++) PMPIC_TRY(dalloc32(&b.grid[i], c->gsz));
   for (int i = 0; i < 12; i++) PMPIC_TRY(dalloc32(&b.mgrid[i], c->gsz));
   PMPIC_TRY(dalloc32(&b.mtouch, c->gsz));
   PMPIC_TRY(dalloc32(&b.dirty, c->ncell / TILE32 + 1));
@@ -1504,7 +1509,7 @@ void b32_free(Ctx *c) {
   hipFree(b.cell);
   hipFree(b.cello);
   hipFree(b.tag);
-  for (int i = 0; i < 6; i++) hipFree(b.grid[i]);
+  for (int i = 0; i < 3; i++) hipFree(b.grid[i]);
   for (int i = 0; i < 12; i++) hipFree(b.mgrid[i]);
   hipFree(b.mtouch);
   hipFree(b.dirty);
@@ -1684,8 +1689,7 @@ int b32_par2grid(Ctx *c) {
 int b32_rk_stage(Ctx *c, int stage, int stretch) {
   const int64_t n = c->n;
   if (n == 0) return PMPIC_OK;
-  Grid32Set gs = {{c->b32.grid[0], c->b32.grid[1], c->b32.grid[2], c->b32.grid[3],
-                   c->b32.grid[4], c->b32.grid[5]}};
+  PMPIC_TRY(records_current(c));
   const Scale32 s3 = scale_of(c->g);
   Bulk32 &b = c->b32;
   b.p2g_reuse = false;
@@ -1703,20 +1707,20 @@ int b32_rk_stage(Ctx *c, int stage, int stretch) {
   }
   switch (stage) {
     case 1:
-      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<1>, gb, tb, 0, c->g, c->b32, c->cap, n, gs,
-                             s3, stretch, c->flag, c->dsc, bo));
+      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<1>, gb, tb, 0, c->g, c->b32, c->cap, n,
+                             c->rec32, s3, stretch, c->flag, c->dsc, bo));
       break;
     case 2:
-      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<2>, gb, tb, 0, c->g, c->b32, c->cap, n, gs,
-                             s3, stretch, c->flag, c->dsc, bo));
+      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<2>, gb, tb, 0, c->g, c->b32, c->cap, n,
+                             c->rec32, s3, stretch, c->flag, c->dsc, bo));
       break;
     case 3:
-      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<3>, gb, tb, 0, c->g, c->b32, c->cap, n, gs,
-                             s3, stretch, c->flag, c->dsc, bo));
+      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<3>, gb, tb, 0, c->g, c->b32, c->cap, n,
+                             c->rec32, s3, stretch, c->flag, c->dsc, bo));
       break;
     default:
-      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<4>, gb, tb, 0, c->g, c->b32, c->cap, n, gs,
-                             s3, stretch, c->flag, c->dsc, bo));
+      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<4>, gb, tb, 0, c->g, c->b32, c->cap, n,
+                             c->rec32, s3, stretch, c->flag, c->dsc, bo));
       break;
   }
   PMPIC_CHECK(hipGetLastError());

@@ -230,6 +230,7 @@ int free_all(Ctx *c) {
   hipFree(c->cell_count); hipFree(c->cell_start); hipFree(c->partial); hipFree(c->partial2);
   hipFree(c->npercell); hipFree(c->cellflag);
   for (int g = 0; g < NGRIDS; g++) hipFree(c->grid[g]);
+  hipFree(c->rec); hipFree(c->rec32);
   for (int g = 0; g < 8; g++) hipFree(c->gtmp[g]);
   for (int g = 0; g < 6; g++) hipFree(c->kres[g]);
   double *sp[] = {c->spool, c->sd, c->se, c->sf, c->su, c->sv, c->sw, c->sbs};
@@ -305,7 +306,9 @@ int create(const pmpic_config *cf, Ctx *c) {
   if (c->precision == 1) PMPIC_TRY(dalloc(&c->partial2, pdoubles));
   PMPIC_TRY(dalloc(&c->npercell, c->ncell));
   PMPIC_TRY(dalloc(&c->cellflag, c->ncell));
-  for (int i = 0; i < NGRIDS; i++) PMPIC_TRY(dalloc(&c->grid[i], c->gsz));
+  for (int i = 0; i < GDP; i++) PMPIC_TRY(dalloc(&c->grid[i], c->gsz));
+  if (c->precision == 1) PMPIC_TRY(dalloc(&c->rec32, 2 * c->gsz));
+  else PMPIC_TRY(dalloc(&c->rec, 3 * c->gsz));
   for (int i = 0; i < 8; i++) PMPIC_TRY(dalloc(&c->gtmp[i], c->gsz));
   for (int i = 0; i < 6; i++) PMPIC_TRY(dalloc(&c->kres[i], c->gsz));
   double **sp[] = {&c->sd, &c->se, &c->sf, &c->su, &c->sv, &c->sw, &c->sbs};
@@ -830,16 +833,16 @@ int pmpic_get_grid(pmpic_ctx *ctx, int32_t id, double *grid) {
   if (!ctx || !grid || id < 0 || id >= NGRIDS) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
   std::vector<double> h;
-  const bool vel = id >= GU && id <= GW, tend = id >= GDP && id <= GDR;
-  if (c->precision == 1 && (vel || tend)) {
-    // the FP32-bulk form keeps u, v, w and the tendencies only in the FP32 grids its gathers
-    // read (b32.grid: U, V, W, DP, DQ, DR)
+  if (c->precision == 1 && id <= GW) {
+    // the FP32-bulk form keeps u, v, w only in FP32
     std::vector<float> hf(c->gsz);
-    const float *src32 = c->b32.grid[vel ? id - GU : 3 + (id - GDP)];
-    PMPIC_CHECK(hipMemcpyAsync(hf.data(), src32, sizeof(float) * c->gsz,
+    PMPIC_CHECK(hipMemcpyAsync(hf.data(), c->b32.grid[id - GU], sizeof(float) * c->gsz,
                                hipMemcpyDeviceToHost, c->stream));
     PMPIC_CHECK(hipStreamSynchronize(c->stream));
     h.assign(hf.begin(), hf.end());
+  } else if (id >= GDP) {
+    PMPIC_TRY(export_tendency(c, id - GDP, c->kres[0]));
+    PMPIC_TRY(download(c, h, c->kres[0], c->gsz));
   } else {
     if (c->precision == 1) PMPIC_TRY(b32_export_grid(c, id));
     PMPIC_TRY(download(c, h, c->grid[id], c->gsz));

@@ -46,7 +46,7 @@ struct Bulk32 {
   int32_t *cell;     // cap: cell holding the parcel
   int32_t *cello;    // cap: cell of the RK4 origin
   double *tag;       // cap
-  float *grid[6];    // gathered grids U, V, W, DP, DQ, DR [nzn][ny][nx]
+  float *grid[3];    // U, V, W [nzn][ny][nx]
   float *mgrid[12];  // mixing: kept vol, b, h, p, q, r (0..5), residuals (6..11)
   uint8_t *mtouch;   // mixing, per node: a residual grid is not zero there
   // cell binning: slot[c * capc + rank] lists the parcels of cell c while rank < capc; a cell
@@ -159,7 +159,15 @@ struct Ctx {
   // grids (interior [nzn][ny][nx])
   int64_t gsz, ssz, csz;              // grid; spectral (planes); complex transform intermediate
   int64_t bsz;                        // spectral (tiles)
-  double *grid[NGRIDS];
+  double *grid[NGRIDS];               // GDP, GDQ, GDR null: those are in the node records
+  // Node records, the six values an RK stage interpolates at a node side by side: U, V, W, DP, DQ,
+  // DR as three double2, or in the FP32-bulk form two float4 (the last two floats unused).  A
+  // parcel's eight corners are then 24 (16) vector loads from eight places instead of 48 from as
+  // many: RK stage 4 of 67 M parcels that have moved a few cells 2.59 -> 1.59 ms (FP32-bulk), stage
+  // 2 of 57 M 3.49 -> 2.93 ms (FP64).  Written by vorticity_tendency; rec_stale: vort2vel has made newer velocities since.
+  double2 *rec;
+  float4 *rec32;
+  bool rec_stale;
   double *gtmp[8];                    // vorticity tendency derivative grids (made by vort2vel)
   double *kres[6];                    // mixing residual grids
   // spectral, in tiles (the standalone operators use the sder arrays as planes)
@@ -360,6 +368,8 @@ int vort2vel_columns(Ctx *c);
 int spectral_setup(Ctx *c);
 int vort2vel_spectral(Ctx *c);
 int vorticity_tendency_grids(Ctx *c);
+int records_current(Ctx *c);                           // refreshes the records' velocities if stale
+int export_tendency(Ctx *c, int f, double *grid);      // DP, DQ, DR (f = 0..2) out of the records
 int op_diffx(Ctx *c, const double *in, double *out);
 int op_diffy(Ctx *c, const double *in, double *out);
 int op_filter(Ctx *c, const double *in, double *out);

@@ -51,10 +51,6 @@ __device__ __forceinline__ void block_rank(bool pred, int &rank, int &total, int
   total = tot;
 }
 
-struct GridSet {
-  const double *g[6];
-};
-
 // haloswap direction of a parcel (haloswap.F90:296-437); 0 = stays
 __device__ __forceinline__ int direction(const Geometry &g, double x, double y) {
   const double xmin = g.hs_xmin, xmax = g.hs_xmax, ymin = g.hs_ymin, ymax = g.hs_ymax;
@@ -89,7 +85,8 @@ __device__ __forceinline__ void write_dir_counts(int dir, bool active, int32_t *
 // vorticity and the stage-4 tendencies of the same parcel).
 template <int STAGE>
 __global__ void __launch_bounds__(TPB) k_rk_stage(Geometry g, double *__restrict__ par, int64_t cap,
-                                                  int64_t n, GridSet gs, int stretch,
+                                                  int64_t n, const double2 *__restrict__ rec,
+                                                  int stretch,
                                                   DevScalars *sc,
                                                   uint8_t *__restrict__ flag,
                                                   int32_t *__restrict__ blk, int64_t nblk) {
@@ -124,21 +121,28 @@ __global__ void __launch_bounds__(TPB) k_rk_stage(Geometry g, double *__restrict
     } else {
       const int i1 = (i0 + 1 == g.nx) ? 0 : i0 + 1;
       const int j1 = (j0 + 1 == g.ny) ? 0 : j0 + 1;
-      const int64_t o000 = gidx(g, k0, j0, i0), o001 = gidx(g, k0, j0, i1);
-      const int64_t o010 = gidx(g, k0, j1, i0), o011 = gidx(g, k0, j1, i1);
-      const int64_t o100 = gidx(g, k0 + 1, j0, i0), o101 = gidx(g, k0 + 1, j0, i1);
-      const int64_t o110 = gidx(g, k0 + 1, j1, i0), o111 = gidx(g, k0 + 1, j1, i1);
+      const int64_t o[8] = {gidx(g, k0, j0, i0),     gidx(g, k0, j0, i1),
+                            gidx(g, k0, j1, i0),     gidx(g, k0, j1, i1),
+                            gidx(g, k0 + 1, j0, i0), gidx(g, k0 + 1, j0, i1),
+                            gidx(g, k0 + 1, j1, i0), gidx(g, k0 + 1, j1, i1)};
       double kv[6];
 #pragma unroll
-      for (int f = 0; f < 6; f++) {
-        const double *G = gs.g[f];
-        const double c00 = G[o000] * (1 - delz) + G[o100] * delz;
-        const double c01 = G[o001] * (1 - delz) + G[o101] * delz;
-        const double c10 = G[o010] * (1 - delz) + G[o110] * delz;
-        const double c11 = G[o011] * (1 - delz) + G[o111] * delz;
-        const double c0 = c00 * (1 - dely) + c10 * dely;
-        const double c1 = c01 * (1 - dely) + c11 * dely;
-        kv[f] = c0 * (1 - delx) + c1 * delx;
+      for (int h = 0; h < 3; h++) {  // two values of every corner's record at a time
+        double2 G[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) G[q] = rec[3 * o[q] + h];
+        auto interp = [&](double a0, double a1, double a2, double a3, double a4, double a5,
+                          double a6, double a7) {
+          const double c00 = a0 * (1 - delz) + a4 * delz;
+          const double c01 = a1 * (1 - delz) + a5 * delz;
+          const double c10 = a2 * (1 - delz) + a6 * delz;
+          const double c11 = a3 * (1 - delz) + a7 * delz;
+          const double c0 = c00 * (1 - dely) + c10 * dely;
+          const double c1 = c01 * (1 - dely) + c11 * dely;
+          return c0 * (1 - delx) + c1 * delx;
+        };
+        kv[2 * h] = interp(G[0].x, G[1].x, G[2].x, G[3].x, G[4].x, G[5].x, G[6].x, G[7].x);
+        kv[2 * h + 1] = interp(G[0].y, G[1].y, G[2].y, G[3].y, G[4].y, G[5].y, G[6].y, G[7].y);
       }
       const double dt = sc->dtm;
       const double dt6 = dt / 6, dt2 = dt / 2, dt3 = dt / 3;
@@ -627,23 +631,23 @@ static int haloswap_permute(Ctx *c, int64_t n, int64_t nblk) {
 int rk_stage_update(Ctx *c, int stage, int64_t n, int stretch) {
   const int64_t nblk = cdiv(n > 0 ? n : 1, TPB);
   if (nblk > c->nblk_max) return PMPIC_ERR_ARG;
-  GridSet gs = {{c->grid[GU], c->grid[GV], c->grid[GW], c->grid[GDP], c->grid[GDQ], c->grid[GDR]}};
+  PMPIC_TRY(records_current(c));
   switch (stage) {
     case 1:
       PMPIC_TRY(launch_timed(c, T_RK, k_rk_stage<1>, dim3(nblk), dim3(TPB), 0, c->g, c->par,
-                             c->cap, n, gs, stretch, c->dsc, c->flag, c->blk, nblk));
+                             c->cap, n, c->rec, stretch, c->dsc, c->flag, c->blk, nblk));
       break;
     case 2:
       PMPIC_TRY(launch_timed(c, T_RK, k_rk_stage<2>, dim3(nblk), dim3(TPB), 0, c->g, c->par,
-                             c->cap, n, gs, stretch, c->dsc, c->flag, c->blk, nblk));
+                             c->cap, n, c->rec, stretch, c->dsc, c->flag, c->blk, nblk));
       break;
     case 3:
       PMPIC_TRY(launch_timed(c, T_RK, k_rk_stage<3>, dim3(nblk), dim3(TPB), 0, c->g, c->par,
-                             c->cap, n, gs, stretch, c->dsc, c->flag, c->blk, nblk));
+                             c->cap, n, c->rec, stretch, c->dsc, c->flag, c->blk, nblk));
       break;
     default:
       PMPIC_TRY(launch_timed(c, T_RK, k_rk_stage<4>, dim3(nblk), dim3(TPB), 0, c->g, c->par,
-                             c->cap, n, gs, stretch, c->dsc, c->flag, c->blk, nblk));
+                             c->cap, n, c->rec, stretch, c->dsc, c->flag, c->blk, nblk));
       break;
   }
   PMPIC_CHECK(hipGetLastError());

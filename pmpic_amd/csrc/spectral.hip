@@ -677,19 +677,32 @@ __global__ void __launch_bounds__(64) k_diffz_qn(Geometry g, ColField cf,
     if (q * L + i < NZ) o[(int64_t)(q * L + i) * plane] = F[i];
 }
 
-// vorticity_tendency.F90:169-265, physical interior, accumulation order as written
-// T: the type of the input grids (FP64, or FP32 in the FP32-bulk form, widened exactly); the
-// products are formed in FP64 in both forms
-template <typename T>
+// a node's record (common.h)
+__device__ __forceinline__ void put_record(double2 *rec, int64_t t, double u, double v, double w,
+                                           double dp, double dq, double dr) {
+  rec[3 * t] = make_double2(u, v);
+  rec[3 * t + 1] = make_double2(w, dp);
+  rec[3 * t + 2] = make_double2(dq, dr);
+}
+__device__ __forceinline__ void put_record(float4 *rec, int64_t t, float u, float v, float w,
+                                           double dp, double dq, double dr) {
+  rec[2 * t] = make_float4(u, v, w, (float)dp);
+  rec[2 * t + 1] = make_float4((float)dq, (float)dr, 0.f, 0.f);
+}
+
+// vorticity_tendency.F90:169-265, physical interior, accumulation order as written, and the node
+// records of the RK stage's gathers.
+// T: the type of the grids (FP64, or FP32 in the FP32-bulk form, widened exactly); the products
+// are formed in FP64 in both forms.  Bound by memory (14 grids read, a record written).
+template <typename T, typename REC>
 __global__ void k_tendency(int64_t nnode, const T *__restrict__ P, const T *__restrict__ Q,
                            const T *__restrict__ R, const T *__restrict__ dbdy,
                            const T *__restrict__ dudx, const T *__restrict__ dudy,
                            const T *__restrict__ dwdx, const T *__restrict__ dbdx,
                            const T *__restrict__ dvdx, const T *__restrict__ dvdy,
-                           const T *__restrict__ dwdy, double *__restrict__ DP,
-                           double *__restrict__ DQ, double *__restrict__ DR,
-                           float *__restrict__ DP32, float *__restrict__ DQ32,
-                           float *__restrict__ DR32) {
+                           const T *__restrict__ dwdy, const T *__restrict__ U,
+                           const T *__restrict__ V, const T *__restrict__ W,
+                           REC *__restrict__ rec) {
   int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= nnode) return;
   const double p = P[q], qq = Q[q], r = R[q];
@@ -705,16 +718,33 @@ __global__ void k_tendency(int64_t nnode, const T *__restrict__ P, const T *__re
   dr = dr + qq * (double)dwdy[q];
   dr = dr + r * (-(double)dudx[q]);
   dr = dr + r * (-(double)dvdy[q]);
-  if (DP) {
-    DP[q] = dp;
-    DQ[q] = dq;
-    DR[q] = dr;
-  }
-  if (DP32) {
-    DP32[q] = (float)dp;
-    DQ32[q] = (float)dq;
-    DR32[q] = (float)dr;
-  }
+  put_record(rec, q, U[q], V[q], W[q], dp, dq, dr);
+}
+
+// newer velocities into the records (vort2vel called again without vorticity_tendency)
+__global__ void k_record_velocity(int64_t nnode, const double *__restrict__ U,
+                                  const double *__restrict__ V, const double *__restrict__ W,
+                                  double2 *__restrict__ rec) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= nnode) return;
+  rec[3 * q] = make_double2(U[q], V[q]);
+  rec[3 * q + 1].x = W[q];
+}
+__global__ void k_record_velocity32(int64_t nnode, const float *__restrict__ U,
+                                    const float *__restrict__ V, const float *__restrict__ W,
+                                    float4 *__restrict__ rec) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= nnode) return;
+  rec[2 * q] = make_float4(U[q], V[q], W[q], rec[2 * q].w);
+}
+
+// a tendency grid out of the records, for an export
+__global__ void k_record_tendency(int64_t nnode, int f, const double2 *__restrict__ rec,
+                                  const float4 *__restrict__ rec32, double *__restrict__ out) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= nnode) return;
+  if (rec) out[q] = f == 0 ? rec[3 * q + 1].y : f == 1 ? rec[3 * q + 2].x : rec[3 * q + 2].y;
+  else out[q] = f == 0 ? rec32[2 * q].w : f == 1 ? rec32[2 * q + 1].x : rec32[2 * q + 1].y;
 }
 
 // maxima of u^2, v^2, w^2 and p^2+q^2+r^2 over the interior (vort2vel.F90:331-337,
@@ -981,6 +1011,7 @@ static int vort2vel_spectral_t(Ctx *c) {
                                                  : reinterpret_cast<float *>(c->gtmp[f - 6]);
       dst[f] = nullptr;
     }
+  c->rec_stale = true;
   return fft_backward_t<S>(c, 14, src, dst, dst32, op);
 }
 
@@ -989,26 +1020,50 @@ int vort2vel_spectral(Ctx *c) {
 }
 
 // vorticity_tendency timestep_callback (vorticity_tendency.F90:169-265) from the grids of
-// vort2vel; tendencies into grid[GDP..GDR] (plain FP64 form) or only into the FP32 grids the
-// FP32-bulk gathers read
-template <typename S>
-static int vorticity_tendency_t(Ctx *c) {
+// vort2vel: the tendencies, with the velocities, into the node records
+int vorticity_tendency_grids(Ctx *c) {
   const Geometry &g = c->g;
-  const bool b32 = c->precision == 1;  // the FP32-bulk form: FP32 grids, FP32 tendencies only
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
-  const S *d[8];
-  for (int f = 0; f < 8; f++) d[f] = reinterpret_cast<const S *>(c->gtmp[f]);
-  hipLaunchKernelGGL(k_tendency<S>, dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, nnode,
-                     pqrb<S>(c, 0), pqrb<S>(c, 1), pqrb<S>(c, 2), d[0], d[1], d[2], d[3], d[4],
-                     d[5], d[6], d[7], b32 ? nullptr : c->grid[GDP], b32 ? nullptr : c->grid[GDQ],
-                     b32 ? nullptr : c->grid[GDR], b32 ? c->b32.grid[3] : nullptr,
-                     b32 ? c->b32.grid[4] : nullptr, b32 ? c->b32.grid[5] : nullptr);
+  const dim3 gb(cdiv(nnode, TPB)), tb(TPB);
+  if (c->precision == 1) {
+    const Bulk32 &b = c->b32;
+    const float *d[8];
+    for (int f = 0; f < 8; f++) d[f] = reinterpret_cast<const float *>(c->gtmp[f]);
+    hipLaunchKernelGGL((k_tendency<float, float4>), gb, tb, 0, c->stream, nnode, b.pgrid[0],
+                       b.pgrid[1], b.pgrid[2], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
+                       b.grid[0], b.grid[1], b.grid[2], c->rec32);
+  } else {
+    double *const *d = c->gtmp;
+    hipLaunchKernelGGL((k_tendency<double, double2>), gb, tb, 0, c->stream, nnode, c->grid[GP],
+                       c->grid[GQ], c->grid[GR], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
+                       c->grid[GU], c->grid[GV], c->grid[GW], c->rec);
+  }
+  c->rec_stale = false;
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
 
-int vorticity_tendency_grids(Ctx *c) {
-  return c->precision == 1 ? vorticity_tendency_t<float>(c) : vorticity_tendency_t<double>(c);
+int records_current(Ctx *c) {
+  if (!c->rec_stale) return PMPIC_OK;
+  const int64_t nnode = c->gsz;
+  const dim3 gb(cdiv(nnode, TPB)), tb(TPB);
+  if (c->precision == 1)
+    hipLaunchKernelGGL(k_record_velocity32, gb, tb, 0, c->stream, nnode, c->b32.grid[0],
+                       c->b32.grid[1], c->b32.grid[2], c->rec32);
+  else
+    hipLaunchKernelGGL(k_record_velocity, gb, tb, 0, c->stream, nnode, c->grid[GU], c->grid[GV],
+                       c->grid[GW], c->rec);
+  c->rec_stale = false;
+  PMPIC_CHECK(hipGetLastError());
+  return PMPIC_OK;
+}
+
+int export_tendency(Ctx *c, int f, double *grid) {
+  const int64_t nnode = c->gsz;
+  hipLaunchKernelGGL(k_record_tendency, dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, nnode, f,
+                     c->rec, c->rec32, grid);
+  PMPIC_CHECK(hipGetLastError());
+  return PMPIC_OK;
 }
 
 int grid_max_reduce(Ctx *c) {
