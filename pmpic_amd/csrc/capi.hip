@@ -5,6 +5,7 @@
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
+#include <algorithm>
 #include <array>
 #include <mutex>
 #include <thread>
@@ -46,13 +47,10 @@ int timing_harvest(Ctx *c) {
   return PMPIC_OK;
 }
 
-// the device staging buffer of host-array transfers, allocated at its first use: a parcel field
-// or a parcel array followed by a grid (max(cap, gsz) + max(gsz, ssz) doubles)
+// the device staging buffer of parcel array transfers, allocated at its first use
 int ensure_fbuf(Ctx *c) {
   if (c->fbuf) return PMPIC_OK;
-  const int64_t a = c->cap > c->gsz ? c->cap : c->gsz;
-  const int64_t b = c->gsz > c->ssz ? c->gsz : c->ssz;
-  PMPIC_CHECK(hipMalloc((void **)&c->fbuf, sizeof(double) * (size_t)(a + b)));
+  PMPIC_CHECK(hipMalloc((void **)&c->fbuf, sizeof(double) * (size_t)c->cap));
   return PMPIC_OK;
 }
 
@@ -124,69 +122,26 @@ void make_geometry(const pmpic_config *cf, Geometry &g, std::vector<double> &coo
   g.lz_cfl = (double)g.nzn * g.dz;
 }
 
-// reference grid layout (z fastest, x/y halo 2) <-> device interior [k][j][i]
-void grid_to_device_layout(const Geometry &g, const double *ref, std::vector<double> &dev) {
-  const int nyh = g.ny + 4, nzn = g.nzn;
-  dev.resize((size_t)nzn * g.ny * g.nx);
-  for (int k = 0; k < nzn; k++)
-    for (int j = 0; j < g.ny; j++)
-      for (int i = 0; i < g.nx; i++)
-        dev[((size_t)k * g.ny + j) * g.nx + i] = ref[((size_t)(i + 2) * nyh + (j + 2)) * nzn + k];
-}
-
-void grid_from_device_layout(const Geometry &g, const std::vector<double> &dev, double *ref) {
-  const int nxh = g.nx + 4, nyh = g.ny + 4, nzn = g.nzn;
-  for (int ih = 0; ih < nxh; ih++) {
-    int i = ((ih - 2) % g.nx + g.nx) % g.nx;
-    for (int jh = 0; jh < nyh; jh++) {
-      int j = ((jh - 2) % g.ny + g.ny) % g.ny;
-      for (int k = 0; k < nzn; k++)
-        ref[((size_t)ih * nyh + jh) * nzn + k] = dev[((size_t)k * g.ny + j) * g.nx + i];
-    }
-  }
-}
-
-void spec_to_device_layout(const Geometry &g, const double *ref, std::vector<double> &dev) {
-  dev.resize((size_t)g.nzn * g.sy * g.sx);
-  for (int k = 0; k < g.nzn; k++)
-    for (int jj = 0; jj < g.sy; jj++)
-      for (int ii = 0; ii < g.sx; ii++)
-        dev[((size_t)k * g.sy + jj) * g.sx + ii] = ref[((size_t)ii * g.sy + jj) * g.nzn + k];
-}
-
-void spec_from_device_layout(const Geometry &g, const std::vector<double> &dev, double *ref) {
-  for (int k = 0; k < g.nzn; k++)
-    for (int jj = 0; jj < g.sy; jj++)
-      for (int ii = 0; ii < g.sx; ii++)
-        ref[((size_t)ii * g.sy + jj) * g.nzn + k] = dev[((size_t)k * g.sy + jj) * g.sx + ii];
-}
-
-// the same between the reference's layout and the spectral tiles (common.h)
-void spec_to_tiles(const Geometry &g, const double *ref, std::vector<double> &dev) {
-  dev.assign((size_t)spec_tiles(g) * g.nzn * 64, 0.0);
-  for (int ii = 0; ii < g.sx; ii++)
-    for (int jj = 0; jj < g.sy; jj++) {
-      const double *r = ref + ((size_t)ii * g.sy + jj) * g.nzn;
-      double *d = dev.data() + spec_at(g.nzn, g.sx / 2, 0, jj / 2, ii / 2) + 2 * (jj & 1) + (ii & 1);
-      for (int k = 0; k < g.nzn; k++) d[(size_t)k * 64] = r[k];
-    }
-}
-
-void spec_from_tiles(const Geometry &g, const std::vector<double> &dev, double *ref) {
-  for (int ii = 0; ii < g.sx; ii++)
-    for (int jj = 0; jj < g.sy; jj++) {
-      double *r = ref + ((size_t)ii * g.sy + jj) * g.nzn;
-      const double *d =
-          dev.data() + spec_at(g.nzn, g.sx / 2, 0, jj / 2, ii / 2) + 2 * (jj & 1) + (ii & 1);
-      for (int k = 0; k < g.nzn; k++) r[k] = d[(size_t)k * 64];
-    }
-}
-
 void col_to_device_layout(const Geometry &g, const double *ref, std::vector<double> &dev) {
   dev.resize((size_t)g.sy * g.sx);
   for (int jj = 0; jj < g.sy; jj++)
     for (int ii = 0; ii < g.sx; ii++) dev[(size_t)jj * g.sx + ii] = ref[(size_t)ii * g.sy + jj];
 }
+
+// host array -> device (in stream order; the caller's stream synchronisation ends its use)
+int put_host(Ctx *c, double *dst, const double *host, int64_t n) {
+  PMPIC_CHECK(hipMemcpyAsync(dst, host, sizeof(double) * (size_t)n, hipMemcpyHostToDevice,
+                             c->stream));
+  return PMPIC_OK;
+}
+// device -> host array, complete on return
+int get_host(Ctx *c, double *host, const double *src, int64_t n) {
+  PMPIC_CHECK(hipMemcpyAsync(host, src, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost,
+                             c->stream));
+  PMPIC_CHECK(hipStreamSynchronize(c->stream));
+  return PMPIC_OK;
+}
+int64_t ref_grid_size(const Geometry &g) { return (int64_t)g.nzn * (g.ny + 4) * (g.nx + 4); }
 
 int upload(Ctx *c, double *dst, const std::vector<double> &h) {
   PMPIC_CHECK(hipMemcpyAsync(dst, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice,
@@ -232,7 +187,7 @@ int free_all(Ctx *c) {
   for (int g = 0; g < NGRIDS; g++) hipFree(c->grid[g]);
   hipFree(c->rec); hipFree(c->rec32);
   for (int g = 0; g < 8; g++) hipFree(c->gtmp[g]);
-  for (int g = 0; g < 6; g++) hipFree(c->kres[g]);
+  hipFree(c->kres[0]);
   double *sp[] = {c->spool, c->sd, c->se, c->sf, c->su, c->sv, c->sw, c->sbs};
   for (double *p : sp) hipFree(p);
   for (int g = 1; g < 6; g++) hipFree(c->sder[g]);
@@ -310,7 +265,10 @@ int create(const pmpic_config *cf, Ctx *c) {
   if (c->precision == 1) PMPIC_TRY(dalloc(&c->rec32, 2 * c->gsz));
   else PMPIC_TRY(dalloc(&c->rec, 3 * c->gsz));
   for (int i = 0; i < 8; i++) PMPIC_TRY(dalloc(&c->gtmp[i], c->gsz));
-  for (int i = 0; i < 6; i++) PMPIC_TRY(dalloc(&c->kres[i], c->gsz));
+  PMPIC_TRY(dalloc(&c->kres[0],
+                   c->gsz + std::max({5 * c->gsz, ref_grid_size(g), c->ssz})));
+  for (int i = 1; i < 6; i++) c->kres[i] = c->kres[0] + i * c->gsz;
+  c->refbuf = c->kres[1];
   double **sp[] = {&c->sd, &c->se, &c->sf, &c->su, &c->sv, &c->sw, &c->sbs};
   for (double **p : sp) PMPIC_TRY(dalloc(p, c->bsz));
   for (int i = 1; i < 6; i++) PMPIC_TRY(dalloc(&c->sder[i], c->bsz));
@@ -800,55 +758,40 @@ int pmpic_par2grid(pmpic_ctx *ctx, const double *var, double *grid) {
   if (!ctx || !var || !grid || ctx->c.precision != 0) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
   PMPIC_TRY(ensure_fbuf(c));
-  if (c->n > 0)
-    PMPIC_CHECK(hipMemcpyAsync(c->fbuf, var, sizeof(double) * c->n, hipMemcpyHostToDevice,
-                               c->stream));
-  double *dg = c->fbuf + (c->cap > c->gsz ? c->cap : c->gsz);
-  PMPIC_TRY(par2grid_single(c, c->n, c->fbuf, dg));
+  if (c->n > 0) PMPIC_TRY(put_host(c, c->fbuf, var, c->n));
+  PMPIC_TRY(par2grid_single(c, c->n, c->fbuf, c->kres[0]));
+  PMPIC_TRY(grid_to_ref(c, c->kres[0], 1, c->refbuf));
   PMPIC_TRY(take_status(c));
-  std::vector<double> h;
-  PMPIC_TRY(download(c, h, dg, c->gsz));
-  grid_from_device_layout(c->g, h, grid);
-  return PMPIC_OK;
+  return get_host(c, grid, c->refbuf, ref_grid_size(c->g));
 }
 
 int pmpic_grid2par(pmpic_ctx *ctx, const double *grid, double *var) {
   if (!ctx || !var || !grid || ctx->c.precision != 0) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
   PMPIC_TRY(ensure_fbuf(c));
-  std::vector<double> h;
-  grid_to_device_layout(c->g, grid, h);
-  double *dg = c->fbuf + (c->cap > c->gsz ? c->cap : c->gsz);
-  PMPIC_TRY(upload(c, dg, h));
-  PMPIC_TRY(grid2par_single(c, c->n, dg, c->fbuf));
+  PMPIC_TRY(put_host(c, c->refbuf, grid, ref_grid_size(c->g)));
+  PMPIC_TRY(ref_to_grid(c, c->refbuf, c->kres[0]));
+  PMPIC_TRY(grid2par_single(c, c->n, c->kres[0], c->fbuf));
   PMPIC_TRY(take_status(c));
-  if (c->n > 0)
-    PMPIC_CHECK(hipMemcpyAsync(var, c->fbuf, sizeof(double) * c->n, hipMemcpyDeviceToHost,
-                               c->stream));
-  PMPIC_CHECK(hipStreamSynchronize(c->stream));
-  return PMPIC_OK;
+  return c->n > 0 ? get_host(c, var, c->fbuf, c->n) : PMPIC_OK;
 }
 
 int pmpic_get_grid(pmpic_ctx *ctx, int32_t id, double *grid) {
   if (!ctx || !grid || id < 0 || id >= NGRIDS) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
-  std::vector<double> h;
-  if (c->precision == 1 && id <= GW) {
+  const bool b32 = c->precision == 1;
+  if (b32 && id <= GW) {
     // the FP32-bulk form keeps u, v, w only in FP32
-    std::vector<float> hf(c->gsz);
-    PMPIC_CHECK(hipMemcpyAsync(hf.data(), c->b32.grid[id - GU], sizeof(float) * c->gsz,
-                               hipMemcpyDeviceToHost, c->stream));
-    PMPIC_CHECK(hipStreamSynchronize(c->stream));
-    h.assign(hf.begin(), hf.end());
+    PMPIC_TRY(grid_to_ref(c, c->b32.grid[id - GU], 1, c->refbuf));
   } else if (id >= GDP) {
-    PMPIC_TRY(export_tendency(c, id - GDP, c->kres[0]));
-    PMPIC_TRY(download(c, h, c->kres[0], c->gsz));
+    // dp, dq, dr are the last three of a node record's values
+    if (b32) PMPIC_TRY(grid_to_ref(c, (const float *)c->rec32 + 3 + (id - GDP), 8, c->refbuf));
+    else PMPIC_TRY(grid_to_ref(c, (const double *)c->rec + 3 + (id - GDP), 6, c->refbuf));
   } else {
-    if (c->precision == 1) PMPIC_TRY(b32_export_grid(c, id));
-    PMPIC_TRY(download(c, h, c->grid[id], c->gsz));
+    if (b32) PMPIC_TRY(b32_export_grid(c, id));
+    PMPIC_TRY(grid_to_ref(c, c->grid[id], 1, c->refbuf));
   }
-  grid_from_device_layout(c->g, h, grid);
-  return PMPIC_OK;
+  return get_host(c, grid, c->refbuf, ref_grid_size(c->g));
 }
 
 int pmpic_writebinary_grids(pmpic_ctx *ctx) {
@@ -863,57 +806,43 @@ int pmpic_writebinary_grids(pmpic_ctx *ctx) {
 int pmpic_get_spectral(pmpic_ctx *ctx, int32_t id, double *spec) {
   if (!ctx || !spec || id < 0 || id > 2) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
-  double *src = id == 0 ? c->su : id == 1 ? c->sv : c->sw;
-  std::vector<double> h;
-  if (c->precision == 1) {
-    // the FP32-bulk form's spectral arrays hold FP32 values; widened exactly
-    std::vector<float> h32((size_t)c->bsz);
-    PMPIC_CHECK(hipMemcpyAsync(h32.data(), src, sizeof(float) * (size_t)c->bsz,
-                               hipMemcpyDeviceToHost, c->stream));
-    PMPIC_CHECK(hipStreamSynchronize(c->stream));
-    h.assign(h32.begin(), h32.end());
-  } else {
-    PMPIC_TRY(download(c, h, src, c->bsz));
-  }
-  spec_from_tiles(c->g, h, spec);
-  return PMPIC_OK;
+  const double *src = id == 0 ? c->su : id == 1 ? c->sv : c->sw;
+  // the FP32-bulk form's spectral arrays hold FP32 values; widened exactly
+  if (c->precision == 1) PMPIC_TRY(tiles_to_ref(c, reinterpret_cast<const float *>(src), c->refbuf));
+  else PMPIC_TRY(tiles_to_ref(c, src, c->refbuf));
+  return get_host(c, spec, c->refbuf, c->ssz);
 }
 
 int pmpic_fft_forward(pmpic_ctx *ctx, const double *grid, double *spec) {
   if (!ctx || !grid || !spec) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
-  std::vector<double> h;
-  grid_to_device_layout(c->g, grid, h);
-  PMPIC_TRY(upload(c, c->kres[0], h));
+  PMPIC_TRY(put_host(c, c->refbuf, grid, ref_grid_size(c->g)));
+  PMPIC_TRY(ref_to_grid(c, c->refbuf, c->kres[0]));
   const double *src[1] = {c->kres[0]};
   double *dst[1] = {c->sder[0]};
   PMPIC_TRY(fft_forward(c, 1, src, dst));
-  PMPIC_TRY(download(c, h, c->sder[0], c->bsz));
-  spec_from_tiles(c->g, h, spec);
-  return PMPIC_OK;
+  PMPIC_TRY(tiles_to_ref(c, c->sder[0], c->refbuf));
+  return get_host(c, spec, c->refbuf, c->ssz);
 }
 
 int pmpic_fft_backward(pmpic_ctx *ctx, const double *spec, double *grid) {
   if (!ctx || !grid || !spec) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
-  std::vector<double> h;
-  spec_to_tiles(c->g, spec, h);
-  PMPIC_TRY(upload(c, c->sder[0], h));
+  PMPIC_TRY(put_host(c, c->refbuf, spec, c->ssz));
+  PMPIC_TRY(ref_to_tiles(c, c->refbuf, c->sder[0]));
   const double *src[1] = {c->sder[0]};
   double *dst[1] = {c->kres[0]};
   PMPIC_TRY(fft_backward(c, 1, src, dst));
-  PMPIC_TRY(download(c, h, c->kres[0], c->gsz));
-  grid_from_device_layout(c->g, h, grid);
-  return PMPIC_OK;
+  PMPIC_TRY(grid_to_ref(c, c->kres[0], 1, c->refbuf));
+  return get_host(c, grid, c->refbuf, ref_grid_size(c->g));
 }
 
 static int spectral_unary(pmpic_ctx *ctx, const double *in, double *out, int which,
                           const double *bot, const double *top) {
   if (!ctx || !in || !out) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
-  std::vector<double> h, hb, ht;
-  spec_to_device_layout(c->g, in, h);
-  PMPIC_TRY(upload(c, c->sder[0], h));
+  PMPIC_TRY(put_host(c, c->refbuf, in, c->ssz));
+  PMPIC_TRY(ref_to_planes(c, c->refbuf, c->sder[0]));
   switch (which) {
     case 0: PMPIC_TRY(op_diffx(c, c->sder[0], c->sder[1])); break;
     case 1: PMPIC_TRY(op_diffy(c, c->sder[0], c->sder[1])); break;
@@ -921,6 +850,7 @@ static int spectral_unary(pmpic_ctx *ctx, const double *in, double *out, int whi
     default: {
       const double *db = nullptr, *dt = nullptr;
       if (bot && top) {
+        std::vector<double> hb, ht;
         col_to_device_layout(c->g, bot, hb);
         col_to_device_layout(c->g, top, ht);
         PMPIC_TRY(upload(c, c->atop, ht));
@@ -931,10 +861,9 @@ static int spectral_unary(pmpic_ctx *ctx, const double *in, double *out, int whi
       PMPIC_TRY(op_diffz(c, c->sder[0], c->sder[1], db, dt));
     }
   }
+  PMPIC_TRY(planes_to_ref(c, c->sder[1], c->refbuf));
   PMPIC_TRY(take_status(c));
-  PMPIC_TRY(download(c, h, c->sder[1], c->ssz));
-  spec_from_device_layout(c->g, h, out);
-  return PMPIC_OK;
+  return get_host(c, out, c->refbuf, c->ssz);
 }
 
 int pmpic_diffx(pmpic_ctx *ctx, const double *in, double *out) { return spectral_unary(ctx, in, out, 0, nullptr, nullptr); }
@@ -947,14 +876,12 @@ int pmpic_diffz(pmpic_ctx *ctx, const double *in, double *out, const double *bot
 int pmpic_laplinv(pmpic_ctx *ctx, double *f, int32_t df0) {
   if (!ctx || !f) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
-  std::vector<double> h;
-  spec_to_device_layout(c->g, f, h);
-  PMPIC_TRY(upload(c, c->sder[0], h));
+  PMPIC_TRY(put_host(c, c->refbuf, f, c->ssz));
+  PMPIC_TRY(ref_to_planes(c, c->refbuf, c->sder[0]));
   PMPIC_TRY(op_laplinv(c, c->sder[0], df0 ? 1 : 0));
+  PMPIC_TRY(planes_to_ref(c, c->sder[0], c->refbuf));
   PMPIC_TRY(take_status(c));
-  PMPIC_TRY(download(c, h, c->sder[0], c->ssz));
-  spec_from_device_layout(c->g, h, f);
-  return PMPIC_OK;
+  return get_host(c, f, c->refbuf, c->ssz);
 }
 
 int pmpic_conservation_sums(pmpic_ctx *ctx, double out6[6]) {

@@ -169,7 +169,7 @@ struct Ctx {
   float4 *rec32;
   bool rec_stale;
   double *gtmp[8];                    // vorticity tendency derivative grids (made by vort2vel)
-  double *kres[6];                    // mixing residual grids
+  double *kres[6];                    // mixing residual grids; kres[0] also standalone scratch
   // spectral, in tiles (the standalone operators use the sder arrays as planes)
   double *sa, *sb, *sc, *sd, *se, *sf, *su, *sv, *sw, *sbs;
   double *sder[6];
@@ -185,7 +185,9 @@ struct Ctx {
   double *lap_rcp, *lap_den, *lap_cp, *lpool;
   int *lap_bad;
   double *coords;                     // x_coords (nx+4), y_coords (ny+4), z_coords (nzn)
-  double *fbuf;                       // host-array staging, allocated at first use (ensure_fbuf)
+  double *fbuf;                       // host transfers' staging of a parcel array, allocated at
+                                      // first use (ensure_fbuf)
+  double *refbuf;                     // ... of an array in the reference's layout (over kres[1..5])
   double2 *cbuf;                      // complex FFT intermediates, FFT_FIELDS fields
   double2 *tw_x, *tw_y;               // twiddles W_n^e, e in [0,n)
   float2 *tw_x32, *tw_y32;            // the same rounded to FP32
@@ -327,12 +329,21 @@ struct BinWork {
 };
 
 // ---- launchers implemented in the translation units ----
+// layout.hip: device layouts <-> the reference's (ref: device memory in the host array's order).
+// grid_to_ref reads every stride-th value of src and fills the halos
+template <typename T>
+int grid_to_ref(Ctx *c, const T *src, int stride, double *ref);
+int ref_to_grid(Ctx *c, const double *ref, double *grid);
+int planes_to_ref(Ctx *c, const double *planes, double *ref);
+int ref_to_planes(Ctx *c, const double *ref, double *planes);
+template <typename S>
+int tiles_to_ref(Ctx *c, const S *tiles, double *ref);
+int ref_to_tiles(Ctx *c, const double *ref, double *tiles);
 // interp.hip
 int bin_parcels(Ctx *c, int64_t n);
 int bin_parcels_ws(Ctx *c, int64_t n, const BinWork &w);
 int par2grid_single_ws(Ctx *c, int64_t n, const double *d_var, double *d_grid, const BinWork &w);
 size_t scan_temp_bytes(Ctx *c, int64_t n);  // temporary storage of an exclusive scan of n
-int to_ref_layout(Ctx *c, const double *d_interior, double *d_ref);
 int par2grid_fused(Ctx *c, int64_t n);  // P,Q,R,B grids from p,q,r,btot
 int par2grid_single(Ctx *c, int64_t n, const double *d_var, double *d_grid);
 int grid2par_single(Ctx *c, int64_t n, const double *d_grid, double *d_var);
@@ -369,7 +380,6 @@ int spectral_setup(Ctx *c);
 int vort2vel_spectral(Ctx *c);
 int vorticity_tendency_grids(Ctx *c);
 int records_current(Ctx *c);                           // refreshes the records' velocities if stale
-int export_tendency(Ctx *c, int f, double *grid);      // DP, DQ, DR (f = 0..2) out of the records
 int op_diffx(Ctx *c, const double *in, double *out);
 int op_diffy(Ctx *c, const double *in, double *out);
 int op_filter(Ctx *c, const double *in, double *out);

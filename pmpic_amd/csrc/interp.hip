@@ -525,32 +525,6 @@ int par2grid_single(Ctx *c, int64_t n, const double *d_var, double *d_grid) {
   return par2grid_single_ws(c, n, d_var, d_grid, ctx_work(c));
 }
 
-// interior [nzn][ny][nx] -> the reference layout data(z, y, x) with x/y halo 2 holding the
-// periodic copies of the interior (the layout pmpic_par2grid returns)
-__global__ void k_to_ref_layout(Geometry g, const double *__restrict__ in, double *__restrict__ out) {
-  const int nxh = g.nx + 4, nyh = g.ny + 4;
-  const int64_t total = (int64_t)nxh * nyh * g.nzn;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= total) return;
-  const int k = (int)(t % g.nzn);
-  const int jh = (int)((t / g.nzn) % nyh);
-  const int ih = (int)(t / ((int64_t)g.nzn * nyh));
-  int i = ih - 2, j = jh - 2;
-  if (i < 0) i += g.nx;
-  else if (i >= g.nx) i -= g.nx;
-  if (j < 0) j += g.ny;
-  else if (j >= g.ny) j -= g.ny;
-  out[t] = in[gidx(g, k, j, i)];
-}
-
-int to_ref_layout(Ctx *c, const double *d_interior, double *d_ref) {
-  const int64_t total = (int64_t)(c->g.nx + 4) * (c->g.ny + 4) * c->g.nzn;
-  hipLaunchKernelGGL(k_to_ref_layout, dim3(cdiv(total, TPB)), dim3(TPB), 0, c->stream, c->g,
-                     d_interior, d_ref);
-  PMPIC_CHECK(hipGetLastError());
-  return PMPIC_OK;
-}
-
 // writebinary's grids (writebinary.F90:217-233): b, hg, p, q, r by par2grid of the parcels'
 // b, h, p, q, r (one binning, the five sums of each node in parcel order as five par2grid
 // calls would take them), then hgliq = max(0, hg - exp(-z)) and b += 12.5 hgliq per node

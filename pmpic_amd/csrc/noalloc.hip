@@ -90,6 +90,6 @@ extern "C" int pmpic_par2grid_noalloc(pmpic_ctx *ctx, const double *var, double 
   w.scan_bytes = NA_SCAN_BYTES;
   double *interior = reinterpret_cast<double *>(base + NA_GRID);
   PMPIC_TRY(par2grid_single_ws(c, c->n, var, interior, w));
-  PMPIC_TRY(to_ref_layout(c, interior, grid));
+  PMPIC_TRY(grid_to_ref(c, interior, 1, grid));
   return take_status(c);
 }

@@ -738,15 +738,6 @@ __global__ void k_record_velocity32(int64_t nnode, const float *__restrict__ U,
   rec[2 * q] = make_float4(U[q], V[q], W[q], rec[2 * q].w);
 }
 
-// a tendency grid out of the records, for an export
-__global__ void k_record_tendency(int64_t nnode, int f, const double2 *__restrict__ rec,
-                                  const float4 *__restrict__ rec32, double *__restrict__ out) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nnode) return;
-  if (rec) out[q] = f == 0 ? rec[3 * q + 1].y : f == 1 ? rec[3 * q + 2].x : rec[3 * q + 2].y;
-  else out[q] = f == 0 ? rec32[2 * q].w : f == 1 ? rec32[2 * q + 1].x : rec32[2 * q + 1].y;
-}
-
 // maxima of u^2, v^2, w^2 and p^2+q^2+r^2 over the interior (vort2vel.F90:331-337,
 // vorticity_tendency.F90:279-282), per block; a maximum is exact in any order, so the result
 // is deterministic.
@@ -1054,14 +1045,6 @@ int records_current(Ctx *c) {
     hipLaunchKernelGGL(k_record_velocity, gb, tb, 0, c->stream, nnode, c->grid[GU], c->grid[GV],
                        c->grid[GW], c->rec);
   c->rec_stale = false;
-  PMPIC_CHECK(hipGetLastError());
-  return PMPIC_OK;
-}
-
-int export_tendency(Ctx *c, int f, double *grid) {
-  const int64_t nnode = c->gsz;
-  hipLaunchKernelGGL(k_record_tendency, dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, nnode, f,
-                     c->rec, c->rec32, grid);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
