@@ -98,6 +98,9 @@ void make_geometry(const pmpic_config *cf, Geometry &g, std::vector<double> &coo
   g.dx = (cf->xmax - cf->xmin) / cf->nx;
   g.dy = (cf->ymax - cf->ymin) / cf->ny;
   g.dz = (cf->zmax - cf->zmin) / cf->nz;
+  g.rdx = 1. / g.dx;
+  g.rdy = 1. / g.dy;
+  g.rdz = 1. / g.dz;
   g.xmin_h = (double)(-2) * g.dx + cf->xmin;
   g.ymin_h = (double)(-2) * g.dy + cf->ymin;
   g.zmin_h = (double)0 * g.dz + cf->zmin;

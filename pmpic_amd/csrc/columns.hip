@@ -22,8 +22,7 @@
 //
 // The pivots depend on the column's k^2 only: they are tabled once per context, four columns
 // sharing an entry, and no pass divides.  The FP64 form gets its quotients from the tabled
-// reciprocal with one residual correction (Markstein, IBM J. Res. Dev. 34, 1990), which rounds
-// as the division does; the FP32-bulk form multiplies by the FP64 reciprocal.  All arithmetic is
+// reciprocal with one residual correction (div_by), which rounds as the division does; the FP32-bulk form multiplies by the FP64 reciprocal.  All arithmetic is
 // FP64 in both forms; the arrays between the passes are of the spectral type S.
 //
 // Bound by memory on large grids (26 passes over a spectral array where the separate kernels took
@@ -57,9 +56,8 @@ __device__ __forceinline__ double other_y(S v) { return (double)quad_perm<0x4E>(
 // n / den, with r = 1 / den rounded to nearest
 template <typename S>
 __device__ __forceinline__ double quot(double n, double den, double r) {
-  const double q = n * r;
-  if constexpr (std::is_same<S, float>::value) return q;
-  return fma(fma(-q, den, n), r, q);
+  if constexpr (std::is_same<S, float>::value) return n * r;
+  return div_by(n, den, r);
 }
 
 // Pivots of the compact inverse Laplacian for both boundary conditions (bc 0: zero value, 1: zero

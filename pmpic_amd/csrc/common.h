@@ -93,6 +93,7 @@ struct Geometry {
   int sx, sy;                    // spectral extents
   double xbot, ybot, zbot, xtop, ytop, ztop;  // config bounds
   double dx, dy, dz;
+  double rdx, rdy, rdz;          // 1 / dx, 1 / dy, 1 / dz rounded to nearest
   double xmin_h, ymin_h, zmin_h, zmax_h;      // parcel_interpolation.F90:104-115
   double hs_xmin, hs_xmax, hs_ymin, hs_ymax;  // haloswap.F90:314-318
   double xshift_e, xshift_w, yshift_n, yshift_s;  // haloswap.F90:529-552
@@ -263,6 +264,14 @@ __device__ __forceinline__ void raise_status(DevScalars *s, int code) {
   atomicCAS(&s->status, 0, code);
 }
 
+// a / b rounded as the division rounds it, from r = 1 / b rounded to nearest: the quotient a r is
+// within an ulp and one residual corrects it (Markstein, IBM J. Res. Dev. 34, 1990).  Three
+// operations where the division takes about a dozen.
+__device__ __forceinline__ double div_by(double a, double b, double r) {
+  const double q = a * r;
+  return fma(fma(-q, b, a), r, q);
+}
+
 // cache_parcel_interp_weights for one parcel (parcel_interpolation.F90:206-246), returning the
 // periodic interior cell (i0, j0, k0) and the offsets.  Arithmetic is the reference's, operand
 // for operand.  Returns a status code.
@@ -270,17 +279,17 @@ __device__ __forceinline__ int locate(const Geometry &g, double xp, double yp, d
                                       int &i0, int &j0, int &k0, double &delx, double &dely,
                                       double &delz) {
   const double ax = xp - g.xmin_h, ay = yp - g.ymin_h, az = zp - g.zmin_h;
-  const int i = (int)floor(ax / g.dx) + 1;
-  const int j = (int)floor(ay / g.dy) + 1;
-  const int k = (int)floor(az / g.dz) + 1;
+  const int i = (int)floor(div_by(ax, g.dx, g.rdx)) + 1;
+  const int j = (int)floor(div_by(ay, g.dy, g.rdy)) + 1;
+  const int k = (int)floor(div_by(az, g.dz, g.rdz)) + 1;
   // the reference accepts 1 <= i < nx+4; halo columns 1,2 only arise for a parcel the
   // haloswap failed to wrap, which is rejected here instead of silently mis-deposited
   if (i < 3 || i > g.nx + 3) return PMPIC_ERR_OUT_OF_BOX_X;
   if (j < 3 || j > g.ny + 3) return PMPIC_ERR_OUT_OF_BOX_Y;
   if (k < 1 || k >= g.nzn) return PMPIC_ERR_OUT_OF_BOX_Z;
-  delx = (ax - (double)(i - 1) * g.dx) / g.dx;
-  dely = (ay - (double)(j - 1) * g.dy) / g.dy;
-  delz = (az - (double)(k - 1) * g.dz) / g.dz;
+  delx = div_by(ax - (double)(i - 1) * g.dx, g.dx, g.rdx);
+  dely = div_by(ay - (double)(j - 1) * g.dy, g.dy, g.rdy);
+  delz = div_by(az - (double)(k - 1) * g.dz, g.dz, g.rdz);
   if (delx > 1. || delx < 0) return PMPIC_ERR_DELTA;
   if (dely > 1. || dely < 0) return PMPIC_ERR_DELTA;
   if (delz > 1. || delz < 0) return PMPIC_ERR_DELTA;
@@ -318,14 +327,11 @@ __device__ __forceinline__ int64_t gidx(const Geometry &g, int k, int j, int i) 
 }
 
 // Buffers of one FP64 binning + single-field par2grid: the context's own, or caller-provided
-// memory (pmpic_par2grid_noalloc).  cell, rank, sorted: n entries; count, start: ncell + 1;
-// partial: 16 * ncell doubles; scan_tmp (scan_bytes) the exclusive scan's temporary storage,
-// or null to use the context's (grown on demand).
+// memory (pmpic_par2grid_noalloc).  cell, rank, sorted: n entries; count, start: ncell; cursor: one
+// entry; partial: 12 * ncell doubles.  count and cursor are zero between calls.
 struct BinWork {
-  int32_t *cell, *rank, *count, *start, *sorted;
+  int32_t *cell, *rank, *count, *start, *sorted, *cursor;
   double *partial;
-  void *scan_tmp;
-  size_t scan_bytes;
 };
 
 // ---- launchers implemented in the translation units ----
@@ -343,7 +349,6 @@ int ref_to_tiles(Ctx *c, const double *ref, double *tiles);
 int bin_parcels(Ctx *c, int64_t n);
 int bin_parcels_ws(Ctx *c, int64_t n, const BinWork &w);
 int par2grid_single_ws(Ctx *c, int64_t n, const double *d_var, double *d_grid, const BinWork &w);
-size_t scan_temp_bytes(Ctx *c, int64_t n);  // temporary storage of an exclusive scan of n
 int par2grid_fused(Ctx *c, int64_t n);  // P,Q,R,B grids from p,q,r,btot
 int par2grid_single(Ctx *c, int64_t n, const double *d_var, double *d_grid);
 int grid2par_single(Ctx *c, int64_t n, const double *d_grid, double *d_var);

@@ -8,13 +8,13 @@
 // par2grid is a scatter; here it is a gather over a cell binning so that no floating-point
 // atomics are used and every node sum has a fixed order:
 //   1. bin:   each parcel finds its cell and takes a slot in the cell's bucket (integer atomics,
-//             one per run of equal cells within a wavefront), an exclusive scan turns bucket
-//             sizes into offsets and parcel indices are scattered into the buckets;
-//   2. cell:  a workgroup stages a tile of cells' parcels in LDS (coalesced loads, one
-//             location per parcel), then one thread per cell adds the 8 corner weights (and
-//             weight * value) of its parcels in ascending parcel order;
-//   3. node:  one thread per node adds the matching corner partials of its 8 adjacent cells
-//             (periodic in x, y) in a fixed order and normalises by the summed weights.
+//             one per run of equal cells within a wavefront), the buckets are given room and the
+//             parcel indices are scattered into them;
+//   2. cell:  a wavefront takes eight cells of one x row; its 8 lanes a cell stage the cell's
+//             parcels in LDS eight at a time, then lane q adds corner q's weight and weight *
+//             value over them in ascending parcel order;
+//   3. node:  one thread per node adds the matching corner sums of its adjacent cells (periodic
+//             in x, y) in a fixed order and normalises by the summed weights.
 // The result differs from the reference's sequential sum only by the order of additions.
 #include "common.h"
 
@@ -26,18 +26,14 @@ namespace {
 
 constexpr int TPB = 256;
 
-__global__ void k_fill_i32(int32_t *a, int64_t n, int32_t v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = v;
-}
-
 // cell of every parcel and its slot in the cell's bucket.  Parcels that are neighbours in slot
 // order usually share a cell, so lanes are grouped into runs of equal cell and one lane per run
 // takes the whole run's slots with a single integer atomic.  Each wavefront walks BIN_SEQ
 // consecutive groups of 64 parcels in order, so a cell whose parcels are consecutive in slot
-// order gets ascending bucket slots unless it straddles two wavefronts' ranges.
-constexpr int BIN_SEQ = 16;
-
+// order gets ascending bucket slots unless it straddles two wavefronts' ranges.  16 groups where
+// the parcels fill the chip with wavefronts that long (bin_seq); fewer below, down to one, where
+// the walk is what takes the time (7,680 parcels: 13.3 us a call with 16 groups, 4 with one).
+template <int BIN_SEQ>
 __global__ void k_bin_count(Geometry g, const double *__restrict__ X, const double *__restrict__ Y,
                             const double *__restrict__ Z, int64_t n, int32_t *__restrict__ cell,
                             int32_t *__restrict__ rank, int32_t *__restrict__ count,
@@ -48,7 +44,7 @@ __global__ void k_bin_count(Geometry g, const double *__restrict__ X, const doub
   int base[BIN_SEQ], hls[BIN_SEQ];
   // the positions of the next BIN_AHEAD groups are loaded before the current group is located
   // (clamped index, n >= 1), so the wavefront does not wait on memory once per group
-  constexpr int BIN_AHEAD = 4;
+  constexpr int BIN_AHEAD = BIN_SEQ < 4 ? BIN_SEQ : 4;
   double px[BIN_SEQ], py[BIN_SEQ], pz[BIN_SEQ];
   auto load_group = [&](int it) {
     const int64_t p = min(w0 + (int64_t)it * 64 + lane, n - 1);
@@ -89,6 +85,49 @@ __global__ void k_bin_count(Geometry g, const double *__restrict__ X, const doub
   }
 }
 
+// room for every bucket: start[c] from a running total.  The buckets' order does not matter to the
+// sums, so each block takes its cells' total from the cursor with one atomic, and no scan of the
+// whole array (two more launches) is needed.
+constexpr int ALLOC_CELLS = 4;  // cells per thread
+__global__ void __launch_bounds__(TPB) k_bin_alloc(const int32_t *__restrict__ count, int64_t ncell,
+                                                   int32_t *__restrict__ start,
+                                                   int32_t *__restrict__ cursor) {
+  __shared__ int32_t wave_sum[TPB / 64];
+  __shared__ int32_t base;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t c0 = ((int64_t)blockIdx.x * TPB + threadIdx.x) * ALLOC_CELLS;
+  int32_t k[ALLOC_CELLS], sum = 0;
+#pragma unroll
+  for (int i = 0; i < ALLOC_CELLS; i++) {
+    k[i] = c0 + i < ncell ? count[c0 + i] : 0;
+    sum += k[i];
+  }
+  int32_t incl = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t u = __shfl_up(incl, d);
+    if (lane >= d) incl += u;
+  }
+  if (lane == 63) wave_sum[wave] = incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int32_t t = 0;
+    for (int w = 0; w < TPB / 64; w++) {
+      const int32_t v = wave_sum[w];
+      wave_sum[w] = t;
+      t += v;
+    }
+    base = t > 0 ? atomicAdd(cursor, t) : 0;
+  }
+  __syncthreads();
+  int32_t o = base + wave_sum[wave] + incl - sum;
+#pragma unroll
+  for (int i = 0; i < ALLOC_CELLS; i++) {
+    if (c0 + i < ncell) start[c0 + i] = o;
+    o += k[i];
+  }
+}
+
 __global__ void k_bin_scatter(const int32_t *__restrict__ cell, const int32_t *__restrict__ rank,
                               const int32_t *__restrict__ start, int64_t n,
                               int32_t *__restrict__ sorted) {
@@ -99,170 +138,190 @@ __global__ void k_bin_scatter(const int32_t *__restrict__ cell, const int32_t *_
   sorted[start[c] + rank[p]] = (int32_t)p;
 }
 
-// buckets larger than the LDS tile are sorted by parcel index here (insertion sort; such cells
-// do not occur at the target workloads); smaller buckets are ordered inside the accumulation
-__global__ void k_bin_sort_big(const int32_t *__restrict__ start, int64_t ncell, int sgsize,
-                               int32_t *__restrict__ sorted) {
-  int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  const int32_t b = start[c], e = start[c + 1];
-  if (e - b <= sgsize) return;
-  for (int32_t a = b + 1; a < e; a++) {
-    int32_t v = sorted[a];
-    int32_t q = a - 1;
-    while (q >= b && sorted[q] > v) {
-      sorted[q + 1] = sorted[q];
-      q--;
-    }
-    sorted[q + 1] = v;
-  }
-}
-
 // value sources for the per-cell accumulation
-enum AccMode { ACC_P2G = 0, ACC_SINGLE = 1, ACC_MIX_KEEP = 2, ACC_MIX_RES = 3, ACC_DUMP = 4 };
+enum AccMode { ACC_P2G = 0, ACC_SINGLE = 1, ACC_MIX = 2, ACC_DUMP = 4 };
 
-// Per-cell corner partial sums.
-// A workgroup owns TILE consecutive cells.  Their buckets are consecutive in the bucket array, so
-// the workgroup loads them with coalesced reads (bucket entries are mostly consecutive parcel
-// slots), locates each parcel once and stages (offsets, volume, values, parcel index) in LDS as
-// 16-byte pairs.  The 8 threads of a cell put its rows in ascending parcel order (a pass over
-// adjacent pairs, and a parallel ranking only when a pair is out of order); then one thread per
-// (cell, corner) adds that corner's weight and weight * value over the cell's rows in that
-// order, so within a cell the additions run in the reference's order.
-// MIX mode sums kept parcels into `partial` (and counts them) and residual parcels into
-// `partial2`.  Cells with more than ROWS parcels (never at the target workloads) are summed
-// straight from global memory after k_bin_sort_big ordered their buckets.
-constexpr int TILE = 16;  // cells per workgroup: 8 threads (corners) each
-constexpr int ROWS_P2G = 512, ROWS_MIX = 448;
+// Per-cell corner sums.
+//
+// One wavefront per tile of 8 cells of one x row; lane = 8 q + cl is corner q (bits z<<2 | y<<1 |
+// x) of cell cl.  A cell's parcels are taken eight at a time: lane (q, cl) loads and locates
+// parcel q of the eight and stages (offsets, volume, values) in LDS row 8 q + cl; then every lane
+// adds its corner's weight and weight * value over the cell's eight rows (the wavefront reads
+// eight neighbouring 16-byte pairs at a time, each by eight lanes: no bank conflicts).  The next
+// eight parcels' loads are in flight meanwhile.  With 2-5 KB of LDS and no barrier across
+// wavefronts a CU holds 16 to 20 of them and the loads overlap the sums; the earlier form (a
+// workgroup staging all parcels of 16 cells in 36 KB, 8 wavefronts a CU, its load and sum phases
+// apart) took 2.18 ms for 57 M parcels in slot order and 224 us for 0.9 M well mixed ones, this one
+// 1.78 ms (3.1 TB/s) and 115 us.  It is bound by the loads' latency.  The parcel loads are cached
+// ones: a 128-byte line serves two chunks (streaming loads: 3.02 ms).
+//
+// Within a cell the additions run in ascending parcel order, the reference's: bucket slots come
+// from atomics and may be out of order, so the lanes check their adjacent entries and rank the
+// entries of the tile's cells where a pair is not ascending (in LDS up to LIST entries a cell, else
+// in global memory through `order`).
+//
+// The corner sums are combined along x before they are written: node position i of corner pair
+// bb = (by, bz) adds the bx = 1 corner of cell i - 1 and the bx = 0 corner of cell i.  Value f of
+// entry (bb, row, position) sits at ((f 4 + bb) nrows + row) (nx + ntx) + 9 tx + position - 8 tx,
+// ntx tiles a row; a tile's last position holds its last cell's bx = 1 corner alone, completed by
+// k_node_sum.  180 bytes a cell for five values instead of 320.
+//
+// ACC_MIX sums the kept parcels into `partial` (and counts them) and the residual ones into
+// `partial2`, whose tiles without residual parcels (almost all) are left unwritten and marked so in
+// tileres.  Either output may be null.  `zero`: leaves count and the cursor at zero, as the next
+// binning wants them.
+constexpr int LIST = 64;
 
 template <int MODE, int NV>
 __device__ __forceinline__ void load_values(const double *__restrict__ par, int64_t cap,
-                                            const double *__restrict__ var, int64_t p, double z,
+                                            const double *__restrict__ var, int64_t p,
                                             double *val) {
   if constexpr (MODE == ACC_P2G) {
-    val[0] = ld_stream(&par[FP * cap + p]);
-    val[1] = ld_stream(&par[FQ * cap + p]);
-    val[2] = ld_stream(&par[FR * cap + p]);
-    // total buoyancy, vorticity_tendency.F90:121-126
-    const double hl = ld_stream(&par[FH * cap + p]) - exp(-z);
-    val[3] = ld_stream(&par[FB * cap + p]) + 12.5 * (hl > 0.0 ? hl : 0.0);
+    val[0] = par[FP * cap + p];
+    val[1] = par[FQ * cap + p];
+    val[2] = par[FR * cap + p];
+    val[3] = par[FB * cap + p];
+    val[4] = par[FH * cap + p];
   } else if constexpr (MODE == ACC_SINGLE) {
-    val[0] = ld_stream(&var[p]);
+    val[0] = var[p];
   } else {
-    val[0] = ld_stream(&par[FB * cap + p]);
-    val[1] = ld_stream(&par[FH * cap + p]);
-    val[2] = ld_stream(&par[FP * cap + p]);
-    val[3] = ld_stream(&par[FQ * cap + p]);
-    val[4] = ld_stream(&par[FR * cap + p]);
+    val[0] = par[FB * cap + p];
+    val[1] = par[FH * cap + p];
+    val[2] = par[FP * cap + p];
+    val[3] = par[FQ * cap + p];
+    val[4] = par[FR * cap + p];
   }
 }
 
-template <int MODE, int NV, int ROWS>
-__global__ void __launch_bounds__(256) k_cell_accum_lds(Geometry g, const double *__restrict__ par,
-                                                        int64_t cap, const double *__restrict__ var,
-                                                        const int32_t *__restrict__ start,
-                                                        const int32_t *__restrict__ sorted,
-                                                        int64_t ncell, double *__restrict__ partial,
-                                                        double *__restrict__ partial2,
-                                                        int32_t *__restrict__ npercell) {
+// one parcel's loads
+template <int NL>
+struct Row {
+  double x, y, z, vol, val[NL];
+};
+
+template <int MODE, int NV>
+__global__ void __launch_bounds__(64) k_cell_accum(Geometry g, const double *__restrict__ par,
+                                                   int64_t cap, const double *__restrict__ var,
+                                                   int32_t *__restrict__ count,
+                                                   const int32_t *__restrict__ start,
+                                                   const int32_t *__restrict__ sorted,
+                                                   int32_t *__restrict__ order,
+                                                   double *__restrict__ partial,
+                                                   double *__restrict__ partial2,
+                                                   int32_t *__restrict__ npercell,
+                                                   uint8_t *__restrict__ tileres,
+                                                   int32_t *__restrict__ cursor, int zero) {
   constexpr int NF = NV + 1;
-  constexpr int NVS = (NV + 1) / 2;  // value pairs per row
-  constexpr bool MIX = (MODE == ACC_MIX_KEEP);
-  __shared__ double2 sgeo[2][ROWS];    // (delx, dely), (delz, vol)
-  __shared__ double2 sval[NVS][ROWS];  // values, two per slot
-  __shared__ int32_t sidx[ROWS];
-  __shared__ int16_t sperm[ROWS];
-  __shared__ uint8_t skeep[MIX ? ROWS : 1];
-  __shared__ int32_t sstart[TILE + 1];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int cl = tid >> 3;          // cell within the tile
-  const int q = tid & 7;            // corner: bits z<<2 | y<<1 | x
-  const int bx = q & 1, by = (q >> 1) & 1, bz = (q >> 2) & 1;
-  const int64_t c0 = (int64_t)blockIdx.x * TILE;
-  const int ntile = (int)min((int64_t)TILE, ncell - c0);
-  for (int t = tid; t <= ntile; t += blockDim.x) sstart[t] = start[c0 + t];
+  constexpr int NL = MODE == ACC_P2G ? 5 : NV;  // values loaded: p, q, r, b, h make four
+  constexpr int NVS = (NV + 1) / 2;             // value pairs a row
+  constexpr bool MIX = MODE == ACC_MIX;
+  __shared__ double2 sgeo[2][64];    // (delx, dely), (delz, vol)
+  __shared__ double2 sval[NVS][64];  // values, two per slot
+  __shared__ int32_t slist[LIST * 8];  // entry e of cell cl at 8 e + cl
+  const int lane = threadIdx.x, cl = lane & 7, q = lane >> 3;
+  const int bx = q & 1, by = (q >> 1) & 1, bz = q >> 2;
+  const int ntx = (g.nx + 7) / 8;
+  const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
+  const uint32_t xrow = tile / (uint32_t)ntx;
+  const int tx = (int)(tile - xrow * (uint32_t)ntx), m = min(8, g.nx - 8 * tx);  // cells here
+  const bool live = cl < m;
+  const int64_t c = (int64_t)xrow * g.nx + 8 * tx + cl;
+  const int n = live ? count[c] : 0;
+  const int64_t b = live ? start[c] : 0;
+  int nmax = n;
+#pragma unroll
+  for (int d = 1; d < 8; d <<= 1) nmax = max(nmax, __shfl_xor(nmax, d));
+  nmax = __builtin_amdgcn_readfirstlane(nmax);
+  const int nch = (nmax + 7) >> 3;  // chunks of eight parcels a cell
+  const int32_t *list = sorted + b;
+  const bool small = nmax <= LIST;
+  // entries 8 (i0 + i) + q of the cell, i < 8, ordered by parcel
+  bool bad = false;
+  for (int i0 = 0; i0 < nch; i0 += 8) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      if (i0 + i >= nch) break;
+      const int e = 8 * (i0 + i) + q;
+      const int32_t v = e < n ? list[e] : INT32_MAX;
+      if (small) slist[64 * i + lane] = v;
+      bad |= e + 1 < n && v > list[e + 1];
+    }
+  }
+  if (__any(bad)) {
+    for (int i0 = 0; i0 < nch; i0 += 8) {
+      int32_t v[8];
+      int r[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int e = 8 * (i0 + i) + q;
+        v[i] = e < n ? list[e] : INT32_MAX;
+        r[i] = 0;
+      }
+      for (int e = 0; e < nmax; e++) {
+        const int32_t key = small ? slist[8 * e + cl] : e < n ? list[e] : INT32_MAX;
+#pragma unroll
+        for (int i = 0; i < 8; i++) r[i] += key < v[i] ? 1 : 0;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        if (8 * (i0 + i) + q < n) {
+          if (small) slist[8 * r[i] + cl] = v[i];
+          else order[b + r[i]] = v[i];
+        }
+    }
+    if (!small) {
+      __threadfence_block();
+      list = order + b;
+    }
+  }
   __syncthreads();
   const double *X = par + FX * cap, *Y = par + FY * cap, *Z = par + FZ * cap;
   const double *VOL = par + FVOL * cap;
-  double acc[NF], res[NF];
+  auto fetch = [&](int ch, Row<NL> &row) {
+    const int e = 8 * ch + q;
+    if (e < n) {
+      const int64_t p = small ? slist[64 * ch + lane] : list[e];
+      row.x = X[p];
+      row.y = Y[p];
+      row.z = Z[p];
+      row.vol = VOL[p];
+      load_values<MODE, NV>(par, cap, var, p, row.val);
+    }
+  };
+  double acc[NF], res[MIX ? NF : 1];
 #pragma unroll
-  for (int f = 0; f < NF; f++) { acc[f] = 0.0; res[f] = 0.0; }
+  for (int f = 0; f < NF; f++) acc[f] = 0.0;
+#pragma unroll
+  for (int f = 0; f < (MIX ? NF : 1); f++) res[f] = 0.0;
   int kept = 0;
-  bool big = false;
-  int first = 0;
-  while (first < ntile) {
-    // the group of cells [first, last) whose rows fit in LDS (at least one cell)
-    int last = first + 1;
-    if (sstart[ntile] - sstart[first] <= ROWS) last = ntile;  // the usual case: the rest fits
-    else
-      while (last < ntile && sstart[last + 1] - sstart[first] <= ROWS) last++;
-    const int32_t r0 = sstart[first];
-    const int nrows = sstart[last] - r0;
-    const bool fits = nrows <= ROWS;
-    if (fits) {
-      // all of this thread's rows are fetched before any is used, so the dependent
-      // bucket -> parcel loads of different rows overlap
-      constexpr int RPT = (ROWS + TILE * 8 - 1) / (TILE * 8);
-      int32_t pr[RPT];
+  bool anyres = false;
+  Row<NL> row{};
+  if (nch > 0) fetch(0, row);
+  for (int ch = 0; ch < nch; ch++) {
+    if (8 * ch + q < n) {
+      int i0, j0, k0;
+      double delx, dely, delz;
+      locate(g, row.x, row.y, row.z, i0, j0, k0, delx, dely, delz);
+      sgeo[0][lane] = make_double2(delx, dely);
+      sgeo[1][lane] = make_double2(delz, row.vol);
+      if constexpr (MODE == ACC_P2G) {
+        // total buoyancy, vorticity_tendency.F90:121-126
+        const double hl = row.val[4] - exp(-row.z);
+        sval[0][lane] = make_double2(row.val[0], row.val[1]);
+        sval[1][lane] = make_double2(row.val[2], row.val[3] + 12.5 * (hl > 0.0 ? hl : 0.0));
+      } else {
 #pragma unroll
-      for (int k = 0; k < RPT; k++) {
-        const int r = tid + k * TILE * 8;
-        pr[k] = (r < nrows) ? sorted[r0 + r] : -1;
-      }
-      double px[RPT], py[RPT], pz[RPT], pv[RPT], pval[RPT][2 * NVS];
-#pragma unroll
-      for (int k = 0; k < RPT; k++) {
-        pval[k][2 * NVS - 1] = 0.0;
-        if (pr[k] >= 0) {
-          const int64_t pp = pr[k];
-          px[k] = ld_stream(&X[pp]);
-          py[k] = ld_stream(&Y[pp]);
-          pz[k] = ld_stream(&Z[pp]);
-          pv[k] = ld_stream(&VOL[pp]);
-          load_values<MODE, NV>(par, cap, var, pp, pz[k], pval[k]);
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < RPT; k++) {
-        const int r = tid + k * TILE * 8;
-        if (pr[k] < 0) continue;
-        int i0, j0, k0;
-        double delx, dely, delz;
-        locate(g, px[k], py[k], pz[k], i0, j0, k0, delx, dely, delz);
-        sgeo[0][r] = make_double2(delx, dely);
-        sgeo[1][r] = make_double2(delz, pv[k]);
-#pragma unroll
-        for (int f = 0; f < NVS; f++) sval[f][r] = make_double2(pval[k][2 * f], pval[k][2 * f + 1]);
-        if constexpr (MIX) skeep[r] = (pv[k] < g.vmin) ? 0 : 1;
-        sidx[r] = pr[k];
+        for (int f = 0; f < NVS; f++)
+          sval[f][lane] = make_double2(row.val[2 * f], 2 * f + 1 < NL ? row.val[2 * f + 1 < NL ? 2 * f + 1 : 0] : 0.0);
       }
     }
     __syncthreads();
-    const bool mine = fits && cl >= first && cl < last;
-    const int lo = mine ? sstart[cl] - r0 : 0, hi = mine ? sstart[cl + 1] - r0 : 0;
-    // Canonical order: a cell's rows by ascending parcel index.  Bucket slots come from atomics,
-    // so runs of a cell's parcels filled by different wavefronts may arrive out of order.  The 8
-    // corner lanes of a cell check their share of adjacent pairs; if any pair is out of order,
-    // each lane ranks its share of rows by counting smaller parcel indices in the cell.
-    bool ord = true;
-    for (int a = lo + 1 + q; a < hi; a += 8) ord &= (sidx[a - 1] < sidx[a]);
-    const unsigned long long bad = __ballot(!ord);
-    const bool sort_cell = ((bad >> (lane & ~7)) & 0xffull) != 0ull;
-    if (sort_cell) {
-      for (int a = lo + q; a < hi; a += 8) {
-        const int32_t key = sidx[a];
-        int rk = 0;
-        for (int b = lo; b < hi; b++) rk += (sidx[b] < key) ? 1 : 0;
-        sperm[lo + rk] = (int16_t)a;
-      }
-    } else {
-      for (int a = lo + q; a < hi; a += 8) sperm[a] = (int16_t)a;
-    }
-    __syncthreads();
+    if (ch + 1 < nch) fetch(ch + 1, row);
+    const int rows = min(8, nmax - 8 * ch), mine = n - 8 * ch;
 #pragma unroll 2
-    for (int a = lo; a < hi; a++) {
-      const int r = sperm[a];
+    for (int a = 0; a < rows; a++) {
+      const int r = 8 * a + cl;
       const double2 g0 = sgeo[0][r], g1 = sgeo[1][r];
       double v[2 * NVS];
 #pragma unroll
@@ -275,118 +334,102 @@ __global__ void __launch_bounds__(256) k_cell_accum_lds(Geometry g, const double
       const double fy = by ? g0.y : 1 - g0.y;
       const double fz = bz ? g1.x : 1 - g1.x;
       const double w = fz * fy * fx * g1.y;
-      if (!MIX || skeep[r]) {
-        acc[0] += w;
+      if (a < mine) {
+        if (!MIX || !(g1.y < g.vmin)) {
+          acc[0] += w;
 #pragma unroll
-        for (int f = 0; f < NV; f++) acc[f + 1] += w * v[f];
-        kept++;
-      } else {
-        res[0] += w;
+          for (int f = 0; f < NV; f++) acc[f + 1] += w * v[f];
+          kept++;
+        } else if constexpr (MIX) {
+          anyres = true;
+          res[0] += w;
 #pragma unroll
-        for (int f = 0; f < NV; f++) res[f + 1] += w * v[f];
+          for (int f = 0; f < NV; f++) res[f + 1] += w * v[f];
+        }
       }
     }
-    if (fits == false && cl == first) big = true;
     __syncthreads();
-    first = last;
   }
-  if (cl >= ntile) return;
-  const int64_t c = c0 + cl;
-  if (big) {
-    // bucket already sorted by k_bin_sort_big; the same sums straight from global memory
-    for (int32_t s = sstart[cl]; s < sstart[cl + 1]; s++) {
-      const int32_t p = sorted[s];
-      const double v = VOL[p];
-      int i0, j0, k0;
-      double delx, dely, delz;
-      const double zp = Z[p];
-      locate(g, X[p], Y[p], zp, i0, j0, k0, delx, dely, delz);
-      double val[NV];
-      load_values<MODE, NV>(par, cap, var, p, zp, val);
-      const double fx = bx ? delx : 1 - delx;
-      const double fy = by ? dely : 1 - dely;
-      const double fz = bz ? delz : 1 - delz;
-      const double w = fz * fy * fx * v;
-      if (!MIX || !(v < g.vmin)) {
-        acc[0] += w;
+  const int64_t nrows = (int64_t)g.ny * g.ncz, W = g.nx + ntx;
+  auto write_x = [&](const double *v, double *out) {
+    const int64_t o = ((int64_t)(q >> 1) * nrows + xrow) * W + 9 * tx + (bx ? 8 : cl);
+    const bool mine = bx ? (cl == 7 && m == 8) : cl <= m;
 #pragma unroll
-        for (int f = 0; f < NV; f++) acc[f + 1] += w * val[f];
-        kept++;
-      } else {
-        res[0] += w;
-#pragma unroll
-        for (int f = 0; f < NV; f++) res[f + 1] += w * val[f];
-      }
+    for (int f = 0; f < NF; f++) {
+      const double left = __shfl(v[f], (lane + 7) & 63);  // corner q | 1 of cell cl - 1
+      if (mine) out[f * 4 * nrows * W + o] = bx || cl == 0 ? v[f] : left + v[f];
     }
-  }
-  // MIX: either output may be null (the two-pass form of mixing_grids); the sums are the same
-  if (!MIX || partial) {
-#pragma unroll
-    for (int f = 0; f < NF; f++) partial[((int64_t)q * ncell + c) * NF + f] = acc[f];
-  }
+  };
+  if (!MIX || partial) write_x(acc, partial);
   if constexpr (MIX) {
-    if (partial2) {
-#pragma unroll
-      for (int f = 0; f < NF; f++) partial2[((int64_t)q * ncell + c) * NF + f] = res[f];
-    }
-    if (npercell && q == 0) npercell[c] = kept;
+    const bool any = __any(anyres) != 0;
+    if (tileres && lane == 0) tileres[tile] = any ? 1 : 0;
+    if (partial2 && any) write_x(res, partial2);
+    if (npercell && live && q == 0) npercell[c] = kept;
+  }
+  if (zero) {
+    if (live && q == 0) count[c] = 0;
+    if (tile == 0 && lane == 0) *cursor = 0;
   }
 }
 
-// node sums: NORM = divide by summed weights (par2grid, parcel_interpolation.F90:463-469);
-// otherwise raw sums with the mixing z-boundary doubling (parcel_mixing.F90:141-152).
+// node sums of the x-combined corner sums: NORM = divide by summed weights (par2grid,
+// parcel_interpolation.F90:463-469); otherwise raw sums with the mixing z-boundary doubling
+// (parcel_mixing.F90:141-152).  Node (i, j, k) adds, for each corner pair (by, bz) in a fixed
+// order, the entry of cell row (j - by, k - bz) at its position, and at a tile boundary the left
+// tile's last entry before it.  tileres (may be null): the tiles whose entries were written.
 struct OutTable {
   double *p[6];
 };
 
 template <int NV, bool NORM, bool DBL = true>
-__global__ void k_node_sum(Geometry g, const double *__restrict__ partial, int64_t ncell,
-                           OutTable out) {
+__global__ void k_node_sum(Geometry g, const double *__restrict__ partial, OutTable out,
+                           const uint8_t *__restrict__ tileres) {
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nnode) return;
   const int i = (int)(t % g.nx);
   const int j = (int)((t / g.nx) % g.ny);
   const int k = (int)(t / ((int64_t)g.nx * g.ny));
-  // every corner's partials are loaded first (a corner below the bottom or above the top cell
-  // reads cell 0 and is left out of the sum), then summed in the fixed corner order
-  double v[8][NV + 1];
-  bool ok[8];
+  const int ntx = (g.nx + 7) / 8, tx = i >> 3, pos = i & 7, txl = tx == 0 ? ntx - 1 : tx - 1;
+  const int64_t nrows = (int64_t)g.ny * g.ncz, W = g.nx + ntx, fstride = 4 * nrows * W;
+  const int own = 9 * tx + pos, left = tx == 0 ? (int)W - 1 : 9 * tx - 1;
+  double v[4][NV + 1], vl[4][NV + 1];
+  bool ok[4], okl[4];
 #pragma unroll
-  for (int q = 0; q < 8; q++) {
-    const int bx = q & 1, by = (q >> 1) & 1, bz = q >> 2;
-    int ci = i - bx;
-    if (ci < 0) ci += g.nx;
+  for (int bb = 0; bb < 4; bb++) {
+    const int by = bb & 1, bz = bb >> 1;
     int cj = j - by;
     if (cj < 0) cj += g.ny;
     const int ck = k - bz;
-    ok[q] = ck >= 0 && ck < g.ncz;
-    const int64_t c = ok[q] ? ((int64_t)ck * g.ny + cj) * g.nx + ci : 0;
+    const bool in = ck >= 0 && ck < g.ncz;
+    const int64_t crow = in ? (int64_t)ck * g.ny + cj : 0;
+    ok[bb] = in && (!tileres || tileres[crow * ntx + tx]);
+    okl[bb] = in && pos == 0 && (!tileres || tileres[crow * ntx + txl]);
+    const double *e = partial + ((int64_t)bb * nrows + crow) * W;
 #pragma unroll
-    for (int f = 0; f <= NV; f++) v[q][f] = partial[((int64_t)q * ncell + c) * (NV + 1) + f];
+    for (int f = 0; f <= NV; f++) {
+      v[bb][f] = ok[bb] ? e[f * fstride + own] : 0.0;
+      vl[bb][f] = okl[bb] ? e[f * fstride + left] : 0.0;
+    }
   }
   double s[NV + 1];
 #pragma unroll
   for (int f = 0; f <= NV; f++) s[f] = 0.0;
 #pragma unroll
-  for (int bx = 0; bx < 2; bx++)
+  for (int bb = 0; bb < 4; bb++)
 #pragma unroll
-    for (int by = 0; by < 2; by++)
-#pragma unroll
-      for (int bz = 0; bz < 2; bz++) {
-        const int q = (bz << 2) | (by << 1) | bx;
-#pragma unroll
-        for (int f = 0; f <= NV; f++) s[f] = ok[q] ? s[f] + v[q][f] : s[f];
-      }
+    for (int f = 0; f <= NV; f++)
+      if (ok[bb] || okl[bb]) s[f] = s[f] + (pos == 0 ? vl[bb][f] + v[bb][f] : v[bb][f]);
   if (NORM) {
     double w = s[0];
     if (w == 0.) w = 1.;
 #pragma unroll
     for (int f = 1; f <= NV; f++) out.p[f - 1][t] = s[f] / w;
   } else {
-    const double m = (DBL && (k == 0 || k == g.nzn - 1)) ? 2. : 1.;
+    const double mul = (DBL && (k == 0 || k == g.nzn - 1)) ? 2. : 1.;
 #pragma unroll
-    for (int f = 0; f <= NV; f++) out.p[f][t] = s[f] * m;
+    for (int f = 0; f <= NV; f++) out.p[f][t] = s[f] * mul;
   }
 }
 
@@ -421,14 +464,6 @@ __global__ void k_grid2par(Geometry g, const double *__restrict__ par, int64_t c
 
 }  // namespace
 
-size_t scan_temp_bytes(Ctx *c, int64_t n) {
-  size_t need = 0;
-  if (hipcub::DeviceScan::ExclusiveSum(nullptr, need, (const int32_t *)nullptr, (int32_t *)nullptr,
-                                       (int)n, c->stream) != hipSuccess)
-    return 0;
-  return need;
-}
-
 int scan_exclusive_i32(Ctx *c, const int32_t *in, int32_t *out, int64_t n) {
   size_t need = 0;
   PMPIC_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, need, in, out, (int)n, c->stream));
@@ -443,7 +478,7 @@ int scan_exclusive_i32(Ctx *c, const int32_t *in, int32_t *out, int64_t n) {
   return PMPIC_OK;
 }
 
-// the context's own binning buffers (the scan's temporary storage is grown on demand)
+// the context's own binning buffers
 static BinWork ctx_work(Ctx *c) {
   BinWork w;
   w.cell = c->cell;
@@ -451,57 +486,63 @@ static BinWork ctx_work(Ctx *c) {
   w.count = c->cell_count;
   w.start = c->cell_start;
   w.sorted = c->sorted;
+  w.cursor = c->cell_count + c->ncell;
   w.partial = c->partial;
-  w.scan_tmp = nullptr;  // c->scan_tmp, grown by scan_exclusive_i32
-  w.scan_bytes = 0;
   return w;
 }
 
+// bins n parcels; count and cursor must be zero, and the accumulation that follows zeroes them
 int bin_parcels_ws(Ctx *c, int64_t n, const BinWork &w) {
   const Geometry &g = c->g;
-  const int64_t nc1 = c->ncell + 1;
-  hipLaunchKernelGGL(k_fill_i32, dim3(cdiv(nc1, TPB)), dim3(TPB), 0, c->stream, w.count, nc1, 0);
-  if (n > 0)
-    hipLaunchKernelGGL(k_bin_count, dim3(cdiv(n, (int64_t)TPB * BIN_SEQ)), dim3(TPB), 0, c->stream, g,
+  auto count = [&](auto kernel, int seq) {
+    hipLaunchKernelGGL(kernel, dim3(cdiv(n, (int64_t)TPB * seq)), dim3(TPB), 0, c->stream, g,
                        c->par + FX * c->cap, c->par + FY * c->cap, c->par + FZ * c->cap, n,
                        w.cell, w.rank, w.count, c->dsc);
-  if (w.scan_tmp) {
-    size_t have = w.scan_bytes;
-    PMPIC_CHECK(hipcub::DeviceScan::ExclusiveSum(w.scan_tmp, have, w.count, w.start, (int)nc1,
-                                                 c->stream));
-  } else {
-    PMPIC_TRY(scan_exclusive_i32(c, w.count, w.start, nc1));
-  }
+  };
+  // wavefronts of 16 groups from 2^22 parcels (4,096 of them, four a SIMD), of four from 2^19
+  if (n >= (int64_t)1 << 22) count(k_bin_count<16>, 16);
+  else if (n >= (int64_t)1 << 19) count(k_bin_count<4>, 4);
+  else if (n > 0) count(k_bin_count<1>, 1);
+  hipLaunchKernelGGL(k_bin_alloc, dim3(cdiv(c->ncell, TPB * ALLOC_CELLS)), dim3(TPB), 0, c->stream,
+                     w.count, c->ncell, w.start, w.cursor);
   if (n > 0)
     hipLaunchKernelGGL(k_bin_scatter, dim3(cdiv(n, TPB)), dim3(TPB), 0, c->stream, w.cell, w.rank,
                        w.start, n, w.sorted);
-  hipLaunchKernelGGL(k_bin_sort_big, dim3(cdiv(c->ncell, TPB)), dim3(TPB), 0, c->stream, w.start,
-                     c->ncell, ROWS_MIX, w.sorted);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
 
 int bin_parcels(Ctx *c, int64_t n) { return bin_parcels_ws(c, n, ctx_work(c)); }
 
-template <int MODE, int NV, int ROWS>
-static void launch_accum_lds(Ctx *c, const double *var, double *partial, double *partial2,
-                             int32_t *npc) {
-  hipLaunchKernelGGL((k_cell_accum_lds<MODE, NV, ROWS>), dim3(cdiv(c->ncell, TILE)), dim3(TILE * 8), 0,
-                     c->stream, c->g, c->par, c->cap, var, c->cell_start, c->sorted, c->ncell,
-                     partial, partial2, npc);
+static dim3 accum_tiles(const Ctx *c) {
+  return dim3((unsigned)(cdiv(c->g.nx, 8) * c->g.ny * c->g.ncz));
+}
+
+template <int MODE, int NV>
+static void launch_accum(Ctx *c, const BinWork &w, const double *var, double *partial,
+                         double *partial2, int32_t *npc, uint8_t *tileres, int zero) {
+  hipLaunchKernelGGL((k_cell_accum<MODE, NV>), accum_tiles(c), dim3(64), 0, c->stream, c->g, c->par,
+                     c->cap, var, w.count, w.start, w.sorted, w.rank, partial, partial2, npc,
+                     tileres, w.cursor, zero);
+}
+
+template <int NV, bool NORM, bool DBL>
+static void launch_node_sum(Ctx *c, const double *partial, const OutTable &out,
+                            const uint8_t *tileres) {
+  const int64_t nnode = (int64_t)c->g.nzn * c->g.ny * c->g.nx;
+  hipLaunchKernelGGL((k_node_sum<NV, NORM, DBL>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream,
+                     c->g, partial, out, tileres);
 }
 
 int par2grid_fused(Ctx *c, int64_t n) {
   PMPIC_TRY(bin_parcels(c, n));
-  const int64_t ncell = c->ncell;
-  PMPIC_TRY(launch_timed(c, T_ACCUM, k_cell_accum_lds<ACC_P2G, 4, ROWS_P2G>,
-                         dim3(cdiv(c->ncell, TILE)), dim3(TILE * 8), 0, c->g, c->par, c->cap,
-                         nullptr, c->cell_start, c->sorted, c->ncell, c->partial, nullptr,
-                         nullptr));
-  OutTable table = {{c->grid[GP], c->grid[GQ], c->grid[GR], c->grid[GB], nullptr, nullptr}};
-  const int64_t nnode = (int64_t)c->g.nzn * c->g.ny * c->g.nx;
-  hipLaunchKernelGGL((k_node_sum<4, true>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, c->g,
-                     c->partial, ncell, table);
+  const BinWork w = ctx_work(c);
+  PMPIC_TRY(launch_timed(c, T_ACCUM, k_cell_accum<ACC_P2G, 4>, accum_tiles(c), dim3(64), 0, c->g,
+                         c->par, c->cap, nullptr, w.count, w.start, w.sorted, w.rank, w.partial,
+                         nullptr, nullptr, nullptr, w.cursor, 1));
+  launch_node_sum<4, true, true>(
+      c, w.partial, {{c->grid[GP], c->grid[GQ], c->grid[GR], c->grid[GB], nullptr, nullptr}},
+      nullptr);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
@@ -509,14 +550,9 @@ int par2grid_fused(Ctx *c, int64_t n) {
 int par2grid_single_ws(Ctx *c, int64_t n, const double *d_var, double *d_grid,
                        const BinWork &w) {
   PMPIC_TRY(bin_parcels_ws(c, n, w));
-  const int64_t ncell = c->ncell;
-  hipLaunchKernelGGL((k_cell_accum_lds<ACC_SINGLE, 1, ROWS_P2G>), dim3(cdiv(ncell, TILE)),
-                     dim3(TILE * 8), 0, c->stream, c->g, c->par, c->cap, d_var, w.start, w.sorted,
-                     ncell, w.partial, nullptr, nullptr);
-  OutTable table = {{d_grid, nullptr, nullptr, nullptr, nullptr, nullptr}};
-  const int64_t nnode = (int64_t)c->g.nzn * c->g.ny * c->g.nx;
-  hipLaunchKernelGGL((k_node_sum<1, true>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, c->g,
-                     w.partial, ncell, table);
+  launch_accum<ACC_SINGLE, 1>(c, w, d_var, w.partial, nullptr, nullptr, nullptr, 1);
+  launch_node_sum<1, true, true>(c, w.partial,
+                                 {{d_grid, nullptr, nullptr, nullptr, nullptr, nullptr}}, nullptr);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
@@ -543,11 +579,10 @@ __global__ void k_hgliq(Geometry g, double *__restrict__ B, const double *__rest
 
 int dump_grids_f64(Ctx *c, int64_t n) {
   PMPIC_TRY(bin_parcels(c, n));
-  launch_accum_lds<ACC_DUMP, 5, ROWS_MIX>(c, nullptr, c->partial, nullptr, nullptr);
-  OutTable out = {{c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR], nullptr}};
-  const int64_t nnode = (int64_t)c->g.nzn * c->g.ny * c->g.nx;
-  hipLaunchKernelGGL((k_node_sum<5, true>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, c->g,
-                     c->partial, c->ncell, out);
+  launch_accum<ACC_DUMP, 5>(c, ctx_work(c), nullptr, c->partial, nullptr, nullptr, nullptr, 1);
+  launch_node_sum<5, true, true>(
+      c, c->partial, {{c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR], nullptr}},
+      nullptr);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
@@ -573,27 +608,24 @@ int grid2par_single(Ctx *c, int64_t n, const double *d_grid, double *d_var) {
 // z-boundary doubling of :141-152; kres[0..5] hold the residual grids before the new-parcel
 // correction of :202-207 and before their own doubling (:229-240).
 // Without a residual buffer (partial2 null: a context too large for both) the kept and the
-// residual sums take one pass each over `partial`, with the same sums.
+// residual sums take one pass each over `partial`, with the same sums.  cellflag holds the
+// residual flags of the tiles (at most one a cell).
 int mixing_grids(Ctx *c, int64_t n) {
   PMPIC_TRY(bin_parcels(c, n));
-  const int64_t ncell = c->ncell;
-  OutTable kept = {{c->grid[GVOL], c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ],
-                    c->grid[GR]}};
-  OutTable res = {{c->kres[0], c->kres[1], c->kres[2], c->kres[3], c->kres[4], c->kres[5]}};
-  const int64_t nnode = (int64_t)c->g.nzn * c->g.ny * c->g.nx;
+  const BinWork w = ctx_work(c);
+  const OutTable kept = {{c->grid[GVOL], c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ],
+                          c->grid[GR]}};
+  const OutTable res = {{c->kres[0], c->kres[1], c->kres[2], c->kres[3], c->kres[4], c->kres[5]}};
+  uint8_t *flags = c->cellflag;
   if (c->partial2) {
-    launch_accum_lds<ACC_MIX_KEEP, 5, ROWS_MIX>(c, nullptr, c->partial, c->partial2, c->npercell);
-    hipLaunchKernelGGL((k_node_sum<5, false>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream,
-                       c->g, c->partial, ncell, kept);
-    hipLaunchKernelGGL((k_node_sum<5, false, false>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0,
-                       c->stream, c->g, c->partial2, ncell, res);
+    launch_accum<ACC_MIX, 5>(c, w, nullptr, c->partial, c->partial2, c->npercell, flags, 1);
+    launch_node_sum<5, false, true>(c, c->partial, kept, nullptr);
+    launch_node_sum<5, false, false>(c, c->partial2, res, flags);
   } else {
-    launch_accum_lds<ACC_MIX_KEEP, 5, ROWS_MIX>(c, nullptr, c->partial, nullptr, c->npercell);
-    hipLaunchKernelGGL((k_node_sum<5, false>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream,
-                       c->g, c->partial, ncell, kept);
-    launch_accum_lds<ACC_MIX_KEEP, 5, ROWS_MIX>(c, nullptr, nullptr, c->partial, nullptr);
-    hipLaunchKernelGGL((k_node_sum<5, false, false>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0,
-                       c->stream, c->g, c->partial, ncell, res);
+    launch_accum<ACC_MIX, 5>(c, w, nullptr, c->partial, nullptr, c->npercell, flags, 0);
+    launch_node_sum<5, false, true>(c, c->partial, kept, nullptr);
+    launch_accum<ACC_MIX, 5>(c, w, nullptr, nullptr, c->partial, nullptr, nullptr, 1);
+    launch_node_sum<5, false, false>(c, c->partial, res, flags);
   }
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;

@@ -1,16 +1,16 @@
 // pmpic_par2grid_noalloc: par2grid of a device array that allocates nothing.
 //
-// The same binning and per-cell sums as pmpic_par2grid (k_bin_count, the exclusive scan,
-// k_bin_scatter, k_cell_accum_lds, k_node_sum), so the grid it returns is bit-identical to that
-// entry point's.  Its working memory (cell and rank of each parcel, the per-cell counts and
-// offsets, the cell-sorted parcel list, the corner partial sums, the interior grid and the
-// scan's temporary storage) is carved out of `scratch`, one static device array per GPU that
-// lives until the process ends, instead of the context's buffers or hipMalloc.  Inputs and the
+// The same binning and per-cell sums as pmpic_par2grid (k_bin_count, k_bin_alloc, k_bin_scatter,
+// k_cell_accum, k_node_sum), so the grid it returns is bit-identical to that entry point's.  Its
+// working memory (cell and rank of each parcel, the per-cell counts and offsets, the cell-sorted
+// parcel list, the corner partial sums and the interior grid) is carved out of `scratch`, one
+// static device array per GPU that lives until the process ends, instead of the context's buffers
+// or hipMalloc.  Inputs and the
 // output are the caller's device arrays.
 //
 // Every call on a GPU shares that GPU's array: calls that overlap on one GPU (two host threads,
-// or two streams) race on it.  The per-cell counts are cleared by a fill kernel on each call;
-// every other region is written in full before it is read, so nothing from an earlier call
+// or two streams) race on it.  The per-cell counts are zero at load and each call leaves them zero
+// again; every other region is written in full before it is read, so nothing from an earlier call
 // leaks into a later one.
 #include "common.h"
 
@@ -32,13 +32,13 @@ constexpr size_t NA_RANK = NA_CELL + na_round(4 * NA_MAX_PARCELS);
 constexpr size_t NA_SORTED = NA_RANK + na_round(4 * NA_MAX_PARCELS);
 constexpr size_t NA_COUNT = NA_SORTED + na_round(4 * NA_MAX_PARCELS);
 constexpr size_t NA_START = NA_COUNT + na_round(4 * (NA_MAX_CELLS + 1));
-// 8 corners x (weight, weight * value) per cell
+// at most 12 doubles a cell of x-combined (weight, weight * value) sums
 constexpr size_t NA_PARTIAL = NA_START + na_round(4 * (NA_MAX_CELLS + 1));
 // interior grid [nzn][ny][nx]: nzn * ny * nx = ncell + nx * ny <= 2 ncell since nz >= 2
 constexpr size_t NA_GRID = NA_PARTIAL + na_round(8 * 16 * NA_MAX_CELLS);
-constexpr size_t NA_SCAN = NA_GRID + na_round(8 * 2 * NA_MAX_CELLS);
-constexpr size_t NA_SCAN_BYTES = 256 * 1024;
-constexpr size_t NA_TOTAL = NA_SCAN + NA_SCAN_BYTES;
+constexpr size_t NA_CURSOR = NA_GRID + na_round(8 * 2 * NA_MAX_CELLS);
+// (the size stays what pmpic_hip.h publishes)
+constexpr size_t NA_TOTAL = NA_CURSOR + 256 * 1024;
 static_assert(NA_TOTAL == PMPIC_NOALLOC_SCRATCH_BYTES, "scratch size in pmpic_hip.h");
 
 // Host code must not pass `scratch` itself to a kernel: on the host the name is a stand-in, not
@@ -76,7 +76,6 @@ extern "C" int pmpic_par2grid_noalloc(pmpic_ctx *ctx, const double *var, double 
   if (!ctx || !var || !grid || ctx->c.precision != 0) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
   if (c->n > NA_MAX_PARCELS || c->ncell > NA_MAX_CELLS) return PMPIC_ERR_ARG;
-  if (scan_temp_bytes(c, c->ncell + 1) > NA_SCAN_BYTES) return PMPIC_ERR_ARG;
   unsigned char *base = nullptr;
   PMPIC_TRY(scratch_addr(c->device, &base));
   BinWork w;
@@ -86,8 +85,7 @@ extern "C" int pmpic_par2grid_noalloc(pmpic_ctx *ctx, const double *var, double 
   w.count = reinterpret_cast<int32_t *>(base + NA_COUNT);
   w.start = reinterpret_cast<int32_t *>(base + NA_START);
   w.partial = reinterpret_cast<double *>(base + NA_PARTIAL);
-  w.scan_tmp = base + NA_SCAN;
-  w.scan_bytes = NA_SCAN_BYTES;
+  w.cursor = reinterpret_cast<int32_t *>(base + NA_CURSOR);
   double *interior = reinterpret_cast<double *>(base + NA_GRID);
   PMPIC_TRY(par2grid_single_ws(c, c->n, var, interior, w));
   PMPIC_TRY(grid_to_ref(c, interior, 1, grid));

@@ -1,0 +1,95 @@
+"""The kernels at the edges of their tiles, chunks and dispatch rules, against the oracle.
+
+par2grid: x rows shorter, equal and longer than the eight-cell tiles; cells of 0, 1, 7, 8, 9, 63,
+64, 65 and 130 parcels (chunks of eight, ordered lists of up to 64 in LDS, longer in memory), with
+the parcels in and out of slot order, and parcel counts either side of the binning walks' rule.
+The bar is 1e-12 of the field's maximum, as for every FP64 par2grid; each cell holds few enough
+parcels that sums of 1e3 terms with 1e-16 rounding stay far below it.
+
+The column kernel: levels per column below, at and above its read-ahead (8), rows of wavenumber
+blocks below and above a wavefront's 16, whole steps, 1e-12 (FP64) and 1e-5 (FP32-bulk against
+FP64, that form's bar).
+"""
+import numpy as np
+import pytest
+
+from tests.cases import box, rel_err, thermal_case
+
+pytestmark = pytest.mark.gpu
+
+OCCUPANCY = (0, 1, 7, 8, 9, 63, 64, 65, 130)
+
+
+def _pair(oracle_mod, shape, ic, precision=0):
+    from pmpic_amd.lib import Context
+    b = box(*shape)
+    args = (*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+            2 * len(ic["x"]) + 64)
+    o = oracle_mod.Oracle(*args, 0.01, 0.01, 0.5)
+    g = Context(*args, precision=precision)
+    o.set_parcels(ic)
+    g.set_parcels(ic)
+    return o, g
+
+
+@pytest.mark.parametrize("shuffled", [False, True])
+@pytest.mark.parametrize("nx", [2, 3, 8, 9, 10, 15, 16, 18, 25])
+def test_par2grid_tiles_and_occupancy(oracle_mod, nx, shuffled, bar):
+    shape = (nx, 4, 3)
+    b = box(*shape)
+    rng = np.random.default_rng(nx)
+    d = [(b[k + "max"] - b[k + "min"]) / n for k, n in zip("xyz", shape)]
+    at = []
+    for c in range(nx * 4 * 3):
+        m = OCCUPANCY[c % len(OCCUPANCY)]
+        ijk = np.array([c % nx, c // nx % 4, c // (nx * 4)])
+        at.append((ijk + rng.uniform(0.01, 0.99, (m, 3))) * d)
+    at = np.concatenate(at)
+    n = len(at)
+    if shuffled:
+        at = at[rng.permutation(n)]
+    ic = dict(x=at[:, 0].copy(), y=at[:, 1].copy(), z=at[:, 2].copy(),
+              vol=rng.uniform(0.5, 1.0, n) * np.prod(d) / 8)
+    o, g = _pair(oracle_mod, shape, ic)
+    o.cache_weights()
+    for _ in range(2):  # the second call finds what the first left behind
+        var = rng.standard_normal(n)
+        bar("par2grid", rel_err(g.par2grid(var)[2:-2, 2:-2], o.par2grid(var)[2:-2, 2:-2]), 1e-12)
+    g.close()
+
+
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+@pytest.mark.parametrize("most", [1 << 19, 1 << 22])
+def test_par2grid_binning_walks(oracle_mod, most, extra, bar):
+    """Parcel counts at the changes of the binning's walk length."""
+    shape = (32, 32, 32)
+    rng = np.random.default_rng(1)
+    b = box(*shape)
+    n = most + extra
+    ic = {k: rng.uniform(b[k + "min"], b[k + "max"] * (1 - 1e-9), n) for k in "xyz"}
+    ic["vol"] = np.full(n, 1e-3)
+    o, g = _pair(oracle_mod, shape, ic)
+    o.cache_weights()
+    var = np.cos(ic["x"]) * ic["z"]
+    bar("par2grid", rel_err(g.par2grid(var)[2:-2, 2:-2], o.par2grid(var)[2:-2, 2:-2]), 1e-12)
+    g.close()
+
+
+@pytest.mark.parametrize("shape", [(8, 8, 2), (8, 9, 3), (15, 8, 7), (16, 10, 8), (30, 6, 9),
+                                   (32, 8, 15), (36, 5, 16), (64, 4, 17)])
+def test_column_kernel_lengths(oracle_mod, shape, bar):
+    ic = thermal_case(*shape, 2, vort=1.0)
+    o, g = _pair(oracle_mod, shape, ic)
+    _, f = _pair(oracle_mod, shape, ic, precision=1)
+    for _ in range(2):
+        o.step()
+        g.step()
+        f.step()
+    for k in ("u", "v", "w", "p", "q", "r"):
+        want = o.grid(k)[2:-2, 2:-2]
+        bar(k, rel_err(g.grid(k)[2:-2, 2:-2], want), 1e-12)
+        bar(k + "32", rel_err(f.grid(k)[2:-2, 2:-2], want), 1e-5)
+    for k in ("u_s", "v_s", "w_s"):
+        bar(k, rel_err(g.spectral(k), o.spec(k)), 1e-12)
+    g.close()
+    f.close()
