@@ -1046,13 +1046,6 @@ __global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, int64_
 }
 
 // ---- splitting (parcel_splitting.F90:76-131, then the haloswap's wrap and reflection) ----
-__global__ void k32_split_flags(const float *__restrict__ F, int64_t cap, int64_t n,
-                                uint8_t *__restrict__ flag) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  flag[p] = (F[B_STRETCH * cap + p] > 4.f) ? 1 : 0;
-}
-
 __global__ void k32_split_apply(Geometry g, Bulk32 b, int64_t cap, int64_t n, Scale32 sc3,
                                 const int32_t *__restrict__ parents, int64_t nsplit,
                                 DevScalars *sc) {
@@ -1105,31 +1098,6 @@ __global__ void k32_split_apply(Geometry g, Bulk32 b, int64_t cap, int64_t n, Sc
 }
 
 // ---- mixing (parcel_mixing.F90:157-389) ----
-// KPT parcels per thread, at stride TPB (each a coalesced pass), the loads issued together
-constexpr int KPT = 4;
-__global__ void k32_keep_flags(const float *__restrict__ F, int64_t cap, int64_t n, float vmin,
-                               uint8_t *__restrict__ keep) {
-  const int64_t p0 = (int64_t)blockIdx.x * (TPB * KPT) + threadIdx.x;
-  const float *vol = F + (int64_t)B_VOL * cap;
-  float v[KPT];
-#pragma unroll
-  for (int k = 0; k < KPT; k++) v[k] = vol[min(p0 + (int64_t)k * TPB, n - 1)];
-#pragma unroll
-  for (int k = 0; k < KPT; k++)
-    if (p0 + (int64_t)k * TPB < n) keep[p0 + (int64_t)k * TPB] = (v[k] < vmin) ? 0 : 1;
-}
-
-__global__ void k32_newcell_flags(Geometry g, const int32_t *__restrict__ npercell,
-                                  uint8_t *__restrict__ cellflag, int64_t ncell) {
-  const int64_t ord = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ord >= ncell) return;
-  const int k = (int)(ord % g.ncz);
-  const int j = (int)((ord / g.ncz) % g.ny);
-  const int i = (int)(ord / ((int64_t)g.ncz * g.ny));
-  const int64_t c = ((int64_t)k * g.ny + j) * g.nx + i;
-  cellflag[ord] = (npercell[c] < 3) ? 1 : 0;
-}
-
 struct Mix32 {
   const float *G[6];  // kept vol, b, h, p, q, r (folded, doubled)
   float *R[6];        // residual vol .. r; after k32_mix_residual, divided by the kept volume
@@ -1738,11 +1706,11 @@ int b32_split(Ctx *c) {
   c->b32.p2g_reuse = false;
   if (n > 0) {
     // the stage-4 RK kernel already flagged the parcels to split
-    if (!c->split_flags_fresh)
-      hipLaunchKernelGGL(k32_split_flags, dim3(cdiv(n, TPB)), dim3(TPB), 0, c->stream,
-                         c->b32.f, c->cap, n, c->flag);
+    if (c->split_flags_fresh)
+      PMPIC_TRY(compact_flags(c, c->flag, 1, n, c->list_b, &c->dsc->nsplit));
+    else
+      PMPIC_TRY(split_list(c, c->b32.f + (int64_t)B_STRETCH * c->cap, n));
     c->split_flags_fresh = 0;
-    PMPIC_TRY(compact_flags(c, c->flag, 1, n, c->list_b, &c->dsc->nsplit));
   } else {
     c->hsc.nsplit = 0;
     PMPIC_CHECK(hipMemcpyAsync(&c->dsc->nsplit, &c->hsc.nsplit, sizeof(int64_t),
@@ -1825,13 +1793,7 @@ int b32_mix(Ctx *c) {
   // step reads them there, so b32_export_grid widens them when one is exported
   for (int f = 0; f < 6; f++) b.kept_pending[f] = true;
   for (int f = 0; f < 4; f++) b.p2g_pending[f] = false;
-  if (norig > 0)
-    hipLaunchKernelGGL(k32_keep_flags, dim3(cdiv(norig, TPB * KPT)), dim3(TPB), 0, c->stream, b.f,
-                       c->cap, norig, vmin, c->flag);
-  PMPIC_TRY(compact_flags(c, c->flag, 0, norig, c->list_a, &c->dsc->nzero));
-  hipLaunchKernelGGL(k32_newcell_flags, dim3(cdiv(c->ncell, TPB)), dim3(TPB), 0, c->stream, g,
-                     c->npercell, c->cellflag, c->ncell);
-  PMPIC_TRY(compact_flags(c, c->cellflag, 1, c->ncell, c->sorted, &c->dsc->nadd));
+  PMPIC_TRY(mix_lists(c, (const float *)b.f + (int64_t)B_VOL * c->cap, vmin, norig, nullptr));
   PMPIC_TRY(sync_scalars(c));
   const int64_t Z = c->hsc.nzero, nadd = c->hsc.nadd;
   Mix32 mg = {{b.mgrid[0], b.mgrid[1], b.mgrid[2], b.mgrid[3], b.mgrid[4], b.mgrid[5]},
@@ -1868,7 +1830,8 @@ int b32_mix(Ctx *c) {
     }
     if (slast + 1 > np) np = slast + 1;
   }
-  PMPIC_TRY(sync_scalars(c));
+  // what k32_mix_new raised (nothing else since the last read-back raises anything)
+  if (nadd > 0) PMPIC_TRY(sync_scalars(c));
   c->last_removed = Z;
   c->last_added = nadd;
   if (np == norig) {

@@ -186,7 +186,7 @@ int free_all(Ctx *c) {
   hipFree(c->cell); hipFree(c->rank); hipFree(c->sorted); hipFree(c->flag);
   hipFree(c->list_a); hipFree(c->list_b);
   hipFree(c->cell_count); hipFree(c->cell_start); hipFree(c->partial); hipFree(c->partial2);
-  hipFree(c->npercell); hipFree(c->cellflag);
+  hipFree(c->npercell); hipFree(c->cellflag); hipFree(c->ctouch);
   for (int g = 0; g < NGRIDS; g++) hipFree(c->grid[g]);
   hipFree(c->rec); hipFree(c->rec32);
   for (int g = 0; g < 8; g++) hipFree(c->gtmp[g]);
@@ -264,6 +264,7 @@ int create(const pmpic_config *cf, Ctx *c) {
   if (c->precision == 1) PMPIC_TRY(dalloc(&c->partial2, pdoubles));
   PMPIC_TRY(dalloc(&c->npercell, c->ncell));
   PMPIC_TRY(dalloc(&c->cellflag, c->ncell));
+  if (c->precision == 0) PMPIC_TRY(dalloc(&c->ctouch, c->ncell));
   for (int i = 0; i < GDP; i++) PMPIC_TRY(dalloc(&c->grid[i], c->gsz));
   if (c->precision == 1) PMPIC_TRY(dalloc(&c->rec32, 2 * c->gsz));
   else PMPIC_TRY(dalloc(&c->rec, 3 * c->gsz));
@@ -684,8 +685,10 @@ int pmpic_step(pmpic_ctx *ctx, int32_t nsteps) {
   Ctx *c = &ctx->c;
   for (int s = 0; s < nsteps; s++) {
     c->defer_status = 1;
+    c->whole_step = c->rkstep == 1;
     int st = step_once(ctx);
     c->defer_status = 0;
+    c->whole_step = 0;
     const int ks = take_status(c);
     if (st == PMPIC_OK) st = ks;
     if (st != PMPIC_OK) return st;

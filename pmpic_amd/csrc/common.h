@@ -136,6 +136,7 @@ struct Ctx {
   int precision;
   int device;
   int defer_status;      // set inside pmpic_step: kernel status checked once per step
+  int whole_step;        // set inside pmpic_step where its four stages are 1, 2, 3, 4
   int split_flags_fresh; // flag[] holds the split test of the last stage-4 RK update
   int splitting_enabled, mixing_enabled;
   int64_t last_split, last_removed, last_added;
@@ -157,6 +158,7 @@ struct Ctx {
                                       // FP64 form (then mixing takes two passes over partial)
   int32_t *npercell;                  // ncell
   uint8_t *cellflag;                  // ncell
+  uint8_t *ctouch;                    // ncell, FP64 form: cells whose parcels absorb a residual
   // grids (interior [nzn][ny][nx])
   int64_t gsz, ssz, csz;              // grid; spectral (planes); complex transform intermediate
   int64_t bsz;                        // spectral (tiles)
@@ -425,6 +427,13 @@ int parcel_split(Ctx *c);
 int parcel_mix(Ctx *c);
 int compact_flags(Ctx *c, const uint8_t *flags, uint8_t want, int64_t n, int32_t *out,
                   int64_t *d_count);
+// the parcels to split (list_b, DevScalars::nsplit), from their stretch; n > 0
+template <typename T>
+int split_list(Ctx *c, const T *stretch, int64_t n);
+// mixing's parcels below vmin (flag, list_a, nzero) and cells short of parcels (cellflag, sorted,
+// nadd); clears ctouch (may be null)
+template <typename T>
+int mix_lists(Ctx *c, const T *vol, T vmin, int64_t n, uint8_t *ctouch);
 // bulk32.hip (FP32-bulk form)
 int b32_alloc(Ctx *c);
 void b32_free(Ctx *c);

@@ -20,7 +20,10 @@
 //    compaction and permutation is deterministic.
 #include "common.h"
 
+#include <float.h>
 #include <string.h>
+
+#include <algorithm>
 
 #include <hipcub/hipcub.hpp>
 #include <math.h>
@@ -31,25 +34,6 @@ namespace {
 
 constexpr int TPB = 256;
 constexpr int NWAVE = TPB / 64;
-
-// exclusive rank of `pred` among the block's threads (thread order) and the block total
-__device__ __forceinline__ void block_rank(bool pred, int &rank, int &total, int *lds) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const unsigned long long m = __ballot(pred);
-  const int below = __popcll(m & ((1ull << lane) - 1ull));
-  if (lane == 0) lds[wave] = __popcll(m);
-  __syncthreads();
-  int off = 0, tot = 0;
-#pragma unroll
-  for (int w = 0; w < NWAVE; w++) {
-    const int v = lds[w];
-    if (w < wave) off += v;
-    tot += v;
-  }
-  __syncthreads();
-  rank = off + below;
-  total = tot;
-}
 
 // haloswap direction of a parcel (haloswap.F90:296-437); 0 = stays
 __device__ __forceinline__ int direction(const Geometry &g, double x, double y) {
@@ -65,17 +49,34 @@ __device__ __forceinline__ int direction(const Geometry &g, double x, double y) 
   return 0;
 }
 
-// per-block direction counts: rows 0..7 = directions 1..8, row 8 = all crossing parcels
-__device__ __forceinline__ void write_dir_counts(int dir, bool active, int32_t *blk, int64_t nblk,
-                                                 int *lds) {
-  for (int d = 1; d <= 8; d++) {
-    int r, t;
-    block_rank(active && dir == d, r, t, lds);
-    if (threadIdx.x == 0) blk[(int64_t)(d - 1) * nblk + blockIdx.x] = t;
+// Direction counts of a block: rows 0..7 = directions 1..8, row 8 = all crossing parcels.  Each
+// wavefront's counts, one barrier, nine threads' sums; a wavefront none of whose parcels cross
+// (almost every one) writes zeros.
+__device__ __forceinline__ void wave_dir_counts(int dir, int32_t (*lds)[NWAVE]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int mine = 0;
+  if (__any(dir != 0)) {
+#pragma unroll
+    for (int d = 1; d <= 8; d++) {
+      const int k = __popcll(__ballot(dir == d));
+      if (lane == d - 1) mine = k;
+    }
+    const int k = __popcll(__ballot(dir != 0));
+    if (lane == 8) mine = k;
   }
-  int r, t;
-  block_rank(active && dir != 0, r, t, lds);
-  if (threadIdx.x == 0) blk[(int64_t)8 * nblk + blockIdx.x] = t;
+  if (lane < 9) lds[lane][wave] = mine;
+}
+
+__device__ __forceinline__ void write_dir_counts(int dir, int32_t *blk, int64_t nblk,
+                                                 int32_t (*lds)[NWAVE]) {
+  wave_dir_counts(dir, lds);
+  __syncthreads();
+  if (threadIdx.x < 9) {
+    int t = 0;
+#pragma unroll
+    for (int w = 0; w < NWAVE; w++) t += lds[threadIdx.x][w];
+    blk[(int64_t)threadIdx.x * nblk + blockIdx.x] = t;
+  }
 }
 
 // grid2par of the six tendencies (vort2vel.F90:325-327, vorticity_tendency.F90:273-275) at the
@@ -83,14 +84,18 @@ __device__ __forceinline__ void write_dir_counts(int dir, bool active, int32_t *
 // reflection (haloswap.F90:440-456) and the haloswap direction of each parcel.  At stage 4 the
 // stretch increment of parcel_splitting.F90:64-73 is applied too (it only needs the updated
 // vorticity and the stage-4 tendencies of the same parcel).
+//
+// Bound by the parcel arrays' traffic.  keep_k: the stage's tendencies are stored too.  Inside a
+// whole step only stage 4's are, the ones a caller can see: 48 of stage 2's 265 bytes a parcel
+// (57 M parcels: 2.93 -> 2.43 ms, 4.9 TB/s).
 template <int STAGE>
 __global__ void __launch_bounds__(TPB) k_rk_stage(Geometry g, double *__restrict__ par, int64_t cap,
                                                   int64_t n, const double2 *__restrict__ rec,
-                                                  int stretch,
+                                                  int stretch, int keep_k,
                                                   DevScalars *sc,
                                                   uint8_t *__restrict__ flag,
                                                   int32_t *__restrict__ blk, int64_t nblk) {
-  __shared__ int lds[NWAVE];
+  __shared__ int32_t lds[9][NWAVE];
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool active = p < n;
   int dir = 0;
@@ -170,7 +175,7 @@ __global__ void __launch_bounds__(TPB) k_rk_stage(Geometry g, double *__restrict
       yv[2] = z;
 #pragma unroll
       for (int f = 0; f < 6; f++) {
-        st_stream(&par[(FDXDT + f) * cap + p], kv[f]);
+        if (STAGE == 4 || keep_k) st_stream(&par[(FDXDT + f) * cap + p], kv[f]);
         if (STAGE == 1) st_stream(&par[(f < 3 ? FXO + f : FPO + f - 3) * cap + p], yo[f]);
         st_stream(&par[(f < 3 ? FXF + f : FPF + f - 3) * cap + p], yfn[f]);
         st_stream(&par[(FX + f) * cap + p], yv[f]);
@@ -185,7 +190,7 @@ __global__ void __launch_bounds__(TPB) k_rk_stage(Geometry g, double *__restrict
     }
     flag[p] = (uint8_t)dir;
   }
-  write_dir_counts(dir, active, blk, nblk, lds);
+  write_dir_counts(dir, blk, nblk, lds);
 }
 
 // direction classification only (haloswap after splitting): reflect, then tag
@@ -193,19 +198,76 @@ __global__ void __launch_bounds__(TPB) k_reflect_classify(Geometry g, double *__
                                                           int64_t cap, int64_t n,
                                                           uint8_t *__restrict__ flag,
                                                           int32_t *__restrict__ blk, int64_t nblk) {
-  __shared__ int lds[NWAVE];
+  __shared__ int32_t lds[9][NWAVE];
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool active = p < n;
   int dir = 0;
   if (active) {
-    double z = par[FZ * cap + p];
-    if (z < g.zmin_h) z = g.zmin_h + (g.zmin_h - z);
-    else if (z > g.zmax_h) z = g.zmax_h - (z - g.zmax_h);
-    par[FZ * cap + p] = z;
+    const double z = par[FZ * cap + p];
+    if (z < g.zmin_h) par[FZ * cap + p] = g.zmin_h + (g.zmin_h - z);
+    else if (z > g.zmax_h) par[FZ * cap + p] = g.zmax_h - (z - g.zmax_h);
     dir = direction(g, par[FX * cap + p], par[FY * cap + p]);
     flag[p] = (uint8_t)dir;
   }
-  write_dir_counts(dir, active, blk, nblk, lds);
+  write_dir_counts(dir, blk, nblk, lds);
+}
+
+// Exclusive prefix sums of each of the nine rows of block counts, and the rows' totals (row 8's
+// is the number of crossing parcels), a workgroup a row: every load issued at once (16
+// counts a thread, four side by side) and one barrier.  One launch, 4.0 us at 30 blocks and 4.6
+// at 3,456, up to the blocks it holds; above them the device-wide scan of all nine rows as one
+// (two launches, and one for the total: 8 us and the gaps between them).
+constexpr int SCAN_TPB = 1024, SCAN_TILES = 4, SCAN_MAX = SCAN_TILES * 4 * SCAN_TPB;
+__global__ void __launch_bounds__(SCAN_TPB) k_hs_scan(const int32_t *__restrict__ blk,
+                                                      int32_t *__restrict__ pre, int nblk,
+                                                      int32_t *__restrict__ tot, DevScalars *sc) {
+  constexpr int NW = SCAN_TPB / 64;
+  static_assert(SCAN_TILES * NW == 64, "a (tile, wavefront) pair a lane");
+  __shared__ int32_t wsum[SCAN_TILES * NW];
+  const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  blk += (int64_t)row * nblk;
+  pre += (int64_t)row * nblk;
+  int32_t v[SCAN_TILES][4], incl[SCAN_TILES];
+#pragma unroll
+  for (int t = 0; t < SCAN_TILES; t++)
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int i = 4 * (t * SCAN_TPB + (int)threadIdx.x) + k;
+      v[t][k] = i < nblk ? blk[i] : 0;
+    }
+#pragma unroll
+  for (int t = 0; t < SCAN_TILES; t++) {
+    incl[t] = v[t][0] + v[t][1] + v[t][2] + v[t][3];
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t u = __shfl_up(incl[t], d);
+      if (lane >= d) incl[t] += u;
+    }
+    if (lane == 63) wsum[t * NW + wave] = incl[t];
+  }
+  __syncthreads();
+  const int32_t own = wsum[lane];
+  int32_t s = own;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t u = __shfl_up(s, d);
+    if (lane >= d) s += u;
+  }
+#pragma unroll
+  for (int t = 0; t < SCAN_TILES; t++) {
+    int32_t o = __shfl(s - own, t * NW + wave) + incl[t] -
+                (v[t][0] + v[t][1] + v[t][2] + v[t][3]);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int i = 4 * (t * SCAN_TPB + (int)threadIdx.x) + k;
+      if (i < nblk) pre[i] = o;
+      o += v[t][k];
+    }
+  }
+  if (threadIdx.x == 63) {
+    tot[row] = s;
+    if (row == 8) sc->cross = s;
+  }
 }
 
 __global__ void k_cross_total(const int32_t *__restrict__ pre, const int32_t *__restrict__ blk,
@@ -218,39 +280,63 @@ __global__ void k_cross_total(const int32_t *__restrict__ pre, const int32_t *__
 }
 
 // crossing parcels: record their slot at its rank among vacated slots and copy their fields,
-// shifted by one period, to the staging slot given by their (direction, slot) rank
+// shifted by one period, to the staging slot given by their (direction, slot) rank.  A block
+// without any returns at once; the others list theirs in LDS and copy a field a thread.  pre:
+// prefix sums within each row, with the rows' totals, or (tot null) over all nine rows as one.
 __global__ void __launch_bounds__(TPB) k_hs_gather(Geometry g, const double *__restrict__ par,
                                                    int64_t cap, int64_t n,
                                                    const uint8_t *__restrict__ flag,
+                                                   const int32_t *__restrict__ blk,
                                                    const int32_t *__restrict__ pre, int64_t nblk,
+                                                   const int32_t *__restrict__ tot,
                                                    int32_t *__restrict__ vacated,
                                                    double *__restrict__ tmp, int64_t tcap) {
-  __shared__ int lds[NWAVE];
+  __shared__ int32_t lds[9][NWAVE];
+  __shared__ int2 who[TPB];  // (slot, staging slot) of the block's crossing parcels
+  __shared__ uint8_t wdir[TPB];
+  const int K = blk[8 * nblk + blockIdx.x];
+  if (K == 0) return;
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool active = p < n;
-  const int dir = active ? flag[p] : 0;
-  int wr = 0, wc = 0, t_;
+  const int dir = p < n ? flag[p] : 0;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  wave_dir_counts(dir, lds);
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int wr = 0, wc = 0;  // ranks within the wavefront
   for (int d = 1; d <= 8; d++) {
-    int r;
-    block_rank(active && dir == d, r, t_, lds);
-    if (dir == d) wr = r;
+    const unsigned long long m = __ballot(dir == d);
+    if (dir == d) wr = __popcll(m & below);
   }
-  block_rank(active && dir != 0, wc, t_, lds);
-  if (!active || dir == 0) return;
-  const int64_t t = (int64_t)pre[(int64_t)(dir - 1) * nblk + blockIdx.x] + wr;
-  const int64_t v = (int64_t)pre[(int64_t)8 * nblk + blockIdx.x] - pre[(int64_t)8 * nblk] + wc;
-  vacated[v] = (int32_t)p;
-  double xs = 0, ys = 0;
-  if (dir == 3 || dir == 2 || dir == 4) xs = g.xshift_e;
-  else if (dir == 7 || dir == 8 || dir == 6) xs = g.xshift_w;
-  if (dir == 1 || dir == 2 || dir == 8) ys = g.yshift_n;
-  else if (dir == 5 || dir == 6 || dir == 4) ys = g.yshift_s;
-#pragma unroll 1
-  for (int f = 0; f < NFIELDS; f++) {
-    double val = par[(int64_t)f * cap + p];
-    if (f == FX || f == FXO || f == FXF) val = val + xs;
-    if (f == FY || f == FYO || f == FYF) val = val + ys;
-    tmp[(int64_t)f * tcap + t] = val;
+  wc = __popcll(__ballot(dir != 0) & below);
+  __syncthreads();
+  if (dir != 0) {
+    for (int w = 0; w < wave; w++) {
+      wr += lds[dir - 1][w];
+      wc += lds[8][w];
+    }
+    int32_t t = pre[(int64_t)(dir - 1) * nblk + blockIdx.x] + wr;
+    int32_t v = pre[(int64_t)8 * nblk + blockIdx.x] + wc;
+    if (tot)
+      for (int d = 0; d < dir - 1; d++) t += tot[d];
+    else
+      v -= pre[(int64_t)8 * nblk];
+    vacated[v] = (int32_t)p;
+    who[wc] = make_int2((int32_t)p, t);
+    wdir[wc] = (uint8_t)dir;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < K * NFIELDS; e += TPB) {
+    const int f = e / K, m = e - f * K;
+    const int d = wdir[m];
+    double val = par[(int64_t)f * cap + who[m].x];
+    if (f == FX || f == FXO || f == FXF) {
+      if (d == 2 || d == 3 || d == 4) val = val + g.xshift_e;
+      else if (d == 6 || d == 7 || d == 8) val = val + g.xshift_w;
+    }
+    if (f == FY || f == FYO || f == FYF) {
+      if (d == 1 || d == 2 || d == 8) val = val + g.yshift_n;
+      else if (d == 4 || d == 5 || d == 6) val = val + g.yshift_s;
+    }
+    tmp[(int64_t)f * tcap + who[m].y] = val;
   }
 }
 
@@ -258,11 +344,10 @@ __global__ void k_hs_scatter(double *__restrict__ par, int64_t cap, const double
                              int64_t tcap, const int32_t *__restrict__ vacated,
                              const DevScalars *sc) {
   const int64_t K = sc->cross;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < K;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t s = vacated[t];
-#pragma unroll 1
-    for (int f = 0; f < NFIELDS; f++) par[(int64_t)f * cap + s] = tmp[(int64_t)f * tcap + t];
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < K * NFIELDS;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t f = e / K, t = e - f * K;
+    par[f * cap + vacated[t]] = tmp[f * tcap + t];
   }
 }
 
@@ -314,6 +399,9 @@ __device__ __forceinline__ int block_excl_scan(int v, int &total, int *lds) {
   return off + incl - v;
 }
 
+// The flags `want` of a block counted, from flags that a kernel has made already (k_flag_count)
+// or that the block makes and stores itself (the others: one pass over the parcels or cells
+// instead of two, KPT loads a thread in flight and each pass of them coalesced).
 __global__ void __launch_bounds__(TPB) k_flag_count(const uint8_t *__restrict__ flags,
                                                     uint8_t want, int64_t n,
                                                     int32_t *__restrict__ blk) {
@@ -325,33 +413,107 @@ __global__ void __launch_bounds__(TPB) k_flag_count(const uint8_t *__restrict__ 
   if (threadIdx.x == 0) blk[blockIdx.x] = t;
 }
 
-__global__ void __launch_bounds__(TPB) k_flag_scatter(const uint8_t *__restrict__ flags,
-                                                      uint8_t want, int64_t n,
-                                                      const int32_t *__restrict__ pre,
-                                                      const int32_t *__restrict__ blk,
-                                                      int64_t nblk, int32_t *__restrict__ out,
-                                                      int64_t *__restrict__ count) {
-  __shared__ int lds[NWAVE];
-  const int64_t i0 = ((int64_t)blockIdx.x * TPB + threadIdx.x) * FPT;
-  uint32_t m = (i0 < n) ? flag_bits(flags, want, i0, n) : 0u;
+// flag(i) of the block's items stored and the ones equal to want counted
+template <typename F>
+__device__ __forceinline__ void make_flags(const F &flag, uint8_t want, int64_t n, int64_t block,
+                                           uint8_t *__restrict__ flags, int32_t *__restrict__ blk,
+                                           int *lds) {
+  const int64_t i0 = block * FPB + threadIdx.x;
+  int k = 0;
+  uint8_t v[FPT];
+#pragma unroll
+  for (int q = 0; q < FPT; q++) v[q] = flag(min(i0 + q * TPB, n - 1));
+#pragma unroll
+  for (int q = 0; q < FPT; q++)
+    if (i0 + q * TPB < n) {
+      flags[i0 + q * TPB] = v[q];
+      k += v[q] == want;
+    }
   int t;
-  int64_t o = (int64_t)pre[blockIdx.x] + block_excl_scan(__popc(m), t, lds);
+  block_excl_scan(k, t, lds);
+  if (threadIdx.x == 0) blk[block] = t;
+}
+
+// splitting (parcel_splitting.F90:76)
+template <typename T>
+__global__ void __launch_bounds__(TPB) k_split_flags(const T *__restrict__ stretch, int64_t n,
+                                                     uint8_t *__restrict__ flags,
+                                                     int32_t *__restrict__ blk) {
+  __shared__ int lds[NWAVE];
+  make_flags([&](int64_t i) { return (uint8_t)(stretch[i] > (T)4 ? 1 : 0); }, 1, n, blockIdx.x,
+             flags, blk, lds);
+}
+
+// mixing: the first nblk blocks flag the parcels below vmin with 0 and the kept ones with 1, the
+// others flag the cells with fewer than three kept parcels, in the reference's loop order (i
+// outer, j, k inner; parcel_mixing.F90:160-162), and clear ctouch
+template <typename T>
+__global__ void __launch_bounds__(TPB) k_mix_flags(const T *__restrict__ vol, int64_t n, T vmin,
+                                                   uint8_t *__restrict__ keep,
+                                                   int32_t *__restrict__ blk, int64_t nblk,
+                                                   Geometry g, const int32_t *__restrict__ npercell,
+                                                   int64_t ncell, uint8_t *__restrict__ cellflag,
+                                                   uint8_t *__restrict__ ctouch,
+                                                   int32_t *__restrict__ cblk) {
+  __shared__ int lds[NWAVE];
+  if (blockIdx.x < nblk) {
+    if (n > 0)
+      make_flags([&](int64_t i) { return (uint8_t)(vol[i] < vmin ? 0 : 1); }, 0, n, blockIdx.x,
+                 keep, blk, lds);
+    else if (threadIdx.x == 0) blk[blockIdx.x] = 0;
+    return;
+  }
+  make_flags(
+      [&](int64_t o) {
+        const uint32_t ord = (uint32_t)o, col = ord / (uint32_t)g.ncz;  // cells are below 2^31
+        const uint32_t k = ord - col * (uint32_t)g.ncz, i = col / (uint32_t)g.ny;
+        const uint32_t j = col - i * (uint32_t)g.ny;
+        if (ctouch) ctouch[ord] = 0;
+        return (uint8_t)(npercell[((int64_t)k * g.ny + j) * g.nx + i] < 3 ? 1 : 0);
+      },
+      1, ncell, blockIdx.x - nblk, cellflag, cblk, lds);
+}
+
+// one flag array's compaction: the ascending indices of its flags `want`
+struct FlagList {
+  const uint8_t *flags;
+  int64_t n, nblk;
+  const int32_t *blk, *pre;  // per block: flags counted, and their prefix sums
+  int32_t *out;
+  int64_t *count;
+  uint8_t want;
+};
+
+// up to OWN_PREFIX blocks a block sums the counts before it itself (at most 8 a thread), which
+// takes less than the two launches of a scan; pre is null then
+constexpr int OWN_PREFIX = 8 * TPB;
+
+// the lists of a (its first a.nblk blocks) and b
+__global__ void __launch_bounds__(TPB) k_flag_scatter(FlagList a, FlagList b) {
+  __shared__ int lds[NWAVE];
+  const bool second = blockIdx.x >= a.nblk;
+  const FlagList &l = second ? b : a;
+  const int64_t block = blockIdx.x - (second ? a.nblk : 0);
+  const int64_t i0 = (block * TPB + threadIdx.x) * FPT;
+  uint32_t m = (i0 < l.n) ? flag_bits(l.flags, l.want, i0, l.n) : 0u;
+  int before = 0;
+  if (l.pre) {
+    before = l.pre[block];
+  } else {
+    int own = 0;
+    for (int64_t q = threadIdx.x; q < block; q += TPB) own += l.blk[q];
+    block_excl_scan(own, before, lds);
+  }
+  int t;
+  int64_t o = (int64_t)before + block_excl_scan(__popc(m), t, lds);
   while (m) {
-    out[o++] = (int32_t)(i0 + (__ffs(m) - 1));
+    l.out[o++] = (int32_t)(i0 + (__ffs(m) - 1));
     m &= m - 1u;
   }
-  if (blockIdx.x == nblk - 1 && threadIdx.x == 0 && count)
-    *count = (int64_t)pre[nblk - 1] + blk[nblk - 1];
+  if (block == l.nblk - 1 && threadIdx.x == 0) *l.count = (int64_t)before + t;
 }
 
 // ---- splitting (parcel_splitting.F90:76-131) ----
-__global__ void k_split_flags(const double *__restrict__ par, int64_t cap, int64_t n,
-                              uint8_t *__restrict__ flag) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  flag[p] = (par[FSTRETCH * cap + p] > 4.) ? 1 : 0;
-}
-
 __global__ void k_split_apply(double *__restrict__ par, int64_t cap, int64_t n,
                               const int32_t *__restrict__ parents, int64_t nsplit,
                               DevScalars *sc) {
@@ -392,32 +554,6 @@ __global__ void k_split_apply(double *__restrict__ par, int64_t cap, int64_t n,
 }
 
 // ---- mixing (parcel_mixing.F90:157-389) ----
-// KPT parcels per thread, at stride TPB (each a coalesced pass), the loads issued together
-constexpr int KPT = 4;
-__global__ void k_keep_flags(const double *__restrict__ par, int64_t cap, int64_t n, double vmin,
-                             uint8_t *__restrict__ keep) {
-  const int64_t p0 = (int64_t)blockIdx.x * (TPB * KPT) + threadIdx.x;
-  const double *vol = par + (int64_t)FVOL * cap;
-  double v[KPT];
-#pragma unroll
-  for (int k = 0; k < KPT; k++) v[k] = vol[min(p0 + (int64_t)k * TPB, n - 1)];
-#pragma unroll
-  for (int k = 0; k < KPT; k++)
-    if (p0 + (int64_t)k * TPB < n) keep[p0 + (int64_t)k * TPB] = (v[k] < vmin) ? 0 : 1;
-}
-
-// flags over cells in the reference's loop order (i outer, j, k inner; parcel_mixing.F90:160-162)
-__global__ void k_newcell_flags(Geometry g, const int32_t *__restrict__ npercell,
-                                uint8_t *__restrict__ cellflag, int64_t ncell) {
-  const int64_t ord = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ord >= ncell) return;
-  const int k = (int)(ord % g.ncz);
-  const int j = (int)((ord / g.ncz) % g.ny);
-  const int i = (int)(ord / ((int64_t)g.ncz * g.ny));
-  const int64_t c = ((int64_t)k * g.ny + j) * g.nx + i;
-  cellflag[ord] = (npercell[c] < 3) ? 1 : 0;
-}
-
 struct MixGrids {
   const double *G[6];  // kept vol, b, hg, p, q, r (folded, doubled)
   double *R[6];        // residual vres..rres
@@ -477,8 +613,11 @@ __global__ void k_mix_new(Geometry g, double *__restrict__ par, int64_t cap, int
 
 // residual minus the share of every adjacent new parcel, visiting cells in the reference's
 // loop order, then the z-boundary doubling (parcel_mixing.F90:202-207, 221-240)
+// ... and marks the cells around a node whose residual changes a parcel's values: not zero, or at
+// a node without a (finite) kept volume to divide by
 __global__ void k_mix_residual(Geometry g, MixGrids mg, const int32_t *__restrict__ npercell,
-                               const double *__restrict__ portion_cell) {
+                               const double *__restrict__ portion_cell,
+                               uint8_t *__restrict__ ctouch) {
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nnode) return;
@@ -505,15 +644,32 @@ __global__ void k_mix_residual(Geometry g, MixGrids mg, const int32_t *__restric
         for (int f = 0; f < 6; f++) r[f] = r[f] - portion * gv[f];
       }
   const double mlt = (k == 0 || k == g.nzn - 1) ? 2. : 1.;
+  bool any = !(gv[0] > 0.0 && gv[0] <= DBL_MAX);
 #pragma unroll
-  for (int f = 0; f < 6; f++) mg.R[f][t] = r[f] * mlt;
+  for (int f = 0; f < 6; f++) {
+    const double v = r[f] * mlt;
+    mg.R[f][t] = v;
+    any = any || !(v == 0.0);
+  }
+  if (!any) return;
+  for (int a = 0; a < 2; a++)
+    for (int b = 0; b < 2; b++)
+      for (int kc = k - 1; kc <= k; kc++)
+        if (kc >= 0 && kc < g.ncz) ctouch[((int64_t)kc * g.ny + cj[b]) * g.nx + ci[a]] = 1;
 }
 
-// kept parcels absorb the residuals (parcel_mixing.F90:247-340)
+// Kept parcels absorb the residuals (parcel_mixing.F90:247-340).  A parcel of a cell that
+// k_mix_residual has not marked (almost all of them: residuals arise only around removed parcels
+// and the cells that received new ones) keeps its values, which the arithmetic would return to
+// within rounding: 6 bytes of flags and cells a parcel instead of 73 and the gathers (57 M
+// parcels, none marked: 2.62 -> 0.29 ms).  cell: the mixing's binning.
 __global__ void k_mix_absorb(Geometry g, double *__restrict__ par, int64_t cap, int64_t norig,
-                             const uint8_t *__restrict__ keep, MixGrids mg) {
+                             const uint8_t *__restrict__ keep, const int32_t *__restrict__ cell,
+                             const uint8_t *__restrict__ ctouch, MixGrids mg) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= norig || keep[p] != 1) return;
+  const int32_t c = cell[p];
+  if (c >= 0 && !ctouch[c]) return;
   // all loads first (parcel values, then the gathers), all stores last
   const int fld[5] = {FB, FH, FP, FQ, FR};
   const double x = ld_stream(&par[FX * cap + p]), y = ld_stream(&par[FY * cap + p]),
@@ -584,18 +740,60 @@ int sync_scalars(Ctx *c) {
   return c->hsc.status;
 }
 
+// blk and pre of a list's counts; the scan where its blocks do not sum them themselves
+static int list_prefix(Ctx *c, FlagList &l, int32_t *blk) {
+  l.blk = blk;
+  l.pre = nullptr;
+  if (l.nblk <= OWN_PREFIX) return PMPIC_OK;
+  l.pre = blk + l.nblk;
+  return scan_exclusive_i32(c, blk, blk + l.nblk, l.nblk);
+}
+
 int compact_flags(Ctx *c, const uint8_t *flags, uint8_t want, int64_t n, int32_t *out,
                   int64_t *d_count) {
-  const int64_t nblk = cdiv(n > 0 ? n : 1, FPB);
-  if (nblk > c->nblk_max) return PMPIC_ERR_ARG;
-  int32_t *blk = c->blk, *pre = c->blk + nblk;
-  hipLaunchKernelGGL(k_flag_count, dim3(nblk), dim3(TPB), 0, c->stream, flags, want, n, blk);
-  PMPIC_TRY(scan_exclusive_i32(c, blk, pre, nblk));
-  hipLaunchKernelGGL(k_flag_scatter, dim3(nblk), dim3(TPB), 0, c->stream, flags, want, n, pre, blk,
-                     nblk, out, d_count);
+  FlagList l = {flags, n, cdiv(n > 0 ? n : 1, FPB), nullptr, nullptr, out, d_count, want};
+  if (l.nblk > c->nblk_max) return PMPIC_ERR_ARG;
+  hipLaunchKernelGGL(k_flag_count, dim3(l.nblk), dim3(TPB), 0, c->stream, flags, want, n, c->blk);
+  PMPIC_TRY(list_prefix(c, l, c->blk));
+  hipLaunchKernelGGL(k_flag_scatter, dim3(l.nblk), dim3(TPB), 0, c->stream, l, l);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
+
+template <typename T>
+int split_list(Ctx *c, const T *stretch, int64_t n) {
+  FlagList l = {c->flag, n, cdiv(n, FPB), nullptr, nullptr, c->list_b, &c->dsc->nsplit, 1};
+  if (n <= 0 || l.nblk > c->nblk_max) return PMPIC_ERR_ARG;
+  hipLaunchKernelGGL(k_split_flags<T>, dim3(l.nblk), dim3(TPB), 0, c->stream, stretch, n, c->flag,
+                     c->blk);
+  PMPIC_TRY(list_prefix(c, l, c->blk));
+  hipLaunchKernelGGL(k_flag_scatter, dim3(l.nblk), dim3(TPB), 0, c->stream, l, l);
+  PMPIC_CHECK(hipGetLastError());
+  return PMPIC_OK;
+}
+
+template <typename T>
+int mix_lists(Ctx *c, const T *vol, T vmin, int64_t n, uint8_t *ctouch) {
+  FlagList a = {c->flag, n, cdiv(n > 0 ? n : 1, FPB), nullptr, nullptr, c->list_a,
+                &c->dsc->nzero, 0};
+  FlagList b = {c->cellflag, c->ncell, cdiv(c->ncell, FPB), nullptr, nullptr, c->sorted,
+                &c->dsc->nadd, 1};
+  if (a.nblk > c->nblk_max || b.nblk > c->nblk_max) return PMPIC_ERR_ARG;
+  int32_t *blk_a = c->blk, *blk_b = c->blk + 2 * a.nblk;
+  hipLaunchKernelGGL(k_mix_flags<T>, dim3(a.nblk + b.nblk), dim3(TPB), 0, c->stream, vol, n, vmin,
+                     c->flag, blk_a, a.nblk, c->g, c->npercell, c->ncell, c->cellflag, ctouch,
+                     blk_b);
+  PMPIC_TRY(list_prefix(c, a, blk_a));
+  PMPIC_TRY(list_prefix(c, b, blk_b));
+  hipLaunchKernelGGL(k_flag_scatter, dim3(a.nblk + b.nblk), dim3(TPB), 0, c->stream, a, b);
+  PMPIC_CHECK(hipGetLastError());
+  return PMPIC_OK;
+}
+
+template int split_list<double>(Ctx *, const double *, int64_t);
+template int split_list<float>(Ctx *, const float *, int64_t);
+template int mix_lists<double>(Ctx *, const double *, double, int64_t, uint8_t *);
+template int mix_lists<float>(Ctx *, const float *, float, int64_t, uint8_t *);
 
 static int ensure_tmp(Ctx *c, int64_t need) {
   if (need <= c->tmp_cap) return PMPIC_OK;
@@ -608,20 +806,32 @@ static int ensure_tmp(Ctx *c, int64_t need) {
   return PMPIC_OK;
 }
 
-// permutation part of the haloswap; expects flag[] and the per-block direction counts
+// Permutation part of the haloswap; expects flag[] and the per-block direction counts.  The
+// staging buffer must hold every crossing parcel: up to HS_STAGE parcels it is made to hold them
+// all, so nothing need be read back, which takes the host longer than the two copies take the device
+// where nothing crosses; above, the count is read, and at most that much staged.
+constexpr int64_t HS_STAGE = (int64_t)1 << 20;  // 232 MB of staging
 static int haloswap_permute(Ctx *c, int64_t n, int64_t nblk) {
-  int32_t *blk = c->blk, *pre = c->blk + 9 * nblk;
-  PMPIC_TRY(scan_exclusive_i32(c, blk, pre, 9 * nblk));
-  hipLaunchKernelGGL(k_cross_total, dim3(1), dim3(1), 0, c->stream, pre, blk, nblk, c->dsc);
-  // the staging buffer must hold every crossing parcel; read the count back
-  PMPIC_TRY(read_back(c, &c->hsc.cross, &c->dsc->cross, sizeof(int64_t)));
-  const int64_t K = c->hsc.cross;
-  if (K == 0) return PMPIC_OK;
-  PMPIC_TRY(ensure_tmp(c, K));
+  int32_t *blk = c->blk, *pre = c->blk + 9 * nblk, *tot = nullptr;
+  int64_t most = n;
+  if (nblk <= SCAN_MAX) {
+    tot = c->blk + 18 * nblk;
+    hipLaunchKernelGGL(k_hs_scan, dim3(9), dim3(SCAN_TPB), 0, c->stream, blk, pre, (int)nblk, tot,
+                       c->dsc);
+  } else {
+    PMPIC_TRY(scan_exclusive_i32(c, blk, pre, 9 * nblk));
+    hipLaunchKernelGGL(k_cross_total, dim3(1), dim3(1), 0, c->stream, pre, blk, nblk, c->dsc);
+  }
+  if (n > HS_STAGE) {
+    PMPIC_TRY(read_back(c, &c->hsc.cross, &c->dsc->cross, sizeof(int64_t)));
+    most = c->hsc.cross;
+  }
+  if (most == 0) return PMPIC_OK;
+  PMPIC_TRY(ensure_tmp(c, most));
   hipLaunchKernelGGL(k_hs_gather, dim3(nblk), dim3(TPB), 0, c->stream, c->g, c->par, c->cap, n,
-                     c->flag, pre, nblk, c->list_a, c->tmp, c->tmp_cap);
-  int64_t sb = cdiv(K, TPB);
-  if (sb > 4096) sb = 4096;
+                     c->flag, blk, pre, nblk, tot, c->list_a, c->tmp, c->tmp_cap);
+  // a grid-stride copy: the count is the device's
+  const int64_t sb = std::min<int64_t>(cdiv(most * NFIELDS, TPB), n > HS_STAGE ? 4096 : 256);
   hipLaunchKernelGGL(k_hs_scatter, dim3(sb), dim3(TPB), 0, c->stream, c->par, c->cap, c->tmp,
                      c->tmp_cap, c->list_a, c->dsc);
   PMPIC_CHECK(hipGetLastError());
@@ -632,22 +842,23 @@ int rk_stage_update(Ctx *c, int stage, int64_t n, int stretch) {
   const int64_t nblk = cdiv(n > 0 ? n : 1, TPB);
   if (nblk > c->nblk_max) return PMPIC_ERR_ARG;
   PMPIC_TRY(records_current(c));
+  const int keep_k = c->whole_step ? 0 : 1;
   switch (stage) {
     case 1:
       PMPIC_TRY(launch_timed(c, T_RK, k_rk_stage<1>, dim3(nblk), dim3(TPB), 0, c->g, c->par,
-                             c->cap, n, c->rec, stretch, c->dsc, c->flag, c->blk, nblk));
+                             c->cap, n, c->rec, stretch, keep_k, c->dsc, c->flag, c->blk, nblk));
       break;
     case 2:
       PMPIC_TRY(launch_timed(c, T_RK, k_rk_stage<2>, dim3(nblk), dim3(TPB), 0, c->g, c->par,
-                             c->cap, n, c->rec, stretch, c->dsc, c->flag, c->blk, nblk));
+                             c->cap, n, c->rec, stretch, keep_k, c->dsc, c->flag, c->blk, nblk));
       break;
     case 3:
       PMPIC_TRY(launch_timed(c, T_RK, k_rk_stage<3>, dim3(nblk), dim3(TPB), 0, c->g, c->par,
-                             c->cap, n, c->rec, stretch, c->dsc, c->flag, c->blk, nblk));
+                             c->cap, n, c->rec, stretch, keep_k, c->dsc, c->flag, c->blk, nblk));
       break;
     default:
       PMPIC_TRY(launch_timed(c, T_RK, k_rk_stage<4>, dim3(nblk), dim3(TPB), 0, c->g, c->par,
-                             c->cap, n, c->rec, stretch, c->dsc, c->flag, c->blk, nblk));
+                             c->cap, n, c->rec, stretch, keep_k, c->dsc, c->flag, c->blk, nblk));
       break;
   }
   PMPIC_CHECK(hipGetLastError());
@@ -668,9 +879,7 @@ int parcel_haloswap(Ctx *c, int64_t n, int reflect) {
 int parcel_split(Ctx *c) {
   const int64_t n = c->n;
   if (n > 0) {
-    hipLaunchKernelGGL(k_split_flags, dim3(cdiv(n, TPB)), dim3(TPB), 0, c->stream, c->par, c->cap,
-                       n, c->flag);
-    PMPIC_TRY(compact_flags(c, c->flag, 1, n, c->list_b, &c->dsc->nsplit));
+    PMPIC_TRY(split_list(c, c->par + FSTRETCH * c->cap, n));
   } else {
     c->hsc.nsplit = 0;
     PMPIC_CHECK(hipMemcpyAsync(&c->dsc->nsplit, &c->hsc.nsplit, sizeof(int64_t),
@@ -693,15 +902,8 @@ int parcel_mix(Ctx *c) {
   const Geometry &g = c->g;
   const int64_t norig = c->n;
   PMPIC_TRY(mixing_grids(c, norig));
-  if (norig > 0)
-    hipLaunchKernelGGL(k_keep_flags, dim3(cdiv(norig, TPB * KPT)), dim3(TPB), 0, c->stream, c->par,
-                       c->cap, norig, g.vmin, c->flag);
-  // removed slots, ascending
-  PMPIC_TRY(compact_flags(c, c->flag, 0, norig, c->list_a, &c->dsc->nzero));
-  // sparse cells in the reference's loop order
-  hipLaunchKernelGGL(k_newcell_flags, dim3(cdiv(c->ncell, TPB)), dim3(TPB), 0, c->stream, g,
-                     c->npercell, c->cellflag, c->ncell);
-  PMPIC_TRY(compact_flags(c, c->cellflag, 1, c->ncell, c->sorted, &c->dsc->nadd));
+  // removed slots, ascending, and sparse cells in the reference's loop order
+  PMPIC_TRY(mix_lists(c, c->par + FVOL * c->cap, g.vmin, norig, c->ctouch));
   PMPIC_TRY(sync_scalars(c));
   const int64_t Z = c->hsc.nzero, nadd = c->hsc.nadd;
   MixGrids mg = {{c->grid[GVOL], c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR]},
@@ -714,10 +916,10 @@ int parcel_mix(Ctx *c) {
                        c->dsc);
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
   hipLaunchKernelGGL(k_mix_residual, dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, g, mg,
-                     c->npercell, portion);
+                     c->npercell, portion, c->ctouch);
   if (norig > 0)
     hipLaunchKernelGGL(k_mix_absorb, dim3(cdiv(norig, TPB)), dim3(TPB), 0, c->stream, g, c->par,
-                       c->cap, norig, c->flag, mg);
+                       c->cap, norig, c->flag, c->cell, c->ctouch, mg);
   PMPIC_CHECK(hipGetLastError());
   // new count (parcel_mixing.F90:217)
   int64_t np = norig;
@@ -732,7 +934,8 @@ int parcel_mix(Ctx *c) {
     }
     if (slast + 1 > np) np = slast + 1;
   }
-  PMPIC_TRY(sync_scalars(c));
+  // what k_mix_new raised (nothing else since the last read-back raises anything)
+  if (nadd > 0) PMPIC_TRY(sync_scalars(c));
   c->last_removed = Z;
   c->last_added = nadd;
   if (np == norig) {

@@ -9,6 +9,9 @@ parcels that sums of 1e3 terms with 1e-16 rounding stay far below it.
 The column kernel: levels per column below, at and above its read-ahead (8), rows of wavenumber
 blocks below and above a wavefront's 16, whole steps, 1e-12 (FP64) and 1e-5 (FP32-bulk against
 FP64, that form's bar).
+
+The haloswap's permutation: parcel counts either side of a block, of the staging that needs no
+count read back (2^20 parcels) and of the one-launch scan (16,384 blocks).
 """
 import numpy as np
 import pytest
@@ -93,3 +96,42 @@ def test_column_kernel_lengths(oracle_mod, shape, bar):
         bar(k, rel_err(g.spectral(k), o.spec(k)), 1e-12)
     g.close()
     f.close()
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 4096, 1_048_576, 1_048_577, 4_194_304, 4_194_305])
+@pytest.mark.parametrize("crossing", [0.0, 0.003, 0.5])
+def test_haloswap_counts(n, crossing):
+    """The haloswap's permutation either side of its scan's and its staging's rules: crossing
+    parcels, shifted by a period, in (direction, slot) order in the vacated slots.  Tags are whole
+    numbers; a position takes two additions of up to two periods, so it comes back to within 8
+    roundings of a period."""
+    from pmpic_amd.lib import Context
+    b = box(8, 6, 5)
+    lx, ly = b["xmax"] - b["xmin"], b["ymax"] - b["ymin"]
+    rng = np.random.default_rng(n)
+    ic = dict(x=b["xmin"] + rng.uniform(0.01, 0.99, n) * lx,
+              y=b["ymin"] + rng.uniform(0.01, 0.99, n) * ly,
+              z=b["zmin"] + rng.uniform(0.1, 0.9, n) * (b["zmax"] - b["zmin"]),
+              tag=np.arange(n, dtype=np.float64))
+    step = [rng.choice([-1, 0, 1], n, p=[crossing / 2, 1 - crossing, crossing / 2])
+            for _ in range(2)]
+    x = ic["x"] + step[0] * lx
+    y = ic["y"] + step[1] * ly
+    # N, NE, E, SE, S, SW, W, NW
+    order = {(0, 1): 1, (1, 1): 2, (1, 0): 3, (1, -1): 4, (0, -1): 5, (-1, -1): 6, (-1, 0): 7,
+             (-1, 1): 8, (0, 0): 0}
+    table = np.array([[order[(i, j)] for j in (-1, 0, 1)] for i in (-1, 0, 1)])
+    direction = table[step[0] + 1, step[1] + 1]
+    slots = np.flatnonzero(direction)
+    moved = slots[np.argsort(direction[slots], kind="stable")]
+    tag = ic["tag"].copy()
+    tag[slots] = ic["tag"][moved]
+    g = Context(8, 6, 5, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"], n + 64)
+    g.set_parcels(dict(ic, x=x, y=y))
+    g.parcel_haloswap()
+    out = g.get_parcels()
+    assert np.array_equal(out["tag"], tag)
+    back = np.argsort(tag)
+    for k, start, period in (("x", ic["x"], lx), ("y", ic["y"], ly)):
+        assert np.abs(out[k][back] - start).max() <= 8 * np.finfo(float).eps * period
+    g.close()
