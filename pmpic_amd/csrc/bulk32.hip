@@ -12,7 +12,7 @@
 //    three FP32 offsets in [0,1) inside the cell, so it carries 24 bits relative to the cell
 //    rather than to the whole domain; vorticity, buoyancy, humidity, volume and stretch are
 //    FP32, and interpolation and the par2grid sums run in FP32;
-//  * the RK4 origin of the position is (cell_o, offset_o) and the RK4 accumulator
+//  * the RK4 origin is the other of two sets of positions and vorticity, and the RK4 accumulator
 //    dt/6 k1 + dt/3 k2 + dt/3 k3 + dt/6 k4 is kept in cells relative to it;
 //  * the haloswap becomes index arithmetic: leaving through x or y wraps the cell index and the
 //    z reflection mirrors (cell, offset) about the boundary, so parcels keep their slots (the
@@ -20,10 +20,8 @@
 //  * parcel tendencies dxdt..drdt are stored at stage 4 only (the values that survive a step).
 // The spectral inversion, the timestep selection and the conservation sums stay FP64: the
 // grids are a few percent of the parcel bytes.
-#include "common.h"
+#include "node_sum.h"
 
-#include <hipcub/hipcub.hpp>
-#include <rocprim/iterator/transform_iterator.hpp>
 #include <algorithm>
 #include <math.h>
 #include <stdlib.h>
@@ -39,7 +37,6 @@ namespace pmpic {
 namespace {
 
 constexpr int TPB = 256;
-constexpr int NWAVE = TPB / 64;
 
 // A parcel's cell is stored packed as k << 20 | j << 10 | i (nx, ny <= 1024, nz < 2048), so
 // unpacking is shifts and masks; the linear cell index (k*ny + j)*nx + i is formed only where
@@ -76,6 +73,21 @@ template <typename T>
 __device__ __forceinline__ void stnt(T *base, uint32_t i, T v) {
   __builtin_nontemporal_store(v, reinterpret_cast<T *>(reinterpret_cast<char *>(base) +
                                                        i * (uint32_t)sizeof(T)));
+}
+
+struct Float3 {
+  float x, y, z;
+};
+__device__ __forceinline__ Float3 ld3(const float *base, int64_t i) {
+  const float *a = base + 3 * i;
+  return {__builtin_nontemporal_load(a), __builtin_nontemporal_load(a + 1),
+          __builtin_nontemporal_load(a + 2)};
+}
+__device__ __forceinline__ void st3(float *base, int64_t i, float x, float y, float z) {
+  float *a = base + 3 * i;
+  __builtin_nontemporal_store(x, a);
+  __builtin_nontemporal_store(y, a + 1);
+  __builtin_nontemporal_store(z, a + 2);
 }
 
 // fold an offset outside [0,1) into the cell index
@@ -183,7 +195,7 @@ __global__ void k32_pos_in(Geometry g, int axis, const double *__restrict__ x, i
       i = 0;
     }
   }
-  off[p] = o;
+  off[3 * p + axis] = o;
   cell[p] = (axis == 0 ? 0 : cell[p]) | (i << (10 * axis));
 }
 
@@ -196,17 +208,19 @@ __global__ void k32_pos_out(Geometry g, int axis, const int32_t *__restrict__ ce
   const int idx = axis == 0 ? i : (axis == 1 ? j : k);
   const double bot = axis == 0 ? g.xbot : (axis == 1 ? g.ybot : g.zbot);
   const double d = axis == 0 ? g.dx : (axis == 1 ? g.dy : g.dz);
-  x[p] = bot + ((double)idx + (double)off[p]) * d;
+  x[p] = bot + ((double)idx + (double)off[3 * p + axis]) * d;
 }
 
-__global__ void k32_from_f64(const double *__restrict__ a, int64_t n, float *__restrict__ b) {
+__global__ void k32_from_f64(const double *__restrict__ a, int64_t n, float *__restrict__ b,
+                             int stride) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < n) b[p] = (float)a[p];
+  if (p < n) b[p * stride] = (float)a[p];
 }
 
-__global__ void k32_to_f64(const float *__restrict__ a, int64_t n, double *__restrict__ b) {
+__global__ void k32_to_f64(const float *__restrict__ a, int stride, int64_t n,
+                           double *__restrict__ b) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < n) b[p] = (double)a[p];
+  if (p < n) b[p] = (double)a[p * stride];
 }
 
 // ---- cell binning ----
@@ -214,10 +228,10 @@ __global__ void k32_to_f64(const float *__restrict__ a, int64_t n, double *__res
 // run of equal cells, so a cell whose parcels are consecutive in slot order gets its ranks in
 // ascending parcel order unless it straddles two wavefronts' ranges; the accumulation only has
 // to reorder those cells.  A parcel of rank < capc is listed at slot[cell * capc + rank], so a
-// typical cell needs no scan and no scatter pass.  A parcel of higher rank is appended, with
+// typical cell needs no scatter pass.  A parcel of higher rank is appended, with
 // its rank, to an overflow list; every cell holding more than capc parcels is then laid out
-// densely, all its parcels in rank order, in `sorted` from ostart[cell] (an exclusive scan of
-// those cells' counts).  capc = 0 lays out every cell that way.  capc is chosen per binning:
+// densely, all its parcels in rank order, in `sorted` from ostart[cell] (room by
+// bin_alloc).  capc = 0 lays out every cell that way.  capc is chosen per binning:
 // CAPC_LOW while the mean is at most LOW_PPC parcels per cell, so a sparse grid does not read
 // mostly empty entries, else CAPC.
 constexpr int BIN_SEQ = 16;
@@ -306,11 +320,6 @@ __global__ void k32_bin_slot(Geometry g, const int32_t *__restrict__ cellv, int6
   }
 }
 
-struct OvfCount {
-  int capc;
-  __host__ __device__ int32_t operator()(int32_t k) const { return k > capc ? k : 0; }
-};
-
 // the overflow list into the dense region; the parcel of rank capc also copies its cell's
 // capc slot entries there, so the region holds ranks 0 .. count-1
 __global__ void k32_ovf_scatter(Geometry g, const int32_t *__restrict__ cellv,
@@ -340,49 +349,47 @@ __global__ void k32_dense_scatter(Geometry g, const int32_t *__restrict__ cellv,
   st(sorted, (uint32_t)(start[c] + ld(rankv, (uint32_t)p)), (int32_t)p);
 }
 
-__global__ void k32_sort_big(const int32_t *__restrict__ start, int64_t ncell, int rows,
-                             int32_t *__restrict__ sorted) {
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  const int32_t b = start[c], e = start[c + 1];
-  if (e - b <= rows) return;
-  for (int32_t a = b + 1; a < e; a++) {
-    const int32_t v = sorted[a];
-    int32_t q = a - 1;
-    while (q >= b && sorted[q] > v) {
-      sorted[q + 1] = sorted[q];
-      q--;
-    }
-    sorted[q + 1] = v;
-  }
-}
-
-// ---- per-cell corner partial sums (the plain form's LDS kernel in FP32) ----
-// A workgroup of 8 threads per cell takes a tile of TILE32 cells.  The tile's slot entries are
-// loaded together with the cell counts (their addresses do not depend on the counts), the
-// parcels' values are staged in LDS in dense rows, cell after cell, and thread q of a cell sums
-// corner q over the cell's parcels in ascending parcel order, so the sums are deterministic.
-// P2G: p, q, r and the total buoyancy (vort2vel + vorticity_tendency); MIX: kept / residual
-// vol, b, h, p, q, r (parcel_mixing); DUMP: b, h, p, q, r (writebinary's grids)
-// P2GX, MIXX: P2G and MIX whose tiles are 16 cells of one x row (nx a multiple of 16), each
-// tile writing its corner sums combined along x into the 17 node positions it touches (see
-// k32_node_sum_x); MIXX sums vol, p, q, r, the total buoyancy, b and h, so that its first five
-// planes are the ones P2GX writes (the next par2grid keeps them where mixing changed nothing)
-enum Acc32 { A32_P2G = 0, A32_MIX = 1, A32_DUMP = 2, A32_P2GX = 3, A32_MIXX = 4 };
-constexpr int TILE32 = 16;
-constexpr int ROWS32 = 512;     // LDS rows with the full capacity
-constexpr int ROWS_LOW = 256;   // LDS rows with CAPC_LOW
-__host__ __device__ constexpr int rows_of(int capc) { return capc == CAPC_LOW ? ROWS_LOW : ROWS32; }
-constexpr int ATPB = TILE32 * 8;  // threads of the accumulation workgroup
+// ---- corner sums ----
+// One wavefront per tile of eight cells of one x row; lane = 8 q + cl is corner q (bits z<<2 |
+// y<<1 | x) of cell cl, and the cell's parcels are taken eight at a time: lane (q, cl) stages
+// parcel q of the eight in LDS row 8 q + cl, then every lane adds its corner's weight and weight *
+// value over the cell's rows.  The next eight parcels' loads are in flight meanwhile, and no
+// barrier ties wavefronts together, so the CU's 32 overlap each other's loads and sums.  It is
+// bound by the latency of the gathers: three 12-byte records a parcel, and
+// half by the issue of the sums.  67 M parcels that have moved a few cells: 1.39 ms with nine 4-byte
+// gathers and a workgroup staging all parcels of 16 cells, 1.14 ms (2.6 TB/s); 1.8 M well mixed
+// ones in 221 k cells: 87 -> 58 us.
+//
+// Within a cell the additions run in ascending parcel order, so the sums do not depend on the
+// order in which the binning's atomics came: the lanes check their adjacent entries and rank them
+// where a pair is not ascending (in LDS up to LIST entries a cell, else in memory).
+//
+// A cell of up to capc parcels lists them in the slot table, whose first 16 entries are loaded
+// before the count is known; the others in the dense region.
+//
+// The corner sums are combined along x as they are written: node position i of corner pair
+// bb = (by, bz) adds the bx = 1 corner of cell i - 1 and the bx = 0 corner of cell i.  Value f of
+// entry (bb, row, position) sits at ((f 4 + bb) nrows + row) (nx + ntx) + 9 tx + position - 8 tx,
+// ntx tiles a row; a tile's last position holds its last cell's bx = 1 corner alone, completed by
+// the node sums.
+//
+// A32_P2G: weight, p, q, r, total buoyancy (vort2vel + vorticity_tendency).  A32_MIX: those and
+// b, h, of the kept parcels and (partial2) the residual ones (parcel_mixing), so that its first
+// five planes are the ones the next par2grid would write; the tiles without residual parcels
+// (almost all) are marked so in tileres and write none.  A32_DUMP: weight, b, h, p, q, r
+// (writebinary's grids).
+enum Acc32 { A32_P2G = 0, A32_MIX = 1, A32_DUMP = 2 };
+constexpr int LIST = 64;
 
 struct Zmap {
   float zbot, dz;  // z of a parcel = zbot + (k + oz) dz
 };
 
-// A parcel's weight at corner (bx, by, bz) of its cell, in the form's one order of operations
-// (every accumulation kernel and path uses it, so a cell's sums do not depend on which of them
-// ran): the factor of an axis is |t - offset|, t = 1 for the lower corner (1 - offset) and 0 for
-// the upper (the offset, which lies in [0, 1]); the weight is ((fz fy) vol) fx.
+// A parcel's weight at corner (bx, by, bz) of its cell: the factor of an axis is |t - offset|,
+// t = 1 for the lower corner (1 - offset) and 0 for the upper (the offset, which lies in [0, 1]);
+// the weight is ((fz fy) vol) fx.  No contraction here or in add_parcel: the compiler would
+// otherwise fuse the weight's last product into the first sum in some of the kernels that inline
+// these and not in others, and a tile that mixing left unchanged must have the par2grid's bits.
 __device__ __forceinline__ float corner_weight(float ox, float oy, float oz, float vol, float tx,
                                                float ty, float tz) {
 #pragma clang fp contract(off)
@@ -392,10 +399,7 @@ __device__ __forceinline__ float corner_weight(float ox, float oy, float oz, flo
   return wv * fabsf(tx - ox);
 }
 
-// acc[0] += w, acc[1 + f] += w * v[f], fused.  No contraction here or in corner_weight: the
-// compiler would otherwise fuse the weight's last product into the first sum in some of the
-// kernels that inline these and not in others, and every accumulation path must give the same
-// bits.
+// acc[0] += w, acc[1 + f] += w * v[f], fused
 template <int NV>
 __device__ __forceinline__ void add_parcel(float *acc, float w, const float *v) {
 #pragma clang fp contract(off)
@@ -404,453 +408,215 @@ __device__ __forceinline__ void add_parcel(float *acc, float w, const float *v) 
   for (int f = 0; f < NV; f++) acc[f + 1] = fmaf(w, v[f], acc[f + 1]);
 }
 
-// CAP: the binning's slot capacity (any value when capc = 0); ROWS: LDS rows of a pass
-// The kernel is bound by memory latency, so waves in flight set its speed: with the 16-entry
-// table the LDS rows allow 16 workgroups (32 waves) per CU, and holding the registers to 72
-// allows 7 waves per SIMD (28 per CU) instead of 5 (4-5 % faster at 8 parcels per cell); the
-// x-row form fits 64 registers without spilling, so all 8 (0.95 -> 0.90 ms at 256x256x128).
-// The x-row mixing form's seven sums and three staged values per row allow 12 workgroups (6
-// waves per SIMD) by LDS, so it takes the registers of 6 waves.
-// The 32-entry form is bound by its LDS rows (8 workgroups per CU) instead.
-template <int MODE, int CAP, int ROWS>
-__global__ void __launch_bounds__(ATPB)
-__attribute__((amdgpu_waves_per_eu(CAP == CAPC_LOW ? (MODE == A32_P2GX ? 8 : MODE == A32_MIXX ? 6 : 7) : 1))) k32_cell_accum(Bulk32 b, int64_t cap, Geometry g, Zmap zm,
-                                                       float vmin, const int32_t *__restrict__ count,
-                                                       const int32_t *__restrict__ ostart,
-                                                       const int32_t *__restrict__ sorted,
-                                                       int64_t ncell, float *__restrict__ partial,
-                                                       float *__restrict__ partial2,
-                                                       int32_t *__restrict__ npercell,
-                                                       uint8_t *__restrict__ tileres,
-                                                       const uint8_t *__restrict__ dirty) {
-  constexpr bool MIX = (MODE == A32_MIX || MODE == A32_MIXX);
-  constexpr bool XC = (MODE == A32_P2GX || MODE == A32_MIXX);
-  // BT: the values start p, q, r and the total buoyancy (par2grid's four; the x-row mixing adds
-  // b and h after them, so its first five planes are the ones the x-row par2grid writes);
-  // FIVE: b, h, p, q, r (the other mixing form and the dump)
-  constexpr bool BT = (MODE == A32_P2G || MODE == A32_P2GX || MODE == A32_MIXX);
-  constexpr bool FIVE = !BT;
-  constexpr int NV = MODE == A32_MIXX ? 6 : (FIVE ? 5 : 4);
+__host__ __device__ inline int tiles_x(const Geometry &g) { return (g.nx + 7) / 8; }
+// tile of cell (i, j, k)
+__device__ __forceinline__ int64_t tile_of(const Geometry &g, int i, int j, int k) {
+  return ((int64_t)k * g.ny + j) * tiles_x(g) + (i >> 3);
+}
+
+// The lanes' W entries 8 i + q of eight lists of up to nmax entries (key e of list cl at
+// keys(e)): their ranks among the list's entries
+template <int W, typename K>
+__device__ __forceinline__ void rank_entries(const int32_t *v, int *r, int nmax, K keys) {
+#pragma unroll
+  for (int i = 0; i < W; i++) r[i] = 0;
+  for (int e = 0; e < nmax; e++) {
+    const int32_t key = keys(e);
+#pragma unroll
+    for (int i = 0; i < W; i++) r[i] += key < v[i] ? 1 : 0;
+  }
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(64) k32_cell_accum(
+    Geometry g, Parcels32 P, Zmap zm, float vmin, int capc, const int32_t *__restrict__ slot,
+    int32_t *__restrict__ count, const int32_t *__restrict__ start,
+    const int32_t *__restrict__ sorted, int32_t *__restrict__ order, float *__restrict__ partial,
+    float *__restrict__ partial2, int32_t *__restrict__ npercell, uint8_t *__restrict__ tileres,
+    uint8_t *__restrict__ dirty, int32_t *__restrict__ cursor, DevScalars *sc, int zero) {
+  constexpr bool MIX = MODE == A32_MIX;
+  constexpr int NV = MODE == A32_P2G ? 4 : MODE == A32_MIX ? 6 : 5;
   constexpr int NF = NV + 1;
-  constexpr int SPT = TILE32 * CAP / ATPB;  // slot entries per thread
-  constexpr int RPT = ROWS / ATPB;         // dense rows per thread
-  __shared__ float4 sgeo[ROWS];  // ox, oy, oz, vol
-  __shared__ float4 sva[ROWS];   // values 0..3
-  __shared__ float svb[NV >= 5 ? ROWS : 1];
-  __shared__ float svc[NV >= 6 ? ROWS : 1];
-  __shared__ int32_t sidx[ROWS];
-  __shared__ int16_t sperm[ROWS];  // the rows of a cell in parcel order, as byte offsets 16 r
-  __shared__ uint8_t skeep[MIX ? ROWS : 1];
-  __shared__ int32_t soff[TILE32 + 1];  // first dense row of each cell of the tile
-  __shared__ int32_t scnt[TILE32], sost[TILE32];
-  __shared__ uint32_t sover;            // bit cl: cell cl is listed in the dense overflow region
-  __shared__ float skz[TILE32];         // z level of each cell of the tile
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int cl = tid >> 3;
-  const int q = tid & 7;
-  const int bx = q & 1, by = (q >> 1) & 1, bz = (q >> 2) & 1;
-  // corner factor f = s * offset + t: offset for the upper corner, 1 - offset for the lower
-  // corner factors |t - offset|: t = 1 at the lower corner, 0 at the upper
+  __shared__ float4 sgeo[64];               // offsets, vol
+  __shared__ float4 sval[64];               // the first four values
+  __shared__ float2 sval2[NV > 4 ? 64 : 1];  // the others
+  __shared__ int32_t slist[LIST * 8];       // entry e of cell cl at 8 e + cl
+  const int lane = threadIdx.x, cl = lane & 7, q = lane >> 3;
+  const int bx = q & 1, by = (q >> 1) & 1, bz = q >> 2;
   const float tx = bx ? 0.f : 1.f, ty = by ? 0.f : 1.f, tz = bz ? 0.f : 1.f;
+  const uint32_t ntx = (uint32_t)tiles_x(g);
   const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
-  // a par2grid whose partials the last x-row mixing sums left current: only the tiles mixing
-  // changed (dirty) are summed again
-  if (dirty && !dirty[tile]) return;
-  const int64_t c0 = (int64_t)tile * TILE32;
-  // cell, tile and row numbers are below 2^31, so their divisions are 32-bit; an x-row tile
-  // has ntx tiles per row
-  const uint32_t ntx = XC ? (uint32_t)g.nx / TILE32 : 1u;
-  const int ntile = (int)min((int64_t)TILE32, ncell - c0);
-  const int capc = b.capc;
-  int32_t sl[SPT];
-#pragma unroll
-  for (int k = 0; k < SPT; k++) {
-    const int e = tid + k * ATPB;
-    sl[k] = (capc > 0 && e < ntile * CAP) ? ld(b.slot, (uint32_t)(c0 * CAP + e)) : -1;
+  const uint32_t xrow = tile / ntx, tile_x = tile - xrow * ntx;
+  const int m = min(8, g.nx - 8 * (int)tile_x);  // cells here
+  const bool live = cl < m;
+  const int64_t c = (int64_t)xrow * g.nx + 8 * tile_x + (live ? cl : 0);
+  const int32_t *own = slot + c * capc;
+  int32_t pre[2] = {0, 0};
+  if (capc) {
+    pre[0] = own[q];
+    pre[1] = own[8 + q];
   }
-  if (tid < 64) {
-    const int32_t v = (tid < ntile) ? count[c0 + tid] : 0;
-    const int32_t o = (tid < ntile) ? ostart[c0 + tid] : 0;
-    int32_t incl = v;
-#pragma unroll
-    for (int d = 1; d < TILE32; d <<= 1) {
-      const int32_t u = __shfl_up(incl, d);
-      if (lane >= d) incl += u;
-    }
-    const unsigned long long om = __ballot(tid < TILE32 && v > capc);
-    if (tid < TILE32) {
-      scnt[tid] = v;
-      sost[tid] = o;
-      soff[tid + 1] = incl;
-      const uint32_t kc = XC ? tile / ntx / (uint32_t)g.ny
-                             : (uint32_t)(c0 + tid) / ((uint32_t)g.nx * (uint32_t)g.ny);
-      skz[tid] = (tid < ntile) ? (float)kc : 0.f;
-    }
-    if (tid == 0) {
-      soff[0] = 0;
-      sover = (uint32_t)om;
+  const int n = live ? count[c] : 0;
+  if (zero) {
+    if (live && q == 0) count[c] = 0;
+    if (tile == 0 && lane == 0) {
+      *cursor = 0;
+      sc->novf = 0;
     }
   }
-  __syncthreads();
-  const float *F = b.f;
-  auto fld = [&](int f) { return b.fp[f]; };
-  // one parcel's staged values
-  auto fetch = [&](uint32_t pp, float4 &geo, float4 &va, float &vb) {
-    geo = make_float4(ldnt(fld(B_OX), pp), ldnt(fld(B_OY), pp), ldnt(fld(B_OZ), pp),
-                      ldnt(fld(B_VOL), pp));
-    if constexpr (BT) {
-      va = make_float4(ldnt(fld(B_P), pp), ldnt(fld(B_Q), pp), ldnt(fld(B_R), pp),
-                       ldnt(fld(B_B), pp));
-      vb = ldnt(fld(B_H), pp);  // humidity, for the total buoyancy below
-    } else {
-      va = make_float4(ldnt(fld(B_B), pp), ldnt(fld(B_H), pp), ldnt(fld(B_P), pp),
-                       ldnt(fld(B_Q), pp));
-      vb = ldnt(fld(B_R), pp);
-    }
-  };
-  // kz: the z level of the parcel's cell (known from the tile, so the cell is not read)
-  auto put = [&](int r, int32_t pp, float4 geo, float4 v, float vb, float kz) {
-    if constexpr (BT) {
-      // total buoyancy (vorticity_tendency.F90:121-126)
-      const float z = fmaf(kz + geo.z, zm.dz, zm.zbot);
-      const float hl = vb - expf(-z);
-      const float bv = v.w;
-      v.w = fmaf(12.5f, hl > 0.f ? hl : 0.f, bv);
-      if constexpr (NV >= 6) {
-        svb[r] = bv;
-        svc[r] = vb;
-      }
-    } else {
-      svb[r] = vb;
-    }
-    if constexpr (MIX) skeep[r] = (geo.w < vmin) ? 0 : 1;
-    sgeo[r] = geo;
-    sva[r] = v;
-    sidx[r] = pp;
-  };
-  float acc[NF], res[NF];
+  if constexpr (MODE == A32_P2G) {
+    // a par2grid whose sums the last mixing left current: only the tiles it changed
+    if (dirty && !dirty[tile]) return;
+  }
+  int nmax = n;
 #pragma unroll
-  for (int f = 0; f < NF; f++) { acc[f] = 0.f; res[f] = 0.f; }
-  int kept = 0, nres = 0;
-  bool big = false;
-  int first = 0;
-  while (first < ntile) {
-    int last = first + 1;
-    if (soff[ntile] - soff[first] <= ROWS) last = ntile;  // the usual case: the rest fits
-    else
-      while (last < ntile && soff[last + 1] - soff[first] <= ROWS) last++;
-    const int32_t r0 = soff[first];
-    const int nrows = soff[last] - r0;
-    const bool fits = nrows <= ROWS;
-    if (fits) {
-      // rows of the cells listed in the slot table, from the entries already loaded
-      int32_t pr[SPT], row[SPT];
+  for (int d = 1; d < 8; d <<= 1) nmax = max(nmax, __shfl_xor(nmax, d));
+  nmax = __builtin_amdgcn_readfirstlane(nmax);
+  const int nch = (nmax + 7) >> 3;  // chunks of eight parcels a cell
+  const bool small = nmax <= LIST;
+  const bool dense = n > capc;
+  const int64_t b = dense ? start[c] : 0;
+  const int32_t *list = dense ? sorted + b : own;
+  // entries 8 i + q of the cell, ordered by parcel
+  if (small) {
+    bool bad = false;
 #pragma unroll
-      for (int k = 0; k < SPT; k++) {
-        const int e = tid + k * ATPB;
-        const int ce = e / CAP, j = e % CAP;
-        pr[k] = -1;
-        row[k] = 0;
-        if (sl[k] >= 0 && ce >= first && ce < last && j < scnt[ce] && scnt[ce] <= capc) {
-          pr[k] = sl[k];
-          row[k] = soff[ce] - r0 + j;
-        }
-      }
-      float4 geo[SPT], va[SPT];
-      float vb[SPT];
-#pragma unroll
-      for (int k = 0; k < SPT; k++)
-        if (pr[k] >= 0) fetch((uint32_t)pr[k], geo[k], va[k], vb[k]);
-#pragma unroll
-      for (int k = 0; k < SPT; k++)
-        if (pr[k] >= 0) put(row[k], pr[k], geo[k], va[k], vb[k], skz[(tid + k * ATPB) / CAP]);
-      // rows of the cells listed in the dense overflow region
-      const uint32_t pass = (last - first >= 32 ? ~0u : ((1u << (last - first)) - 1u)) << first;
-      if (sover & pass) {
-        for (int k = 0; k < RPT; k++) {
-          const int r = tid + k * ATPB;
-          if (r >= nrows) break;
-          // the cell of dense row r: the last cell of the pass starting at or before it
-          int lo_ = first, hi_ = last - 1;
-          while (lo_ < hi_) {
-            const int mid = (lo_ + hi_ + 1) >> 1;
-            if (soff[mid] - r0 <= r) lo_ = mid;
-            else hi_ = mid - 1;
-          }
-          if (!((sover >> lo_) & 1u)) continue;
-          const int32_t pp = ld(sorted, (uint32_t)(sost[lo_] + (r + r0 - soff[lo_])));
-          float4 g1, v1;
-          float b1;
-          fetch((uint32_t)pp, g1, v1, b1);
-          put(r, pp, g1, v1, b1, skz[lo_]);
-        }
-      }
+    for (int i = 0; i < LIST / 8; i++) {
+      if (i >= nch) break;
+      const int e = 8 * i + q;
+      slist[64 * i + lane] = e >= n ? INT32_MAX : i < 2 && !dense ? pre[i < 2 ? i : 0] : list[e];
     }
     __syncthreads();
-    const bool mine = fits && cl >= first && cl < last;
-    const int lo = mine ? soff[cl] - r0 : 0, hi = mine ? soff[cl + 1] - r0 : 0;
-    bool ord = true;
-    for (int a = lo + 1 + q; a < hi; a += 8) ord &= (sidx[a - 1] < sidx[a]);
-    const unsigned long long bad = __ballot(!ord);
-    const bool sort_cell = ((bad >> (lane & ~7)) & 0xffull) != 0ull;
-    if (sort_cell) {
-      for (int a = lo + q; a < hi; a += 8) {
-        const int32_t key = sidx[a];
-        int rk = 0;
-        for (int bb = lo; bb < hi; bb++) rk += (sidx[bb] < key) ? 1 : 0;
-        sperm[lo + rk] = (int16_t)(a * 16);
-      }
-    } else {
-      for (int a = lo + q; a < hi; a += 8) sperm[a] = (int16_t)(a * 16);
-    }
-    __syncthreads();
-#pragma unroll 2
-    for (int a = lo; a < hi; a++) {
-      const int off = sperm[a];
-      const float4 gr = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(sgeo) + off);
-      const float4 v = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(sva) + off);
-      const float w = corner_weight(gr.x, gr.y, gr.z, gr.w, tx, ty, tz);
-      float vals[6] = {v.x, v.y, v.z, v.w, 0.f, 0.f};
-      if constexpr (NV >= 5) vals[4] = svb[off >> 4];
-      if constexpr (NV >= 6) vals[5] = svc[off >> 4];
-      if (!MIX || skeep[off >> 4]) {
-        add_parcel<NV>(acc, w, vals);
-        kept++;
-      } else {
-        nres++;
-        add_parcel<NV>(res, w, vals);
-      }
-    }
-    if (fits == false && cl == first) big = true;
-    __syncthreads();
-    first = last;
-  }
-  const bool live = cl < ntile;
-  const int64_t c = c0 + cl;
-  if (live && big) {
-    // more parcels than LDS rows: always in the overflow region, sorted by parcel there
-    const int32_t s0 = sost[cl], s1 = s0 + scnt[cl];
-    for (int32_t s = s0; s < s1; s++) {
-      const int64_t pp = sorted[s];
-      const float ox = F[B_OX * cap + pp], oy = F[B_OY * cap + pp], oz = F[B_OZ * cap + pp];
-      const float vol = F[B_VOL * cap + pp];
-      float vals[6];
-      if constexpr (BT) {
-        const float z = fmaf(skz[cl] + oz, zm.dz, zm.zbot);
-        const float hv = F[B_H * cap + pp], bv = F[B_B * cap + pp];
-        const float hl = hv - expf(-z);
-        vals[0] = F[B_P * cap + pp];
-        vals[1] = F[B_Q * cap + pp];
-        vals[2] = F[B_R * cap + pp];
-        vals[3] = fmaf(12.5f, hl > 0.f ? hl : 0.f, bv);
-        vals[4] = bv;
-        vals[5] = hv;
-      } else {
-        vals[0] = F[B_B * cap + pp];
-        vals[1] = F[B_H * cap + pp];
-        vals[2] = F[B_P * cap + pp];
-        vals[3] = F[B_Q * cap + pp];
-        vals[4] = F[B_R * cap + pp];
-      }
-      const float w = corner_weight(ox, oy, oz, vol, tx, ty, tz);
-      if (!MIX || !(vol < vmin)) {
-        add_parcel<NV>(acc, w, vals);
-        kept++;
-      } else {
-        nres++;
-        add_parcel<NV>(res, w, vals);
-      }
-    }
-  }
-  if constexpr (XC) {
-    // the tile's 16 cells lie in one x row: node position pos (0..16) of corner pair
-    // bb = (by, bz) sums the bx = 1 corner of cell pos - 1 and the bx = 0 corner of cell pos
-    // (left + right); positions 0 and 16 hold one side, completed by k32_node_sum_x.  Value f
-    // of entry (bb, row, tx, pos) sits at ((f 4 + bb) nrows + row) W + 17 tx + pos, W = 17 ntx:
-    // each value's plane is read coalesced by the node sums.
-    static_assert(TILE32 == 16, "x-combined partials of 16-cell tiles");
-    float *cor = reinterpret_cast<float *>(sgeo);  // free after the passes' last barrier
-    static_assert(ATPB * NF <= ROWS * 4, "the corner sums fit the staging rows");
-    const uint32_t xrow = tile / ntx;
-    const int64_t row = xrow;
-    const int tx = (int)(tile - xrow * ntx);
-    const int64_t nrows = (int64_t)g.ny * g.ncz;
-    const int64_t fstride = 4 * nrows * (int64_t)(ntx * 17);
-    auto write_x = [&](const float *v, float *out) {
-      __syncthreads();  // cor free (the passes' staging, or the previous write_x's reads)
 #pragma unroll
-      for (int f = 0; f < NF; f++) cor[tid * NF + f] = v[f];  // tid = cell * 8 + corner
+    for (int i = 0; i < LIST / 8; i++) {
+      if (i >= nch) break;
+      if (8 * i + q + 1 < n) bad |= slist[64 * i + lane] > slist[64 * i + lane + 8];
+    }
+    if (__any(bad)) {
+      auto sort = [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        int32_t v[W];
+        int r[W];
+#pragma unroll
+        for (int i = 0; i < W; i++) v[i] = i < nch ? slist[64 * i + lane] : INT32_MAX;
+        rank_entries<W>(v, r, nmax, [&](int e) { return slist[8 * e + cl]; });
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < W; i++)
+          if (8 * i + q < n) slist[8 * r[i] + cl] = v[i];
+      };
+      if (nch <= 2) sort(std::integral_constant<int, 2>());
+      else sort(std::integral_constant<int, LIST / 8>());
       __syncthreads();
-      if (tid < 4 * 17) {
-        const int bb = tid / 17, pos = tid - bb * 17;
-        float *dst = out + ((int64_t)bb * nrows + row) * (ntx * 17) + tx * 17 + pos;
-        // cell pos - 1, bx = 1 and cell pos, bx = 0 (indices clamped into the tile; the ends
-        // use one side only)
-        const float *L = cor + ((pos > 0 ? pos - 1 : 0) * 8 + 1 + 2 * bb) * NF;
-        const float *R = cor + ((pos < 16 ? pos : 15) * 8 + 2 * bb) * NF;
-#pragma unroll
-        for (int f = 0; f < NF; f++)
-          dst[f * fstride] = pos == 0 ? R[f] : pos == 16 ? L[f] : L[f] + R[f];
-      }
-    };
-    write_x(acc, partial);
-    if constexpr (MIX) {
-      // residual partials only from tiles that have residual parcels (tileres)
-      const bool anyres = __syncthreads_or(nres > 0);
-      if (tid == 0) tileres[tile] = anyres ? 1 : 0;
-      if (q == 0) npercell[c0 + cl] = kept;
-      if (anyres) write_x(res, partial2);
     }
-    return;
+  } else {
+    bool bad = false;
+    for (int i = 0; i < nch; i++)
+      if (8 * i + q + 1 < n) bad |= list[8 * i + q] > list[8 * i + q + 1];
+    if (__any(bad)) {
+      // a cell still in the slot table is ordered into its own entries, after the reads
+      int32_t *out = dense ? order + b : nullptr;
+      for (int i0 = 0; i0 < nch; i0 += 8) {
+        int32_t v[8];
+        int r[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = 8 * (i0 + i) + q < n ? list[8 * (i0 + i) + q] : INT32_MAX;
+        rank_entries<8>(v, r, nmax, [&](int e) { return e < n ? list[e] : INT32_MAX; });
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          if (8 * (i0 + i) + q < n) {
+            if (out) out[r[i]] = v[i];
+            else slist[8 * r[i] + cl] = v[i];  // at most capc <= LIST entries
+          }
+      }
+      __threadfence_block();
+      __syncthreads();
+      if (out) list = out;
+    } else {
+      for (int i = 0; i < LIST / 8; i++)
+        if (!dense && 8 * i + q < n) slist[64 * i + lane] = list[8 * i + q];
+      __syncthreads();
+    }
   }
-  // mixing: a tile without residual parcels writes no residual partials; tileres tells the
-  // residual node sums which tiles have them
+  const bool in_lds = small || !dense;
+  const float kz = (float)(xrow / (uint32_t)g.ny);
+  Float3 off{}, vor{}, vbh{};
+  auto fetch = [&](int ch) {
+    const int e = 8 * ch + q;
+    if (e < n) {
+      const int64_t p = in_lds ? slist[64 * ch + lane] : list[e];
+      off = ld3(P.off, p);
+      vor = ld3(P.vor, p);
+      vbh = ld3(P.vbh, p);
+    }
+  };
+  float acc[NF], res[MIX ? NF : 1];
+#pragma unroll
+  for (int f = 0; f < NF; f++) acc[f] = 0.f;
+#pragma unroll
+  for (int f = 0; f < (MIX ? NF : 1); f++) res[f] = 0.f;
+  int kept = 0;
   bool anyres = false;
-  if constexpr (MIX) {
-    anyres = __syncthreads_or(live && nres > 0);
-    if (tid == 0) tileres[tile] = anyres ? 1 : 0;
-  }
-  if (!live) return;
-#pragma unroll
-  for (int f = 0; f < NF; f++) partial[((int64_t)q * ncell + c) * NF + f] = acc[f];
-  if constexpr (MIX) {
-    if (anyres) {
-#pragma unroll
-      for (int f = 0; f < NF; f++) partial2[((int64_t)q * ncell + c) * NF + f] = res[f];
-    }
-    if (q == 0) npercell[c] = kept;
-  }
-}
-
-// node sums of the FP32 corner partials (the plain form's k_node_sum): NORM divides by the
-// summed weight (par2grid) into FP64 grids; otherwise raw FP32 sums, doubled on the z
-// boundaries when DBL (mixing kept grids)
-template <typename T>
-struct Out32 {
-  T *p[7];  // null: a plane not written
-};
-
-// tileres (may be null): per accumulation tile, whether its cells' partials were written; the
-// cells of a tile without them contribute zero
-template <int NV, bool NORM, bool DBL, typename T>
-__global__ void k32_node_sum(Geometry g, const float *__restrict__ partial, int64_t ncell,
-                             Out32<T> out, const uint8_t *__restrict__ tileres) {
-  const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nnode) return;
-  const int i = (int)(t % g.nx);
-  const int j = (int)((t / g.nx) % g.ny);
-  const int k = (int)(t / ((int64_t)g.nx * g.ny));
-  // every corner's partials are loaded first (a corner below the bottom or above the top cell
-  // reads cell 0 and is left out of the sum), then summed in the fixed corner order
-  float v[8][NV + 1];
-  bool ok[8];
-#pragma unroll
-  for (int q = 0; q < 8; q++) {
-    const int bx = q & 1, by = (q >> 1) & 1, bz = q >> 2;
-    int ci = i - bx;
-    if (ci < 0) ci += g.nx;
-    int cj = j - by;
-    if (cj < 0) cj += g.ny;
-    const int ck = k - bz;
-    ok[q] = ck >= 0 && ck < g.ncz;
-    const int64_t c = ok[q] ? ((int64_t)ck * g.ny + cj) * g.nx + ci : 0;
-    if (ok[q] && tileres && !tileres[c / TILE32]) ok[q] = false;
-#pragma unroll
-    for (int f = 0; f <= NV; f++)
-      v[q][f] = ok[q] ? partial[((int64_t)q * ncell + c) * (NV + 1) + f] : 0.f;
-  }
-  float s[NV + 1];
-#pragma unroll
-  for (int f = 0; f <= NV; f++) s[f] = 0.f;
-#pragma unroll
-  for (int bx = 0; bx < 2; bx++)
-#pragma unroll
-    for (int by = 0; by < 2; by++)
-#pragma unroll
-      for (int bz = 0; bz < 2; bz++) {
-        const int q = (bz << 2) | (by << 1) | bx;
-#pragma unroll
-        for (int f = 0; f <= NV; f++) s[f] = ok[q] ? s[f] + v[q][f] : s[f];
-      }
-  if (NORM) {
-    float w = s[0];
-    if (w == 0.f) w = 1.f;
-#pragma unroll
-    for (int f = 1; f <= NV; f++) out.p[f - 1][t] = (T)(s[f] / w);
-  } else {
-    const float m = (DBL && (k == 0 || k == g.nzn - 1)) ? 2.f : 1.f;
-#pragma unroll
-    for (int f = 0; f <= NV; f++) out.p[f][t] = (T)(s[f] * m);
-  }
-}
-
-// node sums of the x-combined partials of A32_P2GX / A32_MIXX (NF values: the weight and NF - 1
-// weighted sums): node (i, j, k) adds, for each corner pair (by, bz) in a fixed order, the
-// entry of cell row (j - by, k - bz) at its node position, and at a tile boundary the left
-// tile's last position before the right tile's first (the same left + right order as inside a
-// tile).  NORM divides by the summed weight into NF - 1 grids; otherwise the NF raw sums,
-// doubled on the z boundaries when DBL.  tileres (may be null): per tile, whether its entries
-// were written; the entries of a tile without them contribute zero.
-template <int NF, bool NORM, bool DBL>
-__global__ void k32_node_sum_x(Geometry g, const float *__restrict__ partial, Out32<float> out,
-                               const uint8_t *__restrict__ tileres) {
-  const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nnode) return;
-  const int i = (int)(t % g.nx);
-  const int j = (int)((t / g.nx) % g.ny);
-  const int k = (int)(t / ((int64_t)g.nx * g.ny));
-  const int ntx = g.nx / TILE32, tx = i / TILE32, pos = i - tx * TILE32;
-  const int txl = tx == 0 ? ntx - 1 : tx - 1;  // the tile left of a boundary (periodic in x)
-  const int64_t nrows = (int64_t)g.ny * g.ncz, w = (int64_t)ntx * 17;
-  const int64_t fstride = 4 * nrows * w;  // value planes (the layout k32_cell_accum writes)
-  float v[4][NF], vl[4][NF];
-  bool ok[4], okl[4];
-#pragma unroll
-  for (int bb = 0; bb < 4; bb++) {
-    const int by = bb & 1, bz = bb >> 1;
-    int cj = j - by;
-    if (cj < 0) cj += g.ny;
-    const int ck = k - bz;
-    const bool in = ck >= 0 && ck < g.ncz;
-    const int64_t crow = in ? (int64_t)ck * g.ny + cj : 0;
-    ok[bb] = in && (!tileres || tileres[crow * ntx + tx]);
-    okl[bb] = in && pos == 0 && (!tileres || tileres[crow * ntx + txl]);
-    const int64_t base = ((int64_t)bb * nrows + crow) * w;
-    const float *e = partial + base + tx * 17 + pos;
-    const float *el = partial + base + txl * 17 + 16;
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-      v[bb][f] = ok[bb] ? e[f * fstride] : 0.f;
-      vl[bb][f] = okl[bb] ? el[f * fstride] : 0.f;
-    }
-  }
-  float s[NF];
-#pragma unroll
-  for (int f = 0; f < NF; f++) s[f] = 0.f;
-#pragma unroll
-  for (int bb = 0; bb < 4; bb++)
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-      if (pos == 0) {
-        if (okl[bb] || ok[bb]) s[f] = s[f] + (vl[bb][f] + v[bb][f]);
-      } else if (ok[bb]) {
-        s[f] = s[f] + v[bb][f];
+  if (nch > 0) fetch(0);
+  for (int ch = 0; ch < nch; ch++) {
+    if (8 * ch + q < n) {
+      sgeo[lane] = make_float4(off.x, off.y, off.z, vbh.x);
+      if constexpr (MODE == A32_DUMP) {
+        sval[lane] = make_float4(vbh.y, vbh.z, vor.x, vor.y);
+        sval2[lane] = make_float2(vor.z, 0.f);
+      } else {
+        // total buoyancy (vorticity_tendency.F90:121-126)
+        const float z = fmaf(kz + off.z, zm.dz, zm.zbot);
+        const float hl = vbh.z - expf(-z);
+        sval[lane] = make_float4(vor.x, vor.y, vor.z, fmaf(12.5f, hl > 0.f ? hl : 0.f, vbh.y));
+        if constexpr (MIX) sval2[lane] = make_float2(vbh.y, vbh.z);
       }
     }
-  if constexpr (NORM) {
-    float wsum = s[0];
-    if (wsum == 0.f) wsum = 1.f;
+    __syncthreads();
+    if (ch + 1 < nch) fetch(ch + 1);
+    const int rows = min(8, nmax - 8 * ch), mine = n - 8 * ch;
+#pragma unroll 2
+    for (int a = 0; a < rows; a++) {
+      const int r = 8 * a + cl;
+      const float4 ge = sgeo[r], v4 = sval[r];
+      float v[6] = {v4.x, v4.y, v4.z, v4.w, 0.f, 0.f};
+      if constexpr (NV > 4) {
+        v[4] = sval2[r].x;
+        v[5] = sval2[r].y;
+      }
+      const float w = corner_weight(ge.x, ge.y, ge.z, ge.w, tx, ty, tz);
+      if (a < mine) {
+        if (!MIX || !(ge.w < vmin)) {
+          add_parcel<NV>(acc, w, v);
+          kept++;
+        } else if constexpr (MIX) {
+          anyres = true;
+          add_parcel<NV>(res, w, v);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  const int64_t nrows = (int64_t)g.ny * g.ncz, W = g.nx + (int64_t)ntx;
+  auto write_x = [&](const float *v, float *out) {
+    const int64_t o = ((int64_t)(q >> 1) * nrows + xrow) * W + 9 * tile_x + (bx ? 8 : cl);
+    const bool mine = bx ? (cl == 7 && m == 8) : cl <= m;
 #pragma unroll
-    for (int f = 1; f < NF; f++)
-      if (out.p[f - 1]) out.p[f - 1][t] = s[f] / wsum;
-  } else {
-    const float m = (DBL && (k == 0 || k == g.nzn - 1)) ? 2.f : 1.f;
-#pragma unroll
-    for (int f = 0; f < NF; f++)
-      if (out.p[f]) out.p[f][t] = s[f] * m;
+    for (int f = 0; f < NF; f++) {
+      const float left = __shfl(v[f], (lane + 7) & 63);  // corner q | 1 of cell cl - 1
+      if (mine) out[f * 4 * nrows * W + o] = bx || cl == 0 ? v[f] : left + v[f];
+    }
+  };
+  write_x(acc, partial);
+  if constexpr (MIX) {
+    const bool any = __any(anyres) != 0;
+    if (lane == 0) {
+      tileres[tile] = any ? 1 : 0;
+      dirty[tile] = 0;
+    }
+    if (tile == 0 && lane == 0) sc->anydirty = 0;
+    if (any) write_x(res, partial2);
+    if (live && q == 0) npercell[c] = kept;
   }
 }
 
@@ -906,37 +672,43 @@ __device__ __forceinline__ void bin_lane(const Geometry &g, int32_t cell, uint32
   }
 }
 
-// the RK stage of parcel p; returns its new cell, or -1 when it left the box (status raised)
+// the sets a stage reads, takes as the RK4 origin and writes
+struct RkSets {
+  const int32_t *cell, *cello;
+  const float *off, *offo, *vor, *voro;
+  int32_t *cell_to;
+  float *off_to, *vor_to;
+};
+
+// The RK stage of parcel p; returns its new cell, or -1 when it left the box (status raised).  The
+// sets of a stage may be the same arrays: a thread reads its parcel before it writes it.
 template <int STAGE>
-__device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b, int64_t cap,
+__device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b, const RkSets &rs,
                                              const float4 *__restrict__ rec,
                                              const Scale32 &sc3,
                                              int stretch, uint8_t *__restrict__ split_flag,
                                              DevScalars *sc, uint32_t p) {
-  float *F = b.f;
-  auto fld = [&](int f) { return F + (size_t)f * cap; };
-  const int32_t cell = ldnt(b.cell, p);
-  const float ox = ldnt(fld(B_OX), p), oy = ldnt(fld(B_OY), p), oz = ldnt(fld(B_OZ), p);
-  int32_t cello;
-  float oo[3], df[3] = {0.f, 0.f, 0.f}, vo[3] = {0.f, 0.f, 0.f}, vf[3] = {0.f, 0.f, 0.f};
+  const int32_t cell = ldnt(rs.cell, p);
+  const Float3 off = ld3(rs.off, p);
+  const float ox = off.x, oy = off.y, oz = off.z;
+  int32_t cello = cell;
+  float oo[3] = {ox, oy, oz}, df[3] = {0.f, 0.f, 0.f}, vo[3] = {0.f, 0.f, 0.f},
+        vf[3] = {0.f, 0.f, 0.f};
+  auto take = [](float *a, const Float3 &v) {
+    a[0] = v.x;
+    a[1] = v.y;
+    a[2] = v.z;
+  };
   if (STAGE == 1) {
-    cello = cell;
-    oo[0] = ox;
-    oo[1] = oy;
-    oo[2] = oz;
-#pragma unroll
-    for (int a = 0; a < 3; a++) vo[a] = ldnt(fld(B_P + a), p);
+    take(vo, ld3(rs.vor, p));
   } else {
-    cello = ldnt(b.cello, p);
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      oo[a] = ldnt(fld(B_OXO + a), p);
-      df[a] = ldnt(fld(B_DFX + a), p);
-      if (STAGE != 4) vo[a] = ldnt(fld(B_PO + a), p);
-      vf[a] = ldnt(fld(B_PF + a), p);
-    }
+    cello = ldnt(rs.cello, p);
+    take(oo, ld3(rs.offo, p));
+    take(df, ld3(b.df, p));
+    if (STAGE != 4) take(vo, ld3(rs.voro, p));
+    take(vf, ld3(b.pf, p));
   }
-  const float s_old = (STAGE == 4 && stretch) ? ldnt(fld(B_STRETCH), p) : 0.f;
+  const float s_old = (STAGE == 4 && stretch) ? ldnt(b.stretch, p) : 0.f;
   int i, j, k;
   cell_ijk(g, cell, i, j, k);
   int32_t o[8];
@@ -988,35 +760,21 @@ __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b,
     raise_status(sc, PMPIC_ERR_OUT_OF_BOX_Z);
     return -1;
   }
-  stnt(b.cell, p, ncell_);
-  stnt(fld(B_OX), p, nox);
-  stnt(fld(B_OY), p, noy);
-  stnt(fld(B_OZ), p, noz);
-#pragma unroll
-  for (int a = 0; a < 3; a++) stnt(fld(B_P + a), p, vn[a]);
-  if (STAGE == 1) {
-    stnt(b.cello, p, cello);
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      stnt(fld(B_OXO + a), p, oo[a]);
-      stnt(fld(B_PO + a), p, vo[a]);
-    }
-  }
+  stnt(rs.cell_to, p, ncell_);
+  st3(rs.off_to, p, nox, noy, noz);
+  st3(rs.vor_to, p, vn[0], vn[1], vn[2]);
   if (STAGE != 4) {
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      stnt(fld(B_DFX + a), p, dfn[a]);
-      stnt(fld(B_PF + a), p, vfn[a]);
-    }
+    st3(b.df, p, dfn[0], dfn[1], dfn[2]);
+    st3(b.pf, p, vfn[0], vfn[1], vfn[2]);
   } else {
-#pragma unroll
-    for (int f = 0; f < 6; f++) stnt(fld(B_DXDT + f), p, kv[f]);
+    st3(b.dx, p, kv[0], kv[1], kv[2]);
+    st3(b.dp, p, kv[3], kv[4], kv[5]);
     if (stretch) {
       const float third = 1.f / 3.f;
       float ds = vn[0] * kv[3] + vn[1] * kv[4] + vn[2] * kv[5];
       ds = powf(fabsf(ds), third);
       const float snew = s_old + ds * dt;
-      stnt(fld(B_STRETCH), p, snew);
+      stnt(b.stretch, p, snew);
       split_flag[p] = (snew > 4.f) ? 1 : 0;  // the test of parcel_splitting.F90:76
     }
   }
@@ -1024,7 +782,7 @@ __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b,
 }
 
 template <int STAGE>
-__global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, int64_t cap, int64_t n,
+__global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, RkSets rs, int64_t n,
                                                     const float4 *__restrict__ rec, Scale32 sc3,
                                                     int stretch,
                                                     uint8_t *__restrict__ split_flag,
@@ -1036,17 +794,17 @@ __global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, int64_
   // with bo.on, the parcel's new cell is binned for the next stage's par2grid as k32_bin_slot
   // bins it; every lane of the wavefront then takes part, parcels past the count as empty
   if (bo.on) {
-    const int32_t nc = valid ? rk_update<STAGE>(g, b, cap, rec, sc3, stretch, split_flag, sc, p)
+    const int32_t nc = valid ? rk_update<STAGE>(g, b, rs, rec, sc3, stretch, split_flag, sc, p)
                              : -1;
     bin_lane(g, nc, p, bo, sc);
     return;
   }
   if (!valid) return;
-  rk_update<STAGE>(g, b, cap, rec, sc3, stretch, split_flag, sc, p);
+  rk_update<STAGE>(g, b, rs, rec, sc3, stretch, split_flag, sc, p);
 }
 
 // ---- splitting (parcel_splitting.F90:76-131, then the haloswap's wrap and reflection) ----
-__global__ void k32_split_apply(Geometry g, Bulk32 b, int64_t cap, int64_t n, Scale32 sc3,
+__global__ void k32_split_apply(Geometry g, Parcels32 P, int64_t cap, int64_t n, Scale32 sc3,
                                 const int32_t *__restrict__ parents, int64_t nsplit,
                                 DevScalars *sc) {
   const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1057,17 +815,17 @@ __global__ void k32_split_apply(Geometry g, Bulk32 b, int64_t cap, int64_t n, Sc
     raise_status(sc, PMPIC_ERR_MAXPARCELS);
     return;
   }
-  float *F = b.f;
   const float third = 1.f / 3.f;
   const float pi = 3.14159265358979f;
-  const float p = F[B_P * cap + i], q = F[B_Q * cap + i], r = F[B_R * cap + i];
-  const float vol = F[B_VOL * cap + i];
+  const Float3 w = ld3(P.vor, i), vbh = ld3(P.vbh, i), off = ld3(P.off, i);
+  const float p = w.x, q = w.y, r = w.z;
+  const float vol = vbh.x;
   const float rr = powf(vol / 4.f / pi, third);
   const float absw = sqrtf(p * p + q * q + r * r);
   const float d[3] = {rr * p / absw * sc3.idx, rr * q / absw * sc3.idy, rr * r / absw * sc3.idz};
   int ci, cj, ck;
-  cell_ijk(g, b.cell[i], ci, cj, ck);
-  const float ox = F[B_OX * cap + i], oy = F[B_OY * cap + i], oz = F[B_OZ * cap + i];
+  cell_ijk(g, P.cell[i], ci, cj, ck);
+  const float ox = off.x, oy = off.y, oz = off.z;
   int32_t cc, cp;
   float cx, cy, cz, px, py, pz;
   const bool okc = place(g, ci, cj, ck, ox + d[0], oy + d[1], oz + d[2], cc, cx, cy, cz);
@@ -1076,25 +834,19 @@ __global__ void k32_split_apply(Geometry g, Bulk32 b, int64_t cap, int64_t n, Sc
     raise_status(sc, PMPIC_ERR_OUT_OF_BOX_Z);
     return;
   }
-  b.cell[c] = cc;
-  F[B_OX * cap + c] = cx;
-  F[B_OY * cap + c] = cy;
-  F[B_OZ * cap + c] = cz;
-  F[B_P * cap + c] = p;
-  F[B_Q * cap + c] = q;
-  F[B_R * cap + c] = r;
-  for (int f = B_DXDT; f <= B_DRDT; f++) F[(int64_t)f * cap + c] = F[(int64_t)f * cap + i];
-  F[B_H * cap + c] = F[B_H * cap + i];
-  F[B_B * cap + c] = F[B_B * cap + i];
-  F[B_VOL * cap + c] = vol / 2;
-  F[B_STRETCH * cap + c] = 0.f;
-  b.tag[c] = b.tag[i];
-  b.cell[i] = cp;
-  F[B_OX * cap + i] = px;
-  F[B_OY * cap + i] = py;
-  F[B_OZ * cap + i] = pz;
-  F[B_VOL * cap + i] = vol / 2;
-  F[B_STRETCH * cap + i] = 0.f;
+  P.cell[c] = cc;
+  st3(P.off, c, cx, cy, cz);
+  st3(P.vor, c, p, q, r);
+  const Float3 dx = ld3(P.dx, i), dp = ld3(P.dp, i);
+  st3(P.dx, c, dx.x, dx.y, dx.z);
+  st3(P.dp, c, dp.x, dp.y, dp.z);
+  st3(P.vbh, c, vol / 2, vbh.y, vbh.z);
+  P.stretch[c] = 0.f;
+  P.tag[c] = P.tag[i];
+  P.cell[i] = cp;
+  st3(P.off, i, px, py, pz);
+  P.vbh[3 * i] = vol / 2;
+  P.stretch[i] = 0.f;
 }
 
 // ---- mixing (parcel_mixing.F90:157-389) ----
@@ -1103,7 +855,7 @@ struct Mix32 {
   float *R[6];        // residual vol .. r; after k32_mix_residual, divided by the kept volume
 };
 
-__global__ void k32_mix_new(Geometry g, Bulk32 b, int64_t cap, int64_t norig,
+__global__ void k32_mix_new(Geometry g, Parcels32 P, int64_t cap, int64_t norig,
                             const int32_t *__restrict__ newcells, int64_t nadd,
                             const int32_t *__restrict__ zlist, int64_t nz_,
                             uint8_t *__restrict__ keep, Mix32 mg, float vmin,
@@ -1134,25 +886,19 @@ __global__ void k32_mix_new(Geometry g, Bulk32 b, int64_t cap, int64_t norig,
     s6[f] = a;
   }
   const float v = s6[0];
-  float *F = b.f;
-  b.cell[s] = pack_cell(i, j, k);
-  F[B_OX * cap + s] = 0.5f;  // the cell centre
-  F[B_OY * cap + s] = 0.5f;
-  F[B_OZ * cap + s] = 0.5f;
-  F[B_VOL * cap + s] = 2 * vmin;
-  F[B_STRETCH * cap + s] = 0.f;
-  F[B_B * cap + s] = s6[1] / v;
-  F[B_H * cap + s] = s6[2] / v;
-  F[B_P * cap + s] = s6[3] / v;
-  F[B_Q * cap + s] = s6[4] / v;
-  F[B_R * cap + s] = s6[5] / v;
+  P.cell[s] = pack_cell(i, j, k);
+  st3(P.off, s, 0.5f, 0.5f, 0.5f);  // the cell centre
+  st3(P.vor, s, s6[3] / v, s6[4] / v, s6[5] / v);
+  st3(P.vbh, s, 2 * vmin, s6[1] / v, s6[2] / v);
+  P.stretch[s] = 0.f;
   if (s + 1 < norig) keep[s] = 2;
   portion_cell[((int64_t)k * g.ny + j) * g.nx + i] = 2 * vmin / v;
 }
 
 __global__ void k32_mix_residual(Geometry g, Mix32 mg, const int32_t *__restrict__ npercell,
                                  const float *__restrict__ portion_cell,
-                                 uint8_t *__restrict__ touch, uint8_t *__restrict__ dirty) {
+                                 uint8_t *__restrict__ touch, uint8_t *__restrict__ dirty,
+                                 DevScalars *sc) {
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nnode) return;
@@ -1190,51 +936,33 @@ __global__ void k32_mix_residual(Geometry g, Mix32 mg, const int32_t *__restrict
   touch[t] = any ? 1 : 0;
   if (any && dirty) {
     // the parcels of the eight cells around the node absorb: their tiles are summed again
-    const int ntx = g.nx / TILE32;
     for (int kc = k - 1; kc <= k; kc++) {
       if (kc < 0 || kc >= g.ncz) continue;
       for (int bb = 0; bb < 2; bb++)
-        for (int a = 0; a < 2; a++)
-          dirty[((int64_t)kc * g.ny + cj[bb]) * ntx + ci[a] / TILE32] = 1;
+        for (int a = 0; a < 2; a++) dirty[tile_of(g, ci[a], cj[bb], kc)] = 1;
     }
+    sc->anydirty = 1;
   }
 }
 
-// dirty tiles (x-row grids): the tile of each listed parcel's cell (parcels != 0) or of each
+// dirty tiles: the tile of each listed parcel's cell (parcels != 0) or of each
 // listed new cell, given in the new-cell flags' order (z fastest, then y, then x)
 __global__ void k32_mark_tiles(Geometry g, const int32_t *__restrict__ cellv,
                                const int32_t *__restrict__ list, int64_t n, int parcels,
-                               uint8_t *__restrict__ dirty) {
+                               uint8_t *__restrict__ dirty, DevScalars *sc) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int32_t e = list[t];
-  int64_t lc;
+  int i, j, k;
   if (parcels) {
-    lc = linear_cell(g, cellv[e]);
+    cell_ijk(g, cellv[e], i, j, k);
   } else {
-    const int k = (int)(e % g.ncz);
-    const int j = (int)((e / g.ncz) % g.ny);
-    const int i = (int)(e / ((int64_t)g.ncz * g.ny));
-    lc = ((int64_t)k * g.ny + j) * g.nx + i;
+    k = (int)(e % g.ncz);
+    j = (int)((e / g.ncz) % g.ny);
+    i = (int)(e / ((int64_t)g.ncz * g.ny));
   }
-  dirty[lc / TILE32] = 1;
-}
-
-// *any = 1 if a byte of a[0, n) is set (a is read a 32-bit word at a time; n a multiple of 4
-// or the tail read as bytes)
-__global__ void k32_any_u8(const uint8_t *__restrict__ a, int64_t n, int64_t *any) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool set = false;
-  if (4 * t + 3 < n) {
-    set = *reinterpret_cast<const uint32_t *>(a + 4 * t) != 0u;
-  } else {
-    for (int64_t e = 4 * t; e < n; e++) set = set || a[e] != 0;
-  }
-  if (__ballot(set) != 0ull && (threadIdx.x & 63) == 0) *any = 1;
-}
-
-__global__ void k32_zero_i64(int64_t *a) {
-  if (threadIdx.x == 0) *a = 0;
+  dirty[tile_of(g, i, j, k)] = 1;
+  if (t == 0) sc->anydirty = 1;
 }
 
 __global__ void k32_fill_u8(uint8_t *__restrict__ a, int64_t n, uint8_t v) {
@@ -1246,13 +974,13 @@ __global__ void k32_fill_u8(uint8_t *__restrict__ a, int64_t n, uint8_t v) {
 // only around removed parcels and the cells that received new ones) keeps its values as they
 // are, without the reads, the arithmetic (which would return them to within rounding) and the
 // writes; `touch` marks the nodes with a residual.
-__global__ void k32_mix_absorb(Geometry g, Bulk32 b, int64_t cap, int64_t norig,
+__global__ void k32_mix_absorb(Geometry g, Parcels32 P, int64_t norig,
                                const uint8_t *__restrict__ keep, Mix32 mg,
                                const uint8_t *__restrict__ touch) {
   const int64_t p64 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p64 >= norig || keep[p64] != 1) return;
   const uint32_t p = (uint32_t)p64;
-  const int32_t cell = ldnt(b.cell, p);
+  const int32_t cell = ldnt((const int32_t *)P.cell, p);
   int i, j, k;
   cell_ijk(g, cell, i, j, k);
   int32_t o[8];
@@ -1261,14 +989,9 @@ __global__ void k32_mix_absorb(Geometry g, Bulk32 b, int64_t cap, int64_t norig,
 #pragma unroll
   for (int c = 0; c < 8; c++) any |= touch[o[c]];
   if (!any) return;
-  float *F = b.f;
-  auto fp = [&](int f) { return F + (size_t)f * cap; };
-  const int fld[5] = {B_B, B_H, B_P, B_Q, B_R};
-  const float ox = ldnt(fp(B_OX), p), oy = ldnt(fp(B_OY), p), oz = ldnt(fp(B_OZ), p);
-  const float v = ldnt(fp(B_VOL), p);
-  float fv[5];
-#pragma unroll
-  for (int f = 0; f < 5; f++) fv[f] = ldnt(fp(fld[f]), p);
+  const Float3 off = ld3(P.off, p), vor = ld3(P.vor, p), vbh = ld3(P.vbh, p);
+  const float ox = off.x, oy = off.y, oz = off.z, v = vbh.x;
+  const float fv[5] = {vbh.y, vbh.z, vor.x, vor.y, vor.z};
   float w[8];
   w[0] = (1 - oz) * (1 - oy) * (1 - ox) * v;
   w[1] = (1 - oz) * (1 - oy) * (ox) * v;
@@ -1291,28 +1014,35 @@ __global__ void k32_mix_absorb(Geometry g, Bulk32 b, int64_t cap, int64_t norig,
     for (int c = 0; c < 8; c++) acc = acc + w[c] * ld((const float *)mg.R[f + 1], (uint32_t)o[c]);
     out[f] = acc * ivn;
   }
-  stnt(fp(B_VOL), p, vn);
-#pragma unroll
-  for (int f = 0; f < 5; f++) stnt(fp(fld[f]), p, out[f]);
+  st3(P.vbh, p, vn, out[0], out[1]);
+  st3(P.vor, p, out[2], out[3], out[4]);
 }
 
 // backfill: the state fields of the j-th kept slot from the end into the j-th removed slot
 // (the reference copies x, y, z, p, q, r, b, h, vol, tag and stretch)
-__global__ void k32_mix_backfill(Geometry g, Bulk32 b, int64_t cap,
-                                 const int32_t *__restrict__ dst, int64_t R,
-                                 const int32_t *__restrict__ k1, int64_t K1,
-                                 uint8_t *__restrict__ dirty) {
+__global__ void k32_mix_backfill(Geometry g, Parcels32 P, const int32_t *__restrict__ dst,
+                                 int64_t R, const int32_t *__restrict__ k1, int64_t K1,
+                                 uint8_t *__restrict__ dirty, DevScalars *sc) {
   const int64_t jx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (jx >= R) return;
   const int64_t s = k1[K1 - 1 - jx], d = dst[jx];
+  const int32_t cell = P.cell[s];
   // a moved parcel changes the parcel order of its cell's sums
-  if (dirty) dirty[linear_cell(g, b.cell[s]) / TILE32] = 1;
-  float *F = b.f;
-  const int fl[10] = {B_OX, B_OY, B_OZ, B_P, B_Q, B_R, B_B, B_H, B_VOL, B_STRETCH};
+  if (dirty) {
+    int i, j, k;
+    cell_ijk(g, cell, i, j, k);
+    dirty[tile_of(g, i, j, k)] = 1;
+    if (jx == 0) sc->anydirty = 1;
+  }
+  P.cell[d] = cell;
 #pragma unroll
-  for (int c = 0; c < 10; c++) F[(int64_t)fl[c] * cap + d] = F[(int64_t)fl[c] * cap + s];
-  b.cell[d] = b.cell[s];
-  b.tag[d] = b.tag[s];
+  for (int e = 0; e < 3; e++) {
+    P.off[3 * d + e] = P.off[3 * s + e];
+    P.vor[3 * d + e] = P.vor[3 * s + e];
+    P.vbh[3 * d + e] = P.vbh[3 * s + e];
+  }
+  P.stretch[d] = P.stretch[s];
+  P.tag[d] = P.tag[s];
 }
 
 Zmap zmap_of(const Geometry &g) { return Zmap{(float)g.zbot, (float)g.dz}; }
@@ -1328,11 +1058,20 @@ int dalloc32(T **p, int64_t n) {
   return PMPIC_OK;
 }
 
+// the counts, the cursor behind them and the overflow list's length at zero (the accumulation that
+// uses a binning leaves them so)
+int zero_counts(Ctx *c) {
+  if (c->b32.counts_zero) return PMPIC_OK;
+  hipLaunchKernelGGL(k32_bin_reset, dim3(cdiv(c->ncell + 1, TPB)), dim3(TPB), 0, c->stream,
+                     c->cell_count, c->ncell + 1, c->dsc);
+  PMPIC_CHECK(hipGetLastError());
+  c->b32.counts_zero = true;
+  return PMPIC_OK;
+}
+
 int bin32(Ctx *c, int64_t n) {
-  const int64_t nc1 = c->ncell + 1;
   Bulk32 &b = c->b32;
-  // the capacity of this binning: 16 entries while the mean is at most LOW_PPC parcels per
-  // cell (fewer empty entries to read), else 32
+  const int32_t *cells = b.cell[b.cur];
   const int capc = b32_choose_capc(c, n);
   // the launches of a captured graph cover a parcel bound (the kernels read the count)
   const int64_t ln = c->graph_n ? c->graph_n : n;
@@ -1342,39 +1081,50 @@ int bin32(Ctx *c, int64_t n) {
   } else {
     b.prebinned = false;
     b.capc = capc;
-    hipLaunchKernelGGL(k32_bin_reset, dim3(cdiv(nc1, TPB)), dim3(TPB), 0, c->stream,
-                       c->cell_count, nc1, c->dsc);
+    PMPIC_TRY(zero_counts(c));
+    b.counts_zero = false;
     if (ln > 0)
       hipLaunchKernelGGL(k32_bin_slot, dim3(cdiv(ln, (int64_t)TPB * BIN_SEQ)), dim3(TPB), 0,
-                         c->stream, c->g, b.cell, ln, b.capc, b.slot, b.ovf, c->rank,
+                         c->stream, c->g, cells, ln, b.capc, b.slot, b.ovf, c->rank,
                          c->cell_count, c->dsc);
   }
-  // dense-region offsets of the cells past the slot capacity
-  auto it = rocprim::make_transform_iterator(static_cast<const int32_t *>(c->cell_count),
-                                             OvfCount{b.capc});
-  size_t need = 0;
-  PMPIC_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, need, it, c->cell_start, (int)nc1,
-                                               c->stream));
-  if (need > c->scan_tmp_bytes) {
-    if (c->scan_tmp) PMPIC_CHECK(hipFree(c->scan_tmp));
-    c->scan_tmp = nullptr;
-    PMPIC_CHECK(hipMalloc(&c->scan_tmp, need));
-    c->scan_tmp_bytes = need;
-  }
-  size_t have = c->scan_tmp_bytes;
-  PMPIC_CHECK(hipcub::DeviceScan::ExclusiveSum(c->scan_tmp, have, it, c->cell_start, (int)nc1,
-                                               c->stream));
+  // the dense region's buckets, of the cells past the slot capacity
+  bin_alloc(c, c->cell_count, b.capc, c->cell_start, c->cell_count + c->ncell);
   if (ln > 0 && b.capc == 0) {
     hipLaunchKernelGGL(k32_dense_scatter, dim3(cdiv(ln, TPB)), dim3(TPB), 0, c->stream, c->g,
-                       b.cell, c->rank, c->dsc, c->cell_start, c->sorted);
+                       cells, c->rank, c->dsc, c->cell_start, c->sorted);
   } else if (ln > 0) {
     const int64_t nb = std::min<int64_t>(cdiv(ln, TPB), 1024);
-    hipLaunchKernelGGL(k32_ovf_scatter, dim3(nb), dim3(TPB), 0, c->stream, c->g, b.cell, b.ovf,
+    hipLaunchKernelGGL(k32_ovf_scatter, dim3(nb), dim3(TPB), 0, c->stream, c->g, cells, b.ovf,
                        c->dsc, c->cell_start, b.slot, b.capc, c->sorted);
   }
-  hipLaunchKernelGGL(k32_sort_big, dim3(cdiv(c->ncell, TPB)), dim3(TPB), 0, c->stream,
-                     c->cell_start, c->ncell, rows_of(b.capc), c->sorted);
   PMPIC_CHECK(hipGetLastError());
+  return PMPIC_OK;
+}
+
+Parcels32 parcels32(const Bulk32 &b) {
+  return Parcels32{b.cell[b.cur], b.off[b.cur], b.vor[b.cur], b.vbh, b.dx, b.dp, b.stretch, b.tag};
+}
+
+// one accumulation of the current binning; zero: the counts are left at zero
+template <int MODE>
+int accumulate(Ctx *c, float *partial, float *partial2, uint8_t *dirty, bool zero = true,
+               bool timed = false) {
+  Bulk32 &b = c->b32;
+  const dim3 grid(tiles_x(c->g) * c->g.ny * c->g.ncz), blk(64);
+  auto k = k32_cell_accum<MODE>;
+  if (timed)
+    PMPIC_TRY(launch_timed(c, T_ACCUM, k, grid, blk, 0, c->g, parcels32(b), zmap_of(c->g),
+                           (float)c->g.vmin, b.capc, b.slot, c->cell_count, c->cell_start,
+                           c->sorted, c->rank, partial, partial2, c->npercell, c->cellflag, dirty,
+                           c->cell_count + c->ncell, c->dsc, zero ? 1 : 0));
+  else
+    hipLaunchKernelGGL(k, grid, blk, 0, c->stream, c->g, parcels32(b), zmap_of(c->g),
+                       (float)c->g.vmin, b.capc, b.slot, c->cell_count, c->cell_start, c->sorted,
+                       c->rank, partial, partial2, c->npercell, c->cellflag, dirty,
+                       c->cell_count + c->ncell, c->dsc, zero ? 1 : 0);
+  PMPIC_CHECK(hipGetLastError());
+  b.counts_zero = zero;
   return PMPIC_OK;
 }
 
@@ -1390,8 +1140,10 @@ __global__ void k32_set_n(DevScalars *sc, int64_t n) {
 }
 
 int b32_publish_n(Ctx *c) {
+  if (c->hsc.n == c->n) return PMPIC_OK;
   hipLaunchKernelGGL(k32_set_n, dim3(1), dim3(64), 0, c->stream, c->dsc, c->n);
   PMPIC_CHECK(hipGetLastError());
+  c->hsc.n = c->n;
   return PMPIC_OK;
 }
 
@@ -1416,20 +1168,36 @@ int b32_choose_capc(const Ctx *c, int64_t n) {
 int b32_alloc(Ctx *c) {
   Bulk32 &b = c->b32;
   for (int f = 0; f < 6; f++) b.kept_pending[f] = false;
-  PMPIC_TRY(dalloc32(&b.f, (int64_t)NF32 * c->cap));
-  for (int k = 0; k < NF32; k++) b.fp[k] = b.f + (int64_t)k * c->cap;
-  PMPIC_TRY(dalloc32(&b.cell, c->cap));
-  PMPIC_TRY(dalloc32(&b.cello, c->cap));
+  PMPIC_TRY(dalloc32(&b.pool, (int64_t)PARCEL32_WORDS * c->cap));
+  float *at = b.pool;
+  auto take = [&](int words) {
+    float *p = at;
+    at += (int64_t)words * c->cap;
+    return p;
+  };
+  for (int i = 0; i < 2; i++) {
+    b.cell[i] = reinterpret_cast<int32_t *>(take(1));
+    b.off[i] = take(3);
+    b.vor[i] = take(3);
+  }
+  b.vbh = take(3);
+  b.dx = take(3);
+  b.dp = take(3);
+  b.stretch = take(1);
+  b.df = take(3);
+  b.pf = take(3);
+  b.cur = 0;
   PMPIC_TRY(dalloc32(&b.tag, c->cap));
   // a parcel created by mixing takes neither a tag nor tendencies (parcel_mixing.F90 copies
   // tags only when it backfills, :377, and never writes dxdt..drdt): a slot past every earlier
   // count reads 0 for them, as in the FP64 form's arrays, which are cleared at allocation too
-  PMPIC_CHECK(hipMemset(b.f, 0, sizeof(float) * (size_t)NF32 * (size_t)c->cap));
+  PMPIC_CHECK(hipMemset(b.pool, 0, sizeof(float) * PARCEL32_WORDS * (size_t)c->cap));
   PMPIC_CHECK(hipMemset(b.tag, 0, sizeof(double) * (size_t)c->cap));
   for (int i = 0; i < 3; i++) PMPIC_TRY(dalloc32(&b.grid[i], c->gsz));
   for (int i = 0; i < 12; i++) PMPIC_TRY(dalloc32(&b.mgrid[i], c->gsz));
   PMPIC_TRY(dalloc32(&b.mtouch, c->gsz));
-  PMPIC_TRY(dalloc32(&b.dirty, c->ncell / TILE32 + 1));
+  PMPIC_TRY(dalloc32(&b.dirty, (int64_t)tiles_x(c->g) * c->g.ny * c->g.ncz));
+  b.counts_zero = false;
   b.p2g_reuse = false;
   b.dirty_seq = 0;
   const char *renv = getenv("PMPIC_P2G_REUSE");
@@ -1473,9 +1241,7 @@ int b32_alloc(Ctx *c) {
 
 void b32_free(Ctx *c) {
   Bulk32 &b = c->b32;
-  hipFree(b.f);
-  hipFree(b.cell);
-  hipFree(b.cello);
+  hipFree(b.pool);
   hipFree(b.tag);
   for (int i = 0; i < 3; i++) hipFree(b.grid[i]);
   for (int i = 0; i < 12; i++) hipFree(b.mgrid[i]);
@@ -1484,6 +1250,21 @@ void b32_free(Ctx *c) {
   for (int i = 0; i < 4; i++) hipFree(b.pgrid[i]);
   hipFree(b.slot);
   hipFree(b.ovf);
+}
+
+// field f (FP..FSTRETCH) of the parcels
+struct Column {
+  float *p;
+  int stride;
+};
+static Column column(const Bulk32 &b, int f) {
+  if (f >= FP && f <= FR) return {b.vor[b.cur] + (f - FP), 3};
+  if (f >= FDXDT && f <= FDZDT) return {b.dx + (f - FDXDT), 3};
+  if (f >= FDPDT && f <= FDRDT) return {b.dp + (f - FDPDT), 3};
+  if (f == FH) return {b.vbh + 2, 3};
+  if (f == FB) return {b.vbh + 1, 3};
+  if (f == FVOL) return {b.vbh, 3};
+  return {b.stretch, 1};
 }
 
 int b32_set_parcels(Ctx *c, int64_t n, const double *const *fields) {
@@ -1496,16 +1277,16 @@ int b32_set_parcels(Ctx *c, int64_t n, const double *const *fields) {
     if (n > 0) {
       PMPIC_CHECK(hipMemcpyAsync(c->fbuf, fields[a], sizeof(double) * n, hipMemcpyHostToDevice,
                                  c->stream));
-      hipLaunchKernelGGL(k32_pos_in, gb, tb, 0, c->stream, c->g, a, c->fbuf, n, b.cell,
-                         b.f + (int64_t)(B_OX + a) * c->cap, c->dsc);
+      hipLaunchKernelGGL(k32_pos_in, gb, tb, 0, c->stream, c->g, a, c->fbuf, n, b.cell[b.cur],
+                         b.off[b.cur], c->dsc);
     }
   }
   for (int f = FP; f <= FSTRETCH; f++) {
     if (n > 0) {
       PMPIC_CHECK(hipMemcpyAsync(c->fbuf, fields[f], sizeof(double) * n, hipMemcpyHostToDevice,
                                  c->stream));
-      hipLaunchKernelGGL(k32_from_f64, gb, tb, 0, c->stream, c->fbuf, n,
-                         b.f + (int64_t)f * c->cap);
+      const Column col = column(b, f);
+      hipLaunchKernelGGL(k32_from_f64, gb, tb, 0, c->stream, c->fbuf, n, col.p, col.stride);
     }
   }
   if (n > 0)
@@ -1530,10 +1311,12 @@ int b32_get_parcels(Ctx *c, double *const *fields) {
       continue;
     }
     if (f < 3)
-      hipLaunchKernelGGL(k32_pos_out, gb, tb, 0, c->stream, c->g, f, b.cell,
-                         b.f + (int64_t)(B_OX + f) * c->cap, n, c->fbuf);
-    else
-      hipLaunchKernelGGL(k32_to_f64, gb, tb, 0, c->stream, b.f + (int64_t)f * c->cap, n, c->fbuf);
+      hipLaunchKernelGGL(k32_pos_out, gb, tb, 0, c->stream, c->g, f, b.cell[b.cur],
+                         b.off[b.cur], n, c->fbuf);
+    else {
+      const Column col = column(b, f);
+      hipLaunchKernelGGL(k32_to_f64, gb, tb, 0, c->stream, col.p, col.stride, n, c->fbuf);
+    }
     PMPIC_CHECK(hipMemcpyAsync(fields[f], c->fbuf, sizeof(double) * n, hipMemcpyDeviceToHost,
                                c->stream));
   }
@@ -1542,47 +1325,33 @@ int b32_get_parcels(Ctx *c, double *const *fields) {
   return PMPIC_OK;
 }
 
-// the x-combined partials need tiles within one x row
-static bool p2g_xrows(const Ctx *c) { return c->g.nx % TILE32 == 0; }
+// The last mixing's kept sums stand for the next par2grid on x rows of whole 16-cell pieces only:
+// elsewhere every par2grid sums every tile, one full launch a stage, which is what its timer's
+// count has always been there.
+static bool reuse_sums(const Ctx *c) { return c->g.nx % 16 == 0 && !c->b32.reuse_off; }
 
-// A graph of stages 1-3 always captures stage 1's par2grid reading the dirty-tile flags (on
-// x-row grids with the reuse on); where the last mixing's sums are not current, every tile is
-// marked dirty first, so the captured par2grid sums them all.
-void b32_graph_reuse(Ctx *c) {
+// A graph of stages 1-3 always captures stage 1's par2grid reading the dirty-tile flags (with the
+// reuse on) and finding the counts at zero; where the last mixing's sums are not current, every
+// tile is marked dirty first, so the captured par2grid sums them all.
+int b32_graph_reuse(Ctx *c) {
   Bulk32 &b = c->b32;
-  if (!p2g_xrows(c) || b.reuse_off) return;
+  PMPIC_TRY(zero_counts(c));
+  if (!reuse_sums(c)) return PMPIC_OK;
   if (!b.p2g_reuse) {
-    const int64_t nt = c->ncell / TILE32 + 1;
+    const int64_t nt = (int64_t)tiles_x(c->g) * c->g.ny * c->g.ncz;
     hipLaunchKernelGGL(k32_fill_u8, dim3(cdiv(nt, TPB)), dim3(TPB), 0, c->stream, b.dirty, nt,
                        (uint8_t)1);
+    PMPIC_CHECK(hipGetLastError());
   }
   b.p2g_reuse = true;
+  return PMPIC_OK;
 }
 
 // the par2grid accumulation; with `dirty`, only the tiles it marks (the others keep the
 // partials the last mixing summed): that launch is left out of the kernel timer, whose
 // per-launch figures are those of full launches
-static int p2g_accum(Ctx *c, const uint8_t *dirty = nullptr) {
-  const dim3 grid(cdiv(c->ncell, TILE32)), blk(ATPB);
-  const Bulk32 &b = c->b32;
-  if (p2g_xrows(c)) {
-    auto k = b.capc == CAPC_LOW ? k32_cell_accum<A32_P2GX, CAPC_LOW, ROWS_LOW>
-                                : k32_cell_accum<A32_P2GX, CAPC, ROWS32>;
-    if (dirty) {
-      hipLaunchKernelGGL(k, grid, blk, 0, c->stream, b, c->cap, c->g, zmap_of(c->g),
-                         (float)c->g.vmin, c->cell_count, c->cell_start, c->sorted, c->ncell,
-                         partial32(c), nullptr, nullptr, nullptr, dirty);
-      return PMPIC_OK;
-    }
-    return launch_timed(c, T_ACCUM, k, grid, blk, 0, b, c->cap, c->g, zmap_of(c->g),
-                        (float)c->g.vmin, c->cell_count, c->cell_start, c->sorted, c->ncell,
-                        partial32(c), nullptr, nullptr, nullptr, nullptr);
-  }
-  auto k = b.capc == CAPC_LOW ? k32_cell_accum<A32_P2G, CAPC_LOW, ROWS_LOW>
-                              : k32_cell_accum<A32_P2G, CAPC, ROWS32>;
-  return launch_timed(c, T_ACCUM, k, grid, blk, 0, b, c->cap, c->g, zmap_of(c->g),
-                      (float)c->g.vmin, c->cell_count, c->cell_start, c->sorted, c->ncell,
-                      partial32(c), nullptr, nullptr, nullptr, nullptr);
+static int p2g_accum(Ctx *c, uint8_t *dirty = nullptr, bool zero = true) {
+  return accumulate<A32_P2G>(c, partial32(c), nullptr, dirty, zero, dirty == nullptr);
 }
 
 // The capacity tuning: bin at 16 and at 32 slots, time the accumulation of each (its second
@@ -1604,7 +1373,7 @@ static int tune_capacity(Ctx *c, int64_t n) {
   for (int t = 0; t < 2 && rc == PMPIC_OK; t++) {
     b.capfix = caps[t];
     rc = bin32(c, n);
-    if (rc == PMPIC_OK) rc = p2g_accum(c);
+    if (rc == PMPIC_OK) rc = p2g_accum(c, nullptr, false);
     if (rc == PMPIC_OK && hipEventRecord(e0, c->stream) != hipSuccess) rc = PMPIC_ERR_HIP;
     if (rc == PMPIC_OK) rc = p2g_accum(c);
     if (rc == PMPIC_OK && (hipEventRecord(e1, c->stream) != hipSuccess ||
@@ -1631,7 +1400,7 @@ int b32_par2grid(Ctx *c) {
   for (int i = 0; i < 4; i++) b.p2g_pending[i] = true;
   // the last mixing's kept sums, where it left them current, stand for this accumulation
   // except on the tiles it changed
-  const uint8_t *dirty = (b.p2g_reuse && p2g_xrows(c) && !b.captune) ? b.dirty : nullptr;
+  uint8_t *dirty = (b.p2g_reuse && !b.captune) ? b.dirty : nullptr;
   b.p2g_reuse = false;
   // a mixing that changed no tile (known to the host once it has read the device scalars back,
   // and not inside a graph capture): the partials are all current, so no binning or sums
@@ -1642,24 +1411,22 @@ int b32_par2grid(Ctx *c) {
     PMPIC_TRY(bin32(c, n));
     PMPIC_TRY(p2g_accum(c, dirty));
   }
-  Out32<float> out = {{b.pgrid[0], b.pgrid[1], b.pgrid[2], b.pgrid[3], nullptr, nullptr}};
-  const int64_t nnode = (int64_t)c->g.nzn * c->g.ny * c->g.nx;
-  if (p2g_xrows(c))
-    hipLaunchKernelGGL((k32_node_sum_x<5, true, false>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0,
-                       c->stream, c->g, partial32(c), out, nullptr);
-  else
-    hipLaunchKernelGGL((k32_node_sum<4, true, true, float>), dim3(cdiv(nnode, TPB)), dim3(TPB),
-                       0, c->stream, c->g, partial32(c), c->ncell, out, nullptr);
+  launch_node_sum<float, float, 5, true>(
+      c, {partial32(c), {b.pgrid[0], b.pgrid[1], b.pgrid[2], b.pgrid[3]}, nullptr, 1.f});
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
 
 int b32_rk_stage(Ctx *c, int stage, int stretch) {
   const int64_t n = c->n;
-  if (n == 0) return PMPIC_OK;
-  PMPIC_TRY(records_current(c));
-  const Scale32 s3 = scale_of(c->g);
   Bulk32 &b = c->b32;
+  const int from = b.cur, to = stage < 4 ? 1 : 0;
+  const RkSets rs = {b.cell[from], b.cell[0], b.off[from], b.off[0],  b.vor[from],
+                     b.vor[0],     b.cell[to], b.off[to],  b.vor[to]};
+  if (n > 0) PMPIC_TRY(records_current(c));
+  b.cur = to;
+  if (n == 0) return PMPIC_OK;
+  const Scale32 s3 = scale_of(c->g);
   b.p2g_reuse = false;
   const dim3 gb(cdiv(c->graph_n ? c->graph_n : n, b.rk_tpb)), tb(b.rk_tpb);
   // stages 1-3 bin the cells they write for the next stage's par2grid (stage 4 is followed by
@@ -1669,25 +1436,24 @@ int b32_rk_stage(Ctx *c, int stage, int stretch) {
   if (stage < 4 && b.fused_bin && !b.captune) {
     bo.on = 1;
     bo.capc = b32_choose_capc(c, n);
-    const int64_t nc1 = c->ncell + 1;
-    hipLaunchKernelGGL(k32_bin_reset, dim3(cdiv(nc1, TPB)), dim3(TPB), 0, c->stream,
-                       c->cell_count, nc1, c->dsc);
+    PMPIC_TRY(zero_counts(c));
+    b.counts_zero = false;
   }
   switch (stage) {
     case 1:
-      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<1>, gb, tb, 0, c->g, c->b32, c->cap, n,
+      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<1>, gb, tb, 0, c->g, c->b32, rs, n,
                              c->rec32, s3, stretch, c->flag, c->dsc, bo));
       break;
     case 2:
-      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<2>, gb, tb, 0, c->g, c->b32, c->cap, n,
+      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<2>, gb, tb, 0, c->g, c->b32, rs, n,
                              c->rec32, s3, stretch, c->flag, c->dsc, bo));
       break;
     case 3:
-      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<3>, gb, tb, 0, c->g, c->b32, c->cap, n,
+      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<3>, gb, tb, 0, c->g, c->b32, rs, n,
                              c->rec32, s3, stretch, c->flag, c->dsc, bo));
       break;
     default:
-      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<4>, gb, tb, 0, c->g, c->b32, c->cap, n,
+      PMPIC_TRY(launch_timed(c, T_RK, k32_rk_stage<4>, gb, tb, 0, c->g, c->b32, rs, n,
                              c->rec32, s3, stretch, c->flag, c->dsc, bo));
       break;
   }
@@ -1709,7 +1475,7 @@ int b32_split(Ctx *c) {
     if (c->split_flags_fresh)
       PMPIC_TRY(compact_flags(c, c->flag, 1, n, c->list_b, &c->dsc->nsplit));
     else
-      PMPIC_TRY(split_list(c, c->b32.f + (int64_t)B_STRETCH * c->cap, n));
+      PMPIC_TRY(split_list(c, c->b32.stretch, n));
     c->split_flags_fresh = 0;
   } else {
     c->hsc.nsplit = 0;
@@ -1721,7 +1487,7 @@ int b32_split(Ctx *c) {
   if (ns > 0) {
     if (n + ns > c->cap) return PMPIC_ERR_MAXPARCELS;
     hipLaunchKernelGGL(k32_split_apply, dim3(cdiv(ns, TPB)), dim3(TPB), 0, c->stream, c->g,
-                       c->b32, c->cap, n, scale_of(c->g), c->list_b, ns, c->dsc);
+                       parcels32(c->b32), c->cap, n, scale_of(c->g), c->list_b, ns, c->dsc);
     PMPIC_CHECK(hipGetLastError());
   }
   c->n = n + ns;
@@ -1736,64 +1502,32 @@ int b32_mix(Ctx *c) {
   const float vmin = (float)g.vmin;
   // kept and residual grids (construct_grids, parcel_mixing.F90:440-624)
   PMPIC_TRY(bin32(c, norig));
-  const bool xr = p2g_xrows(c);
-  // x-row grids: the kept sums' first five planes (weight, p, q, r, total buoyancy) are what
-  // the next par2grid would sum on every tile this mixing leaves unchanged; the tiles it changes
-  // are marked below (removed, new, absorbing and moved parcels)
+  // the kept sums' first five planes (weight, p, q, r, total buoyancy) are what the next
+  // par2grid would sum on every tile this mixing leaves unchanged; the tiles it changes
+  // are marked below (removed, new, absorbing and moved parcels).  cellflag holds the tiles'
+  // residual flags until the new-parcel flags reuse it.
   b.p2g_reuse = false;
-  const bool reuse = xr && !b.reuse_off;
+  const bool reuse = reuse_sums(c);
   uint8_t *dirty = reuse ? b.dirty : nullptr;
-  if (reuse) {
-    const int64_t nt = c->ncell / TILE32 + 1;
-    hipLaunchKernelGGL(k32_fill_u8, dim3(cdiv(nt, TPB)), dim3(TPB), 0, c->stream, b.dirty, nt,
-                       (uint8_t)0);
-  }
-  if (xr && b.capc == CAPC_LOW)
-    hipLaunchKernelGGL((k32_cell_accum<A32_MIXX, CAPC_LOW, ROWS_LOW>), dim3(cdiv(c->ncell, TILE32)),
-                       dim3(ATPB), 0, c->stream, b, c->cap, g, zmap_of(g), vmin, c->cell_count,
-                       c->cell_start, c->sorted, c->ncell, partial32(c), partial32b(c),
-                       c->npercell, c->cellflag, nullptr);
-  else if (xr)
-    hipLaunchKernelGGL((k32_cell_accum<A32_MIXX, CAPC, ROWS32>), dim3(cdiv(c->ncell, TILE32)),
-                       dim3(ATPB), 0, c->stream, b, c->cap, g, zmap_of(g), vmin, c->cell_count,
-                       c->cell_start, c->sorted, c->ncell, partial32(c), partial32b(c),
-                       c->npercell, c->cellflag, nullptr);
-  else if (b.capc == CAPC_LOW)
-    hipLaunchKernelGGL((k32_cell_accum<A32_MIX, CAPC_LOW, ROWS_LOW>), dim3(cdiv(c->ncell, TILE32)),
-                       dim3(ATPB), 0, c->stream, b, c->cap, g, zmap_of(g), vmin, c->cell_count,
-                       c->cell_start, c->sorted, c->ncell, partial32(c), partial32b(c),
-                       c->npercell, c->cellflag, nullptr);
-  else
-    hipLaunchKernelGGL((k32_cell_accum<A32_MIX, CAPC, ROWS32>), dim3(cdiv(c->ncell, TILE32)),
-                       dim3(ATPB), 0, c->stream, b, c->cap, g, zmap_of(g), vmin, c->cell_count,
-                       c->cell_start, c->sorted, c->ncell, partial32(c), partial32b(c),
-                       c->npercell, c->cellflag, nullptr);
+  PMPIC_TRY(accumulate<A32_MIX>(c, partial32(c), partial32b(c), b.dirty));
+  const Parcels32 P = parcels32(b);
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
-  Out32<float> kept = {{b.mgrid[0], b.mgrid[1], b.mgrid[2], b.mgrid[3], b.mgrid[4], b.mgrid[5]}};
-  Out32<float> res = {{b.mgrid[6], b.mgrid[7], b.mgrid[8], b.mgrid[9], b.mgrid[10], b.mgrid[11]}};
-  // cellflag holds the per-tile residual flags until the new-parcel flags reuse it below
-  if (xr) {
-    // planes weight, p, q, r, total buoyancy (not kept), b, h
-    const Out32<float> keptx = {{b.mgrid[0], b.mgrid[3], b.mgrid[4], b.mgrid[5], nullptr,
-                                 b.mgrid[1], b.mgrid[2]}};
-    const Out32<float> resx = {{b.mgrid[6], b.mgrid[9], b.mgrid[10], b.mgrid[11], nullptr,
-                                b.mgrid[7], b.mgrid[8]}};
-    hipLaunchKernelGGL((k32_node_sum_x<7, false, true>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0,
-                       c->stream, g, partial32(c), keptx, nullptr);
-    hipLaunchKernelGGL((k32_node_sum_x<7, false, false>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0,
-                       c->stream, g, partial32b(c), resx, c->cellflag);
-  } else {
-    hipLaunchKernelGGL((k32_node_sum<5, false, true, float>), dim3(cdiv(nnode, TPB)), dim3(TPB),
-                       0, c->stream, g, partial32(c), c->ncell, kept, nullptr);
-    hipLaunchKernelGGL((k32_node_sum<5, false, false, float>), dim3(cdiv(nnode, TPB)), dim3(TPB),
-                       0, c->stream, g, partial32b(c), c->ncell, res, c->cellflag);
-  }
+  // planes weight, p, q, r, total buoyancy (not kept), b, h
+  const NodeSums<float, float> kept = {
+      partial32(c),
+      {b.mgrid[0], b.mgrid[3], b.mgrid[4], b.mgrid[5], nullptr, b.mgrid[1], b.mgrid[2]},
+      nullptr, 2.f};
+  const NodeSums<float, float> res = {
+      partial32b(c),
+      {b.mgrid[6], b.mgrid[9], b.mgrid[10], b.mgrid[11], nullptr, b.mgrid[7], b.mgrid[8]},
+      c->cellflag, 1.f};
+  launch_node_sum<float, float, 7, false>(c, kept, &res);
   // the reference builds the kept grids in the model's vol, b, hg, p, q, r grids
   // (parcel_mixing.F90:131), which is what a grid export shows after mixing; nothing in the
   // step reads them there, so b32_export_grid widens them when one is exported
   for (int f = 0; f < 6; f++) b.kept_pending[f] = true;
   for (int f = 0; f < 4; f++) b.p2g_pending[f] = false;
-  PMPIC_TRY(mix_lists(c, (const float *)b.f + (int64_t)B_VOL * c->cap, vmin, norig, nullptr));
+  PMPIC_TRY(mix_lists(c, (const float *)b.vbh, 3, vmin, norig, nullptr));
   PMPIC_TRY(sync_scalars(c));
   const int64_t Z = c->hsc.nzero, nadd = c->hsc.nadd;
   Mix32 mg = {{b.mgrid[0], b.mgrid[1], b.mgrid[2], b.mgrid[3], b.mgrid[4], b.mgrid[5]},
@@ -1802,20 +1536,20 @@ int b32_mix(Ctx *c) {
   if (reuse) {
     // the removed parcels' cells (read before new parcels take their slots) and the new cells
     if (Z > 0)
-      hipLaunchKernelGGL(k32_mark_tiles, dim3(cdiv(Z, TPB)), dim3(TPB), 0, c->stream, g, b.cell,
-                         c->list_a, Z, 1, b.dirty);
+      hipLaunchKernelGGL(k32_mark_tiles, dim3(cdiv(Z, TPB)), dim3(TPB), 0, c->stream, g, P.cell,
+                         c->list_a, Z, 1, b.dirty, c->dsc);
     if (nadd > 0)
       hipLaunchKernelGGL(k32_mark_tiles, dim3(cdiv(nadd, TPB)), dim3(TPB), 0, c->stream, g,
-                         b.cell, c->sorted, nadd, 0, b.dirty);
+                         P.cell, c->sorted, nadd, 0, b.dirty, c->dsc);
   }
   if (nadd > 0)
-    hipLaunchKernelGGL(k32_mix_new, dim3(cdiv(nadd, TPB)), dim3(TPB), 0, c->stream, g, b, c->cap,
+    hipLaunchKernelGGL(k32_mix_new, dim3(cdiv(nadd, TPB)), dim3(TPB), 0, c->stream, g, P, c->cap,
                        norig, c->sorted, nadd, c->list_a, Z, c->flag, mg, vmin, portion, c->dsc);
   hipLaunchKernelGGL(k32_mix_residual, dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, g, mg,
-                     c->npercell, portion, b.mtouch, dirty);
+                     c->npercell, portion, b.mtouch, dirty, c->dsc);
   if (norig > 0)
-    hipLaunchKernelGGL(k32_mix_absorb, dim3(cdiv(norig, TPB)), dim3(TPB), 0, c->stream, g, b,
-                       c->cap, norig, c->flag, mg, b.mtouch);
+    hipLaunchKernelGGL(k32_mix_absorb, dim3(cdiv(norig, TPB)), dim3(TPB), 0, c->stream, g, P,
+                       norig, c->flag, mg, b.mtouch);
   PMPIC_CHECK(hipGetLastError());
   // new count (parcel_mixing.F90:217), then the backfill of removed slots (:347-389)
   int64_t np = norig;
@@ -1853,23 +1587,18 @@ int b32_mix(Ctx *c) {
       PMPIC_TRY(sync_scalars(c));
       const int64_t K1 = c->hsc.nkeep1;
       if (R > K1) return PMPIC_ERR_BACKFILL;
-      hipLaunchKernelGGL(k32_mix_backfill, dim3(cdiv(R, TPB)), dim3(TPB), 0, c->stream, g, b,
-                         c->cap, dst, R, c->list_b, K1, dirty);
+      hipLaunchKernelGGL(k32_mix_backfill, dim3(cdiv(R, TPB)), dim3(TPB), 0, c->stream, g, P,
+                         dst, R, c->list_b, K1, dirty, c->dsc);
       PMPIC_CHECK(hipGetLastError());
       np -= R;
     }
   }
   c->n = np;
   b.p2g_reuse = reuse;
-  if (reuse) {
-    // whether any tile changed; the host learns it with the next read-back of the device
-    // scalars (the status check that ends the component or the step)
-    const int64_t nt = c->ncell / TILE32;
-    hipLaunchKernelGGL(k32_zero_i64, dim3(1), dim3(64), 0, c->stream, &c->dsc->anydirty);
-    hipLaunchKernelGGL(k32_any_u8, dim3(cdiv(cdiv(nt, 4), TPB)), dim3(TPB), 0, c->stream, b.dirty,
-                       nt, &c->dsc->anydirty);
-    b.dirty_seq = c->sync_seq;
-  }
+  // whether any tile changed (anydirty) the host learns with the next read-back of the device
+  // scalars (the status check that ends the component or the step)
+  b.dirty_seq = c->sync_seq;
+  b.p2g_reuse = reuse;
   return b32_publish_n(c);
 }
 
@@ -1877,23 +1606,12 @@ int b32_mix(Ctx *c) {
 // parcels' b, h, p, q, r, FP32 sums normalised into the FP64 grids
 int b32_dump_grids(Ctx *c) {
   Bulk32 &b = c->b32;
-  const Geometry &g = c->g;
   b.p2g_reuse = false;  // the dump's sums overwrite the partials
   PMPIC_TRY(bin32(c, c->n));
-  if (b.capc == CAPC_LOW)
-    hipLaunchKernelGGL((k32_cell_accum<A32_DUMP, CAPC_LOW, ROWS_LOW>), dim3(cdiv(c->ncell, TILE32)),
-                       dim3(ATPB), 0, c->stream, b, c->cap, g, zmap_of(g), (float)g.vmin,
-                       c->cell_count, c->cell_start, c->sorted, c->ncell, partial32(c), nullptr,
-                       nullptr, nullptr, nullptr);
-  else
-    hipLaunchKernelGGL((k32_cell_accum<A32_DUMP, CAPC, ROWS32>), dim3(cdiv(c->ncell, TILE32)),
-                       dim3(ATPB), 0, c->stream, b, c->cap, g, zmap_of(g), (float)g.vmin,
-                       c->cell_count, c->cell_start, c->sorted, c->ncell, partial32(c), nullptr,
-                       nullptr, nullptr, nullptr);
-  Out32<double> out = {{c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR], nullptr}};
-  const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
-  hipLaunchKernelGGL((k32_node_sum<5, true, true, double>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0,
-                     c->stream, g, partial32(c), c->ncell, out, nullptr);
+  PMPIC_TRY(accumulate<A32_DUMP>(c, partial32(c), nullptr, nullptr));
+  launch_node_sum<float, double, 6, true>(
+      c, {partial32(c), {c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR]}, nullptr,
+          1.f});
   PMPIC_CHECK(hipGetLastError());
   // these grids now hold writebinary's values, not the kept grids of the last mixing or the
   // step's FP32 grids
@@ -1928,18 +1646,19 @@ int b32_export_grid(Ctx *c, int id) {
 
 int b32_conservation_sums(Ctx *c, double out6[6]) {
   const int64_t n = c->n;
-  std::vector<float> v(n), f(n);
-  if (n > 0)
-    PMPIC_CHECK(hipMemcpy(v.data(), c->b32.f + (int64_t)B_VOL * c->cap, sizeof(float) * n,
+  // vol, b, h and p, q, r of each parcel
+  std::vector<float> vbh(3 * n), vor(3 * n);
+  if (n > 0) {
+    PMPIC_CHECK(hipMemcpy(vbh.data(), c->b32.vbh, sizeof(float) * 3 * n, hipMemcpyDeviceToHost));
+    PMPIC_CHECK(hipMemcpy(vor.data(), c->b32.vor[c->b32.cur], sizeof(float) * 3 * n,
                           hipMemcpyDeviceToHost));
-  const int fl[6] = {-1, B_B, B_H, B_P, B_Q, B_R};
+  }
+  const float *v = vbh.data(), *fl[6] = {nullptr, v + 1, v + 2, vor.data(), vor.data() + 1,
+                                         vor.data() + 2};
   for (int k = 0; k < 6; k++) {
-    if (fl[k] >= 0 && n > 0)
-      PMPIC_CHECK(hipMemcpy(f.data(), c->b32.f + (int64_t)fl[k] * c->cap, sizeof(float) * n,
-                            hipMemcpyDeviceToHost));
     double s = 0.0, comp = 0.0;  // Neumaier summation in parcel order, FP64
     for (int64_t p = 0; p < n; p++) {
-      const double term = fl[k] < 0 ? (double)v[p] : (double)v[p] * (double)f[p];
+      const double term = !fl[k] ? (double)v[3 * p] : (double)v[3 * p] * (double)fl[k][3 * p];
       const double t = s + term;
       if (fabs(s) >= fabs(term)) comp += (s - t) + term;
       else comp += (term - t) + s;

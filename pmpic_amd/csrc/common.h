@@ -29,22 +29,33 @@ enum Field {
   FSTRETCH, FTAG, FXO, FYO, FZO, FXF, FYF, FZF, FPO, FQO, FRO, FPF, FQF, FRF, NFIELDS
 };
 
-// FP32-bulk form: per-parcel FP32 fields (the position is an int32 cell index plus the three
-// offsets B_OX..B_OZ in [0,1) inside that cell; B_OXO..B_OZO and the cell_o array hold the RK4
-// origin, B_DFX..B_DFZ the accumulated RK4 increment in cells relative to it).  Fields 3..15
-// share their numbers with Field.
-enum Field32 {
-  B_OX = 0, B_OY, B_OZ, B_P, B_Q, B_R, B_DXDT, B_DYDT, B_DZDT, B_DPDT, B_DQDT, B_DRDT, B_H, B_B,
-  B_VOL, B_STRETCH, B_OXO, B_OYO, B_OZO, B_DFX, B_DFY, B_DFZ, B_PO, B_QO, B_RO, B_PF, B_QF, B_RF,
-  NF32
+// FP32-bulk form: the position is an int32 cell index plus three FP32 offsets in [0, 1) inside
+// that cell.  Values that the kernels use together lie side by side, three floats a parcel, so
+// that a parcel out of cell order costs three lines in the par2grid gather instead of nine and a
+// kernel a third of the loads.
+//
+// Positions and vorticity are kept twice.  RK stage 1 reads set 0 and writes set 1, stages 2 and 3
+// update set 1, stage 4 reads it and writes set 0: set 0 is the RK4 origin meanwhile, without
+// being copied.  `cur` is the set that holds the parcels.
+struct Parcels32 {
+  int32_t *cell;  // cell holding the parcel
+  float *off;     // 3 a parcel: offsets in it
+  float *vor;     // 3: p, q, r
+  float *vbh;     // 3: vol, b, h
+  float *dx, *dp;  // 3 each: dxdt, dydt, dzdt; dpdt, dqdt, drdt
+  float *stretch;
+  double *tag;
 };
+constexpr int PARCEL32_WORDS = 2 * 7 + 3 + 6 + 1 + 6;  // 32-bit words a parcel besides the tag
 
 struct Bulk32 {
-  float *f;          // NF32 * cap
-  float *fp[NF32];   // fp[k] = f + k * cap: field k (kernels take these from their arguments
-                     // instead of forming them)
-  int32_t *cell;     // cap: cell holding the parcel
-  int32_t *cello;    // cap: cell of the RK4 origin
+  float *pool;        // PARCEL32_WORDS * cap: everything below but the tag
+  int32_t *cell[2];   // the two sets
+  float *off[2], *vor[2];
+  float *vbh, *dx, *dp, *stretch;
+  float *df, *pf;     // 3 a parcel: the RK4 sums of position (in cells, relative to the origin)
+                      // and vorticity
+  int cur;
   double *tag;       // cap
   float *grid[3];    // U, V, W [nzn][ny][nx]
   float *mgrid[12];  // mixing: kept vol, b, h, p, q, r (0..5), residuals (6..11)
@@ -74,8 +85,9 @@ struct Bulk32 {
   // cells are built
   bool fused_bin;
   bool prebinned;
-  // x-row grids: the last mixing's kept sums are the next par2grid's partials except on the
-  // tiles mixing changed (dirty: one byte per 16-cell tile); p2g_reuse while that holds (set by
+  bool counts_zero;   // the cell counts are zero, as a binning wants them
+  // the last mixing's kept sums are the next par2grid's partials except on the
+  // tiles mixing changed (dirty: one byte per 8-cell tile); p2g_reuse while that holds (set by
   // mixing, cleared by the par2grid that uses it and by anything else that changes the
   // parcels or the partials); reuse_off: PMPIC_P2G_REUSE=0
   uint8_t *dirty;
@@ -354,6 +366,8 @@ int par2grid_single_ws(Ctx *c, int64_t n, const double *d_var, double *d_grid, c
 int par2grid_fused(Ctx *c, int64_t n);  // P,Q,R,B grids from p,q,r,btot
 int par2grid_single(Ctx *c, int64_t n, const double *d_var, double *d_grid);
 int grid2par_single(Ctx *c, int64_t n, const double *d_grid, double *d_var);
+// buckets of the cells of more than `held` parcels, from *cursor on
+void bin_alloc(Ctx *c, const int32_t *count, int held, int32_t *start, int32_t *cursor);
 int mixing_grids(Ctx *c, int64_t n);
 int dump_grids_f64(Ctx *c, int64_t n);  // writebinary's b, hg, p, q, r grids
 int hgliq_grid(Ctx *c);                 // hgliq and b += 12.5 hgliq (writebinary.F90:224-233)
@@ -430,10 +444,10 @@ int compact_flags(Ctx *c, const uint8_t *flags, uint8_t want, int64_t n, int32_t
 // the parcels to split (list_b, DevScalars::nsplit), from their stretch; n > 0
 template <typename T>
 int split_list(Ctx *c, const T *stretch, int64_t n);
-// mixing's parcels below vmin (flag, list_a, nzero) and cells short of parcels (cellflag, sorted,
+// mixing's parcels whose volume vol[stride i] is below vmin (flag, list_a, nzero) and cells short of parcels (cellflag, sorted,
 // nadd); clears ctouch (may be null)
 template <typename T>
-int mix_lists(Ctx *c, const T *vol, T vmin, int64_t n, uint8_t *ctouch);
+int mix_lists(Ctx *c, const T *vol, int stride, T vmin, int64_t n, uint8_t *ctouch);
 // bulk32.hip (FP32-bulk form)
 int b32_alloc(Ctx *c);
 void b32_free(Ctx *c);
@@ -446,7 +460,7 @@ int b32_mix(Ctx *c);
 int b32_conservation_sums(Ctx *c, double out6[6]);
 int b32_choose_capc(const Ctx *c, int64_t n);  // the slot capacity a binning of n parcels takes
 int b32_mean_capc(const Ctx *c, int64_t n);    // ... by the mean-occupancy rule alone
-void b32_graph_reuse(Ctx *c);  // stage 1's par2grid reading the dirty-tile flags, all set if stale
+int b32_graph_reuse(Ctx *c);  // stage 1's par2grid reading the dirty-tile flags, all set if stale
 int b32_publish_n(Ctx *c);                     // the parcel count into device memory
 int b32_export_grid(Ctx *c, int id);  // brings grid[id] up to date for a grid export
 int b32_dump_grids(Ctx *c);             // writebinary's b, hg, p, q, r grids

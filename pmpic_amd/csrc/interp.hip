@@ -16,7 +16,7 @@
 //   3. node:  one thread per node adds the matching corner sums of its adjacent cells (periodic
 //             in x, y) in a fixed order and normalises by the summed weights.
 // The result differs from the reference's sequential sum only by the order of additions.
-#include "common.h"
+#include "node_sum.h"
 
 #include <hipcub/hipcub.hpp>
 
@@ -87,10 +87,11 @@ __global__ void k_bin_count(Geometry g, const double *__restrict__ X, const doub
 
 // room for every bucket: start[c] from a running total.  The buckets' order does not matter to the
 // sums, so each block takes its cells' total from the cursor with one atomic, and no scan of the
-// whole array (two more launches) is needed.
+// whole array (two more launches) is needed.  A cell of up to `held` parcels takes none (its
+// parcels are listed elsewhere).
 constexpr int ALLOC_CELLS = 4;  // cells per thread
 __global__ void __launch_bounds__(TPB) k_bin_alloc(const int32_t *__restrict__ count, int64_t ncell,
-                                                   int32_t *__restrict__ start,
+                                                   int held, int32_t *__restrict__ start,
                                                    int32_t *__restrict__ cursor) {
   __shared__ int32_t wave_sum[TPB / 64];
   __shared__ int32_t base;
@@ -100,6 +101,7 @@ __global__ void __launch_bounds__(TPB) k_bin_alloc(const int32_t *__restrict__ c
 #pragma unroll
   for (int i = 0; i < ALLOC_CELLS; i++) {
     k[i] = c0 + i < ncell ? count[c0 + i] : 0;
+    if (k[i] <= held) k[i] = 0;
     sum += k[i];
   }
   int32_t incl = sum;
@@ -123,7 +125,7 @@ __global__ void __launch_bounds__(TPB) k_bin_alloc(const int32_t *__restrict__ c
   int32_t o = base + wave_sum[wave] + incl - sum;
 #pragma unroll
   for (int i = 0; i < ALLOC_CELLS; i++) {
-    if (c0 + i < ncell) start[c0 + i] = o;
+    if (c0 + i < ncell && k[i]) start[c0 + i] = o;
     o += k[i];
   }
 }
@@ -373,66 +375,6 @@ __global__ void __launch_bounds__(64) k_cell_accum(Geometry g, const double *__r
   }
 }
 
-// node sums of the x-combined corner sums: NORM = divide by summed weights (par2grid,
-// parcel_interpolation.F90:463-469); otherwise raw sums with the mixing z-boundary doubling
-// (parcel_mixing.F90:141-152).  Node (i, j, k) adds, for each corner pair (by, bz) in a fixed
-// order, the entry of cell row (j - by, k - bz) at its position, and at a tile boundary the left
-// tile's last entry before it.  tileres (may be null): the tiles whose entries were written.
-struct OutTable {
-  double *p[6];
-};
-
-template <int NV, bool NORM, bool DBL = true>
-__global__ void k_node_sum(Geometry g, const double *__restrict__ partial, OutTable out,
-                           const uint8_t *__restrict__ tileres) {
-  const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nnode) return;
-  const int i = (int)(t % g.nx);
-  const int j = (int)((t / g.nx) % g.ny);
-  const int k = (int)(t / ((int64_t)g.nx * g.ny));
-  const int ntx = (g.nx + 7) / 8, tx = i >> 3, pos = i & 7, txl = tx == 0 ? ntx - 1 : tx - 1;
-  const int64_t nrows = (int64_t)g.ny * g.ncz, W = g.nx + ntx, fstride = 4 * nrows * W;
-  const int own = 9 * tx + pos, left = tx == 0 ? (int)W - 1 : 9 * tx - 1;
-  double v[4][NV + 1], vl[4][NV + 1];
-  bool ok[4], okl[4];
-#pragma unroll
-  for (int bb = 0; bb < 4; bb++) {
-    const int by = bb & 1, bz = bb >> 1;
-    int cj = j - by;
-    if (cj < 0) cj += g.ny;
-    const int ck = k - bz;
-    const bool in = ck >= 0 && ck < g.ncz;
-    const int64_t crow = in ? (int64_t)ck * g.ny + cj : 0;
-    ok[bb] = in && (!tileres || tileres[crow * ntx + tx]);
-    okl[bb] = in && pos == 0 && (!tileres || tileres[crow * ntx + txl]);
-    const double *e = partial + ((int64_t)bb * nrows + crow) * W;
-#pragma unroll
-    for (int f = 0; f <= NV; f++) {
-      v[bb][f] = ok[bb] ? e[f * fstride + own] : 0.0;
-      vl[bb][f] = okl[bb] ? e[f * fstride + left] : 0.0;
-    }
-  }
-  double s[NV + 1];
-#pragma unroll
-  for (int f = 0; f <= NV; f++) s[f] = 0.0;
-#pragma unroll
-  for (int bb = 0; bb < 4; bb++)
-#pragma unroll
-    for (int f = 0; f <= NV; f++)
-      if (ok[bb] || okl[bb]) s[f] = s[f] + (pos == 0 ? vl[bb][f] + v[bb][f] : v[bb][f]);
-  if (NORM) {
-    double w = s[0];
-    if (w == 0.) w = 1.;
-#pragma unroll
-    for (int f = 1; f <= NV; f++) out.p[f - 1][t] = s[f] / w;
-  } else {
-    const double mul = (DBL && (k == 0 || k == g.nzn - 1)) ? 2. : 1.;
-#pragma unroll
-    for (int f = 0; f <= NV; f++) out.p[f][t] = s[f] * mul;
-  }
-}
-
 // grid2par of one field (parcel_interpolation.F90:287-327)
 __global__ void k_grid2par(Geometry g, const double *__restrict__ par, int64_t cap, int64_t n,
                            const double *__restrict__ G, double *__restrict__ var,
@@ -491,6 +433,11 @@ static BinWork ctx_work(Ctx *c) {
   return w;
 }
 
+void bin_alloc(Ctx *c, const int32_t *count, int held, int32_t *start, int32_t *cursor) {
+  hipLaunchKernelGGL(k_bin_alloc, dim3(cdiv(c->ncell, TPB * ALLOC_CELLS)), dim3(TPB), 0, c->stream,
+                     count, c->ncell, held, start, cursor);
+}
+
 // bins n parcels; count and cursor must be zero, and the accumulation that follows zeroes them
 int bin_parcels_ws(Ctx *c, int64_t n, const BinWork &w) {
   const Geometry &g = c->g;
@@ -503,8 +450,7 @@ int bin_parcels_ws(Ctx *c, int64_t n, const BinWork &w) {
   if (n >= (int64_t)1 << 22) count(k_bin_count<16>, 16);
   else if (n >= (int64_t)1 << 19) count(k_bin_count<4>, 4);
   else if (n > 0) count(k_bin_count<1>, 1);
-  hipLaunchKernelGGL(k_bin_alloc, dim3(cdiv(c->ncell, TPB * ALLOC_CELLS)), dim3(TPB), 0, c->stream,
-                     w.count, c->ncell, w.start, w.cursor);
+  bin_alloc(c, w.count, 0, w.start, w.cursor);
   if (n > 0)
     hipLaunchKernelGGL(k_bin_scatter, dim3(cdiv(n, TPB)), dim3(TPB), 0, c->stream, w.cell, w.rank,
                        w.start, n, w.sorted);
@@ -526,12 +472,10 @@ static void launch_accum(Ctx *c, const BinWork &w, const double *var, double *pa
                      tileres, w.cursor, zero);
 }
 
-template <int NV, bool NORM, bool DBL>
-static void launch_node_sum(Ctx *c, const double *partial, const OutTable &out,
-                            const uint8_t *tileres) {
-  const int64_t nnode = (int64_t)c->g.nzn * c->g.ny * c->g.nx;
-  hipLaunchKernelGGL((k_node_sum<NV, NORM, DBL>), dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream,
-                     c->g, partial, out, tileres);
+template <int NF, bool NORM>
+static void node_sums(Ctx *c, const NodeSums<double, double> &first,
+                      const NodeSums<double, double> *second = nullptr) {
+  launch_node_sum<double, double, NF, NORM>(c, first, second);
 }
 
 int par2grid_fused(Ctx *c, int64_t n) {
@@ -540,9 +484,7 @@ int par2grid_fused(Ctx *c, int64_t n) {
   PMPIC_TRY(launch_timed(c, T_ACCUM, k_cell_accum<ACC_P2G, 4>, accum_tiles(c), dim3(64), 0, c->g,
                          c->par, c->cap, nullptr, w.count, w.start, w.sorted, w.rank, w.partial,
                          nullptr, nullptr, nullptr, w.cursor, 1));
-  launch_node_sum<4, true, true>(
-      c, w.partial, {{c->grid[GP], c->grid[GQ], c->grid[GR], c->grid[GB], nullptr, nullptr}},
-      nullptr);
+  node_sums<5, true>(c, {w.partial, {c->grid[GP], c->grid[GQ], c->grid[GR], c->grid[GB]}, nullptr, 1.});
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
@@ -551,8 +493,7 @@ int par2grid_single_ws(Ctx *c, int64_t n, const double *d_var, double *d_grid,
                        const BinWork &w) {
   PMPIC_TRY(bin_parcels_ws(c, n, w));
   launch_accum<ACC_SINGLE, 1>(c, w, d_var, w.partial, nullptr, nullptr, nullptr, 1);
-  launch_node_sum<1, true, true>(c, w.partial,
-                                 {{d_grid, nullptr, nullptr, nullptr, nullptr, nullptr}}, nullptr);
+  node_sums<2, true>(c, {w.partial, {d_grid}, nullptr, 1.});
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
@@ -580,9 +521,8 @@ __global__ void k_hgliq(Geometry g, double *__restrict__ B, const double *__rest
 int dump_grids_f64(Ctx *c, int64_t n) {
   PMPIC_TRY(bin_parcels(c, n));
   launch_accum<ACC_DUMP, 5>(c, ctx_work(c), nullptr, c->partial, nullptr, nullptr, nullptr, 1);
-  launch_node_sum<5, true, true>(
-      c, c->partial, {{c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR], nullptr}},
-      nullptr);
+  node_sums<6, true>(
+      c, {c->partial, {c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR]}, nullptr, 1.});
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
@@ -613,19 +553,21 @@ int grid2par_single(Ctx *c, int64_t n, const double *d_grid, double *d_var) {
 int mixing_grids(Ctx *c, int64_t n) {
   PMPIC_TRY(bin_parcels(c, n));
   const BinWork w = ctx_work(c);
-  const OutTable kept = {{c->grid[GVOL], c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ],
-                          c->grid[GR]}};
-  const OutTable res = {{c->kres[0], c->kres[1], c->kres[2], c->kres[3], c->kres[4], c->kres[5]}};
   uint8_t *flags = c->cellflag;
+  const NodeSums<double, double> kept = {
+      c->partial,
+      {c->grid[GVOL], c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR]}, nullptr, 2.};
+  NodeSums<double, double> res = {
+      c->partial2, {c->kres[0], c->kres[1], c->kres[2], c->kres[3], c->kres[4], c->kres[5]}, flags, 1.};
   if (c->partial2) {
     launch_accum<ACC_MIX, 5>(c, w, nullptr, c->partial, c->partial2, c->npercell, flags, 1);
-    launch_node_sum<5, false, true>(c, c->partial, kept, nullptr);
-    launch_node_sum<5, false, false>(c, c->partial2, res, flags);
+    node_sums<6, false>(c, kept, &res);
   } else {
     launch_accum<ACC_MIX, 5>(c, w, nullptr, c->partial, nullptr, c->npercell, flags, 0);
-    launch_node_sum<5, false, true>(c, c->partial, kept, nullptr);
+    node_sums<6, false>(c, kept);
     launch_accum<ACC_MIX, 5>(c, w, nullptr, nullptr, c->partial, nullptr, nullptr, 1);
-    launch_node_sum<5, false, false>(c, c->partial, res, flags);
+    res.partial = c->partial;
+    node_sums<6, false>(c, res);
   }
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;

@@ -448,7 +448,8 @@ __global__ void __launch_bounds__(TPB) k_split_flags(const T *__restrict__ stret
 // others flag the cells with fewer than three kept parcels, in the reference's loop order (i
 // outer, j, k inner; parcel_mixing.F90:160-162), and clear ctouch
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_mix_flags(const T *__restrict__ vol, int64_t n, T vmin,
+__global__ void __launch_bounds__(TPB) k_mix_flags(const T *__restrict__ vol, int stride, int64_t n,
+                                                   T vmin,
                                                    uint8_t *__restrict__ keep,
                                                    int32_t *__restrict__ blk, int64_t nblk,
                                                    Geometry g, const int32_t *__restrict__ npercell,
@@ -458,7 +459,7 @@ __global__ void __launch_bounds__(TPB) k_mix_flags(const T *__restrict__ vol, in
   __shared__ int lds[NWAVE];
   if (blockIdx.x < nblk) {
     if (n > 0)
-      make_flags([&](int64_t i) { return (uint8_t)(vol[i] < vmin ? 0 : 1); }, 0, n, blockIdx.x,
+      make_flags([&](int64_t i) { return (uint8_t)(vol[i * stride] < vmin ? 0 : 1); }, 0, n, blockIdx.x,
                  keep, blk, lds);
     else if (threadIdx.x == 0) blk[blockIdx.x] = 0;
     return;
@@ -773,15 +774,15 @@ int split_list(Ctx *c, const T *stretch, int64_t n) {
 }
 
 template <typename T>
-int mix_lists(Ctx *c, const T *vol, T vmin, int64_t n, uint8_t *ctouch) {
+int mix_lists(Ctx *c, const T *vol, int stride, T vmin, int64_t n, uint8_t *ctouch) {
   FlagList a = {c->flag, n, cdiv(n > 0 ? n : 1, FPB), nullptr, nullptr, c->list_a,
                 &c->dsc->nzero, 0};
   FlagList b = {c->cellflag, c->ncell, cdiv(c->ncell, FPB), nullptr, nullptr, c->sorted,
                 &c->dsc->nadd, 1};
   if (a.nblk > c->nblk_max || b.nblk > c->nblk_max) return PMPIC_ERR_ARG;
   int32_t *blk_a = c->blk, *blk_b = c->blk + 2 * a.nblk;
-  hipLaunchKernelGGL(k_mix_flags<T>, dim3(a.nblk + b.nblk), dim3(TPB), 0, c->stream, vol, n, vmin,
-                     c->flag, blk_a, a.nblk, c->g, c->npercell, c->ncell, c->cellflag, ctouch,
+  hipLaunchKernelGGL(k_mix_flags<T>, dim3(a.nblk + b.nblk), dim3(TPB), 0, c->stream, vol, stride, n,
+                     vmin, c->flag, blk_a, a.nblk, c->g, c->npercell, c->ncell, c->cellflag, ctouch,
                      blk_b);
   PMPIC_TRY(list_prefix(c, a, blk_a));
   PMPIC_TRY(list_prefix(c, b, blk_b));
@@ -792,8 +793,8 @@ int mix_lists(Ctx *c, const T *vol, T vmin, int64_t n, uint8_t *ctouch) {
 
 template int split_list<double>(Ctx *, const double *, int64_t);
 template int split_list<float>(Ctx *, const float *, int64_t);
-template int mix_lists<double>(Ctx *, const double *, double, int64_t, uint8_t *);
-template int mix_lists<float>(Ctx *, const float *, float, int64_t, uint8_t *);
+template int mix_lists<double>(Ctx *, const double *, int, double, int64_t, uint8_t *);
+template int mix_lists<float>(Ctx *, const float *, int, float, int64_t, uint8_t *);
 
 static int ensure_tmp(Ctx *c, int64_t need) {
   if (need <= c->tmp_cap) return PMPIC_OK;
@@ -903,7 +904,7 @@ int parcel_mix(Ctx *c) {
   const int64_t norig = c->n;
   PMPIC_TRY(mixing_grids(c, norig));
   // removed slots, ascending, and sparse cells in the reference's loop order
-  PMPIC_TRY(mix_lists(c, c->par + FVOL * c->cap, g.vmin, norig, c->ctouch));
+  PMPIC_TRY(mix_lists(c, c->par + FVOL * c->cap, 1, g.vmin, norig, c->ctouch));
   PMPIC_TRY(sync_scalars(c));
   const int64_t Z = c->hsc.nzero, nadd = c->hsc.nadd;
   MixGrids mg = {{c->grid[GVOL], c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR]},

@@ -10,6 +10,8 @@ The column kernel: levels per column below, at and above its read-ahead (8), row
 blocks below and above a wavefront's 16, whole steps, 1e-12 (FP64) and 1e-5 (FP32-bulk against
 FP64, that form's bar).
 
+The FP32-bulk accumulation: the same tiles and occupancies, and those around its slot capacities.
+
 The haloswap's permutation: parcel counts either side of a block, of the staging that needs no
 count read back (2^20 parcels) and of the one-launch scan (16,384 blocks).
 """
@@ -135,3 +137,42 @@ def test_haloswap_counts(n, crossing):
     for k, start, period in (("x", ic["x"], lx), ("y", ic["y"], ly)):
         assert np.abs(out[k][back] - start).max() <= 8 * np.finfo(float).eps * period
     g.close()
+
+
+@pytest.mark.parametrize("shuffled", [False, True])
+@pytest.mark.parametrize("slots", ["16", "32", "0"])
+@pytest.mark.parametrize("nx", [2, 3, 8, 9, 16, 25])
+def test_bulk32_tiles_and_occupancy(monkeypatch, nx, slots, shuffled):
+    """The FP32-bulk accumulation and its lists (slot table, overflow region, LDS and memory
+    orderings) against the FP64 form.  A node adds up to 8 cells of up to 300 parcels: a chain of
+    300 roundings of 6e-8 is 1.8e-5 of values between 0.5 and 1, so 3.6e-5 of a grid's least
+    maximum."""
+    from pmpic_amd.lib import Context
+    monkeypatch.setenv("PMPIC_SLOT_CAPACITY", slots)
+    occupancy = (0, 1, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 300)
+    shape = (nx, 4, 3)
+    b = box(*shape)
+    rng = np.random.default_rng(nx)
+    d = [(b[k + "max"] - b[k + "min"]) / n for k, n in zip("xyz", shape)]
+    at = []
+    for c in range(nx * 4 * 3):
+        ijk = np.array([c % nx, c // nx % 4, c // (nx * 4)])
+        at.append((ijk + rng.uniform(0.01, 0.99, (occupancy[c % len(occupancy)], 3))) * d)
+    at = np.concatenate(at)
+    n = len(at)
+    if shuffled:
+        at = at[rng.permutation(n)]
+    ic = dict(x=at[:, 0].copy(), y=at[:, 1].copy(), z=at[:, 2].copy(),
+              vol=rng.uniform(0.5, 1.0, n) * np.prod(d) / 8,
+              **{k: rng.uniform(0.5, 1.0, n) for k in ("b", "h", "p", "q", "r")})
+    grids = []
+    for precision in (0, 1):
+        g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                    2 * n + 64, precision=precision)
+        g.set_parcels(ic)
+        for _ in range(2):  # the second call finds what the first left behind
+            g.writebinary_grids()
+        grids.append({k: g.grid(k)[2:-2, 2:-2] for k in ("b", "hg", "p", "q", "r")})
+        g.close()
+    for k, want in grids[0].items():
+        assert rel_err(grids[1][k], want) < 3.6e-5, k
