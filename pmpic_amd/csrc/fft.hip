@@ -12,12 +12,14 @@
 // so the layout follows from one real-to-complex pass along the contiguous x rows and one
 // complex pass along y.  Each pass is one kernel: a workgroup stages a batch of rows (or of
 // adjacent columns, for coalesced strided access) in LDS and runs a mixed radix-4/2/3/5
-// Stockham FFT there, so each pass reads and writes HBM once.  The inverse builds, per (z, m),
+// Stockham FFT there, so each pass reads and writes HBM once.  A plane that fits the LDS takes both
+// passes in one kernel.  The inverse builds, per (z, m),
 // the complex row H = A_m + i B_m of the two real x-spectra, transforms it along x, and finishes
 // with a complex-to-real pass along y.
 #include "common.h"
 
 #include <math.h>
+#include <algorithm>
 #include <type_traits>
 #include <vector>
 
@@ -334,6 +336,17 @@ struct alignas(4 * sizeof(S) > 16 ? 16 : 4 * sizeof(S)) Quad {
   S v[4];  // a = 0: (Re, Im) of the x transform, a = 1: (Re, Im)
 };
 
+// a block's derivative along x or y (kw: its wavenumber), element for element as the standalone
+// diffx / diffy compute it (fft_ops.F90:266-269, :366-369)
+template <typename S>
+__device__ __forceinline__ Quad<S> derivative(const Quad<S> &u, int op, S kw) {
+  if (op == SPEC_DX)  // pair swap along x
+    return Quad<S>{((S)-1. * u.v[1]) * kw, u.v[0] * kw, ((S)-1. * u.v[3]) * kw, u.v[2] * kw};
+  if (op == SPEC_DY)  // pair swap along y
+    return Quad<S>{((S)-1. * u.v[2]) * kw, ((S)-1. * u.v[3]) * kw, u.v[0] * kw, u.v[1] * kw};
+  return u;
+}
+
 // forward pass 2: complex FFT along y of nb adjacent columns l of one z level, then the
 // (Re,Im)-pair split into the semi-spectral layout
 template <typename S, int NT>
@@ -422,14 +435,9 @@ __global__ void __launch_bounds__(FFT_TPB) k_rows_inv(Plan p, const cx_t<S> *__r
       const int k = div_small(r0 + t, nm, rnm, m);  // row = k * nm + m
       q[i] = *reinterpret_cast<const Quad<S> *>(src + spec_at(nzn, nl, k, m, l));
       if (op != SPEC_PLAIN) {
-        // the derivative, element for element as the standalone diffx / diffy compute it
-        // (fft_ops.F90:266-269, :366-369); kx depends on l and ky on m only
+        // kx depends on l and ky on m only
         const S kw = (S)(op == SPEC_DX ? fp.kx[2 * l] : fp.ky[(int64_t)(2 * m) * (2 * nl)]);
-        const Quad<S> u = q[i];
-        if (op == SPEC_DX)  // pair swap along x
-          q[i] = Quad<S>{((S)-1. * u.v[1]) * kw, u.v[0] * kw, ((S)-1. * u.v[3]) * kw, u.v[2] * kw};
-        else  // pair swap along y
-          q[i] = Quad<S>{((S)-1. * u.v[2]) * kw, ((S)-1. * u.v[3]) * kw, u.v[0] * kw, u.v[1] * kw};
+        q[i] = derivative(q[i], op, kw);
       }
     }
   }
@@ -526,6 +534,212 @@ __global__ void __launch_bounds__(FFT_TPB) k_cols_c2r(Plan p, const cx_t<S> *__r
   }
 }
 
+// ---- both passes of a plane in one workgroup ----
+// A small plane fits the LDS whole: its x and y transforms are then one launch, without the
+// intermediate in memory.  Small grids are bound by the latency of a launch and of its chain of
+// loads, stages and stores, not by the rate.  The forward and inverse calls of a timestep, before
+// and after: 11.0 + 17.4 -> 8.5 + 13.5 us at 48^3 FP32, 16.6 + 32 -> 12.1 + 20.3 at 90x60x41 FP32,
+// 8.9 + 10.0 -> 5.7 + 5.7 at 12x10x8 FP64, each with a gap between launches less.  The transforms
+// are the two-pass kernels', value for value.
+
+// exact q = a / d for a < 2^23 and 0 < d <= 512, m = floor(2^32 / d) + 1 (0 stands for 2^32, d = 1)
+__device__ __forceinline__ int div_magic(int a, uint32_t m) {
+  return m ? (int)__umulhi((uint32_t)a, m) : a;
+}
+inline uint32_t magic_of(int d) { return d == 1 ? 0u : (uint32_t)((1ull << 32) / d) + 1u; }
+
+// a transform of a plane: `count` of them of length n, and the stages' divisors
+struct PlanePass {
+  Plan p;
+  int count;
+  uint32_t mn, mnq[10], mns[10];
+};
+PlanePass plane_pass(int n, int count) {
+  PlanePass pp{};
+  pp.p = make_plan(n);
+  pp.count = count;
+  pp.mn = magic_of(n);
+  int ns = 1;
+  for (int s = 0; s < pp.p.nrad; s++) {
+    const int r = (int)((pp.p.code >> (4 * s)) & 15u);
+    pp.mnq[s] = magic_of(n / r);
+    pp.mns[s] = magic_of(ns);
+    ns *= r;
+  }
+  return pp;
+}
+
+template <int R, bool INV, int TPBP, typename C>
+__device__ __forceinline__ void plane_stage(const C *x, C *y, const C *tw, int n, int Ns, int nb,
+                                            uint32_t mnq, uint32_t mns) {
+  const int nq = n / R;  // R divides n
+  const int tstep = div_magic(nq, mns);
+  const int tot = nb * nq;
+  for (int bi = threadIdx.x; bi < tot; bi += TPBP) {
+    const int t = div_magic(bi, mnq), i = bi - t * nq;
+    const int j = div_magic(i, mns), k = i - j * Ns;
+    const C *xs = x + t * n + i;
+    C v[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+      const C e = xs[q * nq];
+      v[q] = (q == 0 || k == 0) ? e : cmul(e, tw[q * k * tstep]);
+    }
+    dft<R, INV>(v);
+    C *ys = y + t * n + j * Ns * R + k;
+#pragma unroll
+    for (int o = 0; o < R; o++) ys[o * Ns] = v[o];
+  }
+}
+
+template <bool INV, int TPBP, typename C>
+__device__ __forceinline__ void plane_fft(C *&a, C *&b, const C *tw, const PlanePass &pp) {
+  int Ns = 1;
+  for (int s = 0; s < pp.p.nrad; s++) {
+    const int r = (int)((pp.p.code >> (4 * s)) & 15u);
+    const uint32_t mq = pp.mnq[s], ms = pp.mns[s];
+    if (r == 4) plane_stage<4, INV, TPBP>(a, b, tw, pp.p.n, Ns, pp.count, mq, ms);
+    else if (r == 2) plane_stage<2, INV, TPBP>(a, b, tw, pp.p.n, Ns, pp.count, mq, ms);
+    else if (r == 3) plane_stage<3, INV, TPBP>(a, b, tw, pp.p.n, Ns, pp.count, mq, ms);
+    else plane_stage<5, INV, TPBP>(a, b, tw, pp.p.n, Ns, pp.count, mq, ms);
+    __syncthreads();
+    C *sw = a;
+    a = b;
+    b = sw;
+    Ns *= r;
+  }
+}
+
+// loads of a thread in flight at once
+constexpr int PLANE_BATCH = 4;
+
+// forward: x rows in pairs, as k_rows_r2c takes them, then the columns, as k_cols_fwd does
+template <typename S, int TPBP>
+__global__ void __launch_bounds__(TPBP) k_plane_fwd(PlanePass px, PlanePass py,
+                                                    const cx_t<S> *__restrict__ twx,
+                                                    const cx_t<S> *__restrict__ twy, FieldPtrs fp,
+                                                    int cap, int nzn, uint32_t mnl, uint32_t mrows) {
+  using C = cx_t<S>;
+  extern __shared__ double2 plane_lds[];
+  C *a = reinterpret_cast<C *>(plane_lds), *b = a + cap, *tx = b + cap, *ty = tx + px.p.n;
+  const int k = blockIdx.x, f = blockIdx.y, tid = threadIdx.x;
+  const int nx = px.p.n, ny = py.p.n, nl = nx / 2 + 1, rows = px.count;
+  const S *src = static_cast<const S *>(fp.in[f]) + (int64_t)k * ny * nx;
+  for (int e = tid; e < nx; e += TPBP) tx[e] = twx[e];
+  for (int e = tid; e < ny; e += TPBP) ty[e] = twy[e];
+  for (int e0 = tid; e0 < rows * nx; e0 += PLANE_BATCH * TPBP) {
+    C v[PLANE_BATCH];
+#pragma unroll
+    for (int i = 0; i < PLANE_BATCH; i++) {
+      const int e = e0 + i * TPBP;
+      if (e < rows * nx) {
+        const int t = div_magic(e, px.mn), x = e - t * nx;
+        v[i].x = src[2 * t * nx + x];
+        v[i].y = 2 * t + 1 < ny ? src[(2 * t + 1) * nx + x] : (S)0;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PLANE_BATCH; i++)
+      if (e0 + i * TPBP < rows * nx) a[e0 + i * TPBP] = v[i];
+  }
+  __syncthreads();
+  plane_fft<false, TPBP>(a, b, tx, px);
+  // columns: transform l, element y at l ny + y
+  for (int e = tid; e < nl * rows; e += TPBP) {
+    const int l = div_magic(e, mrows), t = e - l * rows;
+    const C z = a[t * nx + l], w = a[t * nx + (l == 0 ? 0 : nx - l)];
+    b[l * ny + 2 * t] = mkc<C, S>((z.x + w.x) / 2, (z.y - w.y) / 2);
+    if (2 * t + 1 < ny) b[l * ny + 2 * t + 1] = mkc<C, S>((z.y + w.y) / 2, (w.x - z.x) / 2);
+  }
+  __syncthreads();
+  plane_fft<false, TPBP>(b, a, ty, py);
+  S *dst = static_cast<S *>(fp.out[f]);
+  for (int e = tid; e < (ny / 2 + 1) * nl; e += TPBP) {
+    const int m = div_magic(e, mnl), l = e - m * nl;
+    const C g = b[l * ny + m], h = b[l * ny + (m == 0 ? 0 : ny - m)];
+    const C s = mkc<C, S>(g.x + h.x, g.y + h.y), d = mkc<C, S>(g.x - h.x, g.y - h.y);
+    *reinterpret_cast<Quad<S> *>(dst + spec_at(nzn, nl, k, m, l)) =
+        Quad<S>{s.x / 2, s.y / 2, d.y / 2, -d.x / 2};
+  }
+}
+
+// inverse: the rows m as k_rows_inv takes them, then the columns in pairs, as k_cols_c2r does
+template <typename S, int TPBP>
+__global__ void __launch_bounds__(TPBP) k_plane_inv(PlanePass px, PlanePass py,
+                                                    const cx_t<S> *__restrict__ twx,
+                                                    const cx_t<S> *__restrict__ twy, FieldPtrs fp,
+                                                    int cap, int nzn, uint32_t mnl, uint32_t mcols) {
+  using C = cx_t<S>;
+  constexpr int BATCH = PLANE_BATCH * 4 / sizeof(S);  // half as many FP64 blocks
+  extern __shared__ double2 plane_lds[];
+  C *a = reinterpret_cast<C *>(plane_lds), *b = a + cap, *tx = b + cap, *ty = tx + px.p.n;
+  const int k = blockIdx.x, f = blockIdx.y, tid = threadIdx.x, op = fp.op[f];
+  const int nx = px.p.n, ny = py.p.n, nl = nx / 2 + 1, nm = px.count, cols = py.count;
+  const S *src = static_cast<const S *>(fp.in[f]);
+  for (int e = tid; e < nx; e += TPBP) tx[e] = mkc<C, S>(twx[e].x, -twx[e].y);
+  for (int e = tid; e < ny; e += TPBP) ty[e] = mkc<C, S>(twy[e].x, -twy[e].y);
+  for (int e0 = tid; e0 < nm * nl; e0 += BATCH * TPBP) {
+    Quad<S> q[BATCH];
+    S kw[BATCH];
+#pragma unroll
+    for (int i = 0; i < BATCH; i++) {
+      const int e = e0 + i * TPBP;
+      if (e < nm * nl) {
+        const int m = div_magic(e, mnl), l = e - m * nl;
+        q[i] = *reinterpret_cast<const Quad<S> *>(src + spec_at(nzn, nl, k, m, l));
+        if (op != SPEC_PLAIN)
+          kw[i] = (S)(op == SPEC_DX ? fp.kx[2 * l] : fp.ky[(int64_t)(2 * m) * (2 * nl)]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < BATCH; i++) {
+      const int e = e0 + i * TPBP;
+      if (e < nm * nl) {
+        const int m = div_magic(e, mnl), l = e - m * nl;
+        const Quad<S> u = derivative(q[i], op, kw[i]);
+        const S ar = u.v[0], ai = u.v[1], br = u.v[2], bi = u.v[3];
+        if (l == 0 || 2 * l == nx) {
+          a[m * nx + l] = mkc<C, S>(ar, br);
+        } else {
+          a[m * nx + l] = mkc<C, S>(ar - bi, ai + br);
+          a[m * nx + nx - l] = mkc<C, S>(ar + bi, -ai + br);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  plane_fft<true, TPBP>(a, b, tx, px);
+  const S dnx = (S)1 / (S)nx, dny = (S)1 / (S)ny;
+  const bool even = (ny % 2) == 0;
+  // columns 2 t, 2 t + 1 as one transform: element y at t ny + y
+  for (int e = tid; e < cols * ny; e += TPBP) {
+    const int y = div_magic(e, mcols), t = e - y * cols;
+    const int m = y < nm ? y : ny - y;
+    C wa = a[m * nx + 2 * t], wb = 2 * t + 1 < nx ? a[m * nx + 2 * t + 1] : mkc<C, S>(0, 0);
+    wa.x *= dnx; wa.y *= dnx; wb.x *= dnx; wb.y *= dnx;
+    if (m == 0 || (even && m == ny / 2)) { wa.y = 0; wb.y = 0; }
+    if (y >= nm) { wa.y = -wa.y; wb.y = -wb.y; }
+    b[t * ny + y] = mkc<C, S>(wa.x - wb.y, wa.y + wb.x);
+  }
+  __syncthreads();
+  plane_fft<true, TPBP>(b, a, ty, py);
+  double *out = static_cast<double *>(fp.out[f]);
+  float *o32 = fp.out32[f];
+  for (int e = tid; e < cols * ny; e += TPBP) {
+    const int y = div_magic(e, mcols), t = e - y * cols;
+    const C v = b[t * ny + y];
+    const int64_t at = ((int64_t)k * ny + y) * nx + 2 * t;
+    if (out) {
+      out[at] = v.x * dny;
+      if (2 * t + 1 < nx) out[at + 1] = v.y * dny;
+    }
+    if (o32) {
+      o32[at] = (float)(v.x * dny);
+      if (2 * t + 1 < nx) o32[at + 1] = (float)(v.y * dny);
+    }
+  }
+}
+
 // W_n^e for e in [0, n), in FP64 and rounded to FP32
 int upload_twiddles(int n, double2 **dptr, float2 **dptr32) {
   std::vector<double2> h(n);
@@ -586,12 +800,47 @@ int with_length(int n, F &&f) {
 }
 static_assert(sizeof(FIXED_N) / sizeof(int) == 8, "with_length lists every fixed length");
 
+// LDS of a plane kernel (two buffers of `cap` elements and the twiddles), or 0 where the two-pass
+// kernels run: planes past 64 KB, and grids of more than 2^18 nodes whose lengths both have kernels
+// compiled for them (the two passes then run at the memory's rate).  FP32 steps, plane / two-pass:
+// 48^3 524 / 548 us, 72x72x30 614 / 682, 80x80x48 851 / 928, but 64^3 834 / 822, 96x64x64 1045 /
+// 1028; FP64 64x48x64 1203 / 1245 us.
+constexpr size_t PLANE_LDS = 64 * 1024;
+constexpr int64_t PLANE_NODES = (int64_t)1 << 18;
+inline bool fixed_length(int n) {
+  for (int f : FIXED_N)
+    if (f == n) return true;
+  return false;
+}
+template <typename S>
+static size_t plane_lds(const Geometry &g, int &cap) {
+  const int nl = g.nx / 2 + 1, nm = g.ny / 2 + 1;
+  cap = std::max(std::max((g.ny + 1) / 2 * g.nx, nl * g.ny),
+                 std::max(nm * g.nx, (g.nx + 1) / 2 * g.ny));
+  const size_t bytes = sizeof(cx_t<S>) * (2 * (size_t)cap + g.nx + g.ny);
+  if (fixed_length(g.nx) && fixed_length(g.ny) && (int64_t)g.nzn * g.ny * g.nx > PLANE_NODES) return 0;
+  return bytes <= PLANE_LDS ? bytes : 0;
+}
+// two wavefronts for planes of up to 512 points, eight above
+constexpr int PLANE_SMALL = 512;
+
 template <typename S>
 int fft_forward_t(Ctx *c, int nf, const S *const *src, S *const *dst) {
   const Geometry &g = c->g;
   if (nf < 1 || nf > MAXF) return PMPIC_ERR_ARG;
   FieldPtrs fp{};
   for (int f = 0; f < nf; f++) { fp.in[f] = src[f]; fp.out[f] = dst[f]; }
+  int cap;
+  if (const size_t lds = plane_lds<S>(g, cap)) {
+    const int rows = (g.ny + 1) / 2, nl = g.nx / 2 + 1;
+    const bool small = g.nx * g.ny <= PLANE_SMALL;
+    auto kernel = small ? k_plane_fwd<S, 128> : k_plane_fwd<S, 512>;
+    hipLaunchKernelGGL(kernel, dim3(g.nzn, nf), dim3(small ? 128 : 512), lds, c->stream,
+                       plane_pass(g.nx, rows), plane_pass(g.ny, nl), twiddles_x<S>(c),
+                       twiddles_y<S>(c), fp, cap, g.nzn, magic_of(nl), magic_of(rows));
+    PMPIC_CHECK(hipGetLastError());
+    return PMPIC_OK;
+  }
   const Plan px = make_plan(g.nx), py = make_plan(g.ny);
   const int64_t c1f = c1_field_size(g);
   const int nrows = g.nzn * g.ny;
@@ -628,6 +877,17 @@ int fft_backward_t(Ctx *c, int nf, const S *const *src, double *const *dst, floa
     fp.out32[f] = dst32 ? dst32[f] : nullptr;
     fp.op[f] = deriv ? deriv[f] : SPEC_PLAIN;
     if (fp.op[f] < SPEC_PLAIN || fp.op[f] > SPEC_DY) return PMPIC_ERR_ARG;
+  }
+  int cap;
+  if (const size_t lds = plane_lds<S>(g, cap)) {
+    const int nl = g.nx / 2 + 1, cols = (g.nx + 1) / 2;
+    const bool small = g.nx * g.ny <= PLANE_SMALL;
+    auto kernel = small ? k_plane_inv<S, 128> : k_plane_inv<S, 512>;
+    hipLaunchKernelGGL(kernel, dim3(g.nzn, nf), dim3(small ? 128 : 512), lds, c->stream,
+                       plane_pass(g.nx, g.ny / 2 + 1), plane_pass(g.ny, cols), twiddles_x<S>(c),
+                       twiddles_y<S>(c), fp, cap, g.nzn, magic_of(nl), magic_of(cols));
+    PMPIC_CHECK(hipGetLastError());
+    return PMPIC_OK;
   }
   const Plan px = make_plan(g.nx), py = make_plan(g.ny);
   const int64_t c2f = c2_field_size(g);

@@ -176,3 +176,27 @@ def test_bulk32_tiles_and_occupancy(monkeypatch, nx, slots, shuffled):
         g.close()
     for k, want in grids[0].items():
         assert rel_err(grids[1][k], want) < 3.6e-5, k
+
+
+@pytest.mark.parametrize("nx,ny", [(2, 2), (2, 5), (5, 2), (3, 16), (16, 32), (18, 32), (25, 16),
+                                   (45, 27), (64, 60), (60, 64), (64, 64), (81, 48)])
+def test_plane_transforms(nx, ny):
+    """Both transforms at the smallest planes, the change of workgroup (512 points) and the largest
+    plane that fits one (60 x 64 in FP64), against numpy: FP64 sums of a few thousand terms, 1e-13
+    of the maximum."""
+    from pmpic_amd.lib import Context
+    b = box(nx, ny, 3)
+    g = Context(nx, ny, 3, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"], 64)
+    rng = np.random.default_rng(nx * ny)
+    field = np.zeros(g.gshape)
+    field[2:-2, 2:-2] = rng.standard_normal(field[2:-2, 2:-2].shape)
+    got = g.fft_forward(field)
+    y = np.fft.rfft(field[2:-2, 2:-2], axis=1)  # [x, y, z]
+    want = np.zeros_like(got)
+    for a, part in enumerate((y.real, y.imag)):
+        x = np.fft.rfft(part, axis=0)
+        want[0::2, a::2], want[1::2, a::2] = x.real, x.imag
+    assert np.abs(got - want).max() <= 1e-13 * np.abs(want).max()
+    back = g.fft_backward(got)[2:-2, 2:-2]
+    assert np.abs(back - field[2:-2, 2:-2]).max() <= 1e-13 * np.abs(field).max()
+    g.close()
