@@ -191,7 +191,7 @@ int free_all(Ctx *c) {
   hipFree(c->rec); hipFree(c->rec32);
   for (int g = 0; g < 8; g++) hipFree(c->gtmp[g]);
   hipFree(c->kres[0]);
-  double *sp[] = {c->spool, c->sd, c->se, c->sf, c->su, c->sv, c->sw, c->sbs};
+  double *sp[] = {c->spool, c->sd, c->se, c->sw, c->sbs};
   for (double *p : sp) hipFree(p);
   for (int g = 1; g < 6; g++) hipFree(c->sder[g]);
   hipFree(c->atop); hipFree(c->abot);
@@ -273,14 +273,14 @@ int create(const pmpic_config *cf, Ctx *c) {
                    c->gsz + std::max({5 * c->gsz, ref_grid_size(g), c->ssz})));
   for (int i = 1; i < 6; i++) c->kres[i] = c->kres[0] + i * c->gsz;
   c->refbuf = c->kres[1];
-  double **sp[] = {&c->sd, &c->se, &c->sf, &c->su, &c->sv, &c->sw, &c->sbs};
+  double **sp[] = {&c->sd, &c->se, &c->sw, &c->sbs};
   for (double **p : sp) PMPIC_TRY(dalloc(p, c->bsz));
   for (int i = 1; i < 6; i++) PMPIC_TRY(dalloc(&c->sder[i], c->bsz));
   const int64_t plane = (int64_t)g.sy * g.sx;
   // the arrays the column kernel reads ahead in, one after another between COLUMN_PAD levels
-  PMPIC_TRY(dalloc(&c->spool, 4 * c->bsz + 2 * COLUMN_PAD * 64));
-  double **rp[] = {&c->sa, &c->sb, &c->sc, &c->sder[0]};
-  for (int i = 0; i < 4; i++) *rp[i] = c->spool + COLUMN_PAD * 64 + i * c->bsz;
+  double **rp[] = {&c->sa, &c->sb, &c->sc, &c->sder[0], &c->sf, &c->su, &c->sv};
+  PMPIC_TRY(dalloc(&c->spool, 7 * c->bsz + 2 * COLUMN_PAD * 64));
+  for (int i = 0; i < 7; i++) *rp[i] = c->spool + COLUMN_PAD * 64 + i * c->bsz;
   PMPIC_TRY(dalloc(&c->atop, plane));
   PMPIC_TRY(dalloc(&c->abot, plane));
   PMPIC_TRY(dalloc(&c->ubar, g.nzn));

@@ -28,7 +28,7 @@
 // Bound by memory on large grids (26 passes over a spectral array where the separate kernels took
 // 41) and by the instruction latency of one wavefront on small ones.  A call, against the sum of
 // the ten kernels it stands for: 199 / 540 us at 256x256x128 FP32 (4.6 TB/s), 143 / 280 us at
-// 128x128x128 FP64, 31 / 91 us at 48x48x48 FP32, 13 / 26 us at 12x10x8 FP64.
+// 128x128x128 FP64, 22 / 91 us at 48x48x48 FP32, 9 / 26 us at 12x10x8 FP64.
 #include "common.h"
 
 #include <type_traits>
@@ -104,7 +104,7 @@ __global__ void k_dz_rcp(Geometry g, const double *__restrict__ den, double *__r
 template <typename S>
 struct ColumnArrays {
   S *a, *b, *c;        // in: vorticity spectra; overwritten by the intermediates
-  S *f;                // scratch
+  S *f;                // scratch; a, b, c, f, fc, us and vs are padded (COLUMN_PAD)
   S *fa, *fb, *fc;     // out: filtered corrected vorticity
   S *u, *v, *w;        // out: velocity spectra
   S *us, *vs, *ws;     // out: filtered velocity spectra
@@ -170,13 +170,23 @@ __device__ void mean_flow(const Geometry &g, const ColumnArrays<S> &ca) {
 // both ends of the arrays and tables), so the loop has no bounds, branches or clamps on its memory
 // accesses: loads and stores retire in a known order, and no wait for a load covers the stores
 // behind it.  LV = 8 against 4: 201 / 212 us at 256x256x128 FP32, 143 / 160 us at 128x128x128 FP64.
+//
+// before(): the steps below s0, whose values the caller has loaded.  EARLY: after the first loads
+// are issued, so that a pass waits on memory once at its start and not twice (the values past its
+// end are then loaded at its start too); the registers for it are there where a wavefront has a
+// SIMD to itself.
 constexpr int LV = 8;
 static_assert(COLUMN_PAD >= 2 * LV, "padding of the arrays the sweeps read");
-template <class T, class Load, class Body>
-__device__ __forceinline__ void sweep(int s0, int n, Load load, Body body) {
+template <class T, bool EARLY, class Load, class Body, class Before>
+__device__ __forceinline__ void sweep(int s0, int n, Load load, Body body, Before before) {
   T v[LV];
+  if constexpr (!EARLY) before();
 #pragma unroll
   for (int i = 0; i < LV; i++) v[i] = load(s0, i);
+  if constexpr (EARLY) {
+    __builtin_amdgcn_sched_barrier(0x7);
+    before();
+  }
   int s = s0;
   for (; s + LV <= n; s += LV) {
 #pragma unroll
@@ -197,22 +207,40 @@ struct Piv {
   double r, d;
 };
 
-// The column work of a wavefront.  KEEP: some of its columns pass the filter (where none does, the
+// The column work of a tile.  KEEP: some of its columns pass the filter (where none does, the
 // correction of the vorticity is zero).  FIRST: it holds the k^2 = 0 columns, which laplinv leaves
 // alone, and of them the column (0, 0), whose u and v belong to the mean flow.
-template <bool KEEP, bool FIRST, typename S>
-__device__ __forceinline__ void columns(const Geometry &g, const ColumnArrays<S> &ca) {
+//
+// SPLIT: four wavefronts share the tile instead of one.  One wavefront issues an instruction every
+// four cycles or so, and a small grid has fewer tiles than the chip has CUs, so its time is the
+// instructions of one wavefront (8,000 at 49 levels), and the loads of its unrolled code from cold
+// caches.  The divergence is taken level by level by
+// all four, into LDS; then the recurrences of a pass that do not depend on each other go to
+// different wavefronts, those that several need (f's solution, a's and b's) computed by each of
+// them; a barrier between the passes.  No pass may then overwrite what another wavefront still
+// reads: the intermediates of dz(f), dz(a) and dz(b) lie in fc, vs and us, read last by the
+// wavefront that writes the results there (and padded, like a, b, c and f, for its read-ahead).
+// A call: 31 -> 22.5 us at 48^3 FP32, 29 -> 21 at 32^3 FP64, 12.9 -> 9.4 at 12x10x8 FP64.  With
+// four or six levels ahead instead of eight 28 and 24 us at 48^3, with 16 (twice the code) 44; with
+// the whole tile in LDS and rolled loops 25 to 27.
+template <bool KEEP, bool FIRST, bool SPLIT, typename S>
+__device__ __forceinline__ void columns(const Geometry &g, const ColumnArrays<S> &ca,
+                                        double *lds) {
   // fused multiply-adds: fewer instructions and roundings in the recurrences
 #pragma clang fp contract(fast)
   constexpr bool F32 = std::is_same<S, float>::value;
-  // the wavefront takes one tile (16 blocks) of the spectral layout, a lane one of its 64 columns:
-  // lane bits 0 the column of the pair, 1 the row of the pair, 2-5 the block
-  const int lane = threadIdx.x, tile = blockIdx.x, ntile = spec_tiles(g), nz = g.nzn;
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  // a lane takes one of the 64 columns of a tile (16 blocks) of the spectral layout: lane bits 0
+  // the column of the pair, 1 the row of the pair, 2-5 the block
+  const int lane = threadIdx.x & 63, tile = blockIdx.x, ntile = spec_tiles(g), nz = g.nzn;
+  const int role = SPLIT ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int nl = g.sx / 2, blk = min(tile * 16 + (lane >> 2), nl * (g.sy / 2) - 1);
   const int m = blk / nl, l = blk - m * nl;
   const int col = (2 * m + ((lane >> 1) & 1)) * g.sx + 2 * l + (lane & 1);  // in the planes of k, filt
   const double k2 = ca.k2[col];
   const bool pass = KEEP && ca.filt[col] != 0.;  // the filter is 0 or 1
+  S *const ef = SPLIT ? ca.fc : ca.f, *const za = SPLIT ? ca.vs : ca.a, *const zb = SPLIT ? ca.us : ca.b;
   // level k + i of an array, k uniform and 0 <= i < LV an immediate
   auto at = [&](S *p, int k, int i) { return p + ((int64_t)tile * nz + k) * 64 + (lane + i * 64); };
   auto get = [&](S *p, int k, int i) { return *at(p, k, i); };
@@ -265,45 +293,98 @@ __device__ __forceinline__ void columns(const Geometry &g, const ColumnArrays<S>
 
   // ---- up: divergence (vort2vel.F90:158-174) and its elimination ----
   if constexpr (KEEP) {
-    struct T { S a, b, c1; Piv p; };
     const double h = 1. / 2. / dz;
-    const double cA = (double)get(ca.c, 0, 0), cB = (double)get(ca.c, 1, 0),
-                 cC = (double)get(ca.c, 2, 0);
     auto horizontal = [&](S a, S b) { return other_x(a) * kx + other_y(b) * ky; };
-    double dm = horizontal(get(ca.a, 0, 0), get(ca.b, 0, 0)) + h * (4. * cB - cC - 3. * cA);
-    double d0 = horizontal(get(ca.a, 1, 0), get(ca.b, 1, 0)) + (cC - cA) * h;
-    if (FIRST && lane == 0) dm = d0 = 0.;
-    double fp = row_first(dm, d0, piv(1, 0, 0));
-    put(ca.f, 0, 0, fp);
-    double cmm = cA, cm = cB, c0 = cC;  // c at levels k - 2, k - 1, k
-    auto step = [&](int k, int i, double fz, S a, S b, const Piv &p) {
-      double d1 = horizontal(a, b) + fz;
-      if (FIRST && lane == 0) d1 = 0.;
-      fp = row(dm, d0, d1, fp, p);  // row k + i - 1
-      put(ca.f, k - 1, i, fp);
-      dm = d0; d0 = d1;
-    };
-    sweep<T>(2, nz - 1,
-        [&](int k, int i) {
-          return T{get(ca.a, k, i), get(ca.b, k, i), get(ca.c, k + 1, i), piv(1, k - 1, i)};
-        },
-        [&](int k, int i, const T &t) {
-          const double c1 = (double)t.c1;
-          step(k, i, (c1 - cm) * h, t.a, t.b, t.p);
-          cmm = cm; cm = c0; c0 = c1;
+    if constexpr (SPLIT) {
+      constexpr int DB = 4;  // levels of a wavefront in flight
+      for (int k0 = role; k0 < nz; k0 += 4 * DB) {
+        S a[DB], b[DB], cl[DB], ch[DB];
+#pragma unroll
+        for (int i = 0; i < DB; i++) {
+          const int k = min(k0 + 4 * i, nz - 1);
+          a[i] = get(ca.a, k, 0);
+          b[i] = get(ca.b, k, 0);
+          cl[i] = get(ca.c, max(k - 1, 0), 0);
+          ch[i] = get(ca.c, min(k + 1, nz - 1), 0);
+        }
+#pragma unroll
+        for (int i = 0; i < DB; i++) {
+          const int k = k0 + 4 * i;
+          if (k >= nz) break;
+          double fz = ((double)ch[i] - (double)cl[i]) * h;
+          if (k == 0)  // cl: level 0, ch: level 1
+            fz = h * (4. * (double)ch[i] - (double)get(ca.c, 2, 0) - 3. * (double)cl[i]);
+          if (k == nz - 1)
+            fz = h * ((double)get(ca.c, nz - 3, 0) + 3. * (double)ch[i] - 4. * (double)cl[i]);
+          const double d = horizontal(a[i], b[i]) + fz;
+          lds[k * 64 + lane] = FIRST && lane == 0 ? 0. : d;
+        }
+      }
+      __syncthreads();
+      if (role == 0) {
+        struct T { double d; Piv p; };
+        double dm = lds[lane], d0 = lds[64 + lane], fp = 0.;
+        const Piv first = piv(1, 0, 0), end = piv(1, nz - 1, 0);
+        auto step = [&](int k, int i, const T &t) {
+          fp = row(dm, d0, t.d, fp, t.p);  // row k + i - 1
+          put(ca.f, k - 1, i, fp);
+          dm = d0; d0 = t.d;
+        };
+        auto load = [&](int k, int i) { return T{lds[(k + i) * 64 + lane], piv(1, k - 1, i)}; };
+        sweep<T, SPLIT>(2, nz, load, step, [&]() {
+          fp = row_first(dm, d0, first);
+          put(ca.f, 0, 0, fp);
         });
-    step(nz - 1, 0, h * (cmm + 3. * c0 - 4. * cm), get(ca.a, nz - 1, 0), get(ca.b, nz - 1, 0),
-         piv(1, nz - 2, 0));
-    put(ca.f, nz - 1, 0, row_last(dm, d0, fp, piv(1, nz - 1, 0)));
+        put(ca.f, nz - 1, 0, row_last(dm, d0, fp, end));
+      }
+      __syncthreads();
+    } else {
+      struct T { S a, b, c1; Piv p; };
+      const S a0 = get(ca.a, 0, 0), a1 = get(ca.a, 1, 0), b0 = get(ca.b, 0, 0),
+              b1 = get(ca.b, 1, 0);
+      const double cA = (double)get(ca.c, 0, 0), cB = (double)get(ca.c, 1, 0),
+                   cC = (double)get(ca.c, 2, 0);
+      const Piv first = piv(1, 0, 0);
+      double dm = 0., d0 = 0., fp = 0.;
+      double cmm = cA, cm = cB, c0 = cC;  // c at levels k - 2, k - 1, k
+      auto step = [&](int k, int i, double fz, S a, S b, const Piv &p) {
+        double d1 = horizontal(a, b) + fz;
+        if (FIRST && lane == 0) d1 = 0.;
+        fp = row(dm, d0, d1, fp, p);  // row k + i - 1
+        put(ca.f, k - 1, i, fp);
+        dm = d0; d0 = d1;
+      };
+      sweep<T, SPLIT>(2, nz - 1,
+          [&](int k, int i) {
+            return T{get(ca.a, k, i), get(ca.b, k, i), get(ca.c, k + 1, i), piv(1, k - 1, i)};
+          },
+          [&](int k, int i, const T &t) {
+            const double c1 = (double)t.c1;
+            step(k, i, (c1 - cm) * h, t.a, t.b, t.p);
+            cmm = cm; cm = c0; c0 = c1;
+          },
+          [&]() {
+            dm = horizontal(a0, b0) + h * (4. * cB - cC - 3. * cA);
+            d0 = horizontal(a1, b1) + (cC - cA) * h;
+            if (FIRST && lane == 0) dm = d0 = 0.;
+            fp = row_first(dm, d0, first);
+            put(ca.f, 0, 0, fp);
+          });
+      step(nz - 1, 0, h * (cmm + 3. * c0 - 4. * cm), get(ca.a, nz - 1, 0), get(ca.b, nz - 1, 0),
+           piv(1, nz - 2, 0));
+      put(ca.f, nz - 1, 0, row_last(dm, d0, fp, piv(1, nz - 1, 0)));
+    }
   }
 
   // ---- down: the correction of a and b (vort2vel.F90:176-194), eliminations of dz(f), a, b ----
-  double atop, abot, btop, bbot;
-  {
+  double atop = 0., abot = 0., btop = 0., bbot = 0.;
+  auto down = [&](auto do_a, auto do_b, auto do_e) {
+    constexpr bool A = decltype(do_a)::value, B = decltype(do_b)::value,
+                   E = KEEP && decltype(do_e)::value;
     struct T { S f, a, b; double cp; Piv p; };
     double fn = 0., f0 = 0., f1 = 0., f2 = 0.;   // unfiltered; filtered at this level, +1, +2
-    double a0, a1 = 0., a2, b0, b1 = 0., b2;     // corrected
-    double ep = 0., ap, bp;                      // eliminated values of the previous row
+    double a0 = 0., a1 = 0., a2 = 0., b0 = 0., b1 = 0., b2 = 0.;  // corrected
+    double ep = 0., ap = 0., bp = 0.;            // eliminated values of the previous row
     // level k + i; cf: the c of its row (for the back-substitution), sub: below the top
     auto level = [&](int k, int i, const T &t, double cf, bool sub) {
       f2 = f1; f1 = f0;
@@ -314,14 +395,17 @@ __device__ __forceinline__ void columns(const Geometry &g, const ColumnArrays<S>
         fn = sub ? (double)t.f - cp_of(cf, t.cp) * fn : (double)t.f;
         const S ff = pass ? (S)fn : (S)0;
         f0 = (double)ff;
-        a0 = (double)(S)(a0 - other_x(ff) * kx);
-        b0 = (double)(S)(b0 - other_y(ff) * ky);
+        if constexpr (A) a0 = (double)(S)(a0 - other_x(ff) * kx);
+        if constexpr (B) b0 = (double)(S)(b0 - other_y(ff) * ky);
       }
-      put_filtered(ca.fa, k, i, (S)a0);
-      put_filtered(ca.fb, k, i, (S)b0);
+      if constexpr (A) put_filtered(ca.fa, k, i, (S)a0);
+      if constexpr (B) put_filtered(ca.fb, k, i, (S)b0);
     };
     auto load = [&](int s, int k, int i, int r) {  // level k + r, elimination step s - 1 + i
-      T t{(S)0, get(ca.a, k, r), get(ca.b, k, r), 0., piv(0, s - 1, i)};
+      T t{};
+      if constexpr (A) t.a = get(ca.a, k, r);
+      if constexpr (B) t.b = get(ca.b, k, r);
+      if constexpr (A || B) t.p = piv(0, s - 1, i);
       if constexpr (KEEP) {
         t.f = get(ca.f, k, r);
         t.cp = back(1, k, r);
@@ -329,45 +413,64 @@ __device__ __forceinline__ void columns(const Geometry &g, const ColumnArrays<S>
       return t;
     };
     const T top = load(1, nz - 1, 0, 0), next = load(1, nz - 2, 0, 0);
-    level(nz - 1, 0, top, 0., false);
-    atop = a0; btop = b0;
-    a1 = a0; b1 = b0;
-    level(nz - 2, 0, next, off, true);
-    ap = row_end(a1);
-    bp = row_end(b1);
-    if constexpr (KEEP) put(ca.f, nz - 1, 0, 0.);
-    put(ca.a, nz - 1, 0, ap);
-    put(ca.b, nz - 1, 0, bp);
-    a2 = a1; a1 = a0;
-    b2 = b1; b1 = b0;
+    T bottom{};
+    if constexpr (SPLIT) bottom = load(nz - 1, 0, 0, 0);
     auto rows = [&](int s, int k, int i, int r, const T &t, double cf) {  // row above level k + r
       const double aa = a1, ab = a2, ba = b1, bb = b2;
       level(k, r, t, cf, true);
-      if constexpr (KEEP) {
+      if constexpr (E) {
         ep = quot<S>(half_dz(f2 - f0) - f16 * ep, zd0[s + i - 1], zr0[s + i - 1]);
-        put(ca.f, k + 1, r, ep);
+        put(ef, k + 1, r, ep);
       }
-      ap = row(a0, aa, ab, ap, t.p);
-      bp = row(b0, ba, bb, bp, t.p);
-      put(ca.a, k + 1, r, ap);
-      put(ca.b, k + 1, r, bp);
+      if constexpr (A) {
+        ap = row(a0, aa, ab, ap, t.p);
+        put(ca.a, k + 1, r, ap);
+      }
+      if constexpr (B) {
+        bp = row(b0, ba, bb, bp, t.p);
+        put(ca.b, k + 1, r, bp);
+      }
       a2 = aa; a1 = a0;
       b2 = ba; b1 = b0;
     };
     // steps 2 .. nz - 2 are levels nz - 3 .. 1; a chunk's lowest level is k
-    sweep<T>(2, nz - 1,
+    sweep<T, SPLIT>(2, nz - 1,
         [&](int s, int i) { return load(s, nz - s - LV, i, LV - 1 - i); },
-        [&](int s, int i, const T &t) { rows(s, nz - s - LV, i, LV - 1 - i, t, off); });
-    rows(nz - 1, 0, 0, 0, load(nz - 1, 0, 0, 0), cend);
+        [&](int s, int i, const T &t) { rows(s, nz - s - LV, i, LV - 1 - i, t, off); },
+        [&]() {
+          level(nz - 1, 0, top, 0., false);
+          atop = a0; btop = b0;
+          a1 = a0; b1 = b0;
+          level(nz - 2, 0, next, off, true);
+          ap = row_end(a1);
+          bp = row_end(b1);
+          if constexpr (E) put(ef, nz - 1, 0, 0.);
+          if constexpr (A) put(ca.a, nz - 1, 0, ap);
+          if constexpr (B) put(ca.b, nz - 1, 0, bp);
+          a2 = a1; a1 = a0;
+          b2 = b1; b1 = b0;
+        });
+    if constexpr (!SPLIT) bottom = load(nz - 1, 0, 0, 0);
+    rows(nz - 1, 0, 0, 0, bottom, cend);
     abot = a0;
     bbot = b0;
-    if constexpr (KEEP) put(ca.f, 0, 0, 0.);
-    put(ca.a, 0, 0, row_end(a0));
-    put(ca.b, 0, 0, row_end(b0));
+    if constexpr (E) put(ef, 0, 0, 0.);
+    if constexpr (A) put(ca.a, 0, 0, row_end(a0));
+    if constexpr (B) put(ca.b, 0, 0, row_end(b0));
+  };
+  if constexpr (SPLIT) {
+    if (role == 0) down(yes, no, no);
+    if (role == 1) down(no, yes, no);
+    if (KEEP && role == 2) down(no, no, yes);
+    __syncthreads();
+  } else {
+    down(yes, yes, yes);
   }
 
   // ---- up: the correction of c (vort2vel.F90:197-218), a and b solved, w; eliminations ----
-  {
+  auto up = [&](auto do_a, auto do_b, auto do_c, auto do_w) {
+    constexpr bool A = decltype(do_a)::value, B = decltype(do_b)::value;
+    constexpr bool C = decltype(do_c)::value, W = decltype(do_w)::value;
     struct T { S f, c, a, b; double cp; Piv p; };
     double fn = 0., an = 0., bn = 0.;                       // solved values
     double cm = 0., c0 = 0., c1 = 0., cp1 = 0.;             // corrected c below, at row; eliminated
@@ -375,106 +478,158 @@ __device__ __forceinline__ void columns(const Geometry &g, const ColumnArrays<S>
     double zap = 0., zbp = 0.;
     // level k + i; zc: the dz solve's c' (unused at the bottom)
     auto level = [&](int k, int i, const T &t, double cf, double zc, bool sub) {
-      cm = c0; c0 = c1;
-      am = a0; a0 = a1;
-      bm = b0; b0 = b1;
-      c1 = (double)t.c;
-      if constexpr (KEEP) {
-        fn = sub ? (double)t.f - zc * fn : (double)t.f;
-        c1 = (double)(S)(c1 - (double)(S)fn);
+      if constexpr (C) {
+        cm = c0; c0 = c1;
+        c1 = (double)t.c;
+        if constexpr (KEEP) {
+          fn = sub ? (double)t.f - zc * fn : (double)t.f;
+          c1 = (double)(S)(c1 - (double)(S)fn);
+        }
+        if (!sub) c1 = 0.;
+        put_filtered(ca.fc, k, i, (S)c1);
       }
-      if (!sub) c1 = 0.;
-      put_filtered(ca.fc, k, i, (S)c1);
       const double cp = cp_of(cf, t.cp);
-      an = sub ? (double)t.a - cp * an : (double)t.a;
-      bn = sub ? (double)t.b - cp * bn : (double)t.b;
-      const S as = (S)an, bs = (S)bn;
-      a1 = (double)as;
-      b1 = (double)bs;
-      const double w = other_y(as) * ky - other_x(bs) * kx;
-      put(ca.w, k, i, w);
-      put_filtered(ca.ws, k, i, (S)w);
+      if constexpr (A || W) {
+        am = a0; a0 = a1;
+        an = sub ? (double)t.a - cp * an : (double)t.a;
+        a1 = (double)(S)an;
+      }
+      if constexpr (B || W) {
+        bm = b0; b0 = b1;
+        bn = sub ? (double)t.b - cp * bn : (double)t.b;
+        b1 = (double)(S)bn;
+      }
+      if constexpr (W) {
+        const double w = other_y((S)an) * ky - other_x((S)bn) * kx;
+        put(ca.w, k, i, w);
+        put_filtered(ca.ws, k, i, (S)w);
+      }
     };
     auto store = [&](int k, int i, int z, double ra, double rb) {  // row k + i
-      put(ca.c, k, i, cp1);
-      zap = quot<S>(ra, zd1[z], zr1[z]);
-      zbp = quot<S>(rb, zd1[z], zr1[z]);
+      if constexpr (C) put(ca.c, k, i, cp1);
+      if constexpr (A) zap = quot<S>(ra, zd1[z], zr1[z]);
+      if constexpr (B) zbp = quot<S>(rb, zd1[z], zr1[z]);
       if (FIRST && lane == 0) return;  // column (0, 0) of a and b stays: the mean flow's input
-      put(ca.a, k, i, zap);
-      put(ca.b, k, i, zbp);
+      if constexpr (A) put(za, k, i, zap);
+      if constexpr (B) put(zb, k, i, zbp);
     };
     auto load = [&](int k, int i, int s, int r, int q) {  // level k + i, its step s + r; row q + i
-      T t{(S)0, get(ca.c, k, i), get(ca.a, k, i), get(ca.b, k, i), back(0, s, r), piv(1, q, i)};
-      if constexpr (KEEP) t.f = get(ca.f, k, i);
+      T t{};
+      if constexpr (A || W) t.a = get(ca.a, k, i);
+      if constexpr (B || W) t.b = get(ca.b, k, i);
+      if constexpr (A || B || W) t.cp = back(0, s, r);
+      if constexpr (C) {
+        t.c = get(ca.c, k, i);
+        t.p = piv(1, q, i);
+        if constexpr (KEEP) t.f = get(ef, k, i);
+      }
       return t;
     };
     const T bottom = load(0, 0, nz - 2, 0, 0), next = load(1, 0, nz - 2, 0, 0);
-    level(0, 0, bottom, 0., 0., false);
-    level(1, 0, next, off, zc0[nz - 1], true);
-    cp1 = row_first(c0, c1, next.p);
-    store(0, 0, 0, per_dz(a1) - f16 * abot * dz, per_dz(b1) - f16 * bbot * dz);
+    T top{};
+    Piv end{};
+    auto load_end = [&]() {
+      top = load(nz - 1, 0, 0, 0, nz - 2);
+      if constexpr (C) end = piv(1, nz - 1, 0);
+    };
+    if constexpr (SPLIT) load_end();
     auto rows = [&](int k, int i, const T &t, double cf, double zc) {
       level(k, i, t, cf, zc, true);
-      cp1 = row(cm, c0, c1, cp1, t.p);
+      if constexpr (C) cp1 = row(cm, c0, c1, cp1, t.p);
       store(k - 1, i, k + i - 1, half_dz(a1 - am) - f16 * zap, half_dz(b1 - bm) - f16 * zbp);
     };
     // levels 2 .. nz - 2; a chunk's levels k .. k + LV - 1 are steps nz - 1 - k downwards
-    sweep<T>(2, nz - 1,
+    sweep<T, SPLIT>(2, nz - 1,
         [&](int k, int i) { return load(k, i, nz - k - LV, LV - 1 - i, k - 1); },
-        [&](int k, int i, const T &t) { rows(k, i, t, off, zc0[nz - k - i]); });
+        [&](int k, int i, const T &t) { rows(k, i, t, off, zc0[nz - k - i]); },
+        [&]() {
+          level(0, 0, bottom, 0., 0., false);
+          level(1, 0, next, off, zc0[nz - 1], true);
+          if constexpr (C) cp1 = row_first(c0, c1, next.p);
+          store(0, 0, 0, per_dz(a1) - f16 * abot * dz, per_dz(b1) - f16 * bbot * dz);
+        });
+    if constexpr (!SPLIT) load_end();
     // the top level's c' is that of the first step: no coupling with a zero value
-    rows(nz - 1, 0, load(nz - 1, 0, 0, 0, nz - 2), 0., zc0[1]);
-    cp1 = row_last(c0, c1, cp1, piv(1, nz - 1, 0));
+    rows(nz - 1, 0, top, 0., zc0[1]);
+    if constexpr (C) cp1 = row_last(c0, c1, cp1, end);
     store(nz - 1, 0, nz - 1, -per_dz(a0) + f16 * atop * dz - f13 * zap,
           -per_dz(b0) + f16 * btop * dz - f13 * zbp);
+  };
+  if constexpr (SPLIT) {
+    if (role == 0) up(yes, no, no, no);
+    if (role == 1) up(no, yes, no, no);
+    if (role == 2) up(no, no, yes, no);
+    if (role == 3) up(no, no, no, yes);
+    __syncthreads();
+  } else {
+    up(yes, yes, yes, yes);
   }
 
   // ---- down: c, dz(a), dz(b) solved; u and v (vort2vel.F90:251-320) ----
-  {
+  auto last = [&](auto do_u, auto do_v) {
+    constexpr bool U = decltype(do_u)::value, V = decltype(do_v)::value;
     struct T { S c, a, b; double cp; };
     double cn = 0., zan = 0., zbn = 0.;
     auto level = [&](int k, int i, const T &t, double cf, double zc, bool sub) {
       cn = sub ? (double)t.c - cp_of(cf, t.cp) * cn : (double)t.c;
-      zan = sub ? (double)t.a - zc * zan : (double)t.a;
-      zbn = sub ? (double)t.b - zc * zbn : (double)t.b;
       const S cs = (S)cn;
+      if constexpr (V) zan = sub ? (double)t.a - zc * zan : (double)t.a;
+      if constexpr (U) zbn = sub ? (double)t.b - zc * zbn : (double)t.b;
       const double u = (double)(S)zbn - other_y(cs) * ky;
       const double v = other_x(cs) * kx - (double)(S)zan;
       if (FIRST && lane == 0) return;
-      put(ca.u, k, i, u);
-      put(ca.v, k, i, v);
-      put_filtered(ca.us, k, i, (S)u);
-      put_filtered(ca.vs, k, i, (S)v);
+      if constexpr (U) {
+        put(ca.u, k, i, u);
+        put_filtered(ca.us, k, i, (S)u);
+      }
+      if constexpr (V) {
+        put(ca.v, k, i, v);
+        put_filtered(ca.vs, k, i, (S)v);
+      }
     };
     auto load = [&](int k, int i) {
-      return T{get(ca.c, k, i), get(ca.a, k, i), get(ca.b, k, i), back(1, k, i)};
+      T t{get(ca.c, k, i), (S)0, (S)0, back(1, k, i)};
+      if constexpr (V) t.a = get(za, k, i);
+      if constexpr (U) t.b = get(zb, k, i);
+      return t;
     };
     const T top = load(nz - 1, 0);
-    level(nz - 1, 0, top, 0., 0., false);
-    sweep<T>(1, nz - 1,
+    T bottom{};
+    if constexpr (SPLIT) bottom = load(0, 0);
+    sweep<T, SPLIT>(1, nz - 1,
         [&](int s, int i) { return load(nz - s - LV, LV - 1 - i); },
         [&](int s, int i, const T &t) {
           level(nz - s - LV, LV - 1 - i, t, off, zc1[nz - s - i], true);
-        });
-    level(0, 0, load(0, 0), cend, zc1[1], true);
+        },
+        [&]() { level(nz - 1, 0, top, 0., 0., false); });
+    if constexpr (!SPLIT) bottom = load(0, 0);
+    level(0, 0, bottom, cend, zc1[1], true);
+  };
+  if constexpr (SPLIT) {
+    if (role == 0) last(yes, no);
+    if (role == 1) last(no, yes);
+  } else {
+    last(yes, yes);
   }
 }
 
-template <typename S>
-__global__ void __launch_bounds__(64) k_vort2vel_columns(Geometry g, ColumnArrays<S> ca,
-                                                         DevScalars *sc) {
+template <typename S, bool SPLIT>
+__global__ void __launch_bounds__(SPLIT ? 256 : 64) k_vort2vel_columns(Geometry g,
+                                                                       ColumnArrays<S> ca,
+                                                                       DevScalars *sc) {
+  extern __shared__ double columns_lds[];
   const int ntile = spec_tiles(g);
   if ((int)blockIdx.x == ntile) {
     if (threadIdx.x == 0 && *ca.bad) raise_status(sc, PMPIC_ERR_ZERO_PIVOT);
-    mean_flow(g, ca);
+    if (threadIdx.x < 64) mean_flow(g, ca);
     return;
   }
-  const int nl = g.sx / 2, blk = min((int)blockIdx.x * 16 + ((int)threadIdx.x >> 2),
+  const int nl = g.sx / 2, blk = min((int)blockIdx.x * 16 + ((int)(threadIdx.x & 63) >> 2),
                                      nl * (g.sy / 2) - 1);
   const bool kept = ca.filt[(int64_t)(2 * (blk / nl)) * g.sx + 2 * (blk % nl)] != 0.;
-  if (blockIdx.x == 0) columns<true, true, S>(g, ca);
-  else if (__any(kept)) columns<true, false, S>(g, ca);
-  else columns<false, false, S>(g, ca);
+  if (blockIdx.x == 0) columns<true, true, SPLIT, S>(g, ca, columns_lds);
+  else if (__any(kept)) columns<true, false, SPLIT, S>(g, ca, columns_lds);
+  else columns<false, false, SPLIT, S>(g, ca, columns_lds);
 }
 
 }  // namespace
@@ -491,6 +646,11 @@ int columns_setup(Ctx *c) {
   return PMPIC_OK;
 }
 
+// Four wavefronts a tile while there are at most as many tiles as CUs: above, one wavefront a SIMD
+// fills the chip and shares no work (a step of 128x128x96 FP64, 265 tiles: 6.67 ms split, 6.65 not;
+// 96x96x64, 150 tiles: 2.72, 2.77).
+constexpr int SPLIT_TILES = 256;
+
 template <typename S>
 int vort2vel_columns(Ctx *c) {
   const Geometry &g = c->g;
@@ -500,8 +660,15 @@ int vort2vel_columns(Ctx *c) {
                            sp(c->sv), sp(c->sw), c->kx, c->ky, c->k2, c->filt, c->lap_rcp,
                            c->lap_den, c->lap_cp, c->dz_rcp, c->dz_den, c->dz_cp, c->ubar, c->vbar,
                            c->lap_bad};
-  hipLaunchKernelGGL(k_vort2vel_columns<S>, dim3(spec_tiles(g) + 1), dim3(64), 0, c->stream, g,
-                     ca, c->dsc);
+  const int tiles = spec_tiles(g);
+  // the divergence of a tile's levels, with those the sweep reads past the last
+  const size_t lds = sizeof(double) * 64 * (g.nzn + 2 * LV);
+  if (tiles <= SPLIT_TILES && lds <= 64 * 1024)
+    hipLaunchKernelGGL((k_vort2vel_columns<S, true>), dim3(tiles + 1), dim3(256), lds, c->stream, g,
+                       ca, c->dsc);
+  else
+    hipLaunchKernelGGL((k_vort2vel_columns<S, false>), dim3(tiles + 1), dim3(64), 0, c->stream, g,
+                       ca, c->dsc);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }

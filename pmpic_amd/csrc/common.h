@@ -188,7 +188,7 @@ struct Ctx {
   // spectral, in tiles (the standalone operators use the sder arrays as planes)
   double *sa, *sb, *sc, *sd, *se, *sf, *su, *sv, *sw, *sbs;
   double *sder[6];
-  double *spool;                      // holds sa, sb, sc and sder[0] (COLUMN_PAD)
+  double *spool;                      // holds sa, sb, sc, sder[0], sf, su, sv (COLUMN_PAD)
   double *abot, *atop;                // [sy][sx], standalone diffz's boundary planes
   double *ubar, *vbar;                // [nzn]
   double *kx, *ky, *k2, *filt;        // [sy][sx]

@@ -200,3 +200,19 @@ def test_plane_transforms(nx, ny):
     back = g.fft_backward(got)[2:-2, 2:-2]
     assert np.abs(back - field[2:-2, 2:-2]).max() <= 1e-13 * np.abs(field).max()
     g.close()
+
+
+@pytest.mark.parametrize("shape", [(8, 6, 111), (8, 6, 112), (120, 128, 3), (128, 128, 3)])
+def test_column_kernel_split(oracle_mod, shape, bar):
+    """Either side of the four-wavefront form's rule: 112 and 113 levels, 248 and 265 tiles."""
+    ic = thermal_case(*shape, 1, vort=1.0)
+    o, g = _pair(oracle_mod, shape, ic)
+    _, f = _pair(oracle_mod, shape, ic, precision=1)
+    for c in (o, g, f):
+        c.step()
+    for k in ("u", "v", "w", "p", "q", "r"):
+        want = o.grid(k)[2:-2, 2:-2]
+        bar(k, rel_err(g.grid(k)[2:-2, 2:-2], want), 1e-12)
+        bar(k + "32", rel_err(f.grid(k)[2:-2, 2:-2], want), 1e-5)
+    g.close()
+    f.close()
