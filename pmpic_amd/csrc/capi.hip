@@ -250,9 +250,10 @@ int create(const pmpic_config *cf, Ctx *c) {
   const int64_t big = c->cap > c->ncell ? c->cap : c->ncell;
   if (c->precision == 1) PMPIC_TRY(b32_alloc(c));
   else PMPIC_TRY(dalloc(&c->par, (int64_t)NFIELDS * c->cap));
-  PMPIC_TRY(dalloc(&c->cell, c->cap));
-  PMPIC_TRY(dalloc(&c->rank, c->cap));
-  PMPIC_TRY(dalloc(&c->sorted, big));
+  if (c->precision == 0) PMPIC_TRY(dalloc(&c->cell, c->cap));
+  const int64_t room = c->precision == 1 ? c->b32.room : c->cap;
+  PMPIC_TRY(dalloc(&c->rank, room));
+  PMPIC_TRY(dalloc(&c->sorted, room > big ? room : big));
   PMPIC_TRY(dalloc(&c->flag, c->cap));
   PMPIC_TRY(dalloc(&c->list_a, c->cap));
   PMPIC_TRY(dalloc(&c->list_b, c->cap));
@@ -628,7 +629,7 @@ static int graph_capture(pmpic_ctx *ctx, int capc) {
   c->g123x = x;
   c->g123_n = bound;
   c->g123_capc = capc;
-  c->g123_prebinned = c->b32.prebinned;
+  c->g123_binned = c->b32.binned;
   c->g123_captures++;
   return PMPIC_OK;
 }
@@ -657,11 +658,11 @@ static int graph_stages123(pmpic_ctx *ctx) {
     c->b32.kept_pending[1] = c->b32.kept_pending[3] = false;
     c->b32.kept_pending[4] = c->b32.kept_pending[5] = false;
     for (int i = 0; i < 4; i++) c->b32.p2g_pending[i] = true;
-    c->b32.prebinned = c->g123_prebinned;
-    c->b32.counts_zero = !c->g123_prebinned;
-    c->b32.cur = 1;
+    c->b32.binned = c->g123_binned;
+    c->b32.counts_zero = !c->g123_binned;
+    c->b32.binned_set = c->b32.cur = 1;
+    c->b32.binned_n = c->n;
     c->b32.p2g_reuse = false;  // consumed by stage 1's par2grid, as the eager call does
-    if (c->b32.prebinned) c->b32.capc = capc;
   }
   PMPIC_CHECK(hipGraphLaunch(c->g123x, c->stream));
   c->g123_replays++;

@@ -65,7 +65,9 @@ struct Bulk32 {
   // entries per cell (none, and capc = 0, when its byte offsets would exceed 32 bits); each
   // binning uses capc = 16 or 32 of them by the mean parcels per cell.
   int32_t *slot;
-  int2 *ovf;         // cap: (parcel, rank) of the parcels past the slot capacity
+  int2 *ovf;         // (parcel, rank) of the parcels past the slot capacity
+  int32_t *ovfc;     // ... and their cells
+  int64_t room;      // entries of ovf, and of Ctx::sorted and rank: cap, or twice that (moving)
   int capc;          // capacity of the current binning (0, 16 or 32)
   int capmax;        // entries per cell allocated (0 or 32)
   int capfix;        // capacity forced by PMPIC_SLOT_CAPACITY (16 or 32), or 0 for the mean rule
@@ -81,10 +83,15 @@ struct Bulk32 {
   float *pgrid[4];
   bool p2g_pending[4];
   // RK stages 1-3 bin the cells they write for the next par2grid (fused_bin: grids of 2^21
-  // cells or more, or as PMPIC_FUSED_BINNING says); prebinned: the cell lists of the current
-  // cells are built
+  // cells or more, or as PMPIC_FUSED_BINNING says)
   bool fused_bin;
-  bool prebinned;
+  // The lists built last still stand (`binned`): for the cells of set binned_set, binned_n parcels
+  // and the capacity capc.  moving: stages 2 and 4, which hardly move a parcel out of the cell that
+  // the stage before put it in, and splitting move the few entries that change instead of
+  // building the lists again (room for the entries that can come: up to 2^27 parcels).
+  bool binned, moving;
+  int binned_set;
+  int64_t binned_n;
   bool counts_zero;   // the cell counts are zero, as a binning wants them
   // the last mixing's kept sums are the next par2grid's partials except on the
   // tiles mixing changed (dirty: one byte per 8-cell tile); p2g_reuse while that holds (set by
@@ -228,7 +235,7 @@ struct Ctx {
   int graph_on;         // PMPIC_GRAPH=1 in the environment at creation
   int64_t eager_steps;  // steps run without the graph (the first sets up the scan storage)
   int64_t g123_captures, g123_replays;  // graphs captured and launched
-  bool g123_prebinned;                  // the binning state the captured stages leave
+  bool g123_binned;                     // the binning state the captured stages leave
   // HIP-event timing: 0 = par2grid cell accumulation kernel, 1 = gather + RK stage kernel,
   // 2..6 = the component callbacks (timer regions named as the reference's timers)
   int timing;

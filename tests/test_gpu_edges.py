@@ -216,3 +216,45 @@ def test_column_kernel_split(oracle_mod, shape, bar):
         bar(k + "32", rel_err(f.grid(k)[2:-2, 2:-2], want), 1e-5)
     g.close()
     f.close()
+
+
+@pytest.mark.parametrize("case,shape", [("8ppc", (32, 16, 8)), ("27ppc", (18, 12, 8)),
+                                        ("crowded", (18, 12, 8))])
+@pytest.mark.parametrize("fused", ["0", "1"])
+@pytest.mark.parametrize("mixing", [True, False])
+def test_moved_entries_change_no_result(monkeypatch, case, shape, fused, mixing):
+    """Lists whose entries stages 2 and 4, splitting and mixing move (16 and 32 slots) against lists
+    built again each time (no slot table): strong random vorticity and the largest timestep that the
+    limits allow, so that many parcels change cell, split and are mixed.  Every list is summed in
+    parcel order, so the runs stay bit-identical."""
+    from pmpic_amd.lib import Context
+    from tests.cases import crowded_case
+    ic = (crowded_case(*shape) if case == "crowded" else
+          thermal_case(*shape, 3 if case == "27ppc" else 2, vort=30.0, shrink=0.05, thin=0.1,
+                       near_split=0.05))
+    if case == "crowded":
+        for k in "pqr":
+            ic[k] = 30.0 * ic[k]
+    monkeypatch.setenv("PMPIC_FUSED_BINNING", fused)
+    b = box(*shape)
+    runs = {}
+    for slots in ("0", "16", "32"):
+        monkeypatch.setenv("PMPIC_SLOT_CAPACITY", slots)
+        g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                    4 * len(ic["x"]), dtm=1.0, dtmax=1.0, mixing=mixing, precision=1)
+        g.set_parcels(ic)
+        runs[slots] = g
+    for s in range(4):
+        for g in runs.values():
+            g.step()
+        want = runs["0"].get_parcels()
+        for slots in ("16", "32"):
+            g = runs[slots]
+            assert (g.n, g.last_counts()) == (runs["0"].n, runs["0"].last_counts()), (slots, s)
+            got = g.get_parcels()
+            for k in want:
+                np.testing.assert_array_equal(got[k], want[k], err_msg=f"{slots} step {s}: {k}")
+            for k in ("u", "v", "w", "p", "q", "r", "b"):
+                np.testing.assert_array_equal(g.grid(k), runs["0"].grid(k), err_msg=f"{slots} {s}: {k}")
+    for g in runs.values():
+        g.close()
