@@ -1366,6 +1366,15 @@ static Column column(const Bulk32 &b, int f) {
   return {b.stretch, 1};
 }
 
+static int put_field(Ctx *c, double *dev, const double *host, int64_t n) {
+  const HostPart p{const_cast<double *>(host), dev, sizeof(double) * (size_t)n};
+  return copy_host(c, &p, 1, false);
+}
+static int get_field(Ctx *c, double *host, double *dev, int64_t n) {
+  const HostPart p{host, dev, sizeof(double) * (size_t)n};
+  return copy_host(c, &p, 1, true);
+}
+
 int b32_set_parcels(Ctx *c, int64_t n, const double *const *fields) {
   PMPIC_TRY(ensure_fbuf(c));
   Bulk32 &b = c->b32;
@@ -1374,23 +1383,20 @@ int b32_set_parcels(Ctx *c, int64_t n, const double *const *fields) {
   const dim3 gb(cdiv(n > 0 ? n : 1, TPB)), tb(TPB);
   for (int a = 0; a < 3; a++) {
     if (n > 0) {
-      PMPIC_CHECK(hipMemcpyAsync(c->fbuf, fields[a], sizeof(double) * n, hipMemcpyHostToDevice,
-                                 c->stream));
+      PMPIC_TRY(put_field(c, c->fbuf, fields[a], n));
       hipLaunchKernelGGL(k32_pos_in, gb, tb, 0, c->stream, c->g, a, c->fbuf, n, b.cell[b.cur],
                          b.off[b.cur], c->dsc);
     }
   }
   for (int f = FP; f <= FSTRETCH; f++) {
     if (n > 0) {
-      PMPIC_CHECK(hipMemcpyAsync(c->fbuf, fields[f], sizeof(double) * n, hipMemcpyHostToDevice,
-                                 c->stream));
+      PMPIC_TRY(put_field(c, c->fbuf, fields[f], n));
       const Column col = column(b, f);
       hipLaunchKernelGGL(k32_from_f64, gb, tb, 0, c->stream, c->fbuf, n, col.p, col.stride);
     }
   }
   if (n > 0)
-    PMPIC_CHECK(hipMemcpyAsync(b.tag, fields[FTAG], sizeof(double) * n, hipMemcpyHostToDevice,
-                               c->stream));
+    PMPIC_TRY(put_field(c, b.tag, fields[FTAG], n));
   PMPIC_CHECK(hipGetLastError());
   PMPIC_CHECK(hipStreamSynchronize(c->stream));
   return PMPIC_OK;
@@ -1405,8 +1411,7 @@ int b32_get_parcels(Ctx *c, double *const *fields) {
   for (int f = 0; f < 17; f++) {
     if (!fields[f]) continue;
     if (f == FTAG) {
-      PMPIC_CHECK(hipMemcpyAsync(fields[f], b.tag, sizeof(double) * n, hipMemcpyDeviceToHost,
-                                 c->stream));
+      PMPIC_TRY(get_field(c, fields[f], b.tag, n));
       continue;
     }
     if (f < 3)
@@ -1416,8 +1421,7 @@ int b32_get_parcels(Ctx *c, double *const *fields) {
       const Column col = column(b, f);
       hipLaunchKernelGGL(k32_to_f64, gb, tb, 0, c->stream, col.p, col.stride, n, c->fbuf);
     }
-    PMPIC_CHECK(hipMemcpyAsync(fields[f], c->fbuf, sizeof(double) * n, hipMemcpyDeviceToHost,
-                               c->stream));
+    PMPIC_TRY(get_field(c, fields[f], c->fbuf, n));
   }
   PMPIC_CHECK(hipGetLastError());
   PMPIC_CHECK(hipStreamSynchronize(c->stream));

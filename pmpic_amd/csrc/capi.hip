@@ -131,18 +131,14 @@ void col_to_device_layout(const Geometry &g, const double *ref, std::vector<doub
     for (int ii = 0; ii < g.sx; ii++) dev[(size_t)jj * g.sx + ii] = ref[(size_t)ii * g.sy + jj];
 }
 
-// host array -> device (in stream order; the caller's stream synchronisation ends its use)
+// host array -> device, in stream order
 int put_host(Ctx *c, double *dst, const double *host, int64_t n) {
-  PMPIC_CHECK(hipMemcpyAsync(dst, host, sizeof(double) * (size_t)n, hipMemcpyHostToDevice,
-                             c->stream));
-  return PMPIC_OK;
+  const HostPart p{const_cast<double *>(host), dst, sizeof(double) * (size_t)n};
+  return copy_host(c, &p, 1, false);
 }
-// device -> host array, complete on return
 int get_host(Ctx *c, double *host, const double *src, int64_t n) {
-  PMPIC_CHECK(hipMemcpyAsync(host, src, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost,
-                             c->stream));
-  PMPIC_CHECK(hipStreamSynchronize(c->stream));
-  return PMPIC_OK;
+  const HostPart p{host, const_cast<double *>(src), sizeof(double) * (size_t)n};
+  return copy_host(c, &p, 1, true);
 }
 int64_t ref_grid_size(const Geometry &g) { return (int64_t)g.nzn * (g.ny + 4) * (g.nx + 4); }
 
@@ -201,6 +197,7 @@ int free_all(Ctx *c) {
   hipFree(c->lpool); hipFree(c->lap_bad);
   hipFree(c->fbuf);
   hipFree(c->cbuf); hipFree(c->tw_x); hipFree(c->tw_y); hipFree(c->tw_x32); hipFree(c->tw_y32);
+  free_host_slots(c);
   hipFree(c->scan_tmp); hipFree(c->blk); hipFree(c->maxblk); hipFree(c->dsc);
   for (int w = 0; w < NTIMERS; w++)
     for (int e = 0; e < 64; e++) {
@@ -433,11 +430,10 @@ int pmpic_set_parcels(pmpic_ctx *ctx, int64_t n, const double *const *fields) {
     PMPIC_TRY(b32_publish_n(c));
     return take_status(c);
   }
-  for (int f = 0; f < 17; f++) {
-    if (n > 0)
-      PMPIC_CHECK(hipMemcpyAsync(c->par + (int64_t)f * c->cap, fields[f], sizeof(double) * n,
-                                 hipMemcpyHostToDevice, c->stream));
-  }
+  HostPart part[17];
+  for (int f = 0; f < 17; f++)
+    part[f] = {const_cast<double *>(fields[f]), c->par + (int64_t)f * c->cap, sizeof(double) * (size_t)n};
+  PMPIC_TRY(copy_host(c, part, 17, false));
   PMPIC_CHECK(hipStreamSynchronize(c->stream));
   c->n = n;
   return PMPIC_OK;
@@ -448,11 +444,13 @@ int pmpic_get_parcels(pmpic_ctx *ctx, int64_t *n, double *const *fields) {
   Ctx *c = &ctx->c;
   if (n) *n = c->n;
   if (fields && c->precision == 1) return b32_get_parcels(c, fields);
+  HostPart part[17];
+  int parts = 0;
   if (fields)
     for (int f = 0; f < 17; f++)
-      if (fields[f] && c->n > 0)
-        PMPIC_CHECK(hipMemcpyAsync(fields[f], c->par + (int64_t)f * c->cap, sizeof(double) * c->n,
-                                   hipMemcpyDeviceToHost, c->stream));
+      if (fields[f])
+        part[parts++] = {fields[f], c->par + (int64_t)f * c->cap, sizeof(double) * (size_t)c->n};
+  PMPIC_TRY(copy_host(c, part, parts, true));
   PMPIC_CHECK(hipStreamSynchronize(c->stream));
   return PMPIC_OK;
 }

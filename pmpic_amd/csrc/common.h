@@ -146,6 +146,8 @@ __host__ __device__ inline int64_t spec_at(int nzn, int nl, int k, int m, int l)
 
 enum TimerId { T_ACCUM = 0, T_RK = 1, T_VORT2VEL, T_VORT_TEND, T_RK4, T_SPLIT, T_MIX, NTIMERS };
 
+constexpr int HOST_SLOTS = 8;  // pinned slots of the large host copies (copy_host)
+
 struct Ctx {
   Geometry g;
   int64_t cap;
@@ -223,6 +225,8 @@ struct Ctx {
   DevScalars hsc;                     // host mirror
   void *pin;                          // pinned host staging for small read-backs (256 B)
   hipEvent_t sync_ev;                 // read-back completion (spin wait)
+  char *hc_pin;                       // copy_host's slots, allocated at its first large copy
+  hipEvent_t hc_ev[HOST_SLOTS];
   // FP32-bulk form with PMPIC_GRAPH=1: RK stages 1-3 of a step (vort2vel, vorticity_tendency,
   // rk4_integrator; the splitting and mixing callbacks do nothing there) captured once as a HIP
   // graph and replayed by later steps; the stage-4 work, whose launches depend on data read
@@ -391,6 +395,15 @@ int fft_backward(Ctx *c, int nf, const double *const *src, double *const *dst,
 // the same transforms with spectral arrays (and the transforms' arithmetic) of type S; the
 // forward transform reads physical grids of type S, the inverse writes dst (FP64) and dst32
 // (FP32), either of which may be NULL
+// Copies between the caller's arrays and the device, on the context's stream.  To the host: complete
+// on return; from it: the caller's arrays may change on return, and the work queued next sees the
+// data.
+struct HostPart {
+  void *host, *dev;
+  size_t bytes;
+};
+int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host);
+void free_host_slots(Ctx *c);
 template <typename S>
 int fft_forward_t(Ctx *c, int nf, const S *const *src, S *const *dst);
 template <typename S>

@@ -258,3 +258,31 @@ def test_moved_entries_change_no_result(monkeypatch, case, shape, fused, mixing)
                 np.testing.assert_array_equal(g.grid(k), runs["0"].grid(k), err_msg=f"{slots} {s}: {k}")
     for g in runs.values():
         g.close()
+
+
+@pytest.mark.parametrize("n", [123_361, 123_362, 131_072, 131_073, 400_001])
+def test_large_host_copies(n):
+    """Parcel arrays to the device and back either side of the size from which several threads
+    carry them (16 MB in 17 arrays), with whole and odd last chunks of 1 MB, from two contexts at a
+    time: every value comes back as it went."""
+    import threading
+    from pmpic_amd.lib import PARCEL_FIELDS, Context
+    b = box(8, 6, 5)
+
+    def round_trip(seed, out):
+        rng = np.random.default_rng(seed)
+        ic = {k: rng.standard_normal(n) for k in PARCEL_FIELDS}
+        g = Context(8, 6, 5, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"], n)
+        for _ in range(2):
+            g.set_parcels(ic)
+            got = g.get_parcels()
+        g.close()
+        out.append(all(np.array_equal(got[k], ic[k]) for k in PARCEL_FIELDS))
+
+    out = []
+    th = [threading.Thread(target=round_trip, args=(s, out)) for s in (n, n + 1)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert out == [True, True]
