@@ -223,6 +223,13 @@ __global__ void k32_to_f64(const float *__restrict__ a, int stride, int64_t n,
   if (p < n) b[p] = (double)a[p * stride];
 }
 
+// ---- tiles of eight cells of an x row ----
+__host__ __device__ inline int tiles_x(const Geometry &g) { return (g.nx + 7) / 8; }
+// tile of cell (i, j, k)
+__device__ __forceinline__ int64_t tile_of(const Geometry &g, int i, int j, int k) {
+  return ((int64_t)k * g.ny + j) * tiles_x(g) + (i >> 3);
+}
+
 // ---- cell binning ----
 // A wavefront walks BIN_SEQ consecutive groups of 64 parcels in order and takes one atomic per
 // run of equal cells, so a cell whose parcels are consecutive in slot order gets its ranks in
@@ -238,6 +245,7 @@ constexpr int BIN_SEQ = 16;
 constexpr int CAPC = 32;      // slot entries per cell of the table, and the full capacity
 constexpr int CAPC_LOW = 16;
 constexpr int LOW_PPC = 10;
+constexpr int MIX_MOVES = 16;  // mixing's changes that the lists follow: up to 1 in so many parcels
 
 __global__ void k32_bin_reset(int32_t *__restrict__ count, int64_t nc1, DevScalars *dsc) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -249,7 +257,8 @@ __global__ void k32_bin_reset(int32_t *__restrict__ count, int64_t nc1, DevScala
 // k32_dense_scatter lays all cells out densely after the scan
 __global__ void k32_bin_slot(Geometry g, const int32_t *__restrict__ cellv, int64_t n, int capc,
                              int32_t *__restrict__ slot, int2 *__restrict__ ovf,
-                             int32_t *__restrict__ ovfc, int32_t *__restrict__ rankv, int32_t *__restrict__ count,
+                             int32_t *__restrict__ ovfc, int32_t *__restrict__ where,
+                             int32_t *__restrict__ rankv, int32_t *__restrict__ count,
                              DevScalars *dsc) {
   // parcel indices fit 32 bits (capacity < 2^30)
   const int lane = threadIdx.x & 63;
@@ -319,16 +328,16 @@ __global__ void k32_bin_slot(Geometry g, const int32_t *__restrict__ cellv, int6
         const int32_t o = ob + __popcll(om & ((1ull << lane) - 1ull));
         ovf[o] = make_int2(p, rk);
         ovfc[o] = ch[it] >> 6;
+        if (where) where[p] = o;
       }
     }
   }
 }
 
 // the overflow list into the dense region; the parcel of rank capc also copies its cell's
-// capc slot entries there, so the region holds ranks 0 .. count-1.  A parcel that has left the cell
-// since leaves a hole (-1).
-__global__ void k32_ovf_scatter(Geometry g, const int32_t *__restrict__ cellv,
-                                const int2 *__restrict__ ovf, const int32_t *__restrict__ ovfc,
+// capc slot entries there, so the region holds ranks 0 .. count-1.  Entries that have left
+// are holes (-1).
+__global__ void k32_ovf_scatter(const int2 *__restrict__ ovf, const int32_t *__restrict__ ovfc,
                                 const DevScalars *dsc, const int32_t *__restrict__ ostart,
                                 const int32_t *__restrict__ slot, int capc,
                                 int32_t *__restrict__ sorted) {
@@ -338,7 +347,7 @@ __global__ void k32_ovf_scatter(Geometry g, const int32_t *__restrict__ cellv,
     const int2 e = ovf[i];
     const int32_t c = ovfc[i];
     const int32_t b0 = ostart[c];
-    sorted[b0 + e.y] = linear_cell(g, cellv[e.x]) == c ? e.x : -1;
+    sorted[b0 + e.y] = e.x;
     if (e.y == capc)
       for (int r = 0; r < capc; r++) sorted[b0 + r] = slot[c * capc + r];
   }
@@ -352,34 +361,38 @@ struct BinOut {
   int32_t *slot;         // [cell * capc + rank]
   int2 *ovf;             // (parcel, rank) past the capacity; their number in DevScalars::novf
   int32_t *ovfc;         // ... their cells
+  int32_t *where;        // ... a parcel's entry there (may be null)
   int32_t *rank;         // per parcel, when capc = 0
 };
 
-// Parcel p's entry from cell `from` (linear; -1: it has none) to cell `to`.  Its old entry becomes a
-// hole (-1), which the accumulation leaves out; one in the overflow list is found out by its cell
-// when that list is scattered.  The first match is the entry: those past the count the lists were
-// built with may hold anything, but there are none below the capacity where the entry is not in the
-// table.  One move a parcel and binning, so no list can hold it twice.
-__device__ __forceinline__ void move_entry(int32_t p, int32_t from, int32_t to, const BinOut &bo,
-                                           DevScalars *sc) {
-  if (from >= 0) {
-    int32_t *row = bo.slot + (int64_t)from * bo.capc;
-    for (int r = 0; r < bo.capc; r += 4) {
-      const int4 e = *reinterpret_cast<const int4 *>(row + r);
-      const int at = e.x == p ? 0 : e.y == p ? 1 : e.z == p ? 2 : e.w == p ? 3 : -1;
-      if (at >= 0) {
-        row[r + at] = -1;
-        break;
-      }
+// Parcel p's entry in cell c's list becomes a hole (-1), which the accumulation leaves out.  rows:
+// the slot entries to search.  Where appends run meanwhile that is all of them, and p has an entry:
+// the first match is it, since entries past the count the list had before may hold anything, but
+// there are none below the capacity where p's entry is not in the table.
+__device__ __forceinline__ void remove_entry(int32_t p, int32_t c, int rows, const BinOut &bo,
+                                             const DevScalars *sc) {
+  int32_t *row = bo.slot + (int64_t)c * bo.capc;
+  for (int r = 0; r < rows; r += 4) {
+    const int4 e = *reinterpret_cast<const int4 *>(row + r);
+    const int at = e.x == p ? 0 : e.y == p ? 1 : e.z == p ? 2 : e.w == p ? 3 : -1;
+    if (at >= 0 && r + at < rows) {
+      row[r + at] = -1;
+      return;
     }
   }
-  const int32_t rk = atomicAdd(&bo.count[to], 1);
+  const int32_t o = bo.where[p];
+  if ((uint32_t)o < (uint32_t)sc->novf && bo.ovf[o].x == p) bo.ovf[o].x = -1;
+}
+__device__ __forceinline__ void append_entry(int32_t p, int32_t c, const BinOut &bo,
+                                             DevScalars *sc) {
+  const int32_t rk = atomicAdd(&bo.count[c], 1);
   if (rk < bo.capc) {
-    bo.slot[(int64_t)to * bo.capc + rk] = p;
+    bo.slot[(int64_t)c * bo.capc + rk] = p;
   } else {
     const int32_t o = atomicAdd(&sc->novf, 1);
     bo.ovf[o] = make_int2(p, rk);
-    bo.ovfc[o] = to;
+    bo.ovfc[o] = c;
+    bo.where[p] = o;
   }
 }
 
@@ -393,7 +406,29 @@ __global__ void k32_bin_move(Geometry g, const int32_t *__restrict__ was,
   if (p >= n) return;
   const int32_t from = p < n_old ? was[p] : -1, to = is[p];
   if (from == to) return;
-  move_entry((int32_t)p, p < n_old ? linear_cell(g, from) : -1, linear_cell(g, to), bo, sc);
+  if (p < n_old) remove_entry((int32_t)p, linear_cell(g, from), bo.capc, bo, sc);
+  append_entry((int32_t)p, linear_cell(g, to), bo, sc);
+}
+
+// Parcels that leave the lists (bo.on) and the sums (dirty, may be null: their tiles): the n listed
+// ones, or without a list those from `base` on.  Nothing is appended meanwhile, so a cell's list
+// ends at its count, and a parcel without an entry finds none.
+__global__ void k32_unlist(Geometry g, const int32_t *__restrict__ cellv,
+                           const int32_t *__restrict__ list, int64_t base, int64_t n, BinOut bo,
+                           uint8_t *__restrict__ dirty, DevScalars *sc) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int32_t p = list ? list[t] : (int32_t)(base + t), cell = cellv[p];
+  if (dirty) {
+    int i, j, k;
+    cell_ijk(g, cell, i, j, k);
+    dirty[tile_of(g, i, j, k)] = 1;
+    if (t == 0) sc->anydirty = 1;
+  }
+  if (bo.on) {
+    const int32_t c = linear_cell(g, cell);
+    remove_entry(p, c, min(bo.count[c], bo.capc), bo, sc);
+  }
 }
 
 // without a slot table: parcel p at its cell's dense offset plus its rank
@@ -420,7 +455,7 @@ __global__ void k32_dense_scatter(Geometry g, const int32_t *__restrict__ cellv,
 // Within a cell the additions run in ascending parcel order, so the sums do not depend on the
 // order in which the binning's atomics came: the lanes check their adjacent entries and rank them
 // where a pair is not ascending (in LDS up to LIST entries a cell, else in memory).  Holes (-1:
-// move_entry) are left out there too.
+// remove_entry) are left out there too.
 //
 // A cell of up to capc parcels lists them in the slot table, whose first 16 entries are loaded
 // before the count is known; the others in the dense region.
@@ -464,12 +499,6 @@ __device__ __forceinline__ void add_parcel(float *acc, float w, const float *v) 
   acc[0] += w;
 #pragma unroll
   for (int f = 0; f < NV; f++) acc[f + 1] = fmaf(w, v[f], acc[f + 1]);
-}
-
-__host__ __device__ inline int tiles_x(const Geometry &g) { return (g.nx + 7) / 8; }
-// tile of cell (i, j, k)
-__device__ __forceinline__ int64_t tile_of(const Geometry &g, int i, int j, int k) {
-  return ((int64_t)k * g.ny + j) * tiles_x(g) + (i >> 3);
 }
 
 // The lanes' W entries 8 i + q of eight lists of up to nmax entries (key e of list cl at
@@ -742,6 +771,7 @@ __device__ __forceinline__ void bin_lane(const Geometry &g, int32_t cell, uint32
       const int32_t o = ob + __popcll(om & ((1ull << lane) - 1ull));
       bo.ovf[o] = make_int2((int32_t)p, rk);
       bo.ovfc[o] = c;
+      if (bo.where) bo.where[p] = o;
     }
   }
 }
@@ -877,8 +907,10 @@ __global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, RkSets
   const int32_t was = STAGE == 2 && bo.on ? rs.cell[p] : -1;  // (the stage updates it in place)
   const int32_t nc = rk_update<STAGE>(g, b, rs, rec, sc3, stretch, split_flag, sc, p);
   // with bo.on = 2, the entries of the parcels that change cell move
-  if (STAGE == 2 && bo.on && nc >= 0 && nc != was)
-    move_entry((int32_t)p, linear_cell(g, was), linear_cell(g, nc), bo, sc);
+  if (STAGE == 2 && bo.on && nc >= 0 && nc != was) {
+    remove_entry((int32_t)p, linear_cell(g, was), bo.capc, bo, sc);
+    append_entry((int32_t)p, linear_cell(g, nc), bo, sc);
+  }
 }
 
 // ---- splitting (parcel_splitting.F90:76-131, then the haloswap's wrap and reflection) ----
@@ -937,7 +969,8 @@ __global__ void k32_mix_new(Geometry g, Parcels32 P, int64_t cap, int64_t norig,
                             const int32_t *__restrict__ newcells, int64_t nadd,
                             const int32_t *__restrict__ zlist, int64_t nz_,
                             uint8_t *__restrict__ keep, Mix32 mg, float vmin,
-                            float *__restrict__ portion_cell, DevScalars *sc) {
+                            float *__restrict__ portion_cell, uint8_t *__restrict__ dirty,
+                            DevScalars *sc) {
   const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= nadd) return;
   const int64_t ord = newcells[m];
@@ -970,13 +1003,28 @@ __global__ void k32_mix_new(Geometry g, Parcels32 P, int64_t cap, int64_t norig,
   st3(P.vbh, s, 2 * vmin, s6[1] / v, s6[2] / v);
   P.stretch[s] = 0.f;
   if (s + 1 < norig) keep[s] = 2;
-  portion_cell[((int64_t)k * g.ny + j) * g.nx + i] = 2 * vmin / v;
+  const int32_t c = (k * g.ny + j) * g.nx + i;
+  portion_cell[c] = 2 * vmin / v;
+  if (dirty) {
+    dirty[tile_of(g, i, j, k)] = 1;
+    if (m == 0) sc->anydirty = 1;
+  }
 }
 
+// the new parcels into the lists (after the absorption, which reads the lists as they were scattered)
+__global__ void k32_list_new(Geometry g, const int32_t *__restrict__ cellv, int64_t norig,
+                             int64_t nadd, const int32_t *__restrict__ zlist, int64_t nz_, BinOut bo,
+                             DevScalars *sc) {
+  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= nadd) return;
+  const int32_t s = m < nz_ ? zlist[m] : (int32_t)(norig + (m - nz_));
+  append_entry(s, linear_cell(g, cellv[s]), bo, sc);
+}
+
+// ... and marks the cells around a node with a residual
 __global__ void k32_mix_residual(Geometry g, Mix32 mg, const int32_t *__restrict__ npercell,
                                  const float *__restrict__ portion_cell,
-                                 uint8_t *__restrict__ touch, uint8_t *__restrict__ dirty,
-                                 DevScalars *sc) {
+                                 uint8_t *__restrict__ ctouch) {
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nnode) return;
@@ -1011,36 +1059,12 @@ __global__ void k32_mix_residual(Geometry g, Mix32 mg, const int32_t *__restrict
     mg.R[f][t] = v;
     any = any || v != 0.f;  // a NaN counts as not zero
   }
-  touch[t] = any ? 1 : 0;
-  if (any && dirty) {
-    // the parcels of the eight cells around the node absorb: their tiles are summed again
-    for (int kc = k - 1; kc <= k; kc++) {
-      if (kc < 0 || kc >= g.ncz) continue;
-      for (int bb = 0; bb < 2; bb++)
-        for (int a = 0; a < 2; a++) dirty[tile_of(g, ci[a], cj[bb], kc)] = 1;
-    }
-    sc->anydirty = 1;
+  if (!any) return;
+  for (int kc = k - 1; kc <= k; kc++) {
+    if (kc < 0 || kc >= g.ncz) continue;
+    for (int bb = 0; bb < 2; bb++)
+      for (int a = 0; a < 2; a++) ctouch[((int64_t)kc * g.ny + cj[bb]) * g.nx + ci[a]] = 1;
   }
-}
-
-// dirty tiles: the tile of each listed parcel's cell (parcels != 0) or of each
-// listed new cell, given in the new-cell flags' order (z fastest, then y, then x)
-__global__ void k32_mark_tiles(Geometry g, const int32_t *__restrict__ cellv,
-                               const int32_t *__restrict__ list, int64_t n, int parcels,
-                               uint8_t *__restrict__ dirty, DevScalars *sc) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int32_t e = list[t];
-  int i, j, k;
-  if (parcels) {
-    cell_ijk(g, cellv[e], i, j, k);
-  } else {
-    k = (int)(e % g.ncz);
-    j = (int)((e / g.ncz) % g.ny);
-    i = (int)(e / ((int64_t)g.ncz * g.ny));
-  }
-  dirty[tile_of(g, i, j, k)] = 1;
-  if (t == 0) sc->anydirty = 1;
 }
 
 __global__ void k32_fill_u8(uint8_t *__restrict__ a, int64_t n, uint8_t v) {
@@ -1048,25 +1072,9 @@ __global__ void k32_fill_u8(uint8_t *__restrict__ a, int64_t n, uint8_t v) {
   if (t < n) a[t] = v;
 }
 
-// A parcel none of whose corner nodes carries a residual (almost all of them: residuals arise
-// only around removed parcels and the cells that received new ones) keeps its values as they
-// are, without the reads, the arithmetic (which would return them to within rounding) and the
-// writes; `touch` marks the nodes with a residual.
-__global__ void k32_mix_absorb(Geometry g, Parcels32 P, int64_t norig,
-                               const uint8_t *__restrict__ keep, Mix32 mg,
-                               const uint8_t *__restrict__ touch) {
-  const int64_t p64 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p64 >= norig || keep[p64] != 1) return;
-  const uint32_t p = (uint32_t)p64;
-  const int32_t cell = ldnt((const int32_t *)P.cell, p);
-  int i, j, k;
-  cell_ijk(g, cell, i, j, k);
-  int32_t o[8];
-  corner_nodes(g, i, j, k, o);
-  int any = 0;
-#pragma unroll
-  for (int c = 0; c < 8; c++) any |= touch[o[c]];
-  if (!any) return;
+// the absorption of parcel p in cell (i, j, k), corners at o
+__device__ __forceinline__ void absorb(const Parcels32 &P, int64_t p, const int32_t o[8],
+                                       const Mix32 &mg) {
   const Float3 off = ld3(P.off, p), vor = ld3(P.vor, p), vbh = ld3(P.vbh, p);
   const float ox = off.x, oy = off.y, oz = off.z, v = vbh.x;
   const float fv[5] = {vbh.y, vbh.z, vor.x, vor.y, vor.z};
@@ -1096,11 +1104,63 @@ __global__ void k32_mix_absorb(Geometry g, Parcels32 P, int64_t norig,
   st3(P.vor, p, out[2], out[3], out[4]);
 }
 
+// Kept parcels absorb the residuals (parcel_mixing.F90:247-340): those in the lists of the cells
+// that k32_mix_residual marked.  The parcels of the others (almost all: residuals arise only around
+// removed parcels and the cells that received new ones) keep their values, which the arithmetic
+// would return to within rounding, and are not read.  A wavefront looks at `per` tiles (up
+// to eight) and takes those with marked cells one after another, a cell's parcels eight at a time:
+// 67 M parcels in 8.4 M cells 0.40 ms from the parcels' flags and cells -> 0.15 ms.  zero: leaves
+// the counts at zero.
+__global__ void __launch_bounds__(64) k32_mix_absorb(
+    Geometry g, Parcels32 P, int64_t norig, const uint8_t *__restrict__ keep, Mix32 mg, int capc,
+    const int32_t *__restrict__ slot, int32_t *__restrict__ count,
+    const int32_t *__restrict__ start, const int32_t *__restrict__ sorted,
+    const uint8_t *__restrict__ ctouch, uint8_t *__restrict__ dirty, DevScalars *sc, int per,
+    int zero) {
+  const int lane = threadIdx.x, cl = lane & 7, q = lane >> 3;
+  const uint32_t ntx = (uint32_t)tiles_x(g), ntile = ntx * (uint32_t)(g.ny * g.ncz);
+  // a lane's cell among the wavefront's tiles
+  const uint32_t t0 = per * xcd_block(blockIdx.x, gridDim.x), own = t0 + q;
+  const uint32_t row = own / ntx;
+  const int x = 8 * (int)(own - row * ntx) + cl;
+  const bool live = q < per && own < ntile && x < g.nx;
+  const bool touched = live && ctouch[(int64_t)row * g.nx + x] != 0;
+  const int held = live ? count[(int64_t)row * g.nx + x] : 0;
+  if (zero) {
+    if (live) count[(int64_t)row * g.nx + x] = 0;
+    if (t0 == 0 && lane == 0) sc->novf = 0;
+  }
+  uint64_t left = __ballot(touched);
+  while (left) {
+    const int t = (__ffsll((unsigned long long)left) - 1) >> 3;  // a tile with touched cells
+    const bool mine = (left >> (8 * t + cl)) & 1ull;
+    left &= ~(0xffull << (8 * t));
+    const uint32_t tile = t0 + t, xrow = tile / ntx;
+    if (dirty && lane == 0) {
+      dirty[tile] = 1;
+      sc->anydirty = 1;
+    }
+    const int n = __shfl(held, 8 * t + cl);
+    if (!mine || n == 0) continue;
+    const int i = 8 * (int)(tile - xrow * ntx) + cl;
+    const int64_t c = (int64_t)xrow * g.nx + i;
+    const int32_t *list = n > capc ? sorted + start[c] : slot + c * capc;
+    const int k = (int)(xrow / (uint32_t)g.ny), j = (int)(xrow - (uint32_t)k * (uint32_t)g.ny);
+    int32_t o[8];
+    corner_nodes(g, i, j, k, o);
+    for (int e = q; e < n; e += 8) {
+      const int32_t p = list[e];
+      if (p >= 0 && p < norig && keep[p] == 1) absorb(P, p, o, mg);
+    }
+  }
+}
+
 // backfill: the state fields of the j-th kept slot from the end into the j-th removed slot
 // (the reference copies x, y, z, p, q, r, b, h, vol, tag and stretch)
 __global__ void k32_mix_backfill(Geometry g, Parcels32 P, const int32_t *__restrict__ dst,
                                  int64_t R, const int32_t *__restrict__ k1, int64_t K1,
-                                 uint8_t *__restrict__ dirty, DevScalars *sc) {
+                                 int64_t n, BinOut bo, uint8_t *__restrict__ dirty,
+                                 DevScalars *sc) {
   const int64_t jx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (jx >= R) return;
   const int64_t s = k1[K1 - 1 - jx], d = dst[jx];
@@ -1121,6 +1181,8 @@ __global__ void k32_mix_backfill(Geometry g, Parcels32 P, const int32_t *__restr
   }
   P.stretch[d] = P.stretch[s];
   P.tag[d] = P.tag[s];
+  // n: the parcels there are from now on
+  if (bo.on && d < n) append_entry((int32_t)d, linear_cell(g, cell), bo, sc);
 }
 
 Zmap zmap_of(const Geometry &g) { return Zmap{(float)g.zbot, (float)g.dz}; }
@@ -1149,7 +1211,7 @@ int zero_counts(Ctx *c) {
 
 BinOut bin_out(const Ctx *c, int on, int capc) {
   const Bulk32 &b = c->b32;
-  return BinOut{on, capc, c->cell_count, b.slot, b.ovf, b.ovfc, c->rank};
+  return BinOut{on, capc, c->cell_count, b.slot, b.ovf, b.ovfc, b.where, c->rank};
 }
 
 // the lists built last no longer stand
@@ -1175,7 +1237,7 @@ int bin32(Ctx *c, int64_t n) {
     b.counts_zero = false;
     if (ln > 0)
       hipLaunchKernelGGL(k32_bin_slot, dim3(cdiv(ln, (int64_t)TPB * BIN_SEQ)), dim3(TPB), 0,
-                         c->stream, c->g, cells, ln, b.capc, b.slot, b.ovf, b.ovfc, c->rank,
+                         c->stream, c->g, cells, ln, b.capc, b.slot, b.ovf, b.ovfc, b.where, c->rank,
                          c->cell_count, c->dsc);
   }
   b.binned = true;
@@ -1188,8 +1250,8 @@ int bin32(Ctx *c, int64_t n) {
                        cells, c->rank, c->dsc, c->cell_start, c->sorted);
   } else if (ln > 0) {
     const int64_t nb = std::min<int64_t>(cdiv(ln, TPB), 1024);
-    hipLaunchKernelGGL(k32_ovf_scatter, dim3(nb), dim3(TPB), 0, c->stream, c->g, cells, b.ovf,
-                       b.ovfc, c->dsc, c->cell_start, b.slot, b.capc, c->sorted);
+    hipLaunchKernelGGL(k32_ovf_scatter, dim3(nb), dim3(TPB), 0, c->stream, b.ovf, b.ovfc, c->dsc,
+                       c->cell_start, b.slot, b.capc, c->sorted);
   }
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
@@ -1290,7 +1352,7 @@ int b32_alloc(Ctx *c) {
   PMPIC_CHECK(hipMemset(b.tag, 0, sizeof(double) * (size_t)c->cap));
   for (int i = 0; i < 3; i++) PMPIC_TRY(dalloc32(&b.grid[i], c->gsz));
   for (int i = 0; i < 12; i++) PMPIC_TRY(dalloc32(&b.mgrid[i], c->gsz));
-  PMPIC_TRY(dalloc32(&b.mtouch, c->gsz));
+  PMPIC_TRY(dalloc32(&b.newcells, c->ncell));
   PMPIC_TRY(dalloc32(&b.dirty, (int64_t)tiles_x(c->g) * c->g.ny * c->g.ncz));
   b.counts_zero = false;
   b.p2g_reuse = false;
@@ -1320,7 +1382,8 @@ int b32_alloc(Ctx *c) {
   b.fused_bin = fenv ? fenv[0] == '1' : c->ncell >= ((int64_t)1 << 21);
   b.binned = false;
   b.moving = c->cap <= (int64_t)1 << 27;
-  b.room = b.moving ? 2 * c->cap : c->cap;
+  // every parcel past its cell's capacity, every one moved there, and what mixing adds (MIX_MOVES)
+  b.room = b.moving ? 2 * c->cap + c->cap / MIX_MOVES + 64 : c->cap;
   const char *env = getenv("PMPIC_SLOT_CAPACITY");
   if (env && strcmp(env, "tune") == 0) {
     b.captune = b.capmax == CAPC;
@@ -1334,6 +1397,8 @@ int b32_alloc(Ctx *c) {
   if (b.capmax > 0) PMPIC_TRY(dalloc32(&b.slot, c->ncell * b.capmax));
   PMPIC_TRY(dalloc32(&b.ovf, b.room));
   PMPIC_TRY(dalloc32(&b.ovfc, b.room));
+  b.where = nullptr;
+  if (b.moving) PMPIC_TRY(dalloc32(&b.where, c->cap));
   return PMPIC_OK;
 }
 
@@ -1343,12 +1408,13 @@ void b32_free(Ctx *c) {
   hipFree(b.tag);
   for (int i = 0; i < 3; i++) hipFree(b.grid[i]);
   for (int i = 0; i < 12; i++) hipFree(b.mgrid[i]);
-  hipFree(b.mtouch);
+  hipFree(b.newcells);
   hipFree(b.dirty);
   for (int i = 0; i < 4; i++) hipFree(b.pgrid[i]);
   hipFree(b.slot);
   hipFree(b.ovf);
   hipFree(b.ovfc);
+  hipFree(b.where);
 }
 
 // field f (FP..FSTRETCH) of the parcels
@@ -1621,7 +1687,8 @@ int b32_mix(Ctx *c) {
   b.p2g_reuse = false;
   const bool reuse = reuse_sums(c);
   uint8_t *dirty = reuse ? b.dirty : nullptr;
-  PMPIC_TRY(accumulate<A32_MIX>(c, partial32(c), partial32b(c), b.dirty));
+  PMPIC_TRY(accumulate<A32_MIX>(c, partial32(c), partial32b(c), b.dirty, false));
+  unbin(c);  // until mixing is through
   const Parcels32 P = parcels32(b);
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
   // planes weight, p, q, r, total buoyancy (not kept), b, h
@@ -1639,29 +1706,38 @@ int b32_mix(Ctx *c) {
   // step reads them there, so b32_export_grid widens them when one is exported
   for (int f = 0; f < 6; f++) b.kept_pending[f] = true;
   for (int f = 0; f < 4; f++) b.p2g_pending[f] = false;
-  PMPIC_TRY(mix_lists(c, (const float *)b.vbh, 3, vmin, norig, nullptr));
+  PMPIC_TRY(mix_lists(c, (const float *)b.vbh, 3, vmin, norig, b.newcells));
   PMPIC_TRY(sync_scalars(c));
   const int64_t Z = c->hsc.nzero, nadd = c->hsc.nadd;
   Mix32 mg = {{b.mgrid[0], b.mgrid[1], b.mgrid[2], b.mgrid[3], b.mgrid[4], b.mgrid[5]},
               {b.mgrid[6], b.mgrid[7], b.mgrid[8], b.mgrid[9], b.mgrid[10], b.mgrid[11]}};
   float *portion = partial32b(c);  // the residual partials are consumed by now
-  if (reuse) {
-    // the removed parcels' cells (read before new parcels take their slots) and the new cells
-    if (Z > 0)
-      hipLaunchKernelGGL(k32_mark_tiles, dim3(cdiv(Z, TPB)), dim3(TPB), 0, c->stream, g, P.cell,
-                         c->list_a, Z, 1, b.dirty, c->dsc);
-    if (nadd > 0)
-      hipLaunchKernelGGL(k32_mark_tiles, dim3(cdiv(nadd, TPB)), dim3(TPB), 0, c->stream, g,
-                         P.cell, c->sorted, nadd, 0, b.dirty, c->dsc);
-  }
+  // The lists follow where few parcels change (a captured graph builds its own first ones).  The
+  // removed parcels leave them before new ones take their slots.
+  const bool none = reuse && Z + nadd == 0;  // the next par2grid wants no lists
+  const bool lists = b.moving && b.capc > 0 && !c->graph_on && !none && norig + nadd < c->cap &&
+                     Z + nadd <= norig / MIX_MOVES;
+  const BinOut bo = bin_out(c, lists ? 2 : 0, b.capc);
+  if (Z > 0 && (lists || reuse))
+    hipLaunchKernelGGL(k32_unlist, dim3(cdiv(Z, TPB)), dim3(TPB), 0, c->stream, g, P.cell,
+                       c->list_a, 0, Z, bo, dirty, c->dsc);
   if (nadd > 0)
     hipLaunchKernelGGL(k32_mix_new, dim3(cdiv(nadd, TPB)), dim3(TPB), 0, c->stream, g, P, c->cap,
-                       norig, c->sorted, nadd, c->list_a, Z, c->flag, mg, vmin, portion, c->dsc);
+                       norig, b.newcells, nadd, c->list_a, Z, c->flag, mg, vmin, portion, dirty,
+                       c->dsc);
   hipLaunchKernelGGL(k32_mix_residual, dim3(cdiv(nnode, TPB)), dim3(TPB), 0, c->stream, g, mg,
-                     c->npercell, portion, b.mtouch, dirty, c->dsc);
-  if (norig > 0)
-    hipLaunchKernelGGL(k32_mix_absorb, dim3(cdiv(norig, TPB)), dim3(TPB), 0, c->stream, g, P,
-                       norig, c->flag, mg, b.mtouch);
+                     c->npercell, portion, c->ctouch);
+  // eight tiles a wavefront where that leaves the chip full of them (150 us against 271 with one in
+  // 1.05 M tiles; but 27 against 22 in 29 k)
+  const int64_t tiles = (int64_t)tiles_x(g) * g.ny * g.ncz;
+  const int per = tiles >= (1 << 17) ? 8 : 1;
+  hipLaunchKernelGGL(k32_mix_absorb, dim3(cdiv(tiles, per)), dim3(64), 0, c->stream, g, P,
+                     norig, c->flag, mg, b.capc, b.slot, c->cell_count, c->cell_start, c->sorted,
+                     c->ctouch, dirty, c->dsc, per, lists ? 0 : 1);
+  b.counts_zero = !lists;
+  if (lists && nadd > 0)
+    hipLaunchKernelGGL(k32_list_new, dim3(cdiv(nadd, TPB)), dim3(TPB), 0, c->stream, g, P.cell,
+                       norig, nadd, c->list_a, Z, bo, c->dsc);
   PMPIC_CHECK(hipGetLastError());
   // new count (parcel_mixing.F90:217), then the backfill of removed slots (:347-389)
   int64_t np = norig;
@@ -1699,14 +1775,18 @@ int b32_mix(Ctx *c) {
       PMPIC_TRY(sync_scalars(c));
       const int64_t K1 = c->hsc.nkeep1;
       if (R > K1) return PMPIC_ERR_BACKFILL;
-      hipLaunchKernelGGL(k32_mix_backfill, dim3(cdiv(R, TPB)), dim3(TPB), 0, c->stream, g, P,
-                         dst, R, c->list_b, K1, dirty, c->dsc);
-      PMPIC_CHECK(hipGetLastError());
       np -= R;
+      if (lists)  // the slots past the new count
+        hipLaunchKernelGGL(k32_unlist, dim3(cdiv(R, TPB)), dim3(TPB), 0, c->stream, g, P.cell,
+                           nullptr, np, R, bo, nullptr, c->dsc);
+      hipLaunchKernelGGL(k32_mix_backfill, dim3(cdiv(R, TPB)), dim3(TPB), 0, c->stream, g, P,
+                         dst, R, c->list_b, K1, np, bo, dirty, c->dsc);
+      PMPIC_CHECK(hipGetLastError());
     }
   }
   c->n = np;
-  b.p2g_reuse = reuse;
+  b.binned = lists;
+  b.binned_n = np;
   // whether any tile changed (anydirty) the host learns with the next read-back of the device
   // scalars (the status check that ends the component or the step)
   b.dirty_seq = c->sync_seq;

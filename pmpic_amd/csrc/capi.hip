@@ -262,7 +262,7 @@ int create(const pmpic_config *cf, Ctx *c) {
   if (c->precision == 1) PMPIC_TRY(dalloc(&c->partial2, pdoubles));
   PMPIC_TRY(dalloc(&c->npercell, c->ncell));
   PMPIC_TRY(dalloc(&c->cellflag, c->ncell));
-  if (c->precision == 0) PMPIC_TRY(dalloc(&c->ctouch, c->ncell));
+  PMPIC_TRY(dalloc(&c->ctouch, c->ncell));
   for (int i = 0; i < GDP; i++) PMPIC_TRY(dalloc(&c->grid[i], c->gsz));
   if (c->precision == 1) PMPIC_TRY(dalloc(&c->rec32, 2 * c->gsz));
   else PMPIC_TRY(dalloc(&c->rec, 3 * c->gsz));

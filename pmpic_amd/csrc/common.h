@@ -59,7 +59,7 @@ struct Bulk32 {
   double *tag;       // cap
   float *grid[3];    // U, V, W [nzn][ny][nx]
   float *mgrid[12];  // mixing: kept vol, b, h, p, q, r (0..5), residuals (6..11)
-  uint8_t *mtouch;   // mixing, per node: a residual grid is not zero there
+  int32_t *newcells; // ncell: mixing's cells short of parcels
   // cell binning: slot[c * capc + rank] lists the parcels of cell c while rank < capc; a cell
   // with more parcels lists all of them in the dense overflow region.  The table holds 32
   // entries per cell (none, and capc = 0, when its byte offsets would exceed 32 bits); each
@@ -67,7 +67,8 @@ struct Bulk32 {
   int32_t *slot;
   int2 *ovf;         // (parcel, rank) of the parcels past the slot capacity
   int32_t *ovfc;     // ... and their cells
-  int64_t room;      // entries of ovf, and of Ctx::sorted and rank: cap, or twice that (moving)
+  int32_t *where;    // cap (moving): a parcel's entry in ovf, where it has one
+  int64_t room;      // entries of ovf, and of Ctx::sorted and rank: cap, or over twice that (moving)
   int capc;          // capacity of the current binning (0, 16 or 32)
   int capmax;        // entries per cell allocated (0 or 32)
   int capfix;        // capacity forced by PMPIC_SLOT_CAPACITY (16 or 32), or 0 for the mean rule
@@ -87,7 +88,7 @@ struct Bulk32 {
   bool fused_bin;
   // The lists built last still stand (`binned`): for the cells of set binned_set, binned_n parcels
   // and the capacity capc.  moving: stages 2 and 4, which hardly move a parcel out of the cell that
-  // the stage before put it in, and splitting move the few entries that change instead of
+  // the stage before put it in, splitting and mixing move the few entries that change instead of
   // building the lists again (room for the entries that can come: up to 2^27 parcels).
   bool binned, moving;
   int binned_set;
@@ -179,7 +180,7 @@ struct Ctx {
                                       // FP64 form (then mixing takes two passes over partial)
   int32_t *npercell;                  // ncell
   uint8_t *cellflag;                  // ncell
-  uint8_t *ctouch;                    // ncell, FP64 form: cells whose parcels absorb a residual
+  uint8_t *ctouch;                    // ncell: cells whose parcels absorb a residual
   // grids (interior [nzn][ny][nx])
   int64_t gsz, ssz, csz;              // grid; spectral (planes); complex transform intermediate
   int64_t bsz;                        // spectral (tiles)
@@ -464,10 +465,10 @@ int compact_flags(Ctx *c, const uint8_t *flags, uint8_t want, int64_t n, int32_t
 // the parcels to split (list_b, DevScalars::nsplit), from their stretch; n > 0
 template <typename T>
 int split_list(Ctx *c, const T *stretch, int64_t n);
-// mixing's parcels whose volume vol[stride i] is below vmin (flag, list_a, nzero) and cells short of parcels (cellflag, sorted,
-// nadd); clears ctouch (may be null)
+// mixing's parcels whose volume vol[stride i] is below vmin (flag, list_a, nzero) and cells short
+// of parcels (cellflag, cells, nadd); clears ctouch
 template <typename T>
-int mix_lists(Ctx *c, const T *vol, int stride, T vmin, int64_t n, uint8_t *ctouch);
+int mix_lists(Ctx *c, const T *vol, int stride, T vmin, int64_t n, int32_t *cells);
 // bulk32.hip (FP32-bulk form)
 int b32_alloc(Ctx *c);
 void b32_free(Ctx *c);

@@ -469,7 +469,7 @@ __global__ void __launch_bounds__(TPB) k_mix_flags(const T *__restrict__ vol, in
         const uint32_t ord = (uint32_t)o, col = ord / (uint32_t)g.ncz;  // cells are below 2^31
         const uint32_t k = ord - col * (uint32_t)g.ncz, i = col / (uint32_t)g.ny;
         const uint32_t j = col - i * (uint32_t)g.ny;
-        if (ctouch) ctouch[ord] = 0;
+        ctouch[ord] = 0;
         return (uint8_t)(npercell[((int64_t)k * g.ny + j) * g.nx + i] < 3 ? 1 : 0);
       },
       1, ncell, blockIdx.x - nblk, cellflag, cblk, lds);
@@ -774,16 +774,16 @@ int split_list(Ctx *c, const T *stretch, int64_t n) {
 }
 
 template <typename T>
-int mix_lists(Ctx *c, const T *vol, int stride, T vmin, int64_t n, uint8_t *ctouch) {
+int mix_lists(Ctx *c, const T *vol, int stride, T vmin, int64_t n, int32_t *cells) {
   FlagList a = {c->flag, n, cdiv(n > 0 ? n : 1, FPB), nullptr, nullptr, c->list_a,
                 &c->dsc->nzero, 0};
-  FlagList b = {c->cellflag, c->ncell, cdiv(c->ncell, FPB), nullptr, nullptr, c->sorted,
+  FlagList b = {c->cellflag, c->ncell, cdiv(c->ncell, FPB), nullptr, nullptr, cells,
                 &c->dsc->nadd, 1};
   if (a.nblk > c->nblk_max || b.nblk > c->nblk_max) return PMPIC_ERR_ARG;
   int32_t *blk_a = c->blk, *blk_b = c->blk + 2 * a.nblk;
   hipLaunchKernelGGL(k_mix_flags<T>, dim3(a.nblk + b.nblk), dim3(TPB), 0, c->stream, vol, stride, n,
-                     vmin, c->flag, blk_a, a.nblk, c->g, c->npercell, c->ncell, c->cellflag, ctouch,
-                     blk_b);
+                     vmin, c->flag, blk_a, a.nblk, c->g, c->npercell, c->ncell, c->cellflag,
+                     c->ctouch, blk_b);
   PMPIC_TRY(list_prefix(c, a, blk_a));
   PMPIC_TRY(list_prefix(c, b, blk_b));
   hipLaunchKernelGGL(k_flag_scatter, dim3(a.nblk + b.nblk), dim3(TPB), 0, c->stream, a, b);
@@ -793,8 +793,8 @@ int mix_lists(Ctx *c, const T *vol, int stride, T vmin, int64_t n, uint8_t *ctou
 
 template int split_list<double>(Ctx *, const double *, int64_t);
 template int split_list<float>(Ctx *, const float *, int64_t);
-template int mix_lists<double>(Ctx *, const double *, int, double, int64_t, uint8_t *);
-template int mix_lists<float>(Ctx *, const float *, int, float, int64_t, uint8_t *);
+template int mix_lists<double>(Ctx *, const double *, int, double, int64_t, int32_t *);
+template int mix_lists<float>(Ctx *, const float *, int, float, int64_t, int32_t *);
 
 static int ensure_tmp(Ctx *c, int64_t need) {
   if (need <= c->tmp_cap) return PMPIC_OK;
@@ -904,7 +904,7 @@ int parcel_mix(Ctx *c) {
   const int64_t norig = c->n;
   PMPIC_TRY(mixing_grids(c, norig));
   // removed slots, ascending, and sparse cells in the reference's loop order
-  PMPIC_TRY(mix_lists(c, c->par + FVOL * c->cap, 1, g.vmin, norig, c->ctouch));
+  PMPIC_TRY(mix_lists(c, c->par + FVOL * c->cap, 1, g.vmin, norig, c->sorted));
   PMPIC_TRY(sync_scalars(c));
   const int64_t Z = c->hsc.nzero, nadd = c->hsc.nadd;
   MixGrids mg = {{c->grid[GVOL], c->grid[GB], c->grid[GHG], c->grid[GP], c->grid[GQ], c->grid[GR]},

@@ -286,3 +286,26 @@ def test_large_host_copies(n):
     for t in th:
         t.join()
     assert out == [True, True]
+
+
+@pytest.mark.parametrize("shape", [(128, 128, 63), (128, 128, 64)])
+def test_bulk32_mixing_tiles_a_wavefront(shape):
+    """Absorption either side of 2^17 tiles, from which a wavefront looks at eight of them: what
+    mixing takes from removed parcels and gives to new ones the absorbing parcels make up for, so the
+    volume stays (to 1e-6 after three steps, as in the small form of this test), with parcels removed
+    and added in one cell of fifty."""
+    from pmpic_amd.lib import Context
+    ic = thermal_case(*shape, 2, vort=1.0, shrink=0.02, thin=0.02, near_split=0.01)
+    b = box(*shape)
+    g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                2 * len(ic["x"]), precision=1)
+    g.set_parcels(ic)
+    s0 = g.conservation_sums()
+    changed = 0
+    for _ in range(3):
+        g.step()
+        changed += sum(g.last_counts()[1:])
+    s1 = g.conservation_sums()
+    g.close()
+    assert changed > 0
+    assert abs(s1[0] - s0[0]) <= 1e-6 * s0[0]
