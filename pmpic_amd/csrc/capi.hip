@@ -226,6 +226,7 @@ int create(const pmpic_config *cf, Ctx *c) {
   c->dtmax = cf->dtmax;
   c->prefactor = cf->timestep_prefactor;
   c->rkstep = 1;
+  c->bins_n = BINS_NONE;
   c->precision = cf->precision;
   c->device = cf->device;
   c->splitting_enabled = cf->splitting_enabled;
@@ -430,6 +431,7 @@ int pmpic_set_parcels(pmpic_ctx *ctx, int64_t n, const double *const *fields) {
     PMPIC_TRY(b32_publish_n(c));
     return take_status(c);
   }
+  PMPIC_TRY(drop_bins(c));
   HostPart part[17];
   for (int f = 0; f < 17; f++)
     part[f] = {const_cast<double *>(fields[f]), c->par + (int64_t)f * c->cap, sizeof(double) * (size_t)n};

@@ -149,6 +149,8 @@ enum TimerId { T_ACCUM = 0, T_RK = 1, T_VORT2VEL, T_VORT_TEND, T_RK4, T_SPLIT, T
 
 constexpr int HOST_SLOTS = 8;  // pinned slots of the large host copies (copy_host)
 
+constexpr int64_t BINS_NONE = -1, BINS_STALE = -2;  // Ctx::bins_n
+
 struct Ctx {
   Geometry g;
   int64_t cap;
@@ -178,6 +180,9 @@ struct Ctx {
   double *partial;                    // corner partial sums: 48 * ncell doubles (FP32 form: 24)
   double *partial2;                   // mixing residual partials, same size; may be null in the
                                       // FP64 form (then mixing takes two passes over partial)
+  // FP64 form: the number of parcels that the binning in cell_count, cell_start, sorted and cell
+  // lists as they are, or none: counts at zero (as a binning wants them), or not
+  int64_t bins_n;
   int32_t *npercell;                  // ncell
   uint8_t *cellflag;                  // ncell
   uint8_t *ctouch;                    // ncell: cells whose parcels absorb a residual
@@ -378,6 +383,7 @@ int par2grid_single_ws(Ctx *c, int64_t n, const double *d_var, double *d_grid, c
 int par2grid_fused(Ctx *c, int64_t n);  // P,Q,R,B grids from p,q,r,btot
 int par2grid_single(Ctx *c, int64_t n, const double *d_var, double *d_grid);
 int grid2par_single(Ctx *c, int64_t n, const double *d_grid, double *d_var);
+int drop_bins(Ctx *c);  // before the parcels change their cells or slots
 // buckets of the cells of more than `held` parcels, from *cursor on
 void bin_alloc(Ctx *c, const int32_t *count, int held, int32_t *start, int32_t *cursor);
 int mixing_grids(Ctx *c, int64_t n);

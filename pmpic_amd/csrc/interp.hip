@@ -458,7 +458,26 @@ int bin_parcels_ws(Ctx *c, int64_t n, const BinWork &w) {
   return PMPIC_OK;
 }
 
-int bin_parcels(Ctx *c, int64_t n) { return bin_parcels_ws(c, n, ctx_work(c)); }
+__global__ void k_zero_i32(int32_t *__restrict__ a, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) a[i] = 0;
+}
+
+// the context's binning no longer stands: counts and cursor at zero
+int drop_bins(Ctx *c) {
+  if (c->bins_n != BINS_NONE)
+    hipLaunchKernelGGL(k_zero_i32, dim3(cdiv(c->ncell + 1, TPB)), dim3(TPB), 0, c->stream,
+                       c->cell_count, c->ncell + 1);
+  c->bins_n = BINS_NONE;
+  PMPIC_CHECK(hipGetLastError());
+  return PMPIC_OK;
+}
+
+int bin_parcels(Ctx *c, int64_t n) {
+  if (c->bins_n == n) return PMPIC_OK;  // mixing's, which changed no parcel's cell or slot
+  PMPIC_TRY(drop_bins(c));
+  return bin_parcels_ws(c, n, ctx_work(c));
+}
 
 static dim3 accum_tiles(const Ctx *c) {
   return dim3((unsigned)(cdiv(c->g.nx, 8) * c->g.ny * c->g.ncz));
@@ -467,6 +486,7 @@ static dim3 accum_tiles(const Ctx *c) {
 template <int MODE, int NV>
 static void launch_accum(Ctx *c, const BinWork &w, const double *var, double *partial,
                          double *partial2, int32_t *npc, uint8_t *tileres, int zero) {
+  if (w.count == c->cell_count) c->bins_n = zero ? BINS_NONE : BINS_STALE;
   hipLaunchKernelGGL((k_cell_accum<MODE, NV>), accum_tiles(c), dim3(64), 0, c->stream, c->g, c->par,
                      c->cap, var, w.count, w.start, w.sorted, w.rank, partial, partial2, npc,
                      tileres, w.cursor, zero);
@@ -481,6 +501,7 @@ static void node_sums(Ctx *c, const NodeSums<double, double> &first,
 int par2grid_fused(Ctx *c, int64_t n) {
   PMPIC_TRY(bin_parcels(c, n));
   const BinWork w = ctx_work(c);
+  c->bins_n = BINS_NONE;
   PMPIC_TRY(launch_timed(c, T_ACCUM, k_cell_accum<ACC_P2G, 4>, accum_tiles(c), dim3(64), 0, c->g,
                          c->par, c->cap, nullptr, w.count, w.start, w.sorted, w.rank, w.partial,
                          nullptr, nullptr, nullptr, w.cursor, 1));
@@ -491,7 +512,8 @@ int par2grid_fused(Ctx *c, int64_t n) {
 
 int par2grid_single_ws(Ctx *c, int64_t n, const double *d_var, double *d_grid,
                        const BinWork &w) {
-  PMPIC_TRY(bin_parcels_ws(c, n, w));
+  if (w.count == c->cell_count) PMPIC_TRY(bin_parcels(c, n));
+  else PMPIC_TRY(bin_parcels_ws(c, n, w));
   launch_accum<ACC_SINGLE, 1>(c, w, d_var, w.partial, nullptr, nullptr, nullptr, 1);
   node_sums<2, true>(c, {w.partial, {d_grid}, nullptr, 1.});
   PMPIC_CHECK(hipGetLastError());
@@ -549,7 +571,7 @@ int grid2par_single(Ctx *c, int64_t n, const double *d_grid, double *d_var) {
 // correction of :202-207 and before their own doubling (:229-240).
 // Without a residual buffer (partial2 null: a context too large for both) the kept and the
 // residual sums take one pass each over `partial`, with the same sums.  cellflag holds the
-// residual flags of the tiles (at most one a cell).
+// residual flags of the tiles (at most one a cell).  Leaves the binning as it is.
 int mixing_grids(Ctx *c, int64_t n) {
   PMPIC_TRY(bin_parcels(c, n));
   const BinWork w = ctx_work(c);
@@ -560,12 +582,12 @@ int mixing_grids(Ctx *c, int64_t n) {
   NodeSums<double, double> res = {
       c->partial2, {c->kres[0], c->kres[1], c->kres[2], c->kres[3], c->kres[4], c->kres[5]}, flags, 1.};
   if (c->partial2) {
-    launch_accum<ACC_MIX, 5>(c, w, nullptr, c->partial, c->partial2, c->npercell, flags, 1);
+    launch_accum<ACC_MIX, 5>(c, w, nullptr, c->partial, c->partial2, c->npercell, flags, 0);
     node_sums<6, false>(c, kept, &res);
   } else {
     launch_accum<ACC_MIX, 5>(c, w, nullptr, c->partial, nullptr, c->npercell, flags, 0);
     node_sums<6, false>(c, kept);
-    launch_accum<ACC_MIX, 5>(c, w, nullptr, nullptr, c->partial, nullptr, nullptr, 1);
+    launch_accum<ACC_MIX, 5>(c, w, nullptr, nullptr, c->partial, nullptr, nullptr, 0);
     res.partial = c->partial;
     node_sums<6, false>(c, res);
   }

@@ -843,6 +843,7 @@ int rk_stage_update(Ctx *c, int stage, int64_t n, int stretch) {
   const int64_t nblk = cdiv(n > 0 ? n : 1, TPB);
   if (nblk > c->nblk_max) return PMPIC_ERR_ARG;
   PMPIC_TRY(records_current(c));
+  PMPIC_TRY(drop_bins(c));
   const int keep_k = c->whole_step ? 0 : 1;
   switch (stage) {
     case 1:
@@ -868,6 +869,7 @@ int rk_stage_update(Ctx *c, int stage, int64_t n, int stretch) {
 
 int parcel_haloswap(Ctx *c, int64_t n, int reflect) {
   (void)reflect;
+  PMPIC_TRY(drop_bins(c));
   const int64_t nblk = cdiv(n > 0 ? n : 1, TPB);
   if (nblk > c->nblk_max) return PMPIC_ERR_ARG;
   hipLaunchKernelGGL(k_reflect_classify, dim3(nblk), dim3(TPB), 0, c->stream, c->g, c->par, c->cap,
@@ -966,6 +968,9 @@ int parcel_mix(Ctx *c) {
     }
   }
   c->n = np;
+  // no parcel removed or added: the binning stands for the next par2grid (else c->sorted holds the
+  // sparse cells now)
+  if (Z == 0 && nadd == 0) c->bins_n = np;
   return PMPIC_OK;
 }
 

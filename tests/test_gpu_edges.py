@@ -309,3 +309,37 @@ def test_bulk32_mixing_tiles_a_wavefront(shape):
     g.close()
     assert changed > 0
     assert abs(s1[0] - s0[0]) <= 1e-6 * s0[0]
+
+
+@pytest.mark.parametrize("change", ["none", "set_parcels", "haloswap", "par2grid", "grids"])
+def test_binning_after_mixing(oracle_mod, change, bar):
+    """The binning that a mixing without removed or new parcels leaves for the next par2grid, with
+    the parcels as they were or changed meanwhile in each way a caller has: against the oracle,
+    1e-12."""
+    shape = (12, 10, 8)
+    ic = thermal_case(*shape, 2, vort=1.0)
+    o, g = _pair(oracle_mod, shape, ic)
+    for c in (o, g):
+        c.step()
+    assert g.last_counts() == o.last_counts() == (0, 0, 0)
+    if change == "set_parcels":
+        other = thermal_case(*shape, 2, seed=9, vort=1.0)
+        for c in (o, g):
+            c.set_parcels(other)
+    elif change == "haloswap":
+        for c in (o, g):
+            c.parcel_haloswap()
+    elif change == "par2grid":
+        o.cache_weights()
+        var = np.arange(o.n, dtype=np.float64)
+        bar("par2grid", rel_err(g.par2grid(var)[2:-2, 2:-2], o.par2grid(var)[2:-2, 2:-2]), 1e-12)
+    elif change == "grids":
+        g.writebinary_grids()
+    for c in (o, g):
+        c.step()
+    for k in ("u", "v", "w", "p", "q", "r"):
+        bar(k, rel_err(g.grid(k)[2:-2, 2:-2], o.grid(k)[2:-2, 2:-2]), 1e-12)
+    got, want = g.get_parcels(), o.get_parcels()
+    for k in ("x", "y", "z", "p", "q", "r"):
+        bar(k, rel_err(got[k], want[k]), 1e-12)
+    g.close()
