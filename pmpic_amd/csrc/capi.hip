@@ -306,7 +306,7 @@ int create(const pmpic_config *cf, Ctx *c) {
   PMPIC_TRY(dalloc(&c->cbuf, (c->precision == 1 ? FFT_FIELDS / 2 : FFT_FIELDS) * c->csz));
   c->nblk_max = cdiv(big, 256) + 1;
   PMPIC_TRY(dalloc(&c->blk, 20 * c->nblk_max + 64));
-  PMPIC_TRY(dalloc(&c->maxblk, 4 * 1024));
+  PMPIC_TRY(dalloc(&c->maxblk, 4 * MAXBLK));
   PMPIC_TRY(dalloc(&c->dsc, 1));
   PMPIC_CHECK(hipHostMalloc(&c->pin, 256));
   PMPIC_CHECK(hipEventCreateWithFlags(&c->sync_ev, hipEventDisableTiming));
@@ -519,10 +519,7 @@ int pmpic_vorticity_tendency(pmpic_ctx *ctx) {
   Ctx *c = &ctx->c;
   const int stage = stage_of(c->it_vt);
   PMPIC_TRY(timing_begin(c, T_VORT_TEND));
-  PMPIC_TRY(vorticity_tendency_grids(c));
-  if (stage == 1) {
-    PMPIC_TRY(grid_max_reduce(c));
-  }
+  PMPIC_TRY(vorticity_tendency_grids(c, stage == 1));
   PMPIC_TRY(timing_end(c, T_VORT_TEND));
   c->it_vt++;
   return PMPIC_OK;

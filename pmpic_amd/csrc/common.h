@@ -147,6 +147,7 @@ __host__ __device__ inline int64_t spec_at(int nzn, int nl, int k, int m, int l)
 
 enum TimerId { T_ACCUM = 0, T_RK = 1, T_VORT2VEL, T_VORT_TEND, T_RK4, T_SPLIT, T_MIX, NTIMERS };
 
+constexpr int MAXBLK = 1024;   // blocks of the timestep reduction
 constexpr int HOST_SLOTS = 8;  // pinned slots of the large host copies (copy_host)
 
 constexpr int64_t BINS_NONE = -1, BINS_STALE = -2;  // Ctx::bins_n
@@ -426,14 +427,13 @@ int vort2vel_columns(Ctx *c);
 // spectral.hip
 int spectral_setup(Ctx *c);
 int vort2vel_spectral(Ctx *c);
-int vorticity_tendency_grids(Ctx *c);
+int vorticity_tendency_grids(Ctx *c, bool maxima);  // maxima: and the timestep
 int records_current(Ctx *c);                           // refreshes the records' velocities if stale
 int op_diffx(Ctx *c, const double *in, double *out);
 int op_diffy(Ctx *c, const double *in, double *out);
 int op_filter(Ctx *c, const double *in, double *out);
 int op_diffz(Ctx *c, const double *in, double *out, const double *bot, const double *top);
 int op_laplinv(Ctx *c, double *f, int df0);
-int grid_max_reduce(Ctx *c);
 // parcels.hip
 int rk_stage_update(Ctx *c, int stage, int64_t n, int stretch);
 // Component timers (timing mode 1) bracket a component with events on the stream.

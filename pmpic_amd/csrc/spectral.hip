@@ -690,10 +690,26 @@ __device__ __forceinline__ void put_record(float4 *rec, int64_t t, float u, floa
   rec[2 * t + 1] = make_float4((float)dq, (float)dr, 0.f, 0.f);
 }
 
+// the block's maxima, one value per block and quantity; k_max4_final reduces them (no contended
+// atomics)
+__device__ __forceinline__ void block_max4(const double m[4], double *__restrict__ blkmax) {
+  __shared__ double sm[4][TPB];
+  for (int f = 0; f < 4; f++) sm[f][threadIdx.x] = m[f];
+  __syncthreads();
+  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
+    if (threadIdx.x < s)
+      for (int f = 0; f < 4; f++) sm[f][threadIdx.x] = fmax(sm[f][threadIdx.x], sm[f][threadIdx.x + s]);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0)
+    for (int f = 0; f < 4; f++) blkmax[(int64_t)f * gridDim.x + blockIdx.x] = sm[f][0];
+}
+
 // vorticity_tendency.F90:169-265, physical interior, accumulation order as written, and the node
 // records of the RK stage's gathers.
 // T: the type of the grids (FP64, or FP32 in the FP32-bulk form, widened exactly); the products
 // are formed in FP64 in both forms.  Bound by memory (14 grids read, a record written).
+// blkmax (may be null): the block's maxima for the timestep as well, of the grids that it reads.
 template <typename T, typename REC>
 __global__ void k_tendency(int64_t nnode, const T *__restrict__ P, const T *__restrict__ Q,
                            const T *__restrict__ R, const T *__restrict__ dbdy,
@@ -702,9 +718,10 @@ __global__ void k_tendency(int64_t nnode, const T *__restrict__ P, const T *__re
                            const T *__restrict__ dvdx, const T *__restrict__ dvdy,
                            const T *__restrict__ dwdy, const T *__restrict__ U,
                            const T *__restrict__ V, const T *__restrict__ W,
-                           REC *__restrict__ rec) {
-  int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nnode) return;
+                           REC *__restrict__ rec, double *__restrict__ blkmax) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nnode && !blkmax) return;
+  const int64_t q = min(t, nnode - 1);  // past the end the last node again: the same record
   const double p = P[q], qq = Q[q], r = R[q];
   double dp = dbdy[q];
   dp = dp + p * (double)dudx[q];
@@ -718,7 +735,12 @@ __global__ void k_tendency(int64_t nnode, const T *__restrict__ P, const T *__re
   dr = dr + qq * (double)dwdy[q];
   dr = dr + r * (-(double)dudx[q]);
   dr = dr + r * (-(double)dvdy[q]);
-  put_record(rec, q, U[q], V[q], W[q], dp, dq, dr);
+  const double u = U[q], v = V[q], w = W[q];
+  put_record(rec, q, u, v, w, dp, dq, dr);
+  if (blkmax) {
+    const double m[4] = {u * u, v * v, w * w, p * p + qq * qq + r * r};
+    block_max4(m, blkmax);
+  }
 }
 
 // newer velocities into the records (vort2vel called again without vorticity_tendency)
@@ -747,7 +769,6 @@ __global__ void k_max4(int64_t nnode, const TU *__restrict__ U, const TU *__rest
                        const TU *__restrict__ W, const TU *__restrict__ P,
                        const TU *__restrict__ Q, const TU *__restrict__ R,
                        double *__restrict__ blkmax) {
-  __shared__ double sm[4][TPB];
   double m[4] = {0, 0, 0, 0};
   // MPT nodes per pass, their loads issued together; an index past the end is clamped to the
   // last node, which the maximum tolerates
@@ -771,20 +792,33 @@ __global__ void k_max4(int64_t nnode, const TU *__restrict__ U, const TU *__rest
       m[3] = fmax(m[3], o);
     }
   }
-  for (int f = 0; f < 4; f++) sm[f][threadIdx.x] = m[f];
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s)
-      for (int f = 0; f < 4; f++) sm[f][threadIdx.x] = fmax(sm[f][threadIdx.x], sm[f][threadIdx.x + s]);
-    __syncthreads();
-  }
-  // one value per block and quantity; k_max4_final reduces them (no contended atomics)
-  if (threadIdx.x == 0)
-    for (int f = 0; f < 4; f++) blkmax[(int64_t)f * gridDim.x + blockIdx.x] = sm[f][0];
+  block_max4(m, blkmax);
 }
 
-// the maxima over the nb blocks of k_max4 (one workgroup); a maximum is exact in any order
-__global__ void k_max4_final(int nb, const double *__restrict__ blkmax, DevScalars *sc) {
+// timestep selection at RK stage 1: vort2vel.F90:329-381 then vorticity_tendency.F90:277-321
+__device__ __forceinline__ void select_dt(const Geometry &g, DevScalars *sc) {
+  double umax = sqrt(sc->umax2), vmax = sqrt(sc->vmax2), wmax = sqrt(sc->wmax2);
+  const double tiny = (double)1.E-15f;
+  if (umax == 0) umax = tiny;
+  if (vmax == 0) vmax = tiny;
+  if (wmax == 0) wmax = tiny;
+  const double t1 = g.lx_cfl / umax, t2 = g.ly_cfl / vmax, t3 = g.lz_cfl / wmax;
+  double dtmaxg = t1;
+  if (t2 < dtmaxg) dtmaxg = t2;
+  if (t3 < dtmaxg) dtmaxg = t3;
+  double dtm = (sc->dtmax > dtmaxg) ? dtmaxg : sc->dtmax;
+  const double omax = sqrt(sc->omax2);
+  double dtv;
+  if (omax > 0.) dtv = sc->prefactor / omax;
+  else dtv = sc->dtmax;
+  if (dtm > dtv) dtm = dtv;
+  sc->dtm = dtm;
+}
+
+// the maxima over the nb blocks (one workgroup), a maximum being exact in any order, and the
+// timestep from them
+__global__ void k_max4_final(Geometry g, int nb, const double *__restrict__ blkmax,
+                             DevScalars *sc) {
   __shared__ double sm[4][TPB];
   double m[4] = {0, 0, 0, 0};
   for (int i = threadIdx.x; i < nb; i += blockDim.x)
@@ -802,28 +836,8 @@ __global__ void k_max4_final(int nb, const double *__restrict__ blkmax, DevScala
     sc->vmax2 = sm[1][0];
     sc->wmax2 = sm[2][0];
     sc->omax2 = sm[3][0];
+    select_dt(g, sc);
   }
-}
-
-// timestep selection at RK stage 1: vort2vel.F90:329-381 then vorticity_tendency.F90:277-321
-__global__ void k_select_dt(Geometry g, DevScalars *sc) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double umax = sqrt(sc->umax2), vmax = sqrt(sc->vmax2), wmax = sqrt(sc->wmax2);
-  const double tiny = (double)1.E-15f;
-  if (umax == 0) umax = tiny;
-  if (vmax == 0) vmax = tiny;
-  if (wmax == 0) wmax = tiny;
-  const double t1 = g.lx_cfl / umax, t2 = g.ly_cfl / vmax, t3 = g.lz_cfl / wmax;
-  double dtmaxg = t1;
-  if (t2 < dtmaxg) dtmaxg = t2;
-  if (t3 < dtmaxg) dtmaxg = t3;
-  double dtm = (sc->dtmax > dtmaxg) ? dtmaxg : sc->dtmax;
-  const double omax = sqrt(sc->omax2);
-  double dtv;
-  if (omax > 0.) dtv = sc->prefactor / omax;
-  else dtv = sc->dtmax;
-  if (dtm > dtv) dtm = dtv;
-  sc->dtm = dtm;
 }
 
 inline int64_t ssz_of(const Geometry &g) { return (int64_t)g.nzn * g.sy * g.sx; }
@@ -1010,27 +1024,51 @@ int vort2vel_spectral(Ctx *c) {
   return c->precision == 1 ? vort2vel_spectral_t<float>(c) : vort2vel_spectral_t<double>(c);
 }
 
+// the timestep from the grids' maxima: those of nb blocks in maxblk, or with nb = 0 taken here
+static int grid_max_reduce(Ctx *c, int nb) {
+  const Geometry &g = c->g;
+  const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
+  if (nb == 0) {
+    nb = (int)std::min<int64_t>(cdiv(nnode, TPB), MAXBLK);
+    if (c->precision == 1)  // the FP32-bulk form's grids are FP32
+      hipLaunchKernelGGL(k_max4<float>, dim3(nb), dim3(TPB), 0, c->stream, nnode, c->b32.grid[0],
+                         c->b32.grid[1], c->b32.grid[2], c->b32.pgrid[0], c->b32.pgrid[1],
+                         c->b32.pgrid[2], c->maxblk);
+    else
+      hipLaunchKernelGGL(k_max4<double>, dim3(nb), dim3(TPB), 0, c->stream, nnode, c->grid[GU],
+                         c->grid[GV], c->grid[GW], c->grid[GP], c->grid[GQ], c->grid[GR],
+                         c->maxblk);
+  }
+  hipLaunchKernelGGL(k_max4_final, dim3(1), dim3(TPB), 0, c->stream, g, nb, c->maxblk, c->dsc);
+  PMPIC_CHECK(hipGetLastError());
+  return PMPIC_OK;
+}
+
 // vorticity_tendency timestep_callback (vorticity_tendency.F90:169-265) from the grids of
 // vort2vel: the tendencies, with the velocities, into the node records
-int vorticity_tendency_grids(Ctx *c) {
+int vorticity_tendency_grids(Ctx *c, bool maxima) {
   const Geometry &g = c->g;
   const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
   const dim3 gb(cdiv(nnode, TPB)), tb(TPB);
+  // up to MAXBLK blocks the tendency takes the maxima for the timestep along (a launch of 4 us
+  // less); the blocks of a larger grid would be too many for the final reduction
+  double *blkmax = maxima && gb.x <= MAXBLK ? c->maxblk : nullptr;
   if (c->precision == 1) {
     const Bulk32 &b = c->b32;
     const float *d[8];
     for (int f = 0; f < 8; f++) d[f] = reinterpret_cast<const float *>(c->gtmp[f]);
     hipLaunchKernelGGL((k_tendency<float, float4>), gb, tb, 0, c->stream, nnode, b.pgrid[0],
                        b.pgrid[1], b.pgrid[2], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
-                       b.grid[0], b.grid[1], b.grid[2], c->rec32);
+                       b.grid[0], b.grid[1], b.grid[2], c->rec32, blkmax);
   } else {
     double *const *d = c->gtmp;
     hipLaunchKernelGGL((k_tendency<double, double2>), gb, tb, 0, c->stream, nnode, c->grid[GP],
                        c->grid[GQ], c->grid[GR], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7],
-                       c->grid[GU], c->grid[GV], c->grid[GW], c->rec);
+                       c->grid[GU], c->grid[GV], c->grid[GW], c->rec, blkmax);
   }
   c->rec_stale = false;
   PMPIC_CHECK(hipGetLastError());
+  if (maxima) PMPIC_TRY(grid_max_reduce(c, blkmax ? (int)gb.x : 0));
   return PMPIC_OK;
 }
 
@@ -1045,25 +1083,6 @@ int records_current(Ctx *c) {
     hipLaunchKernelGGL(k_record_velocity, gb, tb, 0, c->stream, nnode, c->grid[GU], c->grid[GV],
                        c->grid[GW], c->rec);
   c->rec_stale = false;
-  PMPIC_CHECK(hipGetLastError());
-  return PMPIC_OK;
-}
-
-int grid_max_reduce(Ctx *c) {
-  const Geometry &g = c->g;
-  const int64_t nnode = (int64_t)g.nzn * g.ny * g.nx;
-  int64_t nb = cdiv(nnode, TPB);
-  if (nb > 1024) nb = 1024;  // c->maxblk holds 4 * 1024 block maxima
-  if (c->precision == 1)  // the FP32-bulk form's grids are FP32
-    hipLaunchKernelGGL(k_max4<float>, dim3(nb), dim3(TPB), 0, c->stream, nnode, c->b32.grid[0],
-                       c->b32.grid[1], c->b32.grid[2], c->b32.pgrid[0], c->b32.pgrid[1],
-                       c->b32.pgrid[2], c->maxblk);
-  else
-    hipLaunchKernelGGL(k_max4<double>, dim3(nb), dim3(TPB), 0, c->stream, nnode, c->grid[GU],
-                       c->grid[GV], c->grid[GW], c->grid[GP], c->grid[GQ], c->grid[GR],
-                       c->maxblk);
-  hipLaunchKernelGGL(k_max4_final, dim3(1), dim3(TPB), 0, c->stream, (int)nb, c->maxblk, c->dsc);
-  hipLaunchKernelGGL(k_select_dt, dim3(1), dim3(1), 0, c->stream, g, c->dsc);
   PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
