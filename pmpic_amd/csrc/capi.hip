@@ -192,7 +192,7 @@ int free_all(Ctx *c) {
   for (int g = 1; g < 6; g++) hipFree(c->sder[g]);
   hipFree(c->atop); hipFree(c->abot);
   hipFree(c->ubar); hipFree(c->vbar);
-  hipFree(c->kx); hipFree(c->ky); hipFree(c->k2); hipFree(c->filt); hipFree(c->coords);
+  hipFree(c->kx); hipFree(c->ky); hipFree(c->k2); hipFree(c->filt); hipFree(c->lcut); hipFree(c->coords);
   hipFree(c->dz_den); hipFree(c->dz_cp); hipFree(c->dz_rcp);
   hipFree(c->lpool); hipFree(c->lap_bad);
   hipFree(c->fbuf);
@@ -288,6 +288,7 @@ int create(const pmpic_config *cf, Ctx *c) {
   PMPIC_TRY(dalloc(&c->ky, plane));
   PMPIC_TRY(dalloc(&c->k2, plane));
   PMPIC_TRY(dalloc(&c->filt, plane));
+  PMPIC_TRY(dalloc(&c->lcut, g.sy / 2));
   PMPIC_TRY(dalloc(&c->dz_den, 2 * (int64_t)g.nzn));
   PMPIC_TRY(dalloc(&c->dz_cp, 2 * (int64_t)g.nzn));
   PMPIC_TRY(dalloc(&c->dz_rcp, 2 * (int64_t)g.nzn));

@@ -27,8 +27,8 @@
 //
 // Bound by memory on large grids (26 passes over a spectral array where the separate kernels took
 // 41) and by the instruction latency of one wavefront on small ones.  A call, against the sum of
-// the ten kernels it stands for: 199 / 540 us at 256x256x128 FP32 (4.6 TB/s), 143 / 280 us at
-// 128x128x128 FP64, 22 / 91 us at 48x48x48 FP32, 9 / 26 us at 12x10x8 FP64.
+// the ten kernels it stands for: 170 / 540 us at 256x256x128 FP32, 125 / 280 us at
+// 128x128x128 FP64 (197 and 143 before the tiles that the filter clears left its zeros alone), 22 / 91 us at 48x48x48 FP32, 9 / 26 us at 12x10x8 FP64.
 #include "common.h"
 
 #include <type_traits>
@@ -245,7 +245,10 @@ __device__ __forceinline__ void columns(const Geometry &g, const ColumnArrays<S>
   auto at = [&](S *p, int k, int i) { return p + ((int64_t)tile * nz + k) * 64 + (lane + i * 64); };
   auto get = [&](S *p, int k, int i) { return *at(p, k, i); };
   auto put = [&](S *p, int k, int i, double v) { *at(p, k, i) = (S)v; };
-  auto put_filtered = [&](S *p, int k, int i, S v) { *at(p, k, i) = pass ? v : (S)0; };
+  // (where none of the tile's columns passes, the zeros are there since the arrays were allocated)
+  auto put_filtered = [&](S *p, int k, int i, S v) {
+    if (KEEP || SPLIT) *at(p, k, i) = pass ? v : (S)0;
+  };
   auto tab = [&](const double *t, int bc, int s, int i) {
     return (t + (((int64_t)bc * ntile + tile) * nz + s) * 16)[(lane >> 2) + i * 16];
   };

@@ -208,6 +208,10 @@ struct Ctx {
   double *abot, *atop;                // [sy][sx], standalone diffz's boundary planes
   double *ubar, *vbar;                // [nzn]
   double *kx, *ky, *k2, *filt;        // [sy][sx]
+  // the filter's extent: x wavenumbers it passes at y wavenumber m (the first lcut[m] of them), and
+  // the y wavenumbers at which it passes any (the first mcut)
+  int *lcut;
+  int mcut;
   // Thomas elimination: diffz's denominators and c' [bt][k] (the same for every column)
   double *dz_den, *dz_cp, *dz_rcp;
   // and the inverse Laplacian's by boundary condition, step and (m, l) block of columns:
@@ -396,8 +400,9 @@ int fft_setup(Ctx *c);
 int fft_forward(Ctx *c, int nf, const double *const *src, double *const *dst);
 // dst32 (optional, entries may be NULL): an FP32 copy of each real output.
 // deriv (optional): per field, SPEC_PLAIN, or SPEC_DX / SPEC_DY to transform diffx / diffy of
-// the input (applied while the input is read, so the derivative is never stored)
-enum SpecOp { SPEC_PLAIN = 0, SPEC_DX = 1, SPEC_DY = 2 };
+// the input (applied while the input is read, so the derivative is never stored); SPEC_FILTERED is
+// added where the input is zero outside the filter
+enum SpecOp { SPEC_PLAIN = 0, SPEC_DX = 1, SPEC_DY = 2 , SPEC_FILTERED = 4};
 int fft_backward(Ctx *c, int nf, const double *const *src, double *const *dst,
                  float *const *dst32 = nullptr, const int *deriv = nullptr);
 // the same transforms with spectral arrays (and the transforms' arithmetic) of type S; the

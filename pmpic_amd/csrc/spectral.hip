@@ -871,6 +871,15 @@ int spectral_setup(Ctx *c) {
   PMPIC_CHECK(hipMemcpy(c->ky, ky.data(), b, hipMemcpyHostToDevice));
   PMPIC_CHECK(hipMemcpy(c->k2, k2.data(), b, hipMemcpyHostToDevice));
   PMPIC_CHECK(hipMemcpy(c->filt, fl.data(), b, hipMemcpyHostToDevice));
+  std::vector<int> lcut(sy / 2, 0);
+  c->mcut = 0;
+  for (int m = 0; m < sy / 2; m++)
+    for (int l = 0; l < sx / 2; l++)
+      if (fl[(2 * m) * sx + 2 * l] != 0.) {
+        lcut[m] = l + 1;
+        c->mcut = m + 1;
+      }
+  PMPIC_CHECK(hipMemcpy(c->lcut, lcut.data(), sizeof(int) * lcut.size(), hipMemcpyHostToDevice));
   const int64_t plane = (int64_t)sx * sy;
   hipLaunchKernelGGL(k_dz_tables, dim3(1), dim3(1), 0, c->stream, g, c->dz_den, c->dz_cp);
   PMPIC_CHECK(hipGetLastError());
@@ -1003,9 +1012,10 @@ static int vort2vel_spectral_t(Ctx *c) {
   S *su = sp<S>(c->su), *sv = sp<S>(c->sv), *sw = sp<S>(c->sw);
   const S *src[14] = {sp<S>(c->sd), sp<S>(c->se), sp<S>(c->sf), sp<S>(c->sder[2]),
                       sp<S>(c->sder[3]), sp<S>(c->sder[4]), sbs, su, su, sw, sbs, sv, sv, sw};
-  const int op[14] = {SPEC_PLAIN, SPEC_PLAIN, SPEC_PLAIN, SPEC_PLAIN, SPEC_PLAIN,
-                      SPEC_PLAIN, SPEC_DY,    SPEC_DX,    SPEC_DY,    SPEC_DX,
-                      SPEC_DX,    SPEC_DX,    SPEC_DY,    SPEC_DY};
+  constexpr int F = SPEC_FILTERED;
+  const int op[14] = {SPEC_PLAIN | F, SPEC_PLAIN | F, SPEC_PLAIN | F, SPEC_PLAIN,  SPEC_PLAIN,
+                      SPEC_PLAIN,     SPEC_DY,        SPEC_DX | F,    SPEC_DY | F, SPEC_DX | F,
+                      SPEC_DX,        SPEC_DX | F,    SPEC_DY | F,    SPEC_DY | F};
   double *dst[14] = {c->grid[GP], c->grid[GQ], c->grid[GR], c->grid[GU], c->grid[GV], c->grid[GW]};
   float *dst32[14] = {};
   for (int f = 0; f < 8; f++) dst[6 + f] = c->gtmp[f];
