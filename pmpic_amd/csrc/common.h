@@ -235,6 +235,7 @@ struct Ctx {
   DevScalars *dsc;                    // device scalars
   DevScalars hsc;                     // host mirror
   void *pin;                          // pinned host staging for small read-backs (256 B)
+  double *ref_pin;                    // pinned, for small arrays in the reference's layout (ref_out)
   hipEvent_t sync_ev;                 // read-back completion (spin wait)
   char *hc_pin;                       // copy_host's slots, allocated at its first large copy
   hipEvent_t hc_ev[HOST_SLOTS];

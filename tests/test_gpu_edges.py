@@ -343,3 +343,22 @@ def test_binning_after_mixing(oracle_mod, change, bar):
     for k in ("x", "y", "z", "p", "q", "r"):
         bar(k, rel_err(got[k], want[k]), 1e-12)
     g.close()
+
+
+@pytest.mark.parametrize("shape", [(12, 10, 55), (60, 60, 63), (60, 60, 64)])
+def test_exports_around_the_pinned_size(oracle_mod, shape, bar):
+    """Arrays handed out through pinned memory (up to 2^18 values with halos: 64 x 64 x 64) and
+    through a copy: the transforms and exports one after another, none changing the one before
+    it, halos included; 1e-12 of the maximum."""
+    o, g = _pair(oracle_mod, shape, thermal_case(*shape, ppc_dir=1, vort=0.5))
+    grid = np.random.default_rng(7).standard_normal(o.gshape)
+    spec, want = g.fft_forward(grid), o.fft_forward(grid)
+    back = g.fft_backward(want)
+    g.step(1)
+    o.step()
+    u, v = g.grid("u"), g.grid("v")
+    bar("forward", rel_err(spec, want), 1e-12)
+    for name, got, ref in (("back", back, o.fft_backward(want)), ("u", u, o.grid("u")),
+                           ("v", v, o.grid("v"))):
+        inner = ref[2:-2, 2:-2]
+        bar(name, rel_err(got, np.pad(inner, ((2, 2), (2, 2), (0, 0)), mode="wrap")), 1e-12)
