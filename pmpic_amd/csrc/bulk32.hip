@@ -1201,6 +1201,7 @@ int dalloc32(T **p, int64_t n) {
 // the counts, the cursor behind them and the overflow list's length at zero (the accumulation that
 // uses a binning leaves them so)
 int zero_counts(Ctx *c) {
+  c->b32.mix_moves = 0;
   if (c->b32.counts_zero) return PMPIC_OK;
   hipLaunchKernelGGL(k32_bin_reset, dim3(cdiv(c->ncell + 1, TPB)), dim3(TPB), 0, c->stream,
                      c->cell_count, c->ncell + 1, c->dsc);
@@ -1375,11 +1376,12 @@ int b32_alloc(Ctx *c) {
   b.captune = false;
   b.captuned = 0;
   b.rk_tpb = TPB;
-  // binning fused into RK stages 1-3: it costs the RK kernel more than the separate binning
-  // pass on small grids (the 32^3..96^3 ensemble members: 1% slower) and saves on large ones
-  // (256 x 256 x 128: 1.6% faster), so from 2^21 cells on; PMPIC_FUSED_BINNING=0 or 1 forces it
+  // Binning fused into the RK stages (1 and 3; stage 2 moves entries): a pass of its own reads the
+  // cells again and is one more launch a stage (ms a step, apart and fused: 16x12x12 0.232 and 0.220,
+  // 48^3 0.474 and 0.462, a stirred 90x60x41 1.035 and 1.014, eight members together 9.73 and 9.68,
+  // 128^3 3.97 and 3.86, 256x256x128 15.68 and 15.38).  PMPIC_FUSED_BINNING=0 forces the pass.
   const char *fenv = getenv("PMPIC_FUSED_BINNING");
-  b.fused_bin = fenv ? fenv[0] == '1' : c->ncell >= ((int64_t)1 << 21);
+  b.fused_bin = fenv ? fenv[0] == '1' : true;
   b.binned = false;
   b.moving = c->cap <= (int64_t)1 << 27;
   // every parcel past its cell's capacity, every one moved there, and what mixing adds (MIX_MOVES)
@@ -1602,8 +1604,9 @@ int b32_rk_stage(Ctx *c, int stage, int stretch) {
   b.p2g_reuse = false;
   const dim3 gb(cdiv(c->graph_n ? c->graph_n : n, b.rk_tpb)), tb(b.rk_tpb);
   // Stage 2 moves the entries of the parcels that its better velocity takes to another cell (per
-  // mille of them; 67 M parcels: 2.38 -> 1.62 ms against binning them all).  Otherwise stages 1-3 may bin the cells they write for the next stage's par2grid
-  // (not while the capacity is being tuned).  Stage 4 is followed by splitting and mixing, whose
+  // mille of them; 67 M parcels: 2.38 -> 1.62 ms against binning them all).  Otherwise stages 1-3
+  // may bin the cells they write for the next stage's par2grid (not while the capacity is being
+  // tuned).  Stage 4 is followed by splitting and mixing, whose
   // binning compares the cells of both sets.
   const int capc = b32_choose_capc(c, n);
   const bool stands = b.binned && b.binned_set == from && b.binned_n == n && b.capc == capc;
@@ -1716,7 +1719,8 @@ int b32_mix(Ctx *c) {
   // removed parcels leave them before new ones take their slots.
   const bool none = reuse && Z + nadd == 0;  // the next par2grid wants no lists
   const bool lists = b.moving && b.capc > 0 && !c->graph_on && !none && norig + nadd < c->cap &&
-                     Z + nadd <= norig / MIX_MOVES;
+                     b.mix_moves + Z + nadd <= norig / MIX_MOVES;
+  if (lists) b.mix_moves += Z + nadd;
   const BinOut bo = bin_out(c, lists ? 2 : 0, b.capc);
   if (Z > 0 && (lists || reuse))
     hipLaunchKernelGGL(k32_unlist, dim3(cdiv(Z, TPB)), dim3(TPB), 0, c->stream, g, P.cell,

@@ -83,8 +83,8 @@ struct Bulk32 {
   // into FP64 grid GP, GQ, GR, GB (k = 0..3) while p2g_pending[k]
   float *pgrid[4];
   bool p2g_pending[4];
-  // RK stages 1-3 bin the cells they write for the next par2grid (fused_bin: grids of 2^21
-  // cells or more, or as PMPIC_FUSED_BINNING says)
+  // RK stages 1 and 3 (and 2 where no entries can move) bin the cells they write for the next
+  // par2grid (unless PMPIC_FUSED_BINNING=0 or the tuned configuration says otherwise)
   bool fused_bin;
   // The lists built last still stand (`binned`): for the cells of set binned_set, binned_n parcels
   // and the capacity capc.  moving: stages 2 and 4, which hardly move a parcel out of the cell that
@@ -93,6 +93,7 @@ struct Bulk32 {
   bool binned, moving;
   int binned_set;
   int64_t binned_n;
+  int64_t mix_moves;  // changes of mixing that they followed since they were built
   bool counts_zero;   // the cell counts are zero, as a binning wants them
   // the last mixing's kept sums are the next par2grid's partials except on the
   // tiles mixing changed (dirty: one byte per 8-cell tile); p2g_reuse while that holds (set by
