@@ -449,7 +449,7 @@ __global__ void k32_dense_scatter(Geometry g, const int32_t *__restrict__ cellv,
 // barrier ties wavefronts together, so the CU's 32 overlap each other's loads and sums.  It is
 // bound by the latency of the gathers: three 12-byte records a parcel, and
 // half by the issue of the sums.  67 M parcels that have moved a few cells: 1.39 ms with nine 4-byte
-// gathers and a workgroup staging all parcels of 16 cells, 1.14 ms (2.6 TB/s); 1.8 M well mixed
+// gathers and a workgroup staging all parcels of 16 cells, 1.12 ms (2.6 TB/s); 1.8 M well mixed
 // ones in 221 k cells: 87 -> 58 us.
 //
 // Within a cell the additions run in ascending parcel order, so the sums do not depend on the
@@ -681,12 +681,17 @@ __global__ void __launch_bounds__(64) k32_cell_accum(
         sval[lane] = make_float4(vor.x, vor.y, vor.z, fmaf(12.5f, hl > 0.f ? hl : 0.f, vbh.y));
         if constexpr (MIX) sval2[lane] = make_float2(vbh.y, vbh.z);
       }
+    } else if constexpr (!MIX) {
+      sgeo[lane] = sval[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (NV > 4) sval2[lane] = make_float2(0.f, 0.f);
     }
     __syncthreads();
     if (ch + 1 < nch) fetch(ch + 1);
     const int rows = min(8, nmax - 8 * ch), mine = n - 8 * ch;
-#pragma unroll 2
-    for (int a = 0; a < rows; a++) {
+    // (without a test for each row: those past a cell's parcels hold zeros.  256x256x128: 20.11 ->
+    // 19.93 ms a step; mixing can't, its zero volume would count as a parcel to remove)
+#pragma unroll MIX ? 2 : 4
+    for (int a = 0; a < (MIX ? rows : (rows + 3) / 4 * 4); a++) {
       const int r = 8 * a + cl;
       const float4 ge = sgeo[r], v4 = sval[r];
       float v[6] = {v4.x, v4.y, v4.z, v4.w, 0.f, 0.f};
@@ -695,11 +700,13 @@ __global__ void __launch_bounds__(64) k32_cell_accum(
         v[5] = sval2[r].y;
       }
       const float w = corner_weight(ge.x, ge.y, ge.z, ge.w, tx, ty, tz);
-      if (a < mine) {
-        if (!MIX || !(ge.w < vmin)) {
+      if constexpr (!MIX) {
+        add_parcel<NV>(acc, w, v);
+      } else if (a < mine) {
+        if (!(ge.w < vmin)) {
           add_parcel<NV>(acc, w, v);
           kept++;
-        } else if constexpr (MIX) {
+        } else {
           anyres = true;
           add_parcel<NV>(res, w, v);
         }
