@@ -149,7 +149,7 @@ __host__ __device__ inline int64_t spec_at(int nzn, int nl, int k, int m, int l)
 enum TimerId { T_ACCUM = 0, T_RK = 1, T_VORT2VEL, T_VORT_TEND, T_RK4, T_SPLIT, T_MIX, NTIMERS };
 
 constexpr int MAXBLK = 1024;   // blocks of the timestep reduction
-constexpr int HOST_SLOTS = 8;  // pinned slots of the large host copies (copy_host)
+constexpr int HOST_THREADS = 4;  // of the large host copies (copy_host)
 
 constexpr int64_t BINS_NONE = -1, BINS_STALE = -2;  // Ctx::bins_n
 
@@ -238,8 +238,8 @@ struct Ctx {
   void *pin;                          // pinned host staging for small read-backs (256 B)
   double *ref_pin;                    // pinned, for small arrays in the reference's layout (ref_out)
   hipEvent_t sync_ev;                 // read-back completion (spin wait)
-  char *hc_pin;                       // copy_host's slots, allocated at its first large copy
-  hipEvent_t hc_ev[HOST_SLOTS];
+  char *hc_pin[HOST_THREADS];         // copy_host's slots, two a thread, allocated at their first use
+  hipEvent_t hc_ev[2 * HOST_THREADS];
   // FP32-bulk form with PMPIC_GRAPH=1: RK stages 1-3 of a step (vort2vel, vorticity_tendency,
   // rk4_integrator; the splitting and mixing callbacks do nothing there) captured once as a HIP
   // graph and replayed by later steps; the stage-4 work, whose launches depend on data read

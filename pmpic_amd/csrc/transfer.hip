@@ -2,8 +2,10 @@
 //
 // The caller's memory is pageable, and the runtime's copy of it passes through one thread:
 // 17 GB/s to the host (11 where the pages are new), 29 from it, of a link that carries 57 to pinned
-// memory.  A large copy here is cut into chunks that several threads carry through pinned slots of
-// their own, two each, the link moving one while the thread copies the other.
+// memory; and from about a megabyte on it pins the caller's pages for the copy, which can stall the
+// program for milliseconds when it next maps or releases memory.  Here such a copy is cut into chunks
+// that threads (a large one's four, else the caller's alone) carry through pinned slots of their
+// own, two each, the link moving one while the thread copies the other.
 #include "common.h"
 
 #include <string.h>
@@ -17,11 +19,15 @@ namespace pmpic {
 namespace {
 
 constexpr size_t CHUNK = (size_t)1 << 20;
-constexpr int THREADS = 4;  // the caller's and three more, for the length of the call
-// Below this the threads' start and, where the caller's pages are new, their contention for the
-// address space cost more than they save (grids of 5.4 MB into new arrays: 0.47 ms each through the
-// runtime, 0.42 at best and 1 in the median here).
-constexpr size_t LEAST = (size_t)16 << 20;
+constexpr int THREADS = HOST_THREADS;  // the caller's and three more, for the length of the call
+// Below this the runtime's own copy, which doesn't pin.  Above it, a 60x180x28 run's exports of 2.7 MB
+// left the program's next allocation waiting 4 ms in the median (pass 18.4 ms, now 11.9), and eight
+// members' 59 ms a pass is 57.
+constexpr size_t LEAST_PINNED = CHUNK;
+// Below this one thread: the others' start and, where the caller's pages are new, their contention
+// for the address space cost more than they save (a dump of ten grids of 5.4 MB: 4.7 ms through the
+// runtime, 4.3 with one thread, 4.2 at best and 10 in the median with four).
+constexpr size_t LEAST_THREADS = (size_t)16 << 20;
 
 struct Copy {
   Ctx *c;
@@ -55,8 +61,7 @@ struct Copy {
   // one thread's share, through slots 2 w and 2 w + 1
   void run(int w) {
     if (!ok(hipSetDevice(c->device))) return;
-    char *const slot[2] = {c->hc_pin + (size_t)(2 * w) * CHUNK,
-                           c->hc_pin + (size_t)(2 * w + 1) * CHUNK};
+    char *const slot[2] = {c->hc_pin[w], c->hc_pin[w] + CHUNK};
     hipEvent_t *const ev = c->hc_ev + 2 * w;
     char *host[2], *dev[2];
     size_t len[2] = {0, 0};
@@ -93,15 +98,17 @@ struct Copy {
   }
 };
 
-int ensure_slots(Ctx *c) {
-  if (c->hc_pin) return PMPIC_OK;
-  static_assert(2 * THREADS == HOST_SLOTS, "two slots a thread");
-  for (int i = 0; i < HOST_SLOTS; i++)
-    if (!c->hc_ev[i])
-      PMPIC_CHECK(hipEventCreateWithFlags(&c->hc_ev[i], hipEventDisableTiming));
-  void *p = nullptr;
-  PMPIC_CHECK(hipHostMalloc(&p, HOST_SLOTS * CHUNK));
-  c->hc_pin = static_cast<char *>(p);
+// two slots and their events for each of n threads
+int ensure_slots(Ctx *c, int n) {
+  for (int w = 0; w < n; w++) {
+    for (int i = 2 * w; i < 2 * w + 2; i++)
+      if (!c->hc_ev[i])
+        PMPIC_CHECK(hipEventCreateWithFlags(&c->hc_ev[i], hipEventDisableTiming));
+    if (c->hc_pin[w]) continue;
+    void *p = nullptr;
+    PMPIC_CHECK(hipHostMalloc(&p, 2 * CHUNK));
+    c->hc_pin[w] = static_cast<char *>(p);
+  }
   return PMPIC_OK;
 }
 
@@ -114,7 +121,8 @@ int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
     total += part[k].bytes;
     job.nchunks += (int64_t)((part[k].bytes + CHUNK - 1) / CHUNK);
   }
-  if (total < LEAST || ensure_slots(c) != PMPIC_OK) {
+  const int threads = total < LEAST_THREADS ? 1 : THREADS;
+  if (total < LEAST_PINNED || ensure_slots(c, threads) != PMPIC_OK) {
     for (int k = 0; k < nparts; k++)
       if (part[k].bytes)
         PMPIC_CHECK(hipMemcpyAsync(to_host ? part[k].host : part[k].dev,
@@ -125,7 +133,7 @@ int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
     return PMPIC_OK;
   }
   std::thread th[THREADS - 1];
-  for (int w = 1; w < THREADS; w++) {
+  for (int w = 1; w < threads; w++) {
     try {
       th[w - 1] = std::thread([&job, w]() { job.run(w); });
     } catch (const std::system_error &) {
@@ -139,9 +147,10 @@ int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
 }
 
 void free_host_slots(Ctx *c) {
-  if (c->hc_pin) hipHostFree(c->hc_pin);
-  for (int i = 0; i < HOST_SLOTS; i++)
-    if (c->hc_ev[i]) hipEventDestroy(c->hc_ev[i]);
+  for (char *p : c->hc_pin)
+    if (p) hipHostFree(p);
+  for (hipEvent_t e : c->hc_ev)
+    if (e) hipEventDestroy(e);
 }
 
 }  // namespace pmpic

@@ -260,10 +260,10 @@ def test_moved_entries_change_no_result(monkeypatch, case, shape, fused, mixing)
         g.close()
 
 
-@pytest.mark.parametrize("n", [123_361, 123_362, 131_072, 131_073, 400_001])
+@pytest.mark.parametrize("n", [7_709, 7_710, 15_420, 123_361, 123_362, 131_072, 131_073, 400_001])
 def test_large_host_copies(n):
-    """Parcel arrays to the device and back either side of the size from which several threads
-    carry them (16 MB in 17 arrays), with whole and odd last chunks of 1 MB, from two contexts at a
+    """Parcel arrays to the device and back either side of the sizes from which they go through
+    pinned slots (1 MB in 17 arrays) and from which several threads carry them (16 MB), with whole and odd last chunks of 1 MB, from two contexts at a
     time: every value comes back as it went."""
     import threading
     from pmpic_amd.lib import PARCEL_FIELDS, Context
