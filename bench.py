@@ -32,25 +32,25 @@ METRIC = "parcel-steps/s FP32-bulk vs FP64 on 1 MI355X at ≤1e-5 vel err; HBM G
 HBM_PEAK_GBS = 8000.0
 
 # algorithmic bytes per launch of the two hot kernels
-#  cell accumulation: per parcel the bucket entry (4 B) and x,y,z,vol,p,q,r,b,h (72 B);
-#    per cell two bucket offsets (8 B) and 40 corner partial sums written (320 B)
-#  gather + RK stage: per parcel position (24 B), RK state read/written for the stage, six
-#    tendencies written (48 B), direction flag (1 B); per node the six gathered grids (48 B)
-RK_STAGE_BYTES = {1: 24 + 24 + 18 * 8 + 48 + 1, 2: 24 + 12 * 8 + 12 * 8 + 48 + 1,
-                  3: 24 + 12 * 8 + 12 * 8 + 48 + 1, 4: 24 + 7 * 8 + 13 * 8 + 48 + 1}
-# FP32-bulk form: cell accumulation reads per parcel its slot entry, offsets, vol, p,q,r,b,h
-# (40 B; the z level comes from the cell) and per cell its count and overflow offset (8 B);
-# it writes 40 FP32 corner partials per cell (160 B), or, when nx is a multiple of 16 (tiles
-# of 16 cells in one x row), the partials combined along x: 4 corner pairs x 17 node positions
-# x 5 values per 16 cells (85 B per cell).  The RK stages move cell (4 B) + offsets (12 B) for
-# the position and the FP32 RK state (see bulk32.hip)
-ACC_BYTES = {0: (76, 328), 1: (40, 168)}
-ACC_BYTES_XROWS = (40, 8 + 85)
-RK32_STAGE_BYTES = {1: 28 + 80, 2: 68 + 52, 3: 68 + 52, 4: 60 + 56}
-# on grids of 2^21 cells or more, RK stages 1-3 also bin the cells they write: a 4-byte slot
-# entry per parcel (the count atomics, one per run of a cell's parcels, left out)
+#  cell accumulation: per parcel the bucket entry (4 B) and x,y,z,vol,p,q,r,b,h (72 B); per cell
+#    the bucket's start and count (8 B) and the partials written, combined along x: 4 corner pairs
+#    x 9 node positions x 5 values per 8 cells (180 B per cell)
+#  gather + RK stage: per parcel position (24 B), RK state read/written for the stage, at stage 4
+#    six tendencies written (48 B; within a whole step no other stage's are stored), direction
+#    flag (1 B); per node the record of the six gathered values (48 B)
+RK_STAGE_BYTES = {1: 24 + 3 * 8 + 18 * 8 + 1, 2: 24 + 12 * 8 + 12 * 8 + 1,
+                  3: 24 + 12 * 8 + 12 * 8 + 1, 4: 24 + 7 * 8 + 13 * 8 + 48 + 1}
+# FP32-bulk form: cell accumulation reads per parcel its slot entry, offsets, vorticity and vol, b,
+# h (40 B; the z level comes from the cell) and per cell its count and overflow offset (8 B); the
+# partials are half the size (90 B per cell).  The RK stages move cell (4 B) + offsets (12 B) for
+# the position and the FP32 RK state (see bulk32.hip); a node's record is two float4 (32 B)
+ACC_BYTES = {0: (76, 8 + 180), 1: (40, 8 + 90)}
+RK32_STAGE_BYTES = {1: 28 + 52, 2: 68 + 52, 3: 68 + 52, 4: 60 + 56}
+# RK stages 1 and 3 also bin the cells they write: a 4-byte slot entry per parcel (the count
+# atomics, one per run of a cell's parcels, left out); stage 2 moves the entries of the parcels
+# that change cell
 RK32_BIN_BYTES = 4
-GATHER_NODE_BYTES = {0: 48, 1: 24}
+GATHER_NODE_BYTES = {0: 48, 1: 32}
 
 
 def parse():
@@ -220,23 +220,20 @@ def time_form(precision, ic, args, n, nz):
     nnode = n * n * (nz + 1)
     avg_np = total / max(args.steps, 1)
     form = "fp32" if precision else "fp64"
-    xrows = precision == 1 and n % 16 == 0  # the FP32 accumulation's x-combined partials
-    acc_bytes = ACC_BYTES_XROWS if xrows else ACC_BYTES[precision]
+    acc_bytes = ACC_BYTES[precision]
     acc = {
         "kernel": ("k32_cell_accum (FP32 par2grid cell sums, corner partials combined along x)"
-                   if xrows else
-                   "k32_cell_accum (FP32 par2grid per-cell corner sums)" if precision else
-                   "k_cell_accum (par2grid per-cell corner sums)"),
-        "family": ("k_cell_accum_lds<0>" if not precision else
-                   "k32_cell_accum<3>" if xrows else "k32_cell_accum<0>"),
+                   if precision else
+                   "k_cell_accum (par2grid cell sums, corner partials combined along x)"),
+        "family": "k32_cell_accum<0>" if precision else "k_cell_accum<0>",
         "bytes": avg_np * acc_bytes[0] + ncell * acc_bytes[1],
         "ms": p2g_ms, "calls": p2g_calls,
     }
     table = dict(RK32_STAGE_BYTES if precision else RK_STAGE_BYTES)
     fenv = os.environ.get("PMPIC_FUSED_BINNING")
-    fused = precision == 1 and (fenv == "1" if fenv else ncell >= (1 << 21))
+    fused = precision == 1 and (not fenv or fenv[0] == "1")
     if fused:
-        for s_ in (1, 2, 3):
+        for s_ in (1, 3):
             table[s_] += RK32_BIN_BYTES
     rks = {
         "kernel": ("k32_rk_stage (FP32 grid2par of 6 fields + RK4 stage update"
