@@ -269,9 +269,10 @@ __global__ void k32_bin_slot(Geometry g, const int32_t *__restrict__ cellv, int6
   const int32_t n32 = (int32_t)dsc->n;
   if (n32 == 0 || w0 >= n32) return;
   // all count atomics of the wavefront are issued before any result is used, in group order;
-  // ch[it] = cell << 6 | head lane of the parcel's run (the cell part is only used while the
-  // slot table exists, ncell * capc < 2^30)
-  int base[BIN_SEQ], ch[BIN_SEQ];
+  // run[it]: the cell and the head lane of the parcel's run (the cell is only used while the slot
+  // table exists, whose grids have at most 2^26 cells)
+  int base[BIN_SEQ];
+  uint32_t run[BIN_SEQ];
   int32_t cv[BIN_SEQ];  // every load issued before the first is used (clamped index, n >= 1)
 #pragma unroll
   for (int it = 0; it < BIN_SEQ; it++)
@@ -288,13 +289,13 @@ __global__ void k32_bin_slot(Geometry g, const int32_t *__restrict__ cellv, int6
     const unsigned long long above = hm & ~((2ull << hl) - 1ull);
     const int next = above ? (__ffsll(above) - 1) : 64;
     base[it] = (head && c >= 0) ? atomicAdd(&count[c], next - hl) : 0;
-    ch[it] = (int)((uint32_t)c << 6) | hl;
+    run[it] = pack_run(c, hl);
   }
   if (capc == 0) {
 #pragma unroll
     for (int it = 0; it < BIN_SEQ; it++) {
       const int32_t p = w0 + it * 64 + lane;
-      const int hl = ch[it] & 63;
+      const int hl = run_head(run[it]);
       const int32_t rk = __shfl(base[it], hl) + (lane - hl);
       if (p < n32) st(rankv, (uint32_t)p, rk);
     }
@@ -304,10 +305,10 @@ __global__ void k32_bin_slot(Geometry g, const int32_t *__restrict__ cellv, int6
 #pragma unroll
   for (int it = 0; it < BIN_SEQ; it++) {
     const int32_t p = w0 + it * 64 + lane;
-    const int hl = ch[it] & 63;
+    const int hl = run_head(run[it]);
     const int32_t rk = __shfl(base[it], hl) + (lane - hl);
     if (p < n32) {
-      if (rk < capc) st(slot, (uint32_t)((ch[it] >> 6) * capc + rk), p);
+      if (rk < capc) st(slot, (uint32_t)(run_cell(run[it]) * capc + rk), p);
       else anyover = true;
     }
   }
@@ -315,7 +316,7 @@ __global__ void k32_bin_slot(Geometry g, const int32_t *__restrict__ cellv, int6
 #pragma unroll
   for (int it = 0; it < BIN_SEQ; it++) {
     const int32_t p = w0 + it * 64 + lane;
-    const int hl = ch[it] & 63;
+    const int hl = run_head(run[it]);
     const int32_t rk = __shfl(base[it], hl) + (lane - hl);
     const bool over = (p < n32) && rk >= capc;
     const unsigned long long om = __ballot(over);
@@ -327,7 +328,7 @@ __global__ void k32_bin_slot(Geometry g, const int32_t *__restrict__ cellv, int6
       if (over) {
         const int32_t o = ob + __popcll(om & ((1ull << lane) - 1ull));
         ovf[o] = make_int2(p, rk);
-        ovfc[o] = ch[it] >> 6;
+        ovfc[o] = run_cell(run[it]);
         if (where) where[p] = o;
       }
     }

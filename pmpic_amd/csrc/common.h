@@ -364,6 +364,13 @@ __device__ __forceinline__ int64_t gidx(const Geometry &g, int k, int j, int i) 
   return ((int64_t)k * g.ny + j) * g.nx + i;
 }
 
+// a cell below 2^26 and the head lane of its run of parcels, in 32 bits
+__host__ __device__ inline uint32_t pack_run(int32_t cell, int head) {
+  return (uint32_t)cell << 6 | (uint32_t)head;
+}
+__host__ __device__ inline int32_t run_cell(uint32_t run) { return (int32_t)(run >> 6); }
+__host__ __device__ inline int run_head(uint32_t run) { return (int)(run & 63u); }
+
 // Buffers of one FP64 binning + single-field par2grid: the context's own, or caller-provided
 // memory (pmpic_par2grid_noalloc).  cell, rank, sorted: n entries; count, start: ncell; cursor: one
 // entry; partial: 12 * ncell doubles.  count and cursor are zero between calls.
