@@ -182,13 +182,27 @@ int download(Ctx *c, std::vector<double> &h, const double *src, size_t n) {
 }
 
 
+__global__ void k_set_scalars(DevScalars *sc, double dtm, double dtmax, double prefactor, int64_t n) {
+  if (threadIdx.x || blockIdx.x) return;
+  sc->dtm = dtm;
+  sc->dtmax = dtmax;
+  sc->prefactor = prefactor;
+  sc->n = n;
+  sc->status = 0;
+}
+
+// The device scalars the host sets, in stream order.  The others belong to the kernels (the length
+// of the overflow list, for one, has to fit the lists as they are by now), and the mirror's may be
+// older than theirs.
 int set_dev_scalars(Ctx *c) {
+  hipLaunchKernelGGL(k_set_scalars, dim3(1), dim3(64), 0, c->stream, c->dsc, c->dtm, c->dtmax,
+                     c->prefactor, c->n);
+  PMPIC_CHECK(hipGetLastError());
   c->hsc.dtm = c->dtm;
   c->hsc.dtmax = c->dtmax;
   c->hsc.prefactor = c->prefactor;
   c->hsc.n = c->n;
   c->hsc.status = 0;
-  PMPIC_CHECK(hipMemcpy(c->dsc, &c->hsc, sizeof(DevScalars), hipMemcpyHostToDevice));
   return PMPIC_OK;
 }
 

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from tests.cases import LX, LZ
+from tests.cases import LX, LZ, box, crowded_case
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +49,74 @@ def test_crowded_cells_past_2_25():
             for name, field in (("p", "p"), ("hg", "h")):
                 want = np.sum(w * ic[field][s]) / np.sum(w)
                 assert abs(grids[name][i, j, c[2] + b[2]] - want) < 1e-5, (c, bits, name)
+
+
+@pytest.mark.parametrize("slots", ["16", "32"])
+@pytest.mark.parametrize("nx", [18, 32])
+@pytest.mark.parametrize("where", ["between_steps", "stage_1", "stage_3"])
+def test_set_time_between_components(monkeypatch, nx, slots, where):
+    """pmpic_set_time with the values that stand already changes nothing, wherever a caller puts it:
+    after a vort2vel that has used up the lists of crowded cells, between steps (with a grid export,
+    which waits for the device) or between the components of a stage.  The runs stay bit-identical."""
+    from pmpic_amd.lib import Context
+    monkeypatch.setenv("PMPIC_SLOT_CAPACITY", slots)
+    shape = (nx, 12, 8)
+    ic = crowded_case(*shape)
+    for k in "pqr":
+        ic[k] = 10.0 * ic[k]
+    b = box(*shape)
+    runs = []
+    for _ in range(2):
+        g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                    3 * len(ic["x"]), precision=1)
+        g.set_parcels(ic)
+        runs.append(g)
+
+    def set_same_time(g):
+        g.grid("p")
+        g.set_time(g.time, g.dtm)
+
+    for s in range(3):
+        for i, g in enumerate(runs):
+            if where == "between_steps":
+                if i:
+                    g.vort2vel()
+                    set_same_time(g)
+                g.step()
+                continue
+            for stage in (1, 2, 3, 4):
+                g.vort2vel()
+                if i and where == f"stage_{stage}":
+                    set_same_time(g)
+                g.vorticity_tendency()
+                g.rk4_integrator()
+                g.parcel_splitting()
+                g.parcel_mixing()
+        assert runs[0].n == runs[1].n
+        want, got = (g.get_parcels() for g in runs)
+        for k in want:
+            np.testing.assert_array_equal(got[k], want[k], err_msg=f"step {s}: {k}")
+        for k in ("u", "v", "w", "p", "q", "r", "b"):
+            np.testing.assert_array_equal(runs[1].grid(k), runs[0].grid(k), err_msg=f"{s}: {k}")
+    for g in runs:
+        g.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_set_time_sets_the_step(precision):
+    """The timestep given between vorticity_tendency, which selects one at stage 1, and
+    rk4_integrator is the one that the stage takes."""
+    from pmpic_amd.lib import Context
+    shape = (12, 10, 8)
+    ic = crowded_case(*shape, extra=(3,))
+    b = box(*shape)
+    g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                3 * len(ic["x"]), precision=precision)
+    g.set_parcels(ic)
+    g.vort2vel()
+    g.vorticity_tendency()
+    g.set_time(1.5, 0.00125)
+    assert g.state()[1:] == (1.5, 0.00125)
+    g.rk4_integrator()
+    assert g.state()[1:] == (1.5, 0.00125)
+    g.close()
