@@ -304,7 +304,8 @@ __device__ __forceinline__ void raise_status(DevScalars *s, int code) {
 
 // a / b rounded as the division rounds it, from r = 1 / b rounded to nearest: the quotient a r is
 // within an ulp and one residual corrects it (Markstein, IBM J. Res. Dev. 34, 1990).  Three
-// operations where the division takes about a dozen.
+// operations where the division takes about a dozen.  For finite quotients: of an infinite a, or an
+// a r that overflows, the residual makes a NaN.
 __device__ __forceinline__ double div_by(double a, double b, double r) {
   const double q = a * r;
   return fma(fma(-q, b, a), r, q);
@@ -324,7 +325,9 @@ __device__ __forceinline__ int locate(const Geometry &g, double xp, double yp, d
   // haloswap failed to wrap, which is rejected here instead of silently mis-deposited
   if (i < 3 || i > g.nx + 3) return PMPIC_ERR_OUT_OF_BOX_X;
   if (j < 3 || j > g.ny + 3) return PMPIC_ERR_OUT_OF_BOX_Y;
-  if (k < 1 || k >= g.nzn) return PMPIC_ERR_OUT_OF_BOX_Z;
+  // (the NaN that div_by makes of an infinite quotient converts to 0, which x and y refuse and z,
+  // whose grid has no halo below, would not)
+  if (k < 1 || k >= g.nzn || isinf(az * g.rdz)) return PMPIC_ERR_OUT_OF_BOX_Z;
   delx = div_by(ax - (double)(i - 1) * g.dx, g.dx, g.rdx);
   dely = div_by(ay - (double)(j - 1) * g.dy, g.dy, g.rdy);
   delz = div_by(az - (double)(k - 1) * g.dz, g.dz, g.rdz);

@@ -120,3 +120,28 @@ def test_set_time_sets_the_step(precision):
     g.rk4_integrator()
     assert g.state()[1:] == (1.5, 0.00125)
     g.close()
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, 1e308, -1e308, 1e300])
+@pytest.mark.parametrize("axis,status", [("x", 1), ("y", 2), ("z", 3)])
+def test_positions_without_a_cell_are_refused(axis, status, value):
+    """An infinite position, one whose quotient by the cell size overflows and one that does not:
+    refused in every call that finds a parcel's cell, out of the box or (4, above the box by more cells
+    than an integer holds) by its offset."""
+    from pmpic_amd.lib import Context, PmpicError
+    shape = (12, 10, 8)
+    ic = crowded_case(*shape, extra=(3,))
+    n = len(ic["x"])
+    ic[axis] = ic[axis].copy()
+    ic[axis][n // 2] = value
+    b = box(*shape)
+    g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"], 3 * n)
+    calls = {"cache_weights": g.cache_weights, "par2grid": lambda: g.par2grid(np.ones(n)),
+             "grid2par": lambda: g.grid2par(np.ones(g.gshape)),
+             "writebinary_grids": g.writebinary_grids, "step": g.step}
+    for name, call in calls.items():
+        g.set_parcels(ic)
+        with pytest.raises(PmpicError) as e:
+            call()
+        assert e.value.status in (status, 4 if value == 1e300 else status), name
+    g.close()
