@@ -107,8 +107,8 @@ int pmpic_grid2par(pmpic_ctx *ctx, const double *grid, double *var);
  * memory, written in pmpic_par2grid's layout with the same values, bit for bit.  The working
  * memory is one static device array of PMPIC_NOALLOC_SCRATCH_BYTES per GPU, held until the
  * process ends, so the sizes are capped: at most PMPIC_NOALLOC_MAX_PARCELS parcels and
- * PMPIC_NOALLOC_MAX_CELLS cells, else PMPIC_ERR_ARG.  Calls that overlap on one GPU (from two
- * threads or two contexts' streams) race on that array.  Plain FP64 form only. */
+ * PMPIC_NOALLOC_MAX_CELLS cells, else PMPIC_ERR_ARG.  Calls that overlap on one GPU (contexts
+ * stepped by two threads) take turns.  Plain FP64 form only. */
 #define PMPIC_NOALLOC_MAX_PARCELS (1 << 20)
 #define PMPIC_NOALLOC_MAX_CELLS (1 << 15)
 #define PMPIC_NOALLOC_SCRATCH_BYTES 17826304

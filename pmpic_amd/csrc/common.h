@@ -400,6 +400,7 @@ int par2grid_single_ws(Ctx *c, int64_t n, const double *d_var, double *d_grid, c
 int par2grid_fused(Ctx *c, int64_t n);  // P,Q,R,B grids from p,q,r,btot
 int par2grid_single(Ctx *c, int64_t n, const double *d_var, double *d_grid);
 int grid2par_single(Ctx *c, int64_t n, const double *d_grid, double *d_var);
+int zero_i32(Ctx *c, int32_t *a, int64_t n);
 int drop_bins(Ctx *c);  // before the parcels change their cells or slots
 // buckets of the cells of more than `held` parcels, from *cursor on
 void bin_alloc(Ctx *c, const int32_t *count, int held, int32_t *start, int32_t *cursor);

@@ -463,13 +463,16 @@ __global__ void k_zero_i32(int32_t *__restrict__ a, int64_t n) {
   if (i < n) a[i] = 0;
 }
 
+int zero_i32(Ctx *c, int32_t *a, int64_t n) {
+  hipLaunchKernelGGL(k_zero_i32, dim3(cdiv(n, TPB)), dim3(TPB), 0, c->stream, a, n);
+  PMPIC_CHECK(hipGetLastError());
+  return PMPIC_OK;
+}
+
 // the context's binning no longer stands: counts and cursor at zero
 int drop_bins(Ctx *c) {
-  if (c->bins_n != BINS_NONE)
-    hipLaunchKernelGGL(k_zero_i32, dim3(cdiv(c->ncell + 1, TPB)), dim3(TPB), 0, c->stream,
-                       c->cell_count, c->ncell + 1);
+  if (c->bins_n != BINS_NONE) PMPIC_TRY(zero_i32(c, c->cell_count, c->ncell + 1));
   c->bins_n = BINS_NONE;
-  PMPIC_CHECK(hipGetLastError());
   return PMPIC_OK;
 }
 

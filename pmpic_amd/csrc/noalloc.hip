@@ -8,10 +8,11 @@
 // or hipMalloc.  Inputs and the
 // output are the caller's device arrays.
 //
-// Every call on a GPU shares that GPU's array: calls that overlap on one GPU (two host threads,
-// or two streams) race on it.  The per-cell counts are zero at load and each call leaves them zero
-// again; every other region is written in full before it is read, so nothing from an earlier call
-// leaks into a later one.
+// Every call on a GPU shares that GPU's array, so calls that overlap (two host threads) take turns:
+// a call holds the GPU's lock until the device has finished, as it waits for its status anyway.  The
+// per-cell counts are zero at load and each call leaves them zero again; after one that failed the
+// next clears them first.  Every other region is written in full before it is read, so nothing from
+// an earlier call leaks into a later one.
 #include "common.h"
 
 #include <mutex>
@@ -46,14 +47,18 @@ static_assert(NA_TOTAL == PMPIC_NOALLOC_SCRATCH_BYTES, "scratch size in pmpic_hi
 static __device__ __align__(256) unsigned char scratch[NA_TOTAL];
 
 constexpr int NA_MAX_DEVICES = 64;
-std::mutex na_mutex;
-unsigned char *na_addr[NA_MAX_DEVICES];  // device address of `scratch` per device, once looked up
 
-// The address of `scratch` on `device`, looked up once per device with that device current.
+// A device's array: its address, once looked up, and whether the last call left the counts at zero
+struct Shared {
+  std::mutex turn;
+  unsigned char *addr;
+  bool unclean;
+};
+Shared na_shared[NA_MAX_DEVICES];
+
+// the address of `scratch` on `device`, looked up with that device current
 int scratch_addr(int device, unsigned char **out) {
-  if (device < 0 || device >= NA_MAX_DEVICES) return PMPIC_ERR_ARG;
-  std::lock_guard<std::mutex> lock(na_mutex);
-  if (!na_addr[device]) {
+  if (!*out) {
     int prev = 0;
     PMPIC_CHECK(hipGetDevice(&prev));
     if (prev != device) PMPIC_CHECK(hipSetDevice(device));
@@ -61,9 +66,32 @@ int scratch_addr(int device, unsigned char **out) {
     const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
     if (prev != device) PMPIC_CHECK(hipSetDevice(prev));
     if (e != hipSuccess || p == nullptr) return PMPIC_ERR_HIP;
-    na_addr[device] = static_cast<unsigned char *>(p);
+    *out = static_cast<unsigned char *>(p);
   }
-  *out = na_addr[device];
+  return PMPIC_OK;
+}
+
+int par2grid_in(Ctx *c, Shared &s, const double *var, double *grid) {
+  PMPIC_TRY(scratch_addr(c->device, &s.addr));
+  unsigned char *const base = s.addr;
+  BinWork w;
+  w.cell = reinterpret_cast<int32_t *>(base + NA_CELL);
+  w.rank = reinterpret_cast<int32_t *>(base + NA_RANK);
+  w.sorted = reinterpret_cast<int32_t *>(base + NA_SORTED);
+  w.count = reinterpret_cast<int32_t *>(base + NA_COUNT);
+  w.start = reinterpret_cast<int32_t *>(base + NA_START);
+  w.partial = reinterpret_cast<double *>(base + NA_PARTIAL);
+  w.cursor = reinterpret_cast<int32_t *>(base + NA_CURSOR);
+  double *interior = reinterpret_cast<double *>(base + NA_GRID);
+  if (s.unclean) {
+    PMPIC_TRY(zero_i32(c, w.count, NA_MAX_CELLS));
+    PMPIC_TRY(zero_i32(c, w.cursor, 1));
+  }
+  s.unclean = true;
+  PMPIC_TRY(par2grid_single_ws(c, c->n, var, interior, w));
+  PMPIC_TRY(grid_to_ref(c, interior, 1, grid));
+  PMPIC_TRY(take_status(c));
+  s.unclean = false;
   return PMPIC_OK;
 }
 
@@ -76,18 +104,10 @@ extern "C" int pmpic_par2grid_noalloc(pmpic_ctx *ctx, const double *var, double 
   if (!ctx || !var || !grid || ctx->c.precision != 0) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;
   if (c->n > NA_MAX_PARCELS || c->ncell > NA_MAX_CELLS) return PMPIC_ERR_ARG;
-  unsigned char *base = nullptr;
-  PMPIC_TRY(scratch_addr(c->device, &base));
-  BinWork w;
-  w.cell = reinterpret_cast<int32_t *>(base + NA_CELL);
-  w.rank = reinterpret_cast<int32_t *>(base + NA_RANK);
-  w.sorted = reinterpret_cast<int32_t *>(base + NA_SORTED);
-  w.count = reinterpret_cast<int32_t *>(base + NA_COUNT);
-  w.start = reinterpret_cast<int32_t *>(base + NA_START);
-  w.partial = reinterpret_cast<double *>(base + NA_PARTIAL);
-  w.cursor = reinterpret_cast<int32_t *>(base + NA_CURSOR);
-  double *interior = reinterpret_cast<double *>(base + NA_GRID);
-  PMPIC_TRY(par2grid_single_ws(c, c->n, var, interior, w));
-  PMPIC_TRY(grid_to_ref(c, interior, 1, grid));
-  return take_status(c);
+  if (c->device < 0 || c->device >= NA_MAX_DEVICES) return PMPIC_ERR_ARG;
+  Shared &s = na_shared[c->device];
+  std::lock_guard<std::mutex> turn(s.turn);
+  const int st = par2grid_in(c, s, var, grid);
+  if (st != PMPIC_OK) (void)hipStreamSynchronize(c->stream);  // the array is the next call's
+  return st;
 }

@@ -1,8 +1,10 @@
 """Sizes, values and sequences of calls that went wrong once, in the forms that show it."""
+import threading
+
 import numpy as np
 import pytest
 
-from tests.cases import LX, LZ, box, crowded_case
+from tests.cases import LX, LZ, box, crowded_case, thermal_case
 
 pytestmark = pytest.mark.gpu
 
@@ -144,4 +146,56 @@ def test_positions_without_a_cell_are_refused(axis, status, value):
         with pytest.raises(PmpicError) as e:
             call()
         assert e.value.status in (status, 4 if value == 1e300 else status), name
+    g.close()
+
+
+def _noalloc_pair(shape, ppc, seed):
+    """A context, a call of the allocation-free par2grid of its buoyancy (its status and grid) and
+    the grid that pmpic_par2grid gives."""
+    from pmpic_amd.lib import Context
+    from tests.test_zz_no_alloc import _noalloc
+    ic = thermal_case(*shape, ppc, seed=seed, vort=1.0)
+    b = box(*shape)
+    g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                len(ic["x"]) + 64)
+    g.set_parcels(ic)
+    return g, ic, lambda: _noalloc(g, ic["b"]), g.par2grid(ic["b"])
+
+
+def test_noalloc_calls_of_two_threads():
+    """Allocation-free calls of two contexts, a large and a small one, at the same time, then one
+    after another: all bit-identical to pmpic_par2grid."""
+    pairs = [_noalloc_pair((32, 32, 32), 3, 21), _noalloc_pair((10, 12, 5), 2, 22)]
+    bad = []
+
+    def run(call, want):
+        for _ in range(50):
+            st, got = call()
+            if st != 0 or not np.array_equal(got, want):
+                bad.append(st)
+
+    th = [threading.Thread(target=run, args=p[2:]) for p in pairs]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad
+    for g, _, call, want in pairs:
+        st, got = call()
+        assert st == 0
+        np.testing.assert_array_equal(got, want)
+        g.close()
+
+
+def test_noalloc_after_a_refused_call():
+    """A call that fails on a parcel outside the box leaves nothing to the next one."""
+    g, ic, call, want = _noalloc_pair((12, 10, 8), 2, 23)
+    out_of_box = dict(ic, z=ic["z"].copy())
+    out_of_box["z"][7] = 2 * LZ
+    g.set_parcels(out_of_box)
+    assert call()[0] == 3  # PMPIC_ERR_OUT_OF_BOX_Z
+    g.set_parcels(ic)
+    st, got = call()
+    assert st == 0
+    np.testing.assert_array_equal(got, want)
     g.close()
