@@ -98,18 +98,27 @@ struct Copy {
   }
 };
 
-// two slots and their events for each of n threads
+// two slots and their events for each of up to n threads: how many threads have them.  One that
+// gets none is done without, so the error is taken off the runtime's record, where the caller's next
+// check of a launch would find it.
 int ensure_slots(Ctx *c, int n) {
   for (int w = 0; w < n; w++) {
     for (int i = 2 * w; i < 2 * w + 2; i++)
-      if (!c->hc_ev[i])
-        PMPIC_CHECK(hipEventCreateWithFlags(&c->hc_ev[i], hipEventDisableTiming));
+      if (!c->hc_ev[i] &&
+          hipEventCreateWithFlags(&c->hc_ev[i], hipEventDisableTiming) != hipSuccess) {
+        c->hc_ev[i] = nullptr;
+        (void)hipGetLastError();
+        return w;
+      }
     if (c->hc_pin[w]) continue;
     void *p = nullptr;
-    PMPIC_CHECK(hipHostMalloc(&p, 2 * CHUNK));
+    if (hipHostMalloc(&p, 2 * CHUNK) != hipSuccess) {
+      (void)hipGetLastError();
+      return w;
+    }
     c->hc_pin[w] = static_cast<char *>(p);
   }
-  return PMPIC_OK;
+  return n;
 }
 
 }  // namespace
@@ -121,8 +130,9 @@ int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
     total += part[k].bytes;
     job.nchunks += (int64_t)((part[k].bytes + CHUNK - 1) / CHUNK);
   }
-  const int threads = total < LEAST_THREADS ? 1 : THREADS;
-  if (total < LEAST_PINNED || ensure_slots(c, threads) != PMPIC_OK) {
+  const int threads =
+      total < LEAST_PINNED ? 0 : ensure_slots(c, total < LEAST_THREADS ? 1 : THREADS);
+  if (threads == 0) {
     for (int k = 0; k < nparts; k++)
       if (part[k].bytes)
         PMPIC_CHECK(hipMemcpyAsync(to_host ? part[k].host : part[k].dev,

@@ -28,3 +28,27 @@ def test_packed_runs_hold_every_cell_of_a_slot_table(checks, cell, head):
     out = (ctypes.c_int32 * 2)()
     checks.host_run_round_trip(cell, head, out)
     assert tuple(out) == (cell, head)
+
+
+MB = 1 << 20
+
+
+@pytest.mark.parametrize("to_host", [False, True])
+@pytest.mark.parametrize("bytes_each,parts", [(3 * MB + 17, 1), (5 * MB - 3, 4)])
+@pytest.mark.parametrize("pinned", [0, 1, 2, 4])
+def test_host_copies_without_pinned_memory(checks, bytes_each, parts, to_host, pinned):
+    """Copies of a size that goes through pinned slots (one thread's, or four's from 16 MB on) while
+    the system gives pinned memory to some or none of the threads: every byte arrives, the copy
+    reports success and leaves no error for the caller's next check to find."""
+    rng = np.random.default_rng(bytes_each + pinned)
+    src = rng.integers(0, 256, bytes_each * parts, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    host, dev = (dst, src) if to_host else (src, dst)
+    out = (ctypes.c_int * 4)()
+    checks.host_copy(ctypes.c_void_p(host.ctypes.data), ctypes.c_void_p(dev.ctypes.data),
+                     ctypes.c_int64(bytes_each), parts, int(to_host), pinned, out)
+    assert out[0] == 0 and out[1] == 0
+    np.testing.assert_array_equal(dst, src)
+    threads = 4 if bytes_each * parts >= 16 * MB else 1
+    assert out[2] == min(pinned, threads)
+    assert out[3] == (parts if pinned == 0 else parts * -(-bytes_each // MB))
