@@ -60,7 +60,6 @@ struct Copy {
   }
   // one thread's share, through slots 2 w and 2 w + 1
   void run(int w) {
-    if (!ok(hipSetDevice(c->device))) return;
     char *const slot[2] = {c->hc_pin[w], c->hc_pin[w] + CHUNK};
     hipEvent_t *const ev = c->hc_ev + 2 * w;
     char *host[2], *dev[2];
@@ -121,6 +120,20 @@ int ensure_slots(Ctx *c, int n) {
   return n;
 }
 
+// Makes the context's device the calling thread's current one for the length of the copy.
+struct OnDevice {
+  int was = -1;
+  bool ok = false;
+  explicit OnDevice(int device) {
+    if (hipGetDevice(&was) != hipSuccess) return;
+    ok = was == device || hipSetDevice(device) == hipSuccess;
+    if (was == device) was = -1;
+  }
+  ~OnDevice() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+};
+
 }  // namespace
 
 int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
@@ -130,8 +143,10 @@ int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
     total += part[k].bytes;
     job.nchunks += (int64_t)((part[k].bytes + CHUNK - 1) / CHUNK);
   }
-  const int threads =
-      total < LEAST_PINNED ? 0 : ensure_slots(c, total < LEAST_THREADS ? 1 : THREADS);
+  int threads = 0;
+  OnDevice on(c->device);  // the events are its own
+  if (!on.ok) return PMPIC_ERR_HIP;
+  if (total >= LEAST_PINNED) threads = ensure_slots(c, total < LEAST_THREADS ? 1 : THREADS);
   if (threads == 0) {
     for (int k = 0; k < nparts; k++)
       if (part[k].bytes)
@@ -145,7 +160,9 @@ int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
   std::thread th[THREADS - 1];
   for (int w = 1; w < threads; w++) {
     try {
-      th[w - 1] = std::thread([&job, w]() { job.run(w); });
+      th[w - 1] = std::thread([&job, w]() {
+        if (job.ok(hipSetDevice(job.c->device))) job.run(w);
+      });
     } catch (const std::system_error &) {
       break;  // fewer threads
     }

@@ -10,6 +10,9 @@
 namespace fake {
 thread_local hipError_t pending = hipSuccess;  // what hipGetLastError reports
 std::atomic<int> pinned_left{0}, pinned_taken{0}, copies{0};
+// each thread's current device; an event belongs to the one it was created on, the stream to device 1
+thread_local int device = 0;
+constexpr int STREAM_DEVICE = 1;
 
 hipError_t fail(hipError_t e) { return pending = e; }
 hipError_t host_malloc(void **p, size_t n) {
@@ -28,13 +31,23 @@ hipError_t memcpy_async(void *to, const void *from, size_t n, hipMemcpyKind, hip
   return hipSuccess;
 }
 hipError_t event_create(hipEvent_t *e, unsigned) {
-  *e = reinterpret_cast<hipEvent_t>(1);
+  *e = reinterpret_cast<hipEvent_t>((intptr_t)device + 1);
   return hipSuccess;
 }
 hipError_t event(hipEvent_t) { return hipSuccess; }
-hipError_t event_record(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t event_record(hipEvent_t e, hipStream_t) {
+  return e == reinterpret_cast<hipEvent_t>((intptr_t)STREAM_DEVICE + 1) ? hipSuccess
+                                                                        : fail(hipErrorInvalidHandle);
+}
 hipError_t stream(hipStream_t) { return hipSuccess; }
-hipError_t set_device(int) { return hipSuccess; }
+hipError_t set_device(int d) {
+  device = d;
+  return hipSuccess;
+}
+hipError_t get_device(int *d) {
+  *d = device;
+  return hipSuccess;
+}
 hipError_t last_error() {
   const hipError_t e = pending;
   pending = hipSuccess;
@@ -50,6 +63,7 @@ hipError_t last_error() {
 #define hipEventRecord fake::event_record
 #define hipStreamSynchronize fake::stream
 #define hipSetDevice fake::set_device
+#define hipGetDevice fake::get_device
 #define hipGetLastError fake::last_error
 #include "transfer.hip"
 
@@ -65,10 +79,14 @@ void host_run_round_trip(int32_t cell, int32_t head, int32_t out[2]) {
 }
 
 // `parts` copies of n bytes each, one after another in `host` and `dev`, with pinned memory for
-// `pinned` threads' slots.  out: the status, the error left pending, the blocks of pinned memory
-// taken and the copy commands issued
-void host_copy(char *host, char *dev, int64_t n, int parts, int to_host, int pinned, int out[4]) {
+// `pinned` threads' slots, by a thread whose current device is `device`.  out: the status, the error
+// left pending, the blocks of pinned memory taken, the copy commands issued and the thread's device
+// afterwards
+void host_copy(char *host, char *dev, int64_t n, int parts, int to_host, int pinned, int device,
+               int out[5]) {
   Ctx *c = new Ctx();
+  c->device = fake::STREAM_DEVICE;
+  fake::device = device;
   HostPart part[32];
   for (int i = 0; i < parts; i++) part[i] = {host + i * n, dev + i * n, (size_t)n};
   fake::pinned_left = pinned;
@@ -77,6 +95,7 @@ void host_copy(char *host, char *dev, int64_t n, int parts, int to_host, int pin
   out[1] = (int)fake::last_error();
   out[2] = fake::pinned_taken;
   out[3] = fake::copies;
+  out[4] = fake::device;
   free_host_slots(c);
   delete c;
 }

@@ -33,6 +33,15 @@ def test_packed_runs_hold_every_cell_of_a_slot_table(checks, cell, head):
 MB = 1 << 20
 
 
+def _copy(checks, host, dev, bytes_each, parts, to_host, pinned, device=1):
+    """(status, error left pending, blocks of pinned memory taken, copy commands, the calling
+    thread's device afterwards) of a copy of a context on device 1."""
+    out = (ctypes.c_int * 5)()
+    checks.host_copy(ctypes.c_void_p(host.ctypes.data), ctypes.c_void_p(dev.ctypes.data),
+                     ctypes.c_int64(bytes_each), parts, int(to_host), pinned, device, out)
+    return list(out)
+
+
 @pytest.mark.parametrize("to_host", [False, True])
 @pytest.mark.parametrize("bytes_each,parts", [(3 * MB + 17, 1), (5 * MB - 3, 4)])
 @pytest.mark.parametrize("pinned", [0, 1, 2, 4])
@@ -44,11 +53,23 @@ def test_host_copies_without_pinned_memory(checks, bytes_each, parts, to_host, p
     src = rng.integers(0, 256, bytes_each * parts, dtype=np.uint8)
     dst = np.zeros_like(src)
     host, dev = (dst, src) if to_host else (src, dst)
-    out = (ctypes.c_int * 4)()
-    checks.host_copy(ctypes.c_void_p(host.ctypes.data), ctypes.c_void_p(dev.ctypes.data),
-                     ctypes.c_int64(bytes_each), parts, int(to_host), pinned, out)
-    assert out[0] == 0 and out[1] == 0
+    out = _copy(checks, host, dev, bytes_each, parts, to_host, pinned)
+    assert out[:2] == [0, 0]
     np.testing.assert_array_equal(dst, src)
     threads = 4 if bytes_each * parts >= 16 * MB else 1
     assert out[2] == min(pinned, threads)
     assert out[3] == (parts if pinned == 0 else parts * -(-bytes_each // MB))
+
+
+@pytest.mark.parametrize("to_host", [False, True])
+@pytest.mark.parametrize("size", [1000, 3 * MB, 20 * MB])
+@pytest.mark.parametrize("device", [0, 1])
+def test_host_copies_leave_the_current_device(checks, size, to_host, device):
+    """A copy of a context on device 1 by a thread whose current device is another: it succeeds (its
+    events are made on the context's device) and the thread's device is what it was."""
+    src = np.arange(size, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    host, dev = (dst, src) if to_host else (src, dst)
+    out = _copy(checks, host, dev, size, 1, to_host, 4, device)
+    assert out[:2] == [0, 0] and out[4] == device
+    np.testing.assert_array_equal(dst, src)
