@@ -3,9 +3,9 @@
 // The caller's memory is pageable, and the runtime's copy of it passes through one thread:
 // 17 GB/s to the host (11 where the pages are new), 29 from it, of a link that carries 57 to pinned
 // memory; and from about a megabyte on it pins the caller's pages for the copy, which can stall the
-// program for milliseconds when it next maps or releases memory.  Here such a copy is cut into chunks
-// that threads (a large one's four, else the caller's alone) carry through pinned slots of their
-// own, two each, the link moving one while the thread copies the other.
+// program for milliseconds when it next maps or releases memory.  Here a copy of some size is cut
+// into chunks that threads (a large one's four, else the caller's alone) carry through pinned slots of
+// their own, two each, the link moving one while the thread copies the other.
 #include "common.h"
 
 #include <string.h>
@@ -20,14 +20,30 @@ namespace {
 
 constexpr size_t CHUNK = (size_t)1 << 20;
 constexpr int THREADS = HOST_THREADS;  // the caller's and three more, for the length of the call
-// Below this the runtime's own copy, which doesn't pin.  Above it, a 60x180x28 run's exports of 2.7 MB
-// left the program's next allocation waiting 4 ms in the median (pass 18.4 ms, now 11.9), and eight
-// members' 59 ms a pass is 57.
+// To the host, below this the runtime's own copy, which doesn't pin.  Above it, a 60x180x28 run's
+// exports of 2.7 MB left the program's next allocation waiting 4 ms in the median (pass 18.4 ms, now
+// 11.9), and eight members' 59 ms a pass is 57.
 constexpr size_t LEAST_PINNED = CHUNK;
+// Nor does the runtime pin arrays this small, and a chunk of its own for each costs more than the
+// slots save (17 arrays of 64, 128, 256, 512 KB: 0.21, 0.26, 0.33, 0.53 ms through the runtime, 0.29,
+// 0.30, 0.34, 0.43 through slots).
+constexpr size_t LEAST_PART = CHUNK / 4;
 // Below this one thread: the others' start and, where the caller's pages are new, their contention
 // for the address space cost more than they save (a dump of ten grids of 5.4 MB: 4.7 ms through the
 // runtime, 4.3 with one thread, 4.2 at best and 10 in the median with four).
 constexpr size_t LEAST_THREADS = (size_t)16 << 20;
+// From the host, below this the runtime's copy: one thread's slots take longer (17 arrays of 0.1,
+// 0.9, 1.1 MB: 0.19, 0.45, 0.67 ms through the runtime, 0.31, 0.57, 0.90 through slots; one after
+// another, arrays of 1.1, 1.9, 6.9, 15 MB: 0.85, 1.28, 4.4, 9.4 and 1.47, 1.9, 5.3, 10.9), and four
+// threads' are even from here on (17 of 1.9 MB 1.20 and 1.19, of 15 MB 9.2 and 8.8).
+constexpr size_t LEAST_UPLOAD = (size_t)32 << 20;
+
+// the threads that carry a copy through pinned slots, 0 for the runtime's own
+int slot_threads(size_t total, int nparts, bool to_host) {
+  if (!to_host) return total < LEAST_UPLOAD ? 0 : THREADS;
+  if (total < LEAST_PINNED || total < nparts * LEAST_PART) return 0;
+  return total < LEAST_THREADS ? 1 : THREADS;
+}
 
 struct Copy {
   Ctx *c;
@@ -143,10 +159,9 @@ int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
     total += part[k].bytes;
     job.nchunks += (int64_t)((part[k].bytes + CHUNK - 1) / CHUNK);
   }
-  int threads = 0;
   OnDevice on(c->device);  // the events are its own
   if (!on.ok) return PMPIC_ERR_HIP;
-  if (total >= LEAST_PINNED) threads = ensure_slots(c, total < LEAST_THREADS ? 1 : THREADS);
+  const int threads = ensure_slots(c, slot_threads(total, nparts, to_host));
   if (threads == 0) {
     for (int k = 0; k < nparts; k++)
       if (part[k].bytes)

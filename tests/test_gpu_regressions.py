@@ -199,3 +199,22 @@ def test_noalloc_after_a_refused_call():
     assert st == 0
     np.testing.assert_array_equal(got, want)
     g.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n", [32_767, 32_768, 246_723, 246_724, 4_194_303, 4_194_304])
+def test_parcel_arrays_around_the_copy_rules(n, precision):
+    """Parcel arrays there and back either side of the parts that go through pinned slots to the host
+    (256 KB) and of the uploads that do (32 MB in 17 arrays, or in one where each is taken alone):
+    equal in the FP64 form, rounded to FP32 in the other (cells of unit size, positions in the first)."""
+    from pmpic_amd.lib import PARCEL_FIELDS, Context
+    rng = np.random.default_rng(n)
+    ic = {k: rng.uniform(0.1, 0.9, n) for k in PARCEL_FIELDS}
+    g = Context(8, 6, 5, 0.0, 8.0, 0.0, 6.0, 0.0, 5.0, n, precision=precision)
+    for _ in range(2):
+        g.set_parcels(ic)
+        got = g.get_parcels()
+    g.close()
+    for k in PARCEL_FIELDS:
+        want = ic[k] if precision == 0 or k == "tag" else ic[k].astype(np.float32)
+        np.testing.assert_array_equal(got[k], want.astype(np.float64), err_msg=k)

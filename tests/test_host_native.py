@@ -42,13 +42,14 @@ def _copy(checks, host, dev, bytes_each, parts, to_host, pinned, device=1):
     return list(out)
 
 
-@pytest.mark.parametrize("to_host", [False, True])
-@pytest.mark.parametrize("bytes_each,parts", [(3 * MB + 17, 1), (5 * MB - 3, 4)])
+@pytest.mark.parametrize("bytes_each,parts,to_host,threads",
+                         [(3 * MB + 17, 1, True, 1), (5 * MB - 3, 4, True, 4),
+                          (9 * MB + 1, 4, False, 4)])
 @pytest.mark.parametrize("pinned", [0, 1, 2, 4])
-def test_host_copies_without_pinned_memory(checks, bytes_each, parts, to_host, pinned):
-    """Copies of a size that goes through pinned slots (one thread's, or four's from 16 MB on) while
-    the system gives pinned memory to some or none of the threads: every byte arrives, the copy
-    reports success and leaves no error for the caller's next check to find."""
+def test_host_copies_without_pinned_memory(checks, bytes_each, parts, to_host, threads, pinned):
+    """Copies of a size that goes through pinned slots, one thread's or four's, while the system gives
+    pinned memory to some or none of the threads: every byte arrives, the copy reports success and
+    leaves no error for the caller's next check to find."""
     rng = np.random.default_rng(bytes_each + pinned)
     src = rng.integers(0, 256, bytes_each * parts, dtype=np.uint8)
     dst = np.zeros_like(src)
@@ -56,13 +57,30 @@ def test_host_copies_without_pinned_memory(checks, bytes_each, parts, to_host, p
     out = _copy(checks, host, dev, bytes_each, parts, to_host, pinned)
     assert out[:2] == [0, 0]
     np.testing.assert_array_equal(dst, src)
-    threads = 4 if bytes_each * parts >= 16 * MB else 1
     assert out[2] == min(pinned, threads)
     assert out[3] == (parts if pinned == 0 else parts * -(-bytes_each // MB))
 
 
+@pytest.mark.parametrize("bytes_each,parts,to_host,threads",
+                         [(MB - 1, 1, True, 0), (MB, 1, True, 1), (16 * MB - 1, 1, True, 1),
+                          (16 * MB, 1, True, 4), (MB // 4 - 8, 17, True, 0), (MB // 4, 17, True, 1),
+                          (MB, 17, True, 4), (MB, 1, False, 0), (15 * MB, 1, False, 0),
+                          (32 * MB - 1, 1, False, 0), (32 * MB, 1, False, 4), (MB, 17, False, 0),
+                          (2 * MB, 17, False, 4)])
+def test_host_copies_route(checks, bytes_each, parts, to_host, threads):
+    """Which copies go through pinned slots: to the host from 1 MB in parts of 256 KB or more, by four
+    threads from 16 MB; from the host, where one thread's slots are slower than the runtime, from 32
+    MB by four."""
+    src = np.arange(bytes_each * parts, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    host, dev = (dst, src) if to_host else (src, dst)
+    out = _copy(checks, host, dev, bytes_each, parts, to_host, 4)
+    assert out[:3] == [0, 0, threads]
+    np.testing.assert_array_equal(dst, src)
+
+
 @pytest.mark.parametrize("to_host", [False, True])
-@pytest.mark.parametrize("size", [1000, 3 * MB, 20 * MB])
+@pytest.mark.parametrize("size", [1000, 3 * MB, 40 * MB])
 @pytest.mark.parametrize("device", [0, 1])
 def test_host_copies_leave_the_current_device(checks, size, to_host, device):
     """A copy of a context on device 1 by a thread whose current device is another: it succeeds (its
