@@ -792,8 +792,9 @@ struct RkSets {
   float *off_to, *vor_to;
 };
 
-// The RK stage of parcel p; returns its new cell, or -1 when it left the box (status raised).  The
-// sets of a stage may be the same arrays: a thread reads its parcel before it writes it.
+// The RK stage of parcel p; returns its new cell.  One that would leave the box stays where it is
+// (status raised), in the set that the stage writes too.  The sets of a stage may be the same arrays:
+// a thread reads its parcel before it writes it.
 template <int STAGE>
 __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b, const RkSets &rs,
                                              const float4 *__restrict__ rec,
@@ -870,7 +871,13 @@ __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b,
   float nox, noy, noz;
   if (!place(g, io, jo, ko, tpos[0], tpos[1], tpos[2], ncell_, nox, noy, noz)) {
     raise_status(sc, PMPIC_ERR_OUT_OF_BOX_Z);
-    return -1;
+    if (STAGE == 1 || STAGE == 4) {
+      const Float3 v = ld3(rs.vor, p);
+      stnt(rs.cell_to, p, cell);
+      st3(rs.off_to, p, ox, oy, oz);
+      st3(rs.vor_to, p, v.x, v.y, v.z);
+    }
+    return cell;
   }
   stnt(rs.cell_to, p, ncell_);
   st3(rs.off_to, p, nox, noy, noz);
@@ -915,7 +922,7 @@ __global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, RkSets
   const int32_t was = STAGE == 2 && bo.on ? rs.cell[p] : -1;  // (the stage updates it in place)
   const int32_t nc = rk_update<STAGE>(g, b, rs, rec, sc3, stretch, split_flag, sc, p);
   // with bo.on = 2, the entries of the parcels that change cell move
-  if (STAGE == 2 && bo.on && nc >= 0 && nc != was) {
+  if (STAGE == 2 && bo.on && nc != was) {
     remove_entry((int32_t)p, linear_cell(g, was), bo.capc, bo, sc);
     append_entry((int32_t)p, linear_cell(g, nc), bo, sc);
   }

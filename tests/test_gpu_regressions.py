@@ -218,3 +218,49 @@ def test_parcel_arrays_around_the_copy_rules(n, precision):
     for k in PARCEL_FIELDS:
         want = ic[k] if precision == 0 or k == "tag" else ic[k].astype(np.float32)
         np.testing.assert_array_equal(got[k], want.astype(np.float64), err_msg=k)
+
+
+@pytest.mark.parametrize("fused", ["0", "1"])
+@pytest.mark.parametrize("stage", [1, 2, 3, 4])
+def test_parcels_that_would_leave_the_box_stay(monkeypatch, stage, fused):
+    """An FP32-bulk stage whose timestep takes parcels out of the box (by thousands of cells, where
+    they have a vertical velocity to speak of) reports it and leaves those parcels as they were, in
+    either of the two sets that the stages write, and in the next par2grid."""
+    from pmpic_amd.lib import Context, PmpicError
+    monkeypatch.setenv("PMPIC_FUSED_BINNING", fused)
+    shape = (12, 10, 8)
+    ic = thermal_case(*shape, 2, vort=2.0)
+    b = box(*shape)
+    g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                3 * len(ic["x"]), precision=1)
+    g.set_parcels(ic)
+    g.step(2)
+
+    for _ in range(stage - 1):
+        g.vort2vel()
+        g.vorticity_tendency()
+        g.rk4_integrator()
+        g.parcel_splitting()
+        g.parcel_mixing()
+    g.vort2vel()
+    g.vorticity_tendency()
+    before = g.get_parcels()
+    g.set_time(g.time, 1e6)
+    with pytest.raises(PmpicError) as e:
+        g.rk4_integrator()
+    assert e.value.status == 3  # PMPIC_ERR_OUT_OF_BOX_Z
+    after = g.get_parcels()
+    where = ("x", "y", "z", "p", "q", "r")
+    stayed = np.all([after[k] == before[k] for k in where], axis=0)
+    assert stayed.mean() > 0.9
+    # and they are in the lists: a grid of the parcels is that of a context given them as they are
+    g.writebinary_grids()
+    got = {k: g.grid(k) for k in ("b", "hg", "p", "q", "r")}
+    h = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                3 * len(ic["x"]), precision=1)
+    h.set_parcels(after)
+    h.writebinary_grids()
+    for k, want in got.items():
+        assert np.abs(h.grid(k) - want).max() <= 1e-5 * max(1.0, np.abs(want).max()), k
+    g.close()
+    h.close()
