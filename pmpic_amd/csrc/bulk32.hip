@@ -1451,11 +1451,11 @@ static Column column(const Bulk32 &b, int f) {
 
 static int put_field(Ctx *c, double *dev, const double *host, int64_t n) {
   const HostPart p{const_cast<double *>(host), dev, sizeof(double) * (size_t)n};
-  return copy_host(c, &p, 1, false);
+  return copy_to_device(c, &p, 1);
 }
 static int get_field(Ctx *c, double *host, double *dev, int64_t n) {
   const HostPart p{host, dev, sizeof(double) * (size_t)n};
-  return copy_host(c, &p, 1, true);
+  return copy_to_host(c, &p, 1);
 }
 
 int b32_set_parcels(Ctx *c, int64_t n, const double *const *fields) {

@@ -134,7 +134,7 @@ void col_to_device_layout(const Geometry &g, const double *ref, std::vector<doub
 // host array -> device, in stream order
 int put_host(Ctx *c, double *dst, const double *host, int64_t n) {
   const HostPart p{const_cast<double *>(host), dst, sizeof(double) * (size_t)n};
-  return copy_host(c, &p, 1, false);
+  return copy_to_device(c, &p, 1);
 }
 int get_host(Ctx *c, double *host, const double *src, int64_t n) {
   if (src == c->ref_pin) {
@@ -144,7 +144,7 @@ int get_host(Ctx *c, double *host, const double *src, int64_t n) {
     return PMPIC_OK;
   }
   const HostPart p{host, const_cast<double *>(src), sizeof(double) * (size_t)n};
-  return copy_host(c, &p, 1, true);
+  return copy_to_host(c, &p, 1);
 }
 int64_t ref_grid_size(const Geometry &g) { return (int64_t)g.nzn * (g.ny + 4) * (g.nx + 4); }
 
@@ -476,7 +476,7 @@ int pmpic_set_parcels(pmpic_ctx *ctx, int64_t n, const double *const *fields) {
   HostPart part[17];
   for (int f = 0; f < 17; f++)
     part[f] = {const_cast<double *>(fields[f]), c->par + (int64_t)f * c->cap, sizeof(double) * (size_t)n};
-  PMPIC_TRY(copy_host(c, part, 17, false));
+  PMPIC_TRY(copy_to_device(c, part, 17));
   PMPIC_CHECK(hipStreamSynchronize(c->stream));
   c->n = n;
   return PMPIC_OK;
@@ -493,7 +493,7 @@ int pmpic_get_parcels(pmpic_ctx *ctx, int64_t *n, double *const *fields) {
     for (int f = 0; f < 17; f++)
       if (fields[f])
         part[parts++] = {fields[f], c->par + (int64_t)f * c->cap, sizeof(double) * (size_t)c->n};
-  PMPIC_TRY(copy_host(c, part, parts, true));
+  PMPIC_TRY(copy_to_host(c, part, parts));
   PMPIC_CHECK(hipStreamSynchronize(c->stream));
   return PMPIC_OK;
 }

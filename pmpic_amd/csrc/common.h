@@ -149,7 +149,7 @@ __host__ __device__ inline int64_t spec_at(int nzn, int nl, int k, int m, int l)
 enum TimerId { T_ACCUM = 0, T_RK = 1, T_VORT2VEL, T_VORT_TEND, T_RK4, T_SPLIT, T_MIX, NTIMERS };
 
 constexpr int MAXBLK = 1024;   // blocks of the timestep reduction
-constexpr int HOST_THREADS = 4;  // of the large host copies (copy_host)
+constexpr int HOST_THREADS = 4;  // of the large copies to the host (copy_to_host)
 
 constexpr int64_t BINS_NONE = -1, BINS_STALE = -2;  // Ctx::bins_n
 
@@ -238,7 +238,7 @@ struct Ctx {
   void *pin;                          // pinned host staging for small read-backs (256 B)
   double *ref_pin;                    // pinned, for small arrays in the reference's layout (ref_out)
   hipEvent_t sync_ev;                 // read-back completion (spin wait)
-  char *hc_pin[HOST_THREADS];         // copy_host's slots, two a thread, allocated at their first use
+  char *hc_pin[HOST_THREADS];         // copy_to_host's slots, two a thread, allocated at their first use
   hipEvent_t hc_ev[2 * HOST_THREADS];
   // FP32-bulk form with PMPIC_GRAPH=1: RK stages 1-3 of a step (vort2vel, vorticity_tendency,
   // rk4_integrator; the splitting and mixing callbacks do nothing there) captured once as a HIP
@@ -422,13 +422,13 @@ int fft_backward(Ctx *c, int nf, const double *const *src, double *const *dst,
 // forward transform reads physical grids of type S, the inverse writes dst (FP64) and dst32
 // (FP32), either of which may be NULL
 // Copies between the caller's arrays and the device, on the context's stream.  To the host: complete
-// on return; from it: the caller's arrays may change on return, and the work queued next sees the
-// data.
+// on return.  From it: the caller's arrays may change once the stream has been waited for.
 struct HostPart {
   void *host, *dev;
   size_t bytes;
 };
-int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host);
+int copy_to_device(Ctx *c, const HostPart *part, int nparts);
+int copy_to_host(Ctx *c, const HostPart *part, int nparts);
 void free_host_slots(Ctx *c);
 template <typename S>
 int fft_forward_t(Ctx *c, int nf, const S *const *src, S *const *dst);

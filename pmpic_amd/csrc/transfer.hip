@@ -1,11 +1,18 @@
 // Copies between the caller's arrays and the device.
 //
-// The caller's memory is pageable, and the runtime's copy of it passes through one thread:
-// 17 GB/s to the host (11 where the pages are new), 29 from it, of a link that carries 57 to pinned
-// memory; and from about a megabyte on it pins the caller's pages for the copy, which can stall the
-// program for milliseconds when it next maps or releases memory.  Here a copy of some size is cut
-// into chunks that threads (a large one's four, else the caller's alone) carry through pinned slots of
-// their own, two each, the link moving one while the thread copies the other.
+// The caller's memory is pageable.  The runtime's copy to the host passes through one thread, 17 GB/s
+// (11 where the pages are new) of a link that carries 57 to pinned memory; and from about a megabyte
+// on it pins the caller's pages for the copy, which can stall the program for milliseconds when it
+// next maps or releases memory.  Here such a copy is cut into chunks that threads (a large one's four,
+// else the caller's alone) carry through pinned slots of their own, two each, the link moving one while
+// the thread copies the other.
+//
+// From the host the runtime's copy, 29 to 31 GB/s, stays.  One thread's slots were slower (17 arrays of
+// 0.06, 0.84, 1.07 MB: 0.18, 0.45, 0.67 ms through the runtime, 0.29, 0.57, 0.90 through slots; one
+// after another, arrays of 1.9, 6.9, 15 MB: 1.28, 4.4, 9.4 and 1.9, 5.3, 10.9), four threads' no better
+// than even: 17 arrays of 2.3, 6.3, 23 MB 1.31, 4.0, 13.8 against 1.57, 3.85, 12.9, but with seven of
+// them one array of zeros, as the fields that a caller leaves out are, 1.25, 3.5, 12.2 against 1.62,
+// 3.9, 12.9.
 #include "common.h"
 
 #include <string.h>
@@ -32,15 +39,9 @@ constexpr size_t LEAST_PART = CHUNK / 4;
 // for the address space cost more than they save (a dump of ten grids of 5.4 MB: 4.7 ms through the
 // runtime, 4.3 with one thread, 4.2 at best and 10 in the median with four).
 constexpr size_t LEAST_THREADS = (size_t)16 << 20;
-// From the host, below this the runtime's copy: one thread's slots take longer (17 arrays of 0.1,
-// 0.9, 1.1 MB: 0.19, 0.45, 0.67 ms through the runtime, 0.31, 0.57, 0.90 through slots; one after
-// another, arrays of 1.1, 1.9, 6.9, 15 MB: 0.85, 1.28, 4.4, 9.4 and 1.47, 1.9, 5.3, 10.9), and four
-// threads' are even from here on (17 of 1.9 MB 1.20 and 1.19, of 15 MB 9.2 and 8.8).
-constexpr size_t LEAST_UPLOAD = (size_t)32 << 20;
 
-// the threads that carry a copy through pinned slots, 0 for the runtime's own
-int slot_threads(size_t total, int nparts, bool to_host) {
-  if (!to_host) return total < LEAST_UPLOAD ? 0 : THREADS;
+// the threads that carry a copy to the host through pinned slots, 0 for the runtime's own
+int slot_threads(size_t total, int nparts) {
   if (total < LEAST_PINNED || total < nparts * LEAST_PART) return 0;
   return total < LEAST_THREADS ? 1 : THREADS;
 }
@@ -49,7 +50,6 @@ struct Copy {
   Ctx *c;
   const HostPart *part;
   int nparts;
-  bool to_host;
   int64_t nchunks;
   std::atomic<int64_t> next{0};
   std::atomic<int> failed{0};
@@ -80,35 +80,20 @@ struct Copy {
     hipEvent_t *const ev = c->hc_ev + 2 * w;
     char *host[2], *dev[2];
     size_t len[2] = {0, 0};
-    if (to_host) {
-      auto issue = [&](int s) {
+    auto issue = [&](int s) {
+      len[s] = 0;
+      const int64_t i = next.fetch_add(1);
+      if (i >= nchunks || failed.load()) return;
+      chunk(i, host[s], dev[s], len[s]);
+      if (!ok(hipMemcpyAsync(slot[s], dev[s], len[s], hipMemcpyDeviceToHost, c->stream)) ||
+          !ok(hipEventRecord(ev[s], c->stream)))
         len[s] = 0;
-        const int64_t i = next.fetch_add(1);
-        if (i >= nchunks || failed.load()) return;
-        chunk(i, host[s], dev[s], len[s]);
-        if (!ok(hipMemcpyAsync(slot[s], dev[s], len[s], hipMemcpyDeviceToHost, c->stream)) ||
-            !ok(hipEventRecord(ev[s], c->stream)))
-          len[s] = 0;
-      };
-      issue(0);
-      for (int s = 0; len[s]; s ^= 1) {
-        issue(s ^ 1);
-        if (!ok(hipEventSynchronize(ev[s]))) return;
-        memcpy(host[s], slot[s], len[s]);
-      }
-    } else {
-      for (int s = 0;; s ^= 1) {
-        const int64_t i = next.fetch_add(1);
-        if (i >= nchunks || failed.load()) break;
-        if (len[s] && !ok(hipEventSynchronize(ev[s]))) return;
-        chunk(i, host[s], dev[s], len[s]);
-        memcpy(slot[s], host[s], len[s]);
-        if (!ok(hipMemcpyAsync(dev[s], slot[s], len[s], hipMemcpyHostToDevice, c->stream)) ||
-            !ok(hipEventRecord(ev[s], c->stream)))
-          return;
-      }
-      for (int s = 0; s < 2; s++)  // the slots are free again when the call returns
-        if (len[s]) ok(hipEventSynchronize(ev[s]));
+    };
+    issue(0);
+    for (int s = 0; len[s]; s ^= 1) {
+      issue(s ^ 1);
+      if (!ok(hipEventSynchronize(ev[s]))) return;
+      memcpy(host[s], slot[s], len[s]);
     }
   }
 };
@@ -152,24 +137,30 @@ struct OnDevice {
 
 }  // namespace
 
-int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
+int copy_to_device(Ctx *c, const HostPart *part, int nparts) {
+  for (int k = 0; k < nparts; k++)
+    if (part[k].bytes)
+      PMPIC_CHECK(hipMemcpyAsync(part[k].dev, part[k].host, part[k].bytes, hipMemcpyHostToDevice,
+                                 c->stream));
+  return PMPIC_OK;
+}
+
+int copy_to_host(Ctx *c, const HostPart *part, int nparts) {
   size_t total = 0;
-  Copy job{c, part, nparts, to_host, 0};
+  Copy job{c, part, nparts, 0};
   for (int k = 0; k < nparts; k++) {
     total += part[k].bytes;
     job.nchunks += (int64_t)((part[k].bytes + CHUNK - 1) / CHUNK);
   }
   OnDevice on(c->device);  // the events are its own
   if (!on.ok) return PMPIC_ERR_HIP;
-  const int threads = ensure_slots(c, slot_threads(total, nparts, to_host));
+  const int threads = ensure_slots(c, slot_threads(total, nparts));
   if (threads == 0) {
     for (int k = 0; k < nparts; k++)
       if (part[k].bytes)
-        PMPIC_CHECK(hipMemcpyAsync(to_host ? part[k].host : part[k].dev,
-                                   to_host ? part[k].dev : part[k].host, part[k].bytes,
-                                   to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice,
+        PMPIC_CHECK(hipMemcpyAsync(part[k].host, part[k].dev, part[k].bytes, hipMemcpyDeviceToHost,
                                    c->stream));
-    if (to_host) PMPIC_CHECK(hipStreamSynchronize(c->stream));
+    PMPIC_CHECK(hipStreamSynchronize(c->stream));
     return PMPIC_OK;
   }
   std::thread th[THREADS - 1];
@@ -185,7 +176,9 @@ int copy_host(Ctx *c, const HostPart *part, int nparts, bool to_host) {
   job.run(0);
   for (std::thread &t : th)
     if (t.joinable()) t.join();
-  return job.failed.load() ? PMPIC_ERR_HIP : PMPIC_OK;
+  if (!job.failed.load()) return PMPIC_OK;
+  (void)hipStreamSynchronize(c->stream);  // what is still on its way into a slot
+  return PMPIC_ERR_HIP;
 }
 
 void free_host_slots(Ctx *c) {

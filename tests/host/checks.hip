@@ -91,7 +91,7 @@ void host_copy(char *host, char *dev, int64_t n, int parts, int to_host, int pin
   for (int i = 0; i < parts; i++) part[i] = {host + i * n, dev + i * n, (size_t)n};
   fake::pinned_left = pinned;
   fake::pinned_taken = fake::copies = 0;
-  out[0] = copy_host(c, part, parts, to_host != 0);
+  out[0] = to_host ? copy_to_host(c, part, parts) : copy_to_device(c, part, parts);
   out[1] = (int)fake::last_error();
   out[2] = fake::pinned_taken;
   out[3] = fake::copies;

@@ -202,10 +202,10 @@ def test_noalloc_after_a_refused_call():
 
 
 @pytest.mark.parametrize("precision", [0, 1])
-@pytest.mark.parametrize("n", [32_767, 32_768, 246_723, 246_724, 4_194_303, 4_194_304])
+@pytest.mark.parametrize("n", [32_767, 32_768, 131_071, 131_072, 2_097_151, 2_097_152])
 def test_parcel_arrays_around_the_copy_rules(n, precision):
     """Parcel arrays there and back either side of the parts that go through pinned slots to the host
-    (256 KB) and of the uploads that do (32 MB in 17 arrays, or in one where each is taken alone):
+    (256 KB of 17, or 1 MB where each is taken alone, which 16 MB are by four threads):
     equal in the FP64 form, rounded to FP32 in the other (cells of unit size, positions in the first)."""
     from pmpic_amd.lib import PARCEL_FIELDS, Context
     rng = np.random.default_rng(n)
