@@ -144,7 +144,9 @@ int get_host(Ctx *c, double *host, const double *src, int64_t n) {
     return PMPIC_OK;
   }
   const HostPart p{host, const_cast<double *>(src), sizeof(double) * (size_t)n};
-  return copy_to_host(c, &p, 1);
+  PMPIC_TRY(copy_to_host(c, &p, 1));
+  PMPIC_CHECK(hipStreamSynchronize(c->stream));
+  return PMPIC_OK;
 }
 int64_t ref_grid_size(const Geometry &g) { return (int64_t)g.nzn * (g.ny + 4) * (g.nx + 4); }
 

@@ -35,6 +35,11 @@ constexpr size_t LEAST_PINNED = CHUNK;
 // slots save (17 arrays of 64, 128, 256, 512 KB: 0.21, 0.26, 0.33, 0.53 ms through the runtime, 0.29,
 // 0.30, 0.34, 0.43 through slots).
 constexpr size_t LEAST_PART = CHUNK / 4;
+// The wait for the stream is the caller's, one for several copies, but above this it comes sooner: the
+// runtime's next copy waits longer by itself.  FP32-bulk get_parcels, whose fields are converted and
+// copied one after another, of 2,048 parcels 0.41 ms with a wait for each field and 0.30 with one, of
+// 2,049 0.37 and 0.41, of 20,000 0.47 and 0.50.
+constexpr size_t LEAST_WAITED = (size_t)16 << 10;
 // Below this one thread: the others' start and, where the caller's pages are new, their contention
 // for the address space cost more than they save (a dump of ten grids of 5.4 MB: 4.7 ms through the
 // runtime, 4.3 with one thread, 4.2 at best and 10 in the median with four).
@@ -160,7 +165,7 @@ int copy_to_host(Ctx *c, const HostPart *part, int nparts) {
       if (part[k].bytes)
         PMPIC_CHECK(hipMemcpyAsync(part[k].host, part[k].dev, part[k].bytes, hipMemcpyDeviceToHost,
                                    c->stream));
-    PMPIC_CHECK(hipStreamSynchronize(c->stream));
+    if (total > LEAST_WAITED) PMPIC_CHECK(hipStreamSynchronize(c->stream));
     return PMPIC_OK;
   }
   std::thread th[THREADS - 1];

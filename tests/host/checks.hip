@@ -9,7 +9,7 @@
 // at once, and pinned memory runs out after pinned_left blocks.
 namespace fake {
 thread_local hipError_t pending = hipSuccess;  // what hipGetLastError reports
-std::atomic<int> pinned_left{0}, pinned_taken{0}, copies{0};
+std::atomic<int> pinned_left{0}, pinned_taken{0}, copies{0}, waits{0};
 // each thread's current device; an event belongs to the one it was created on, the stream to device 1
 thread_local int device = 0;
 constexpr int STREAM_DEVICE = 1;
@@ -39,7 +39,10 @@ hipError_t event_record(hipEvent_t e, hipStream_t) {
   return e == reinterpret_cast<hipEvent_t>((intptr_t)STREAM_DEVICE + 1) ? hipSuccess
                                                                         : fail(hipErrorInvalidHandle);
 }
-hipError_t stream(hipStream_t) { return hipSuccess; }
+hipError_t stream(hipStream_t) {
+  waits++;
+  return hipSuccess;
+}
 hipError_t set_device(int d) {
   device = d;
   return hipSuccess;
@@ -80,22 +83,23 @@ void host_run_round_trip(int32_t cell, int32_t head, int32_t out[2]) {
 
 // `parts` copies of n bytes each, one after another in `host` and `dev`, with pinned memory for
 // `pinned` threads' slots, by a thread whose current device is `device`.  out: the status, the error
-// left pending, the blocks of pinned memory taken, the copy commands issued and the thread's device
-// afterwards
+// left pending, the blocks of pinned memory taken, the copy commands issued, the thread's device
+// afterwards and the waits for the stream
 void host_copy(char *host, char *dev, int64_t n, int parts, int to_host, int pinned, int device,
-               int out[5]) {
+               int out[6]) {
   Ctx *c = new Ctx();
   c->device = fake::STREAM_DEVICE;
   fake::device = device;
   HostPart part[32];
   for (int i = 0; i < parts; i++) part[i] = {host + i * n, dev + i * n, (size_t)n};
   fake::pinned_left = pinned;
-  fake::pinned_taken = fake::copies = 0;
+  fake::pinned_taken = fake::copies = fake::waits = 0;
   out[0] = to_host ? copy_to_host(c, part, parts) : copy_to_device(c, part, parts);
   out[1] = (int)fake::last_error();
   out[2] = fake::pinned_taken;
   out[3] = fake::copies;
   out[4] = fake::device;
+  out[5] = fake::waits;
   free_host_slots(c);
   delete c;
 }

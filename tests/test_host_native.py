@@ -35,8 +35,8 @@ MB = 1 << 20
 
 def _copy(checks, host, dev, bytes_each, parts, to_host, pinned, device=1):
     """(status, error left pending, blocks of pinned memory taken, copy commands, the calling
-    thread's device afterwards) of a copy of a context on device 1."""
-    out = (ctypes.c_int * 5)()
+    thread's device afterwards, waits for the stream) of a copy of a context on device 1."""
+    out = (ctypes.c_int * 6)()
     checks.host_copy(ctypes.c_void_p(host.ctypes.data), ctypes.c_void_p(dev.ctypes.data),
                      ctypes.c_int64(bytes_each), parts, int(to_host), pinned, device, out)
     return list(out)
@@ -87,4 +87,16 @@ def test_host_copies_leave_the_current_device(checks, size, to_host, device):
     host, dev = (dst, src) if to_host else (src, dst)
     out = _copy(checks, host, dev, size, 1, to_host, 4, device)
     assert out[:2] == [0, 0] and out[4] == device
+    np.testing.assert_array_equal(dst, src)
+
+
+@pytest.mark.parametrize("to_host", [False, True])
+def test_small_host_copies_wait_for_nothing(checks, to_host):
+    """A copy through the runtime leaves the wait for the stream to the caller: parcel fields taken one
+    after another wait once, not once a field."""
+    src = np.arange(15_360, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    host, dev = (dst, src) if to_host else (src, dst)
+    out = _copy(checks, host, dev, len(src), 1, to_host, 4)
+    assert out == [0, 0, 0, 1, 1, 0]
     np.testing.assert_array_equal(dst, src)
