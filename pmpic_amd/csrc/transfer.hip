@@ -31,10 +31,13 @@ constexpr int THREADS = HOST_THREADS;  // the caller's and three more, for the l
 // exports of 2.7 MB left the program's next allocation waiting 4 ms in the median (pass 18.4 ms, now
 // 11.9), and eight members' 59 ms a pass is 57.
 constexpr size_t LEAST_PINNED = CHUNK;
-// Nor does the runtime pin arrays this small, and a chunk of its own for each costs more than the
-// slots save (17 arrays of 64, 128, 256, 512 KB: 0.21, 0.26, 0.33, 0.53 ms through the runtime, 0.29,
-// 0.30, 0.34, 0.43 through slots).
-constexpr size_t LEAST_PART = CHUNK / 4;
+// Nor does the runtime pin arrays below a megabyte, and slots cost some 40 us at a call's start and a
+// chunk for each array: of arrays below LEAST_PART, or LEAST_SUM in all and LEAST_PART_OF_MANY, they
+// take longer (4 arrays of 64, 256, 512, 768 KB: 43, 75, 118, 159 us through the runtime, 88, 107,
+// 132, 157 through slots; 8 of 256, 512 KB 180, 266 and 183, 230; 17 of 128, 256, 512 KB 265, 355, 537
+// and 311, 354, 448).
+constexpr size_t LEAST_PART = 3 * CHUNK / 4;
+constexpr size_t LEAST_SUM = 4 * CHUNK, LEAST_PART_OF_MANY = CHUNK / 4;
 // The wait for the stream is the caller's, one for several copies, but above this it comes sooner: the
 // runtime's next copy waits longer by itself.  FP32-bulk get_parcels, whose fields are converted and
 // copied one after another, of 2,048 parcels 0.41 ms with a wait for each field and 0.30 with one, of
@@ -47,7 +50,8 @@ constexpr size_t LEAST_THREADS = (size_t)16 << 20;
 
 // the threads that carry a copy to the host through pinned slots, 0 for the runtime's own
 int slot_threads(size_t total, int nparts) {
-  if (total < LEAST_PINNED || total < nparts * LEAST_PART) return 0;
+  const size_t least = total < LEAST_SUM ? LEAST_PART : LEAST_PART_OF_MANY;
+  if (total < LEAST_PINNED || total < nparts * least) return 0;
   return total < LEAST_THREADS ? 1 : THREADS;
 }
 

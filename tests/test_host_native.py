@@ -63,11 +63,12 @@ def test_host_copies_without_pinned_memory(checks, bytes_each, parts, to_host, t
 @pytest.mark.parametrize("bytes_each,parts,to_host,threads",
                          [(MB - 1, 1, True, 0), (MB, 1, True, 1), (16 * MB - 1, 1, True, 1),
                           (16 * MB, 1, True, 4), (MB // 4 - 8, 17, True, 0), (MB // 4, 17, True, 1),
-                          (MB, 17, True, 4), (MB, 1, False, 0), (40 * MB, 1, False, 0),
+                          (MB // 2, 7, True, 0), (MB // 2, 8, True, 1), (3 * MB // 4 - 8, 2, True, 0),
+                          (3 * MB // 4, 2, True, 1), (MB, 17, True, 4), (MB, 1, False, 0), (40 * MB, 1, False, 0),
                           (2 * MB, 17, False, 0)])
 def test_host_copies_route(checks, bytes_each, parts, to_host, threads):
-    """Which copies go through pinned slots: to the host from 1 MB in parts of 256 KB or more, by four
-    threads from 16 MB; from the host, where the runtime is as fast or faster, none."""
+    """Which copies go through pinned slots: to the host from 1 MB in parts of 768 KB or more, from 4 MB
+    in parts of 256 KB or more, by four threads from 16 MB; from the host, where the runtime is as fast or faster, none."""
     src = np.arange(bytes_each * parts, dtype=np.uint8)
     dst = np.zeros_like(src)
     host, dev = (dst, src) if to_host else (src, dst)
