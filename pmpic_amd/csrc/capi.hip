@@ -136,10 +136,14 @@ int put_host(Ctx *c, double *dst, const double *host, int64_t n) {
   const HostPart p{const_cast<double *>(host), dst, sizeof(double) * (size_t)n};
   return copy_to_device(c, &p, 1);
 }
-int get_host(Ctx *c, double *host, const double *src, int64_t n) {
+// device array or pinned one (ref_out) -> host; waited: the stream has been waited for since src was
+// made, by the status check (8 us less where the array is pinned)
+int get_host(Ctx *c, double *host, const double *src, int64_t n, bool waited = false) {
   if (src == c->ref_pin) {
-    PMPIC_CHECK(hipEventRecord(c->sync_ev, c->stream));
-    PMPIC_CHECK(hipEventSynchronize(c->sync_ev));
+    if (!waited) {
+      PMPIC_CHECK(hipEventRecord(c->sync_ev, c->stream));
+      PMPIC_CHECK(hipEventSynchronize(c->sync_ev));
+    }
     memcpy(host, src, sizeof(double) * (size_t)n);
     return PMPIC_OK;
   }
@@ -812,7 +816,7 @@ int pmpic_par2grid(pmpic_ctx *ctx, const double *var, double *grid) {
   double *const ref = ref_out(c, ref_grid_size(c->g));
   PMPIC_TRY(grid_to_ref(c, c->kres[0], 1, ref));
   PMPIC_TRY(take_status(c));
-  return get_host(c, grid, ref, ref_grid_size(c->g));
+  return get_host(c, grid, ref, ref_grid_size(c->g), true);
 }
 
 int pmpic_grid2par(pmpic_ctx *ctx, const double *grid, double *var) {
@@ -918,7 +922,7 @@ static int spectral_unary(pmpic_ctx *ctx, const double *in, double *out, int whi
   double *const ref = ref_out(c, c->ssz);
   PMPIC_TRY(planes_to_ref(c, c->sder[1], ref));
   PMPIC_TRY(take_status(c));
-  return get_host(c, out, ref, c->ssz);
+  return get_host(c, out, ref, c->ssz, true);
 }
 
 int pmpic_diffx(pmpic_ctx *ctx, const double *in, double *out) { return spectral_unary(ctx, in, out, 0, nullptr, nullptr); }
@@ -937,7 +941,7 @@ int pmpic_laplinv(pmpic_ctx *ctx, double *f, int32_t df0) {
   double *const ref = ref_out(c, c->ssz);
   PMPIC_TRY(planes_to_ref(c, c->sder[0], ref));
   PMPIC_TRY(take_status(c));
-  return get_host(c, f, ref, c->ssz);
+  return get_host(c, f, ref, c->ssz, true);
 }
 
 int pmpic_conservation_sums(pmpic_ctx *ctx, double out6[6]) {
