@@ -1457,7 +1457,7 @@ static int put_field(Ctx *c, double *dev, const double *host, int64_t n) {
 }
 static int get_field(Ctx *c, double *host, double *dev, int64_t n) {
   const HostPart p{host, dev, sizeof(double) * (size_t)n};
-  return copy_to_host(c, &p, 1);
+  return copy_to_host(c, &p, 1, false);
 }
 
 int b32_set_parcels(Ctx *c, int64_t n, const double *const *fields) {

@@ -54,7 +54,8 @@ int ensure_fbuf(Ctx *c) {
   return PMPIC_OK;
 }
 
-// status raised by kernels since the last check; clears it
+// status raised by kernels since the last check; clears it.  What a failed stage left for the next
+// par2grid is not used.
 int take_status(Ctx *c) {
   int st = sync_scalars(c);
   if (st != PMPIC_OK) {
@@ -148,9 +149,7 @@ int get_host(Ctx *c, double *host, const double *src, int64_t n, bool waited = f
     return PMPIC_OK;
   }
   const HostPart p{host, const_cast<double *>(src), sizeof(double) * (size_t)n};
-  PMPIC_TRY(copy_to_host(c, &p, 1));
-  PMPIC_CHECK(hipStreamSynchronize(c->stream));
-  return PMPIC_OK;
+  return copy_to_host(c, &p, 1, true);
 }
 int64_t ref_grid_size(const Geometry &g) { return (int64_t)g.nzn * (g.ny + 4) * (g.nx + 4); }
 
@@ -499,9 +498,7 @@ int pmpic_get_parcels(pmpic_ctx *ctx, int64_t *n, double *const *fields) {
     for (int f = 0; f < 17; f++)
       if (fields[f])
         part[parts++] = {fields[f], c->par + (int64_t)f * c->cap, sizeof(double) * (size_t)c->n};
-  PMPIC_TRY(copy_to_host(c, part, parts));
-  PMPIC_CHECK(hipStreamSynchronize(c->stream));
-  return PMPIC_OK;
+  return copy_to_host(c, part, parts, true);
 }
 
 int pmpic_set_rk_arrays(pmpic_ctx *ctx, const double *const *fields) {

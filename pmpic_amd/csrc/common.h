@@ -421,14 +421,15 @@ int fft_backward(Ctx *c, int nf, const double *const *src, double *const *dst,
 // the same transforms with spectral arrays (and the transforms' arithmetic) of type S; the
 // forward transform reads physical grids of type S, the inverse writes dst (FP64) and dst32
 // (FP32), either of which may be NULL
-// Copies between the caller's arrays and the device, on the context's stream: complete once the caller
-// has waited for the stream.
+// Copies between the caller's arrays and the device, on the context's stream.  To the host: complete
+// on return, or without `wait` once the caller has waited for the stream.  From it: the caller's arrays
+// may change once the stream has been waited for.
 struct HostPart {
   void *host, *dev;
   size_t bytes;
 };
 int copy_to_device(Ctx *c, const HostPart *part, int nparts);
-int copy_to_host(Ctx *c, const HostPart *part, int nparts);
+int copy_to_host(Ctx *c, const HostPart *part, int nparts, bool wait);
 void free_host_slots(Ctx *c);
 template <typename S>
 int fft_forward_t(Ctx *c, int nf, const S *const *src, S *const *dst);

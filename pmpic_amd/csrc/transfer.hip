@@ -7,16 +7,17 @@
 // else the caller's alone) carry through pinned slots of their own, two each, the link moving one while
 // the thread copies the other.
 //
-// From the host the runtime's copy, 29 to 31 GB/s, stays.  One thread's slots were slower (17 arrays of
-// 0.06, 0.84, 1.07 MB: 0.18, 0.45, 0.67 ms through the runtime, 0.29, 0.57, 0.90 through slots; one
-// after another, arrays of 1.9, 6.9, 15 MB: 1.28, 4.4, 9.4 and 1.9, 5.3, 10.9), four threads' no better
-// than even: 17 arrays of 2.3, 6.3, 23 MB 1.31, 4.0, 13.8 against 1.57, 3.85, 12.9, but with seven of
-// them one array of zeros, as the fields that a caller leaves out are, 1.25, 3.5, 12.2 against 1.62,
-// 3.9, 12.9.
+// From the host it goes through the runtime's own staging, in pieces below the megabyte: 34 GB/s, where
+// the runtime's copy of a whole array, whose pages it pins, does 29 and leaves the stall behind.  17
+// arrays of 1.9, 6.9, 15, 38 MB: 1.03, 4.7, 10.0, 24.6 ms whole, 0.96, 3.5, 7.7, 19.4 in pieces of 1000
+// KB (1.13, 3.8, 8.0, 19.6 of 768 KB, 1.9, 6.6, 14.5, 35.6 of 256), 1.21, 4.0, 8.9, 21.7 through slots by
+// four threads; FP32-bulk arrays, one after another, of 1.9, 6.9, 15 MB 1.2, 4.7, 10.0 whole, 1.15, 3.7,
+// 7.8 in pieces, 1.8, 5.5, 11.9 through one thread's slots.
 #include "common.h"
 
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <system_error>
 #include <thread>
@@ -38,8 +39,8 @@ constexpr size_t LEAST_PINNED = CHUNK;
 // and 311, 354, 448).
 constexpr size_t LEAST_PART = 3 * CHUNK / 4;
 constexpr size_t LEAST_SUM = 4 * CHUNK, LEAST_PART_OF_MANY = CHUNK / 4;
-// The wait for the stream is the caller's, one for several copies, but above this it comes sooner: the
-// runtime's next copy waits longer by itself.  FP32-bulk get_parcels, whose fields are converted and
+// A caller of several copies may wait for the stream once for all of them, but above this the wait comes
+// with each: the runtime's next copy waits longer by itself.  FP32-bulk get_parcels, whose fields are converted and
 // copied one after another, of 2,048 parcels 0.41 ms with a wait for each field and 0.30 with one, of
 // 2,049 0.37 and 0.41, of 20,000 0.47 and 0.50.
 constexpr size_t LEAST_WAITED = (size_t)16 << 10;
@@ -47,6 +48,8 @@ constexpr size_t LEAST_WAITED = (size_t)16 << 10;
 // for the address space cost more than they save (a dump of ten grids of 5.4 MB: 4.7 ms through the
 // runtime, 4.3 with one thread, 4.2 at best and 10 in the median with four).
 constexpr size_t LEAST_THREADS = (size_t)16 << 20;
+
+constexpr size_t UPLOAD_PIECE = (size_t)1000 << 10;
 
 // the threads that carry a copy to the host through pinned slots, 0 for the runtime's own
 int slot_threads(size_t total, int nparts) {
@@ -148,13 +151,15 @@ struct OnDevice {
 
 int copy_to_device(Ctx *c, const HostPart *part, int nparts) {
   for (int k = 0; k < nparts; k++)
-    if (part[k].bytes)
-      PMPIC_CHECK(hipMemcpyAsync(part[k].dev, part[k].host, part[k].bytes, hipMemcpyHostToDevice,
+    for (size_t at = 0; at < part[k].bytes; at += UPLOAD_PIECE)
+      PMPIC_CHECK(hipMemcpyAsync(static_cast<char *>(part[k].dev) + at,
+                                 static_cast<const char *>(part[k].host) + at,
+                                 std::min(UPLOAD_PIECE, part[k].bytes - at), hipMemcpyHostToDevice,
                                  c->stream));
   return PMPIC_OK;
 }
 
-int copy_to_host(Ctx *c, const HostPart *part, int nparts) {
+int copy_to_host(Ctx *c, const HostPart *part, int nparts, bool wait) {
   size_t total = 0;
   Copy job{c, part, nparts, 0};
   for (int k = 0; k < nparts; k++) {
@@ -169,7 +174,7 @@ int copy_to_host(Ctx *c, const HostPart *part, int nparts) {
       if (part[k].bytes)
         PMPIC_CHECK(hipMemcpyAsync(part[k].host, part[k].dev, part[k].bytes, hipMemcpyDeviceToHost,
                                    c->stream));
-    if (total > LEAST_WAITED) PMPIC_CHECK(hipStreamSynchronize(c->stream));
+    if (wait || total > LEAST_WAITED) PMPIC_CHECK(hipStreamSynchronize(c->stream));
     return PMPIC_OK;
   }
   std::thread th[THREADS - 1];

@@ -10,6 +10,7 @@
 namespace fake {
 thread_local hipError_t pending = hipSuccess;  // what hipGetLastError reports
 std::atomic<int> pinned_left{0}, pinned_taken{0}, copies{0}, waits{0};
+std::atomic<size_t> largest{0};  // copy command
 // each thread's current device; an event belongs to the one it was created on, the stream to device 1
 thread_local int device = 0;
 constexpr int STREAM_DEVICE = 1;
@@ -27,6 +28,7 @@ hipError_t host_free(void *p) {
 }
 hipError_t memcpy_async(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t) {
   copies++;
+  if (n > largest) largest = n;
   memcpy(to, from, n);
   return hipSuccess;
 }
@@ -84,9 +86,9 @@ void host_run_round_trip(int32_t cell, int32_t head, int32_t out[2]) {
 // `parts` copies of n bytes each, one after another in `host` and `dev`, with pinned memory for
 // `pinned` threads' slots, by a thread whose current device is `device`.  out: the status, the error
 // left pending, the blocks of pinned memory taken, the copy commands issued, the thread's device
-// afterwards and the waits for the stream
+// afterwards, the waits for the stream and the largest copy's bytes
 void host_copy(char *host, char *dev, int64_t n, int parts, int to_host, int pinned, int device,
-               int out[6]) {
+               int out[7]) {
   Ctx *c = new Ctx();
   c->device = fake::STREAM_DEVICE;
   fake::device = device;
@@ -94,12 +96,14 @@ void host_copy(char *host, char *dev, int64_t n, int parts, int to_host, int pin
   for (int i = 0; i < parts; i++) part[i] = {host + i * n, dev + i * n, (size_t)n};
   fake::pinned_left = pinned;
   fake::pinned_taken = fake::copies = fake::waits = 0;
-  out[0] = to_host ? copy_to_host(c, part, parts) : copy_to_device(c, part, parts);
+  fake::largest = 0;
+  out[0] = to_host ? copy_to_host(c, part, parts, false) : copy_to_device(c, part, parts);
   out[1] = (int)fake::last_error();
   out[2] = fake::pinned_taken;
   out[3] = fake::copies;
   out[4] = fake::device;
   out[5] = fake::waits;
+  out[6] = (int)fake::largest;
   free_host_slots(c);
   delete c;
 }

@@ -35,8 +35,9 @@ MB = 1 << 20
 
 def _copy(checks, host, dev, bytes_each, parts, to_host, pinned, device=1):
     """(status, error left pending, blocks of pinned memory taken, copy commands, the calling
-    thread's device afterwards, waits for the stream) of a copy of a context on device 1."""
-    out = (ctypes.c_int * 6)()
+    thread's device afterwards, waits for the stream, bytes of the largest command) of a copy of a
+    context on device 1."""
+    out = (ctypes.c_int * 7)()
     checks.host_copy(ctypes.c_void_p(host.ctypes.data), ctypes.c_void_p(dev.ctypes.data),
                      ctypes.c_int64(bytes_each), parts, int(to_host), pinned, device, out)
     return list(out)
@@ -99,5 +100,15 @@ def test_small_host_copies_wait_for_nothing(checks, to_host):
     dst = np.zeros_like(src)
     host, dev = (dst, src) if to_host else (src, dst)
     out = _copy(checks, host, dev, len(src), 1, to_host, 4)
-    assert out == [0, 0, 0, 1, 1, 0]
+    assert out == [0, 0, 0, 1, 1, 0, len(src)]
+    np.testing.assert_array_equal(dst, src)
+
+
+@pytest.mark.parametrize("size", [1, MB - 1, MB, MB + 1, 3_072_000, 3_072_001, 20 * MB])
+def test_uploads_come_in_pieces(checks, size):
+    """Uploads stay below the megabyte from which the runtime pins the caller's pages."""
+    src = np.random.default_rng(size).integers(0, 256, size, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    out = _copy(checks, src, dst, size, 1, False, 4)
+    assert out[:3] == [0, 0, 0] and out[3] == -(-size // 1_024_000) and out[6] < MB
     np.testing.assert_array_equal(dst, src)
