@@ -794,9 +794,10 @@ struct RkSets {
   float *off_to, *vor_to;
 };
 
-// The RK stage of parcel p; returns its new cell.  One that would leave the box stays where it is
-// (status raised), in the set that the stage writes too.  The sets of a stage may be the same arrays:
-// a thread reads its parcel before it writes it.
+// The RK stage of parcel p; returns its new cell, or -1 where it would leave the box (status raised).
+// It then stays where it is, in the set that the stage writes too, but is not in the lists that the
+// stage builds: b32_forget drops those.  The sets of a stage may be the same arrays: a thread reads its
+// parcel before it writes it.
 template <int STAGE>
 __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b, const RkSets &rs,
                                              const float4 *__restrict__ rec,
@@ -874,12 +875,12 @@ __device__ __forceinline__ int32_t rk_update(const Geometry &g, const Bulk32 &b,
   if (!place(g, io, jo, ko, tpos[0], tpos[1], tpos[2], ncell_, nox, noy, noz)) {
     raise_status(sc, PMPIC_ERR_OUT_OF_BOX_Z);
     if (STAGE == 1 || STAGE == 4) {
-      const Float3 v = ld3(rs.vor, p);
-      stnt(rs.cell_to, p, cell);
-      st3(rs.off_to, p, ox, oy, oz);
+      const Float3 at = ld3(rs.off, p), v = ld3(rs.vor, p);
+      stnt(rs.cell_to, p, ldnt(rs.cell, p));
+      st3(rs.off_to, p, at.x, at.y, at.z);
       st3(rs.vor_to, p, v.x, v.y, v.z);
     }
-    return cell;
+    return -1;
   }
   stnt(rs.cell_to, p, ncell_);
   st3(rs.off_to, p, nox, noy, noz);
@@ -924,7 +925,7 @@ __global__ void __launch_bounds__(TPB) k32_rk_stage(Geometry g, Bulk32 b, RkSets
   const int32_t was = STAGE == 2 && bo.on ? rs.cell[p] : -1;  // (the stage updates it in place)
   const int32_t nc = rk_update<STAGE>(g, b, rs, rec, sc3, stretch, split_flag, sc, p);
   // with bo.on = 2, the entries of the parcels that change cell move
-  if (STAGE == 2 && bo.on && nc != was) {
+  if (STAGE == 2 && bo.on && nc >= 0 && nc != was) {
     remove_entry((int32_t)p, linear_cell(g, was), bo.capc, bo, sc);
     append_entry((int32_t)p, linear_cell(g, nc), bo, sc);
   }
@@ -1460,11 +1461,15 @@ static int get_field(Ctx *c, double *host, double *dev, int64_t n) {
   return copy_to_host(c, &p, 1, false);
 }
 
+void b32_forget(Ctx *c) {
+  unbin(c);
+  c->b32.p2g_reuse = false;
+}
+
 int b32_set_parcels(Ctx *c, int64_t n, const double *const *fields) {
   PMPIC_TRY(ensure_fbuf(c));
   Bulk32 &b = c->b32;
-  unbin(c);
-  b.p2g_reuse = false;
+  b32_forget(c);
   const dim3 gb(cdiv(n > 0 ? n : 1, TPB)), tb(TPB);
   for (int a = 0; a < 3; a++) {
     if (n > 0) {

@@ -59,6 +59,7 @@ int ensure_fbuf(Ctx *c) {
 int take_status(Ctx *c) {
   int st = sync_scalars(c);
   if (st != PMPIC_OK) {
+    if (c->precision == 1) b32_forget(c);
     int zero = 0;
     hipMemcpy(&c->dsc->status, &zero, sizeof(int), hipMemcpyHostToDevice);
   }

@@ -497,6 +497,7 @@ int mix_lists(Ctx *c, const T *vol, int stride, T vmin, int64_t n, int32_t *cell
 // bulk32.hip (FP32-bulk form)
 int b32_alloc(Ctx *c);
 void b32_free(Ctx *c);
+void b32_forget(Ctx *c);  // the lists and sums kept for the next par2grid
 int b32_set_parcels(Ctx *c, int64_t n, const double *const *fields);
 int b32_get_parcels(Ctx *c, double *const *fields);
 int b32_par2grid(Ctx *c);                 // P, Q, R, B grids (FP64) from the FP32 parcels
