@@ -17,7 +17,6 @@
 
 #include <string.h>
 
-#include <algorithm>
 #include <atomic>
 #include <system_error>
 #include <thread>
@@ -49,7 +48,8 @@ constexpr size_t LEAST_WAITED = (size_t)16 << 10;
 // runtime, 4.3 with one thread, 4.2 at best and 10 in the median with four).
 constexpr size_t LEAST_THREADS = (size_t)16 << 20;
 
-constexpr size_t UPLOAD_PIECE = (size_t)1000 << 10;
+// an upload's pieces, and the size that the runtime pins from (a piece of exactly that is pinned)
+constexpr size_t UPLOAD_PIECE = (size_t)1000 << 10, PINNED_FROM = (size_t)1 << 20;
 
 // the threads that carry a copy to the host through pinned slots, 0 for the runtime's own
 int slot_threads(size_t total, int nparts) {
@@ -151,11 +151,13 @@ struct OnDevice {
 
 int copy_to_device(Ctx *c, const HostPart *part, int nparts) {
   for (int k = 0; k < nparts; k++)
-    for (size_t at = 0; at < part[k].bytes; at += UPLOAD_PIECE)
+    for (size_t at = 0, n; at < part[k].bytes; at += n) {
+      n = part[k].bytes - at;
+      if (n >= PINNED_FROM) n = UPLOAD_PIECE;
       PMPIC_CHECK(hipMemcpyAsync(static_cast<char *>(part[k].dev) + at,
-                                 static_cast<const char *>(part[k].host) + at,
-                                 std::min(UPLOAD_PIECE, part[k].bytes - at), hipMemcpyHostToDevice,
-                                 c->stream));
+                                 static_cast<const char *>(part[k].host) + at, n,
+                                 hipMemcpyHostToDevice, c->stream));
+    }
   return PMPIC_OK;
 }
 
