@@ -175,9 +175,9 @@ int pmpic_graph_stats(pmpic_ctx *ctx, int64_t *captures, int64_t *launches);
 /* Launch-configuration autotuning of an FP32-bulk context (no reference counterpart; for the
  * batched ensemble, whose members differ in grid size).  A configuration is four numbers:
  * config[0] the binning's slot capacity (16 or 32; 0 where the grid has no slot table),
- * config[1] the binning fused into RK stages 1-3 (1) or a pass of its own (0), config[2] RK
- * stages 1-3 launched as one HIP graph (1, only with timing off) or eagerly (0), config[3] the
- * RK stage's workgroup size (128 or 256).  Every configuration gives the same bits.  The first
+ * config[1] the binning fused into RK stages 1 and 3, and 2 where no list entries can move (1),
+ * or a pass of its own (0), config[2] RK stages 1-3 launched as one HIP graph (1, only with
+ * timing off) or eagerly (0), config[3] the RK stage's workgroup size (128 or 256).  Every configuration gives the same bits.  The first
  * context of a grid size (nx, ny, nz) and occupancy class (the slot capacity the mean rule
  * picks) runs each configuration twice (the list forward, then backward, so that a drift of
  * the step time with the model state cancels) for one settling step and `steps` timed steps,

@@ -1518,9 +1518,9 @@ int b32_get_parcels(Ctx *c, double *const *fields) {
   return PMPIC_OK;
 }
 
-// The last mixing's kept sums stand for the next par2grid on x rows of whole 16-cell pieces only:
-// elsewhere every par2grid sums every tile, one full launch a stage, which is what its timer's
-// count has always been there.
+// The last mixing's kept sums stand for the next par2grid on x rows of whole 16-cell pieces.  The
+// tiles and their flags would serve every length; elsewhere every par2grid sums every tile, one full
+// launch a stage, as the accumulation's timer counts them there.
 static bool reuse_sums(const Ctx *c) { return c->g.nx % 16 == 0 && !c->b32.reuse_off; }
 
 // A graph of stages 1-3 always captures stage 1's par2grid reading the dirty-tile flags (with the

@@ -391,8 +391,8 @@ inline int stage_of(int it) { return (it % 4) + 1; }
 
 // ---- launch-configuration autotuning (FP32-bulk form) ----
 // A configuration: the binning's slot capacity (16 or 32; 0 without a slot table), the binning
-// fused into RK stages 1-3 or run as a pass of its own, RK stages 1-3 as a graph or eagerly,
-// and the RK stage's workgroup size.  Every configuration gives the same bits, so the tuning
+// fused into RK stages 1 and 3 (and 2 where no list entries can move) or run as a pass of its own, RK
+// stages 1-3 as a graph or eagerly, and the RK stage's workgroup size.  Every configuration gives the same bits, so the tuning
 // steps are ordinary steps of the model.  The choice is kept per grid size and occupancy class
 // for the life of the process, so later contexts of that size take it without measuring.
 namespace {
@@ -543,7 +543,7 @@ int pmpic_set_time(pmpic_ctx *ctx, double time, double dtm) {
 
 // vort2vel: par2grid of p, q, r (and, fused into the same pass, the total buoyancy that
 // vorticity_tendency grids from the same cached weights), the spectral solve and the derivative
-// grids vorticity_tendency multiplies; its stage 1 takes the grid maxima for the timestep limits
+// grids that vorticity_tendency multiplies
 int pmpic_vort2vel(pmpic_ctx *ctx) {
   if (!ctx) return PMPIC_ERR_ARG;
   Ctx *c = &ctx->c;

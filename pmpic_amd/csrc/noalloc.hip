@@ -5,8 +5,7 @@
 // working memory (cell and rank of each parcel, the per-cell counts and offsets, the cell-sorted
 // parcel list, the corner partial sums and the interior grid) is carved out of `scratch`, one
 // static device array per GPU that lives until the process ends, instead of the context's buffers
-// or hipMalloc.  Inputs and the
-// output are the caller's device arrays.
+// or hipMalloc.  Inputs and the output are the caller's device arrays.
 //
 // Every call on a GPU shares that GPU's array, so calls that overlap (two host threads) take turns:
 // a call holds the GPU's lock until the device has finished, as it waits for its status anyway.  The

@@ -670,7 +670,7 @@ __global__ void k_mix_absorb(Geometry g, double *__restrict__ par, int64_t cap, 
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= norig || keep[p] != 1) return;
   const int32_t c = cell[p];
-  if (c >= 0 && !ctouch[c]) return;
+  if (c < 0 || !ctouch[c]) return;  // (a parcel without a cell has ended the mixing before this)
   // all loads first (parcel values, then the gathers), all stores last
   const int fld[5] = {FB, FH, FP, FQ, FR};
   const double x = ld_stream(&par[FX * cap + p]), y = ld_stream(&par[FY * cap + p]),

@@ -421,10 +421,7 @@ __global__ void __launch_bounds__(64) k_diffz_reg(Geometry g, ColField cf,
                                                   const double *__restrict__ tcp,
                                                   DevScalars *sc) {
   // the Thomas tables are the same for every column: staged once per block in LDS, so the
-  // recurrence reads them without a memory round trip per level.  The FP32-bulk form (S float)
-  // stages the pivots' reciprocals and multiplies by them, takes 1/dz and 1/(2 dz) as factors
-  // and holds the column in FP32 between the sweeps (the sweeps themselves run in FP64); the
-  // FP64 form divides as the reference does
+  // recurrence reads them without a memory round trip per level
   __shared__ double den[NZ], cpt[NZ];
   const int64_t plane = (int64_t)g.sy * g.sx;
   const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -443,7 +440,7 @@ __global__ void __launch_bounds__(64) k_diffz_reg(Geometry g, ColField cf,
   for (int k = 0; k < NZ; k++) F[k] = fin[(int64_t)k * plane];
   const double bot = bt ? cf.bot[col] : 0.0, top = bt ? cf.top[col] : 0.0;
   const double a1 = (double)(1.f / 6.f), al = (double)(1.f / 3.f);
-  const double dz = g.dz, idz = 1.0 / dz, ih2dz = 0.5 / dz;
+  const double dz = g.dz;
   double fkm2 = F[0], fkm1 = F[1];  // originals f(k-2), f(k-1) of the next row
   const double d0 = bt ? (fkm1 / dz) - a1 * bot * dz : 0.0;
   double fprev = d0 / den[0];
@@ -613,7 +610,7 @@ __global__ void __launch_bounds__(64) k_diffz_qn(Geometry g, ColField cf,
   for (int i = 0; i < L; i++) F[i] = (q * L + i < NZ) ? fin[(int64_t)(q * L + i) * plane] : 0.0;
   const double bot = bt ? cf.bot[col] : 0.0, top = bt ? cf.top[col] : 0.0;
   const double a1 = (double)(1.f / 6.f), al = (double)(1.f / 3.f);
-  const double dz = g.dz, idz = 1.0 / dz, ih2dz = 0.5 / dz;
+  const double dz = g.dz;
   const double nxt0 = __shfl(F[0], lane + CPW);  // the original of the next group's first level
   const int PTOP = (NZ - 1) / L;
   double fprev = 0.0, fkm2 = 0.0, fkm1 = 0.0;  // originals f(k-2), f(k-1) of the next row
@@ -880,7 +877,6 @@ int spectral_setup(Ctx *c) {
         c->mcut = m + 1;
       }
   PMPIC_CHECK(hipMemcpy(c->lcut, lcut.data(), sizeof(int) * lcut.size(), hipMemcpyHostToDevice));
-  const int64_t plane = (int64_t)sx * sy;
   hipLaunchKernelGGL(k_dz_tables, dim3(1), dim3(1), 0, c->stream, g, c->dz_den, c->dz_cp);
   PMPIC_CHECK(hipGetLastError());
   PMPIC_CHECK(hipStreamSynchronize(c->stream));
