@@ -237,7 +237,7 @@ def time_form(precision, ic, args, n, nz):
             table[s_] += RK32_BIN_BYTES
     rks = {
         "kernel": ("k32_rk_stage (FP32 grid2par of 6 fields + RK4 stage update"
-                   + (", cell binning in stages 1-3)" if fused else ")") if precision else
+                   + (", cell binning in stages 1 and 3)" if fused else ")") if precision else
                    "k_rk_stage (grid2par of 6 fields + RK4 stage update)"),
         "family": "k32_rk_stage" if precision else "k_rk_stage",
         "bytes": avg_np * sum(table.values()) / 4 + nnode * GATHER_NODE_BYTES[precision],

@@ -392,8 +392,8 @@ inline int stage_of(int it) { return (it % 4) + 1; }
 // ---- launch-configuration autotuning (FP32-bulk form) ----
 // A configuration: the binning's slot capacity (16 or 32; 0 without a slot table), the binning
 // fused into RK stages 1 and 3 (and 2 where no list entries can move) or run as a pass of its own, RK
-// stages 1-3 as a graph or eagerly, and the RK stage's workgroup size.  Every configuration gives the same bits, so the tuning
-// steps are ordinary steps of the model.  The choice is kept per grid size and occupancy class
+// stages 1-3 as a graph or eagerly, and the RK stage's workgroup size.  Every configuration gives the
+// same bits, so the tuning steps are ordinary steps of the model.  The choice is kept per grid size and occupancy class
 // for the life of the process, so later contexts of that size take it without measuring.
 namespace {
 struct TuneEntry {

@@ -23,7 +23,8 @@
 // The pivots depend on the column's k^2 only: they are tabled once per context, four columns
 // sharing an entry, and no pass divides.  The FP64 form gets its quotients from the tabled
 // reciprocal with one residual correction (div_by), which rounds as the division does for finite
-// values; the FP32-bulk form multiplies by the FP64 reciprocal.  All arithmetic is FP64 in both forms; the arrays between the passes are of the spectral type S.
+// values; the FP32-bulk form multiplies by the FP64 reciprocal.  All arithmetic is FP64 in both forms;
+// the arrays between the passes are of the spectral type S.
 //
 // Bound by memory on large grids (26 passes over a spectral array where the separate kernels took
 // 41) and by the instruction latency of one wavefront on small ones.  A call, against the sum of

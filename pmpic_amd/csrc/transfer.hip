@@ -39,16 +39,17 @@ constexpr size_t LEAST_PINNED = CHUNK;
 constexpr size_t LEAST_PART = 3 * CHUNK / 4;
 constexpr size_t LEAST_SUM = 4 * CHUNK, LEAST_PART_OF_MANY = CHUNK / 4;
 // A caller of several copies may wait for the stream once for all of them, but above this the wait comes
-// with each: the runtime's next copy waits longer by itself.  FP32-bulk get_parcels, whose fields are converted and
-// copied one after another, of 2,048 parcels 0.41 ms with a wait for each field and 0.30 with one, of
-// 2,049 0.37 and 0.41, of 20,000 0.47 and 0.50.
+// with each: the runtime's next copy waits longer by itself.  FP32-bulk get_parcels, whose fields are
+// converted and copied one after another, of 2,048 parcels 0.41 ms with a wait for each field and 0.30
+// with one, of 2,049 0.37 and 0.41, of 20,000 0.47 and 0.50.
 constexpr size_t LEAST_WAITED = (size_t)16 << 10;
 // Below this one thread: the others' start and, where the caller's pages are new, their contention
 // for the address space cost more than they save (a dump of ten grids of 5.4 MB: 4.7 ms through the
 // runtime, 4.3 with one thread, 4.2 at best and 10 in the median with four).
 constexpr size_t LEAST_THREADS = (size_t)16 << 20;
 
-// an upload's pieces, and the size that the runtime pins from (a piece of exactly that is pinned)
+// an upload's pieces, and the size that the runtime pins from (pieces of exactly that took as long as
+// whole arrays: 17 of 15 MB 10.1 ms, of 1000 KB 7.6)
 constexpr size_t UPLOAD_PIECE = (size_t)1000 << 10, PINNED_FROM = (size_t)1 << 20;
 
 // the threads that carry a copy to the host through pinned slots, 0 for the runtime's own
