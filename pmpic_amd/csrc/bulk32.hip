@@ -1369,7 +1369,11 @@ int b32_alloc(Ctx *c) {
   // count reads 0 for them, as in the FP64 form's arrays, which are cleared at allocation too
   PMPIC_CHECK(hipMemset(b.pool, 0, sizeof(float) * PARCEL32_WORDS * (size_t)c->cap));
   PMPIC_CHECK(hipMemset(b.tag, 0, sizeof(double) * (size_t)c->cap));
-  for (int i = 0; i < 3; i++) PMPIC_TRY(dalloc32(&b.grid[i], c->gsz));
+  // (zero until the first vort2vel, as the FP64 form's grids are)
+  for (int i = 0; i < 3; i++) {
+    PMPIC_TRY(dalloc32(&b.grid[i], c->gsz));
+    PMPIC_CHECK(hipMemset(b.grid[i], 0, sizeof(float) * (size_t)c->gsz));
+  }
   for (int i = 0; i < 12; i++) PMPIC_TRY(dalloc32(&b.mgrid[i], c->gsz));
   PMPIC_TRY(dalloc32(&b.newcells, c->ncell));
   PMPIC_TRY(dalloc32(&b.dirty, (int64_t)tiles_x(c->g) * c->g.ny * c->g.ncz));
@@ -1380,6 +1384,7 @@ int b32_alloc(Ctx *c) {
   b.reuse_off = renv && renv[0] == '0';
   for (int i = 0; i < 4; i++) {
     PMPIC_TRY(dalloc32(&b.pgrid[i], c->gsz));
+    PMPIC_CHECK(hipMemset(b.pgrid[i], 0, sizeof(float) * (size_t)c->gsz));
     b.p2g_pending[i] = false;
   }
   // 32-bit byte offsets into the slot table.  PMPIC_SLOT_CAPACITY in the environment: 0 drops

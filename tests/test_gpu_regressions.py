@@ -345,3 +345,26 @@ def test_absorption_against_fp64(nz):
     assert np.abs(vol32 / vol64 - 1).max() < 5e-6
     change = np.abs(vol64 / ic["vol"].max() - 1)
     assert change[change < 0.05].max() > 1e-4  # something was absorbed
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_grids_of_a_new_context_are_zero(precision):
+    """Grids exported, and tendencies taken, before the first vort2vel: zero, not what the memory held
+    for a context before (whose grids are far from it)."""
+    from pmpic_amd.lib import GRID_IDS, Context
+    shape = (32, 24, 16)
+    b = box(*shape)
+    ic = thermal_case(*shape, 2, vort=3.0)
+    for fresh in (False, True):
+        g = Context(*shape, b["xmin"], b["xmax"], b["ymin"], b["ymax"], b["zmin"], b["zmax"],
+                    2 * len(ic["x"]), precision=precision)
+        if not fresh:
+            g.set_parcels(ic)
+            g.step()
+        else:
+            for _ in range(2):
+                for k in GRID_IDS:
+                    assert not g.grid(k).any(), k
+                g.vorticity_tendency()
+            assert g.dtm == 0.01
+        g.close()
